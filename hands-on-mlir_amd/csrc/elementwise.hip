@@ -8,6 +8,7 @@
 //   cu_seqlens   include/NVGPUKernels/CuSeqLen.h:28-74
 //   row stats    include/NVGPUKernels/Layernorm.h:33-195 (ApplyFinalReduction)
 #include "cross_lane.h"
+#include "fast_div.h"
 #include "kernels.h"
 #include "store_policy.h"
 
@@ -45,46 +46,115 @@ template <typename T> __device__ __forceinline__ T applyOp(int op, T a, T b) {
   }
 }
 
-// Out = A op B with B either the same shape (inner == total) or repeating
-// every `inner` elements (broadcast over leading dimensions).  One 16-byte
-// vector per thread per step.
-template <typename T, int OP>
-__global__ __launch_bounds__(256) void elementwiseVecKernel(
-    const T *a, const T *b, T *out, int64_t nvec, int64_t innerVec) {
+// Tensors up to this size are written through (the next kernel of the stream
+// finds them in the last-level cache and nothing dirty is left to write back
+// in between); larger ones stream with the non-temporal hint.
+constexpr int64_t kStreamingBytes = int64_t(16) << 20;
+
+template <typename V, bool STREAM>
+__device__ __forceinline__ void storeResult(V *p, const V &v) {
+  if (STREAM)
+    __builtin_nontemporal_store(v, p);
+  else
+    storeWriteThrough(p, v);
+}
+
+// How B is laid over A's elements once neighbouring dimensions that behave the
+// same are merged: rows of `inner` elements of A, and row r of A meets row
+//   (r / rowDiv) % rowMod
+// of B, which is `inner` contiguous values (kRowOfB) or one value (!kRowOfB).
+//   same shape         one row                     rowDiv 1, rowMod 1
+//   [1, .., 1, n]      the same row every time     rowDiv 1, rowMod 1
+//   [b, 1, n]          one row per rowDiv rows     rowDiv s, rowMod b
+//   [b, s, 1]          one value per row           rowDiv 1, rowMod b*s
+//   [1, s, 1]          values repeat every s rows  rowDiv 1, rowMod s
+struct RowBroadcast {
+  uint32_t inner, rowDiv, rowMod;
+  uint32_t innerMagic, divMagic, modMagic; // see fast_div.h
+  bool rowOfB;
+};
+
+// One 16-byte vector of the output per thread: every access of the launch is
+// in flight at once and nothing is recomputed, so the kernel runs at the
+// memory system's rate (16 x 200 x 768 fp32 times a [16, 200, 1] mask: 13.0 us
+// with the generic index walk below, which pays a 64-bit division per
+// dimension and element, 4.2 us this way).  Rows need not be whole vectors: a
+// vector that crosses a row end (WHOLE false: inner not a multiple of the
+// vector width) looks up B per element.
+template <typename T, int OP, bool ROW_OF_B, bool WHOLE, bool STREAM>
+__global__ __launch_bounds__(256) void elementwiseRowKernel(
+    const T *a, const T *b, T *out, uint32_t total, RowBroadcast m) {
   using V = typename Vec16<T>::type;
   constexpr int N = Vec16<T>::kN;
-  const int64_t step = int64_t(gridDim.x) * blockDim.x;
-  for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < nvec;
-       i += step) {
-    const V va = reinterpret_cast<const V *>(a)[i];
-    const V vb = reinterpret_cast<const V *>(b)[i % innerVec];
+  const uint32_t v = blockIdx.x * 256u + threadIdx.x;
+  const uint32_t e0 = v * N;
+  if (e0 >= total)
+    return;
+  uint32_t r = divByMagic(e0, m.inner, m.innerMagic);
+  uint32_t c = e0 - r * m.inner;
+  auto rowOf = [&](uint32_t row) {
+    const uint32_t q = divByMagic(row, m.rowDiv, m.divMagic);
+    return q - divByMagic(q, m.rowMod, m.modMagic) * m.rowMod;
+  };
+  if (WHOLE || e0 + N <= total) {
+    const V *pa = reinterpret_cast<const V *>(a) + v;
+    const V va = STREAM ? __builtin_nontemporal_load(pa) : *pa;
+    V vb, vo;
+    if (WHOLE && ROW_OF_B) {
+      vb = *reinterpret_cast<const V *>(b + size_t(rowOf(r)) * m.inner + c);
+    } else if (WHOLE) {
+      const T x = b[rowOf(r)];
+#pragma unroll
+      for (int j = 0; j < N; j++)
+        vb[j] = x;
+    } else {
+      uint32_t rb = rowOf(r);
+#pragma unroll
+      for (int j = 0; j < N; j++) {
+        vb[j] = b[ROW_OF_B ? size_t(rb) * m.inner + c : size_t(rb)];
+        if (++c == m.inner) {
+          c = 0;
+          rb = rowOf(++r);
+        }
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < N; j++)
+      vo[j] = applyOp<T>(OP, va[j], vb[j]);
+    storeResult<V, STREAM>(reinterpret_cast<V *>(out) + v, vo);
+  } else { // the last elements of a total that is not a multiple of the width
+    for (uint32_t e = e0; e < total; e++) {
+      const uint32_t rb = rowOf(r);
+      out[e] = applyOp<T>(OP, a[e], b[ROW_OF_B ? size_t(rb) * m.inner + c : size_t(rb)]);
+      if (++c == m.inner) {
+        c = 0;
+        r++;
+      }
+    }
+  }
+}
+
+// Same-shape operands: no index arithmetic at all.
+template <typename T, int OP, bool STREAM>
+__global__ __launch_bounds__(256) void elementwiseSameKernel(
+    const T *a, const T *b, T *out, int64_t total) {
+  using V = typename Vec16<T>::type;
+  constexpr int N = Vec16<T>::kN;
+  const int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
+  if (i * N + N <= total) {
+    const V *pa = reinterpret_cast<const V *>(a) + i;
+    const V *pb = reinterpret_cast<const V *>(b) + i;
+    const V va = STREAM ? __builtin_nontemporal_load(pa) : *pa;
+    const V vb = STREAM ? __builtin_nontemporal_load(pb) : *pb;
     V vo;
 #pragma unroll
     for (int j = 0; j < N; j++)
       vo[j] = applyOp<T>(OP, va[j], vb[j]);
-    reinterpret_cast<V *>(out)[i] = vo;
+    storeResult<V, STREAM>(reinterpret_cast<V *>(out) + i, vo);
+  } else {
+    for (int64_t e = i * N; e < total; e++)
+      out[e] = applyOp<T>(OP, a[e], b[e]);
   }
-}
-
-// Same-shape operands beyond the last-level cache: one vector per thread, every
-// access with the non-temporal hint (nothing is touched twice; measured cold on
-// 16384 x 1024 fp16 triples rotating over 800 MB: 5.2 TB/s with default
-// accesses and a grid-stride loop, 5.9 TB/s this way).
-template <typename T, int OP>
-__global__ __launch_bounds__(256) void elementwiseStreamKernel(
-    const T *a, const T *b, T *out, int64_t nvec) {
-  using V = typename Vec16<T>::type;
-  constexpr int N = Vec16<T>::kN;
-  const int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
-  if (i >= nvec)
-    return;
-  const V va = __builtin_nontemporal_load(reinterpret_cast<const V *>(a) + i);
-  const V vb = __builtin_nontemporal_load(reinterpret_cast<const V *>(b) + i);
-  V vo;
-#pragma unroll
-  for (int j = 0; j < N; j++)
-    vo[j] = applyOp<T>(OP, va[j], vb[j]);
-  __builtin_nontemporal_store(vo, reinterpret_cast<V *>(out) + i);
 }
 
 // Any broadcast pattern, scalar accesses.  The index walk is the reference's:
@@ -105,74 +175,141 @@ __global__ __launch_bounds__(256) void elementwiseGenericKernel(
   }
 }
 
-// Operands larger than this are not expected to be found in the last-level
-// cache by whoever reads the result next.
-constexpr int64_t kStreamingBytes = int64_t(16) << 20;
+// Merges dimensions and recognises the row forms above; false: a contiguous B
+// of another pattern, or a strided B, which take the generic walk.
+bool rowBroadcast(const BroadcastDesc &d, int64_t total, RowBroadcast *m) {
+  // groups of neighbouring dimensions, innermost first: extent, and whether B
+  // is full there (B must be dense over its full dimensions)
+  int64_t extent[kMaxRank];
+  bool full[kMaxRank];
+  int groups = 0;
+  int64_t dense = 1;
+  for (int k = d.rank - 1; k >= 0; k--) {
+    if (d.outSize[k] == 1)
+      continue;
+    const bool f = d.bSize[k] != 1;
+    if (f && d.bStride[k] != dense)
+      return false;
+    if (f)
+      dense *= d.outSize[k];
+    if (groups > 0 && full[groups - 1] == f)
+      extent[groups - 1] *= d.outSize[k];
+    else {
+      extent[groups] = d.outSize[k];
+      full[groups++] = f;
+    }
+  }
+  int64_t inner = 1, div = 1, mod = 1;
+  bool rowOfB = true;
+  if (groups > 3 || (groups == 3 && !full[1] && !full[2]))
+    return false;
+  if (groups >= 1) {
+    inner = extent[0];
+    rowOfB = full[0];
+    if (full[0]) { // [.., n] with B repeating in front of it, or [b, 1, n]
+      if (groups >= 2)
+        div = groups == 3 ? extent[1] : 1;
+      mod = groups == 3 ? extent[2] : 1;
+    } else { // one value per row: [b, 1] or [1, s, 1]
+      mod = groups >= 2 ? extent[1] : 1;
+    }
+  }
+  if (total >= (int64_t(1) << 31))
+    return false;
+  m->inner = uint32_t(inner);
+  m->rowDiv = uint32_t(div);
+  m->rowMod = uint32_t(mod);
+  m->innerMagic = magicFor(m->inner);
+  m->divMagic = magicFor(m->rowDiv);
+  m->modMagic = magicFor(m->rowMod);
+  m->rowOfB = rowOfB;
+  return true;
+}
+
+template <typename T, int OP, bool STREAM>
+void launchRows(const T *a, const T *b, T *out, int64_t total,
+                const RowBroadcast &m, bool whole, hipStream_t s) {
+  constexpr int N = Vec16<T>::kN;
+  const int64_t nvec = (total + N - 1) / N;
+  const dim3 grid((unsigned)((nvec + 255) / 256)), block(256);
+  if (m.rowOfB && whole)
+    elementwiseRowKernel<T, OP, true, true, STREAM>
+        <<<grid, block, 0, s>>>(a, b, out, uint32_t(total), m);
+  else if (m.rowOfB)
+    elementwiseRowKernel<T, OP, true, false, STREAM>
+        <<<grid, block, 0, s>>>(a, b, out, uint32_t(total), m);
+  else if (whole)
+    elementwiseRowKernel<T, OP, false, true, STREAM>
+        <<<grid, block, 0, s>>>(a, b, out, uint32_t(total), m);
+  else
+    elementwiseRowKernel<T, OP, false, false, STREAM>
+        <<<grid, block, 0, s>>>(a, b, out, uint32_t(total), m);
+}
 
 template <typename T, int OP>
 Status elementwiseDispatch(const T *a, const T *b, T *out, int64_t total,
                            const BroadcastDesc &d, hipStream_t s) {
   constexpr int N = Vec16<T>::kN;
-  // inner = number of trailing elements over which B is dense and contiguous;
-  // every dimension in front of them must have B extent 1.
-  int64_t inner = 1;
-  int k = d.rank - 1;
-  for (; k >= 0; k--) {
-    if (d.bSize[k] != d.outSize[k] ||
-        (d.outSize[k] != 1 && d.bStride[k] != inner))
-      break;
-    inner *= d.outSize[k];
-  }
-  bool leadingOnly = true;
-  for (int j = k; j >= 0; j--)
-    leadingOnly = leadingOnly && d.bSize[j] == 1;
-  const int cus = deviceInfo().computeUnits;
-  if (leadingOnly && inner % N == 0 && total % N == 0 && aligned16(a) &&
-      aligned16(b) && aligned16(out)) {
-    const int64_t nvec = total / N;
-    int64_t blocks = (nvec + 255) / 256;
-    if (inner == total && total * int64_t(sizeof(T)) > kStreamingBytes &&
-        blocks < (int64_t(1) << 31)) {
-      elementwiseStreamKernel<T, OP>
-          <<<dim3((unsigned)blocks), dim3(256), 0, s>>>(a, b, out, nvec);
-      HOM_HIP_RET(hipGetLastError(), Status::kInternal);
-      return Status::kSuccess;
-    }
-    if (blocks > int64_t(cus) * 16)
-      blocks = int64_t(cus) * 16;
-    elementwiseVecKernel<T, OP><<<dim3((unsigned)blocks), dim3(256), 0, s>>>(
-        a, b, out, nvec, inner / N);
+  const bool stream = total * int64_t(sizeof(T)) > kStreamingBytes;
+  const int64_t blocks = ((total + N - 1) / N + 255) / 256;
+  const bool vec = aligned16(a) && aligned16(out);
+  RowBroadcast m{};
+  bool same = true; // B has A's shape and is dense
+  for (int k = 0; k < d.rank; k++)
+    same = same && d.bSize[k] == d.outSize[k] &&
+           (d.outSize[k] == 1 || d.bStride[k] == d.outStride[k]);
+  if (same && vec && aligned16(b) && blocks < (int64_t(1) << 31)) {
+    const dim3 grid((unsigned)blocks), block(256);
+    if (stream)
+      elementwiseSameKernel<T, OP, true><<<grid, block, 0, s>>>(a, b, out, total);
+    else
+      elementwiseSameKernel<T, OP, false><<<grid, block, 0, s>>>(a, b, out, total);
+  } else if (vec && rowBroadcast(d, total, &m)) {
+    const bool whole = m.inner % N == 0 && (!m.rowOfB || aligned16(b));
+    if (stream)
+      launchRows<T, OP, true>(a, b, out, total, m, whole, s);
+    else
+      launchRows<T, OP, false>(a, b, out, total, m, whole, s);
   } else {
-    int64_t blocks = (total + 255) / 256;
-    if (blocks > int64_t(cus) * 32)
-      blocks = int64_t(cus) * 32;
+    const int cus = deviceInfo().computeUnits;
+    int64_t generic = (total + 255) / 256;
+    if (generic > int64_t(cus) * 32)
+      generic = int64_t(cus) * 32;
     elementwiseGenericKernel<T, OP>
-        <<<dim3((unsigned)blocks), dim3(256), 0, s>>>(a, b, out, total, d);
+        <<<dim3((unsigned)generic), dim3(256), 0, s>>>(a, b, out, total, d);
   }
   HOM_HIP_RET(hipGetLastError(), Status::kInternal);
   return Status::kSuccess;
 }
 
 // ---------------------------------------------------------------- gather --
+// One 16-byte vector per thread, rowVecs of them per row.  Rows need not be
+// whole vectors: they start at any element boundary (which the hardware's
+// 16-byte accesses take), and the last vector of a row ends with the row,
+// overlapping the one before it with the same values.
 template <typename T>
-__global__ __launch_bounds__(256) void gatherVecKernel(
+__global__ __launch_bounds__(256) void gatherKernel(
     const int64_t *__restrict__ indices, const T *__restrict__ value,
-    T *__restrict__ out, int64_t numIndices, int64_t vocab, int rowVec) {
+    T *__restrict__ out, uint32_t total, int64_t vocab, uint32_t rowLength,
+    uint32_t rowVecs, uint32_t rowMagic) {
   using V = typename Vec16<T>::type;
-  const int64_t total = numIndices * rowVec;
-  const int64_t step = int64_t(gridDim.x) * blockDim.x;
-  for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < total;
-       i += step) {
-    const int64_t r = i / rowVec;
-    const int c = int(i - r * rowVec);
-    int64_t src = indices[r];
-    // An index outside the table would read foreign memory; clamp it.
-    src = src < 0 ? 0 : (src >= vocab ? vocab - 1 : src);
-    reinterpret_cast<V *>(out)[i] =
-        reinterpret_cast<const V *>(value)[src * rowVec + c];
-  }
+  typedef V VAny __attribute__((aligned(sizeof(T))));
+  constexpr uint32_t N = Vec16<T>::kN;
+  const uint32_t v = blockIdx.x * 256u + threadIdx.x;
+  if (v >= total)
+    return;
+  const uint32_t r = divByMagic(v, rowVecs, rowMagic);
+  uint32_t c = (v - r * rowVecs) * N;
+  if (c + N > rowLength)
+    c = rowLength - N;
+  // An index outside the table would read foreign memory; clamp it.
+  int64_t i = indices[r];
+  i = i < 0 ? 0 : (i >= vocab ? vocab - 1 : i);
+  const V got = *reinterpret_cast<const VAny *>(value + i * rowLength + c);
+  storeWriteThrough(out + size_t(r) * rowLength + c, got);
 }
 
+// Rows shorter than a vector, outputs of 2^31 vectors and more.
 template <typename T>
 __global__ __launch_bounds__(256) void gatherScalarKernel(
     const int64_t *__restrict__ indices, const T *__restrict__ value,
@@ -190,31 +327,58 @@ __global__ __launch_bounds__(256) void gatherScalarKernel(
 }
 
 // ------------------------------------------------------------ cu_seqlens --
-// One workgroup: each wavefront sums rows of the mask, then thread 0 runs the
-// (short) inclusive scan.  Row sums pass through the output buffer itself.
+// One workgroup of 16 wavefronts: each sums rows of the mask, 8 loads in flight
+// per lane, into LDS; the first wavefront then turns 64 row sums at a time into
+// the running total with a prefix sum across its lanes.  A chain of memory round
+// trips is all this kernel is made of (a row at a time and a serial scan through
+// memory by one thread: 7.4 us for 16 rows of 200, now 2.7).
 template <typename InT>
-__global__ __launch_bounds__(256) void cuSeqLenKernel(
+__global__ __launch_bounds__(1024) void cuSeqLenKernel(
     const InT *__restrict__ mask, int32_t *out, int64_t bs, int64_t seq) {
-  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-  const int nwaves = blockDim.x / kWave;
-  for (int64_t r = wave; r < bs; r += nwaves) {
-    int32_t sum = 0;
-    for (int64_t j = lane; j < seq; j += kWave)
-      sum += int32_t(mask[r * seq + j]);
-#pragma unroll
-    for (int off = kWave / 2; off > 0; off >>= 1)
-      sum += __shfl_xor(sum, off, kWave);
-    if (lane == 0)
-      out[r + 1] = sum;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    int32_t acc = 0;
+  constexpr int kWaves = 16, kRows = 256; // rows per pass
+  __shared__ int32_t rowSum[kRows];
+  const int lane = threadIdx.x % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  int32_t acc = 0; // total of all rows before this pass (first wavefront)
+  if (threadIdx.x == 0)
     out[0] = 0;
-    for (int64_t r = 0; r < bs; r++) {
-      acc += out[r + 1];
-      out[r + 1] = acc;
+  for (int64_t base = 0; base < bs; base += kRows) {
+    const int rows = int(bs - base < kRows ? bs - base : kRows);
+    for (int r = wave; r < rows; r += kWaves) {
+      const InT *row = mask + (base + r) * seq;
+      int32_t sum = 0;
+      for (int64_t j = 0; j < seq; j += 8 * kWave) {
+        InT v[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) { // (past the end: the last element again)
+          const int64_t at = j + u * kWave + lane;
+          v[u] = row[at < seq ? at : seq - 1];
+        }
+#pragma unroll
+        for (int u = 0; u < 8; u++)
+          sum += j + u * kWave + lane < seq ? int32_t(v[u]) : 0;
+      }
+#pragma unroll
+      for (int off = kWave / 2; off > 0; off >>= 1)
+        sum += __shfl_xor(sum, off, kWave);
+      if (lane == 0)
+        rowSum[r] = sum;
     }
+    __syncthreads();
+    if (wave == 0) {
+      for (int r = 0; r < rows; r += kWave) {
+        int32_t v = r + lane < rows ? rowSum[r + lane] : 0;
+#pragma unroll
+        for (int off = 1; off < kWave; off <<= 1) {
+          const int32_t below = __shfl_up(v, off, kWave);
+          v += lane >= off ? below : 0;
+        }
+        if (r + lane < rows)
+          out[base + r + lane + 1] = acc + v;
+        acc += __shfl(v, kWave - 1, kWave);
+      }
+    }
+    __syncthreads();
   }
 }
 
@@ -325,12 +489,13 @@ Status launchGather(const int64_t *indices, const T *value, T *out,
   if (numIndices == 0 || rowLength == 0)
     return Status::kSuccess;
   constexpr int N = Vec16<T>::kN;
-  if (rowLength % N == 0 && aligned16(value) && aligned16(out) &&
-      rowLength / N < (int64_t(1) << 31)) {
-    const int rowVec = int(rowLength / N);
-    gatherVecKernel<T>
-        <<<dim3(cappedBlocks(numIndices * rowVec, 256, 16)), dim3(256), 0, s>>>(
-            indices, value, out, numIndices, vocab, rowVec);
+  const int64_t rowVecs = (rowLength + N - 1) / N, total = numIndices * rowVecs;
+  if (rowLength >= N && rowLength < (int64_t(1) << 31) &&
+      total < (int64_t(1) << 31)) {
+    const dim3 grid((unsigned)((total + 255) / 256));
+    gatherKernel<T><<<grid, dim3(256), 0, s>>>(
+        indices, value, out, uint32_t(total), vocab, uint32_t(rowLength),
+        uint32_t(rowVecs), magicFor(uint32_t(rowVecs)));
   } else {
     gatherScalarKernel<T>
         <<<dim3(cappedBlocks(numIndices * rowLength, 256, 32)), dim3(256), 0,
@@ -348,7 +513,7 @@ template Status launchGather<float>(const int64_t *, const float *, float *,
 template <typename InT>
 Status launchCuSeqLen(const InT *mask, int32_t *out, int64_t bs, int64_t seq,
                       hipStream_t s) {
-  cuSeqLenKernel<InT><<<dim3(1), dim3(256), 0, s>>>(mask, out, bs, seq);
+  cuSeqLenKernel<InT><<<dim3(1), dim3(1024), 0, s>>>(mask, out, bs, seq);
   HOM_HIP_RET(hipGetLastError(), Status::kInternal);
   return Status::kSuccess;
 }

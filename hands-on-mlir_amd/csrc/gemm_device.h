@@ -34,6 +34,7 @@
 #pragma once
 
 #include "cross_lane.h"
+#include "fast_div.h"
 #include "kernels.h"
 #include "store_policy.h"
 
@@ -189,17 +190,6 @@ __device__ __forceinline__ void tileCoords(int tile, int tilesM, int tilesN,
   const int inGroup = tile - g * groupSize;
   *tileM = firstM + inGroup % rows;
   *tileN = inGroup / rows;
-}
-
-// n / d for n < 2^32 given m = floor(2^32 / d) (0xffffffff for d == 1): the
-// high product is the quotient or one less.
-__device__ __forceinline__ uint32_t divByMagic(uint32_t n, uint32_t d,
-                                               uint32_t m) {
-  const uint32_t q = __umulhi(n, m);
-  return n - q * d >= d ? q + 1 : q;
-}
-inline uint32_t magicFor(uint32_t d) {
-  return d <= 1 ? 0xffffffffu : uint32_t((uint64_t(1) << 32) / d);
 }
 
 // m % cRowPeriod (the row of a shared source that output row m reads).

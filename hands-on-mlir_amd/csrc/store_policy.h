@@ -24,8 +24,9 @@ namespace hom {
 constexpr int kWriteThroughAux = 17;
 
 // *p = v with the sc0 sc1 bits.
+// (p: any element boundary, the hardware's wide stores take it)
 template <typename V>
-__device__ __forceinline__ void storeWriteThrough(V *p, const V &v) {
+__device__ __forceinline__ void storeWriteThrough(void *p, const V &v) {
   static_assert(sizeof(V) == 16 || sizeof(V) == 8 || sizeof(V) == 4 ||
                     sizeof(V) == 2,
                 "store width");
@@ -66,7 +67,7 @@ __device__ __forceinline__ void storeWriteThrough(V *p, const V &v) {
 // loads and stores, 5.72 TB/s with this store policy on top (sc1 nt; sc0 sc1
 // nt is the same); write-through without the hint 5.49 TB/s.
 template <typename V>
-__device__ __forceinline__ void storeStreaming(V *p, const V &v) {
+__device__ __forceinline__ void storeStreaming(void *p, const V &v) {
   static_assert(sizeof(V) == 16, "store width");
   typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
   // (wait states: see storeWriteThrough)

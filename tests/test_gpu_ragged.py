@@ -1,0 +1,79 @@
+"""Sizes off the vector width, broadcast forms and edges of the dispatch rules, against numpy and the oracle."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def dev(a):
+    return torch.from_numpy(np.ascontiguousarray(a)).cuda()
+
+
+def host(t):
+    torch.cuda.synchronize()
+    return t.cpu().numpy()
+
+
+# A's shape, B's shape: same, bias row, row per batch, value per row, repeating values, all the same, a pattern
+# only the generic walk takes; rows of whole vectors and not, totals with and without a remainder, streaming size
+@pytest.mark.parametrize("a,b", [
+    ((3, 5, 16), (3, 5, 16)), ((3, 5, 7), (3, 5, 7)), ((4, 6, 16), (1, 1, 16)), ((4, 6, 13), (1, 1, 13)),
+    ((4, 6, 16), (1, 6, 16)), ((4, 6, 24), (4, 1, 24)), ((4, 6, 9), (4, 1, 9)), ((4, 6, 16), (4, 6, 1)),
+    ((4, 6, 11), (4, 6, 1)), ((4, 6, 8), (1, 6, 1)), ((4, 6, 3), (1, 6, 1)), ((4, 6, 5), (4, 1, 1)),
+    ((2, 3, 4, 8), (2, 1, 4, 1)), ((2, 3, 4, 8), (1, 3, 1, 8)), ((4, 6, 5), (1, 1, 1)), ((1, 1, 1), (1, 1, 1)),
+    ((9, 1001, 1023), (9, 1001, 1)), ((9, 1000, 1024), (9, 1, 1024))])
+@pytest.mark.parametrize("sfx,dtype", [("F16", np.float16), ("F32", np.float32)])
+def test_elementwise_broadcast_forms(gpu, rt, a, b, sfx, dtype):
+    g = np.random.default_rng(len(a) + sum(a))
+    x, y = g.standard_normal(a).astype(dtype), g.standard_normal(b).astype(dtype)
+    M = rt.MemRef.from_tensor
+    for op, want in (("Mul", x * y), ("Sub", x - y)):
+        tx, ty, out = dev(x), dev(y), torch.zeros(a, dtype=torch.from_numpy(x).dtype, device="cuda")
+        getattr(gpu, f"thrustElementwise{op}{sfx}")(*M(tx).args(), *M(ty).args(), *M(out).args())
+        np.testing.assert_array_equal(host(out), want)
+        getattr(gpu, f"thrustElementwise{op}{sfx}")(*M(tx).args(), *M(ty).args(), *M(tx).args())  # in place
+        np.testing.assert_array_equal(host(tx), want)
+
+
+@pytest.mark.parametrize("bs,seq", [(1, 1), (1, 64), (3, 65), (17, 511), (64, 513), (257, 33), (600, 5)])
+def test_cu_seqlens_many_rows(gpu, rt, bs, seq):
+    mask = (np.random.default_rng(bs).random((bs, seq)) < 0.7)
+    want = np.concatenate([[0], np.cumsum(mask.sum(1))]).astype(np.int32)
+    M = rt.MemRef.from_tensor
+    for sfx, dt in (("I64", np.int64), ("I32", np.int32)):
+        t, out = dev(mask.astype(dt)), torch.zeros(bs + 1, dtype=torch.int32, device="cuda")
+        getattr(gpu, "thrustCuSeqLen" + sfx)(*M(t).args(), *M(out).args())
+        np.testing.assert_array_equal(host(out), want)
+
+
+@pytest.mark.parametrize("H", [1, 7, 8, 9, 129, 768, 1001])
+@pytest.mark.parametrize("sfx,dtype", [("F16", np.float16), ("F32", np.float32)])
+def test_gather_row_lengths(gpu, rt, H, sfx, dtype):
+    g = np.random.default_rng(H)
+    table, ids = g.standard_normal((1, 50, H)).astype(dtype), g.integers(0, 50, (3, 11)).astype(np.int64)
+    ids[0, 0], ids[2, 10] = 49, 0
+    t, i, out = dev(table), dev(ids), torch.zeros((3, 11, H), dtype=torch.from_numpy(table).dtype, device="cuda")
+    M = rt.MemRef.from_tensor
+    getattr(gpu, "thrustGather" + sfx)(*M(i).args(), *M(t).args(), *M(out).args())
+    np.testing.assert_array_equal(host(out), table[0][ids])
+
+
+# row lengths at the edges of the kernel variants (fp16: 1, 2, 4 vectors per lane of a wavefront, 2, 4, 8 of a workgroup)
+@pytest.mark.parametrize("H", [3, 8, 9, 511, 513, 1025, 2047, 2056, 4097, 8191, 16391, 16400])
+def test_layernorm_row_lengths(gpu, rt, oracle, H):
+    g = np.random.default_rng(H)
+    rows = 5
+    x, r = (g.standard_normal((rows, H)).astype(np.float16) for _ in range(2))
+    ga, be = (1 + 0.1 * g.standard_normal(H)).astype(np.float16), g.standard_normal(H).astype(np.float16)
+    M = rt.MemRef.from_tensor
+    tx, tr, tg, tb, out = dev(x), dev(r), dev(ga), dev(be), torch.zeros((rows, H), dtype=torch.float16, device="cuda")
+    gpu.homAddLayernormF16(*M(tx).args(), *M(tr).args(), *M(tg).args(), *M(tb).args(), *M(out).args(), 1e-12)
+    want = oracle.layernorm_f16(x, 1e-12, res=r, gamma=ga, beta=be)
+    np.testing.assert_allclose(host(out).astype(np.float64), want, rtol=2e-3, atol=2e-3)
+    gpu.nvteLayernormF16(*M(tx).args(), 1e-12)
+    np.testing.assert_allclose(host(tx).astype(np.float64), oracle.layernorm_f16(x, 1e-12), rtol=2e-3, atol=1e-3)
+    y = torch.from_numpy(g.standard_normal((rows, H)).astype(np.float32)).cuda()
+    want32 = torch.nn.functional.layer_norm(y.cpu().double(), (H,), eps=1e-6).numpy()
+    gpu.nvteLayernormF32(*M(y).args(), 1e-6)
+    np.testing.assert_allclose(host(y), want32, rtol=1e-4, atol=1e-5)
