@@ -8,6 +8,17 @@ import numpy as np
 from . import hom_runtime as rt
 
 
+class _HostBuffer:
+    """Pinned memory from the driver's pool behind a result array; goes back when the array is dropped."""
+
+    def __init__(self, drv, ptr, shape):
+        self._drv, self._ptr = drv, ptr
+        self.__array_interface__ = {"data": (ptr, False), "shape": shape, "typestr": "<f2", "version": 3}
+
+    def __del__(self):
+        self._drv.homHostBufferRelease(self._ptr)
+
+
 class BertEncoder:
     ROLES = ("qkv", "out", "ffn1", "ffn2", "transform", "decoder")
 
@@ -66,11 +77,9 @@ class BertEncoder:
                 raise ValueError("the driver refused to fold the layer norms for this configuration")
 
     def set_inputs(self, ids=None, mask=None, hidden=None):
-        p = lambda a, dt: (np.ascontiguousarray(a, dt).ctypes.data_as(ctypes.c_void_p)
-                           if a is not None else None)
         keep = [np.ascontiguousarray(a, dt) if a is not None else None
                 for a, dt in ((ids, np.int64), (mask, np.int64), (hidden, np.float16))]
-        ptrs = [a.ctypes.data_as(ctypes.c_void_p) if a is not None else None for a in keep]
+        ptrs = [a.ctypes.data if a is not None else None for a in keep]
         assert self.drv.homBertSetInputs(self.h, *ptrs) == 0
 
     def forward(self, from_ids=True):
@@ -87,17 +96,25 @@ class BertEncoder:
     def replay(self):
         assert self.drv.homBertReplay(self.h) == 0
 
+    def _fetch(self, get, shape):
+        """A new array with the result; in pinned memory while the driver's pool has some."""
+        nbytes = 2 * shape[0] * shape[1] * shape[2]
+        ptr = self.drv.homHostBufferAcquire(nbytes)
+        if ptr:
+            out = np.asarray(_HostBuffer(self.drv, ptr, shape))
+        else:
+            out = np.empty(shape, np.float16)
+            ptr = out.ctypes.data
+        assert get(self.h, ptr) == 0
+        return out
+
     def output(self):
         d = self.dims
-        out = np.empty((d["bs"], d["seq"], d["hidden"]), np.float16)
-        assert self.drv.homBertGetOutput(self.h, out.ctypes.data_as(ctypes.c_void_p)) == 0
-        return out
+        return self._fetch(self.drv.homBertGetOutput, (d["bs"], d["seq"], d["hidden"]))
 
     def logits(self):
         d = self.dims
-        out = np.empty((d["bs"], d["seq"], d["vocab"]), np.float16)
-        assert self.drv.homBertGetLogits(self.h, out.ctypes.data_as(ctypes.c_void_p)) == 0
-        return out
+        return self._fetch(self.drv.homBertGetLogits, (d["bs"], d["seq"], d["vocab"]))
 
     def time(self, steps, warmup, graph=True, from_ids=True):
         ms = self.drv.homBertTime(self.h, steps, warmup, int(graph), int(from_ids))

@@ -10,6 +10,7 @@
 #include "cross_lane.h"
 #include "fast_div.h"
 #include "kernels.h"
+#include "mask_sums.h"
 #include "store_policy.h"
 
 namespace hom {
@@ -327,59 +328,12 @@ __global__ __launch_bounds__(256) void gatherScalarKernel(
 }
 
 // ------------------------------------------------------------ cu_seqlens --
-// One workgroup of 16 wavefronts: each sums rows of the mask, 8 loads in flight
-// per lane, into LDS; the first wavefront then turns 64 row sums at a time into
-// the running total with a prefix sum across its lanes.  A chain of memory round
-// trips is all this kernel is made of (a row at a time and a serial scan through
-// memory by one thread: 7.4 us for 16 rows of 200, now 2.7).
+// One workgroup, see mask_sums.h.
 template <typename InT>
 __global__ __launch_bounds__(1024) void cuSeqLenKernel(
     const InT *__restrict__ mask, int32_t *out, int64_t bs, int64_t seq) {
-  constexpr int kWaves = 16, kRows = 256; // rows per pass
-  __shared__ int32_t rowSum[kRows];
-  const int lane = threadIdx.x % kWave;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-  int32_t acc = 0; // total of all rows before this pass (first wavefront)
-  if (threadIdx.x == 0)
-    out[0] = 0;
-  for (int64_t base = 0; base < bs; base += kRows) {
-    const int rows = int(bs - base < kRows ? bs - base : kRows);
-    for (int r = wave; r < rows; r += kWaves) {
-      const InT *row = mask + (base + r) * seq;
-      int32_t sum = 0;
-      for (int64_t j = 0; j < seq; j += 8 * kWave) {
-        InT v[8];
-#pragma unroll
-        for (int u = 0; u < 8; u++) { // (past the end: the last element again)
-          const int64_t at = j + u * kWave + lane;
-          v[u] = row[at < seq ? at : seq - 1];
-        }
-#pragma unroll
-        for (int u = 0; u < 8; u++)
-          sum += j + u * kWave + lane < seq ? int32_t(v[u]) : 0;
-      }
-#pragma unroll
-      for (int off = kWave / 2; off > 0; off >>= 1)
-        sum += __shfl_xor(sum, off, kWave);
-      if (lane == 0)
-        rowSum[r] = sum;
-    }
-    __syncthreads();
-    if (wave == 0) {
-      for (int r = 0; r < rows; r += kWave) {
-        int32_t v = r + lane < rows ? rowSum[r + lane] : 0;
-#pragma unroll
-        for (int off = 1; off < kWave; off <<= 1) {
-          const int32_t below = __shfl_up(v, off, kWave);
-          v += lane >= off ? below : 0;
-        }
-        if (r + lane < rows)
-          out[base + r + lane + 1] = acc + v;
-        acc += __shfl(v, kWave - 1, kWave);
-      }
-    }
-    __syncthreads();
-  }
+  __shared__ int32_t rowSum[256];
+  sumMaskRows<InT, 16>(mask, out, bs, seq, rowSum);
 }
 
 // ------------------------------------------------------------------ gelu --

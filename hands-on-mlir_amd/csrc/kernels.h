@@ -50,6 +50,17 @@ Status launchApplyRowStatsF16(const _Float16 *a, const _Float16 *var,
                               const _Float16 *mean, _Float16 *out, int64_t rows,
                               int64_t k, hipStream_t s);
 
+// The embedding front in one kernel: cu_seqlens of the mask, and
+// out[i, j, :] = LN(word[ids[i, j], :] + pos[j, :]); embedFits() says whether
+// the shapes and alignments allow it.  ids and mask: device or pinned host
+// memory.
+bool embedFits(const _Float16 *word, const _Float16 *pos, const _Float16 *out,
+               int64_t bs, int64_t seq, int64_t hidden, int64_t vocab);
+Status launchEmbed(const int64_t *ids, const int64_t *mask, const _Float16 *word,
+                   const _Float16 *pos, _Float16 *out, int32_t *cu, int64_t bs,
+                   int64_t seq, int64_t hidden, int64_t vocab, float eps,
+                   hipStream_t s);
+
 // ------------------------------------------------------------- attention --
 // qkv [bs, seq, 3*heads*headDim] fp16, cu int32[bs+1], out [bs, seq,
 // heads*headDim].  headDim 64, 128, 192 or 256.

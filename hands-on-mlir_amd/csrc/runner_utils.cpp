@@ -227,6 +227,14 @@ void homColumnSumsF16(int64_t rankB, void *dstB, float *out) {
   (void)runColumnSums(rankB, dstB, out);
 }
 
+void homEmbedF16(int64_t rankIds, void *desIds, int64_t rankMask, void *desMask,
+                 int64_t rankWord, void *desWord, int64_t rankPos, void *desPos,
+                 int64_t rankOut, void *desOut, int64_t rankCu, void *desCu,
+                 float eps) {
+  (void)runEmbed(rankIds, desIds, rankMask, desMask, rankWord, desWord, rankPos,
+                 desPos, rankOut, desOut, rankCu, desCu, eps);
+}
+
 void homGeluF16(int64_t rankA, void *dstA, int64_t rankOut, void *dstOut,
                 int32_t form) {
   (void)runGeluF16(rankA, dstA, rankOut, dstOut, form);

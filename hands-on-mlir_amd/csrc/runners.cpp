@@ -1004,6 +1004,59 @@ Status runCuSeqLen(int64_t rankIn, void *desIn, int64_t rankOut, void *desOut) {
 template Status runCuSeqLen<int64_t>(int64_t, void *, int64_t, void *);
 template Status runCuSeqLen<int32_t>(int64_t, void *, int64_t, void *);
 
+Status runEmbed(int64_t rankIds, void *desIds, int64_t rankMask, void *desMask,
+                int64_t rankWord, void *desWord, int64_t rankPos, void *desPos,
+                int64_t rankOut, void *desOut, int64_t rankCu, void *desCu,
+                float eps) {
+  View<int64_t> I(rankIds, desIds), Mk(rankMask, desMask);
+  View<_Float16> W(rankWord, desWord), P(rankPos, desPos), O(rankOut, desOut);
+  View<int32_t> Cu(rankCu, desCu);
+  HOM_CHECK_RET(I.rank == 2 && Mk.rank == 2 && I.sizes && Mk.sizes &&
+                    I.sizes[0] == Mk.sizes[0] && I.sizes[1] == Mk.sizes[1],
+                Status::kInvalidArgument,
+                "embed: ids and mask must be [b, s] tensors of one shape");
+  const int64_t bs = I.sizes[0], seq = I.sizes[1];
+  HOM_CHECK_RET(W.rank == 3 && W.sizes && W.sizes[0] == 1 && P.rank == 3 &&
+                    P.sizes && P.sizes[0] == 1 && P.sizes[1] == seq &&
+                    P.sizes[2] == W.sizes[2],
+                Status::kInvalidArgument,
+                "embed: word must be [1, V, H] and positions [1, s, H]");
+  const int64_t vocab = W.sizes[1], hidden = W.sizes[2];
+  HOM_CHECK_RET(O.rank == 3 && O.sizes && O.sizes[0] == bs &&
+                    O.sizes[1] == seq && O.sizes[2] == hidden,
+                Status::kInvalidArgument, "embed: out must be [b, s, H]");
+  HOM_CHECK_RET(Cu.rank == 1 && Cu.sizes && Cu.sizes[0] == bs + 1,
+                Status::kInvalidArgument, "embed: cu_seqlens must be int32[%lld]",
+                (long long)bs + 1);
+  HOM_CHECK_RET(I.contiguous() && Mk.contiguous() && W.contiguous() &&
+                    P.contiguous() && O.contiguous(),
+                Status::kInvalidArgument, "embed: tensors must be contiguous");
+  if (embedFits(W.data, P.data, O.data, bs, seq, hidden, vocab))
+    return launchEmbed(I.data, Mk.data, W.data, P.data, O.data, Cu.data, bs, seq,
+                       hidden, vocab, eps, stream());
+  // rows off the vector width or beyond a wavefront's registers: step by step
+  Status st = launchCuSeqLen<int64_t>(Mk.data, Cu.data, bs, seq, stream());
+  if (st == Status::kSuccess)
+    st = launchGather<_Float16>(I.data, W.data, O.data, bs * seq, vocab, hidden,
+                                stream());
+  BroadcastDesc d{};
+  d.rank = 3;
+  const int64_t size[3] = {bs, seq, hidden};
+  for (int i = 2; i >= 0; i--) {
+    d.outSize[i] = size[i];
+    d.outStride[i] = i == 2 ? 1 : d.outStride[i + 1] * size[i + 1];
+    d.bSize[i] = i == 0 ? 1 : size[i];
+    d.bStride[i] = d.bSize[i] == 1 ? 0 : P.strides[i];
+  }
+  if (st == Status::kSuccess)
+    st = launchElementwise<_Float16>(BinOp::kAdd, O.data, P.data, O.data,
+                                     bs * seq * hidden, d, stream());
+  if (st == Status::kSuccess)
+    st = launchLayernorm<_Float16>(O.data, nullptr, nullptr, nullptr, O.data,
+                                   bs * seq, hidden, eps, stream());
+  return st;
+}
+
 Status runGeluF16(int64_t rankA, void *dstA, int64_t rankOut, void *dstOut,
                   int32_t form) {
   View<_Float16> A(rankA, dstA), O(rankOut, dstOut);

@@ -124,6 +124,10 @@ Status runGather(int64_t rankIdx, void *desIdx, int64_t rankValue,
                  void *desValue, int64_t rankOut, void *desOut);
 template <typename InT>
 Status runCuSeqLen(int64_t rankIn, void *desIn, int64_t rankOut, void *desOut);
+Status runEmbed(int64_t rankIds, void *desIds, int64_t rankMask, void *desMask,
+                int64_t rankWord, void *desWord, int64_t rankPos, void *desPos,
+                int64_t rankOut, void *desOut, int64_t rankCu, void *desCu,
+                float eps);
 Status runGeluF16(int64_t rankA, void *dstA, int64_t rankOut, void *dstOut,
                   int32_t form);
 

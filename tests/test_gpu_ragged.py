@@ -77,3 +77,55 @@ def test_layernorm_row_lengths(gpu, rt, oracle, H):
     want32 = torch.nn.functional.layer_norm(y.cpu().double(), (H,), eps=1e-6).numpy()
     gpu.nvteLayernormF32(*M(y).args(), 1e-6)
     np.testing.assert_allclose(host(y), want32, rtol=1e-4, atol=1e-5)
+
+
+# one, two and four vectors per lane, partial last vectors, the step-by-step form (H off 8, H > 2048), row counts
+# around a wavefront's four rows and a workgroup's 64, more sequences than one pass of the length scan
+@pytest.mark.parametrize("b,s,H", [(1, 1, 8), (1, 3, 512), (5, 13, 520), (8, 128, 768), (2, 33, 1032), (3, 7, 2048),
+                                   (2, 5, 2056), (2, 5, 100), (300, 3, 64)])
+@pytest.mark.parametrize("pinned", [False, True])
+def test_embed_equals_its_steps(gpu, rt, b, s, H, pinned):
+    g = np.random.default_rng(b + s + H)
+    V = 97
+    word, pos = g.standard_normal((1, V, H)).astype(np.float16), g.standard_normal((1, s, H)).astype(np.float16)
+    ids, mask = g.integers(0, V, (b, s)), (g.random((b, s)) < 0.8).astype(np.int64)
+    ids.flat[0], ids.flat[-1] = -3, V + 5  # clamped to the table
+    tw, tp = dev(word), dev(pos)
+    ti, tm = (torch.from_numpy(a).pin_memory() if pinned else dev(a) for a in (ids, mask))
+    M = rt.MemRef.from_tensor
+    new = lambda *shape, dt=torch.float16: torch.zeros(shape, dtype=dt, device="cuda")  # noqa: E731
+    out, cu = new(b, s, H), new(b + 1, dt=torch.int32)
+    gpu.homEmbedF16(*M(ti).args(), *M(tm).args(), *M(tw).args(), *M(tp).args(), *M(out).args(), *M(cu).args(), 1e-12)
+    rows, want, wantCu = new(b, s, H), new(b, s, H), new(b + 1, dt=torch.int32)
+    gpu.thrustCuSeqLenI64(*M(dev(mask)).args(), *M(wantCu).args())
+    gpu.thrustGatherF16(*M(dev(ids)).args(), *M(tw).args(), *M(rows).args())
+    gpu.thrustElementwiseAddF16(*M(rows).args(), *M(tp).args(), *M(want).args())
+    gpu.nvteLayernormF16(*M(want).args(), 1e-12)
+    np.testing.assert_array_equal(host(cu), host(wantCu))
+    np.testing.assert_array_equal(host(out), host(want))
+
+
+def test_results_kept_by_the_caller_stay_apart(synth):
+    import importlib
+    bert = importlib.import_module("hands-on-mlir_amd.bert")
+    m = synth.bert_encoder(layers=1, hidden=128, heads=2, ffn=256, bs=2, seq=17, vocab=50, config=4)
+    d = m["dims"]
+    enc = bert.BertEncoder(d["layers"], d["hidden"], d["heads"], d["ffn"], d["bs"], d["seq"], d["vocab"])
+    enc.load(m)
+    enc.set_inputs(ids=m["ids"], mask=m["mask"])
+    enc.capture()
+    kept = []
+    for k in range(6):
+        enc.set_inputs(ids=(m["ids"] + k) % d["vocab"])
+        enc.replay()
+        kept.append(enc.output())
+    copies = [a.copy() for a in kept]
+    del kept[1], kept[3]  # these buffers may serve later results
+    enc.set_inputs(ids=m["ids"])
+    enc.replay()
+    again = enc.output()
+    np.testing.assert_array_equal(again, copies[0])
+    for a, c in zip(kept, [copies[0], copies[2], copies[3], copies[5]]):
+        np.testing.assert_array_equal(a, c)
+    enc.close()
+    np.testing.assert_array_equal(again, copies[0])  # outlives the encoder
