@@ -48,6 +48,16 @@ namespace gemmk {
   HOM_EXTERN_Q(1, true, BM, BN, WM, WN, DIST)                                  \
   HOM_EXTERN_Q(2, false, BM, BN, WM, WN, DIST)                                 \
   HOM_EXTERN_Q(2, true, BM, BN, WM, WN, DIST)
+#define HOM_EXTERN_U(E, NK, BM, BN, WM, WN, DIST)                              \
+  extern template Status launchPipe<BM, BN, WM, WN, DIST, E, NK, false, true>( \
+      const GemmProblem &, hipStream_t);
+#define HOM_PIPE_TILE_U(BM, BN, WM, WN, DIST)                                  \
+  HOM_EXTERN_U(0, false, BM, BN, WM, WN, DIST)                                 \
+  HOM_EXTERN_U(0, true, BM, BN, WM, WN, DIST)                                  \
+  HOM_EXTERN_U(1, false, BM, BN, WM, WN, DIST)                                 \
+  HOM_EXTERN_U(1, true, BM, BN, WM, WN, DIST)                                  \
+  HOM_EXTERN_U(2, false, BM, BN, WM, WN, DIST)                                 \
+  HOM_EXTERN_U(2, true, BM, BN, WM, WN, DIST)
 #define HOM_STAGED_TILE(BM, BN, BK, WM, WN, VEC)                               \
   HOM_EXTERN_STAGED(BM, BN, BK, WM, WN, 0, VEC)                                \
   HOM_EXTERN_STAGED(BM, BN, BK, WM, WN, 1, VEC)                                \
@@ -60,6 +70,7 @@ namespace gemmk {
 #undef HOM_PIPE_TILE_D
 #undef HOM_FINE_TILE
 #undef HOM_PIPE_TILE_Q
+#undef HOM_PIPE_TILE_U
 #undef HOM_STAGED_TILE
 } // namespace gemmk
 
@@ -115,6 +126,27 @@ struct KernelEntry {
   HOM_PIPE_Q_ENTRY(BM, BN, WM, WN, DIST, Epilogue::kLinear, "linear", 0),      \
       HOM_PIPE_Q_ENTRY(BM, BN, WM, WN, DIST, Epilogue::kGeluErf, "gelu", 1),   \
       HOM_PIPE_Q_ENTRY(BM, BN, WM, WN, DIST, Epilogue::kGeluTanh, "gelutanh",  \
+                       1),
+// "u<d>" and align1: the register-staged pipeline for operands at any element
+// alignment and any N, K (below 8 values a row the scalar kernel runs).
+template <int BM, int BN, int WM, int WN, int DIST, int EPI, bool B_NK>
+Status launchAny(const GemmProblem &p, hipStream_t s) {
+  if (p.K < 8 || p.N < 8)
+    return launchStaged<64, 64, 32, 2, 2, EPI, B_NK, 1>(p, s);
+  return launchPipe<BM, BN, WM, WN, DIST, EPI, B_NK, false, true>(p, s);
+}
+#define HOM_PIPE_U_ENTRY(BM, BN, WM, WN, DIST, EPI_ENUM, EPI_STR, ACT)         \
+  {                                                                            \
+    {"hom_gfx950_mfma_f16_s32x32x16gemm_f16_" #BM "x" #BN "_64x2u" #DIST       \
+     "_w" #WM "x" #WN "_nn_align1_" EPI_STR,                                   \
+     BM, BN, 64, WM, WN, 1, 1, ACT, EPI_ENUM},                                 \
+        launchAny<BM, BN, WM, WN, DIST, int(EPI_ENUM), false>,                 \
+        launchAny<BM, BN, WM, WN, DIST, int(EPI_ENUM), true>                   \
+  }
+#define HOM_PIPE_TILE_U(BM, BN, WM, WN, DIST)                                  \
+  HOM_PIPE_U_ENTRY(BM, BN, WM, WN, DIST, Epilogue::kLinear, "linear", 0),      \
+      HOM_PIPE_U_ENTRY(BM, BN, WM, WN, DIST, Epilogue::kGeluErf, "gelu", 1),   \
+      HOM_PIPE_U_ENTRY(BM, BN, WM, WN, DIST, Epilogue::kGeluTanh, "gelutanh",  \
                        1),
 #define HOM_PIPE_TILE_A(BM, BN, WM, WN, DIST)                                  \
   HOM_PIPE_ENTRY(BM, BN, WM, WN, DIST, Epilogue::kLinear, "linear", 0),        \

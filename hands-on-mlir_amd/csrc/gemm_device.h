@@ -359,15 +359,20 @@ epilogueStoreLds(const GemmParams &p, float16v (&acc)[MI][NI], int m0, int n0,
             for (int e = 0; e < 8; e++)
               c[e] = float(cv[e]);
           } else {
-            // rows start at 4-byte boundaries only (N not a multiple of 8):
-            // pairs, and the pair that reaches past column N is dropped (N even)
+            // rows start anywhere (N not a multiple of 8): still one 16-byte
+            // load, and element by element in the row's last vector
+            typedef half8 half8any __attribute__((aligned(2)));
+            if (n + 8 <= p.N) {
+              const half8 cv = *reinterpret_cast<const half8any *>(cPtr);
 #pragma unroll
-            for (int e = 0; e < 8; e += 2)
-              if (n + e < p.N) {
-                const half2v cv = *reinterpret_cast<const half2v *>(cPtr + e);
-                c[e] = float(cv[0]);
-                c[e + 1] = float(cv[1]);
-              }
+              for (int e = 0; e < 8; e++)
+                c[e] = float(cv[e]);
+            } else {
+#pragma unroll
+              for (int e = 0; e < 8; e++)
+                if (n + e < p.N)
+                  c[e] = float(cPtr[e]);
+            }
           }
         }
         float rowScale = 1.f, rowShift = 0.f;
@@ -399,26 +404,22 @@ epilogueStoreLds(const GemmParams &p, float16v (&acc)[MI][NI], int m0, int n0,
         if (vec16) {
           storeWriteThrough(reinterpret_cast<half8 *>(dPtr), o);
         } else if (n + 8 <= p.N) {
-          // rows start at 4-byte boundaries only (N even, not a multiple of 8):
-          // still one 16-byte store, which the hardware takes at dword
-          // alignment (as it does the 16-byte loads of such a B); written as
-          // asm because a C++ store of this type would promise 16-byte
-          // alignment.  Default cache policy: see store_policy.h.
+          // rows start anywhere (N not a multiple of 8): still one 16-byte
+          // store, which the hardware takes at any element boundary (as it does
+          // the 16-byte loads of such a B); written as asm because a C++ store
+          // of this type would promise 16-byte alignment.  Default cache
+          // policy: see store_policy.h.
           typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
           asm volatile("global_store_dwordx4 %0, %1, off\n\ts_nop 1"
                        :
                        : "v"(dPtr), "v"(__builtin_bit_cast(u32x4, o))
                        : "memory");
         } else {
-          // the row's last vector: pairs, the pair past column N is dropped
+          // the row's last vector
 #pragma unroll
-          for (int e = 0; e < 8; e += 2)
-            if (n + e < p.N) {
-              half2v ov;
-              ov[0] = o[e];
-              ov[1] = o[e + 1];
-              *reinterpret_cast<half2v *>(dPtr + e) = ov;
-            }
+          for (int e = 0; e < 8; e++)
+            if (n + e < p.N)
+              dPtr[e] = o[e];
         }
       }
       if constexpr (EPI == kEpiRowStats) {

@@ -27,8 +27,24 @@
   template Status FN<__VA_ARGS__, 2, true, true>(const GemmProblem &,          \
                                                  hipStream_t);
 
+// and for its any-alignment variant (launchPipe<..., false, true>)
+#define HOM_INST_EPILOGUES_ANY(FN, ...)                                        \
+  template Status FN<__VA_ARGS__, 0, false, false, true>(const GemmProblem &,  \
+                                                         hipStream_t);         \
+  template Status FN<__VA_ARGS__, 0, true, false, true>(const GemmProblem &,   \
+                                                        hipStream_t);          \
+  template Status FN<__VA_ARGS__, 1, false, false, true>(const GemmProblem &,  \
+                                                         hipStream_t);         \
+  template Status FN<__VA_ARGS__, 1, true, false, true>(const GemmProblem &,   \
+                                                        hipStream_t);          \
+  template Status FN<__VA_ARGS__, 2, false, false, true>(const GemmProblem &,  \
+                                                         hipStream_t);         \
+  template Status FN<__VA_ARGS__, 2, true, false, true>(const GemmProblem &,   \
+                                                        hipStream_t);
+
 #define HOM_DMA_TILE(...)
 #define HOM_PIPE_TILE_Q(...)
+#define HOM_PIPE_TILE_U(...)
 #define HOM_PIPE_TILE_A(...)
 #define HOM_PIPE_TILE_B(...)
 #define HOM_PIPE_TILE_C(...)

@@ -23,8 +23,20 @@ namespace gemmk {
 // memory.  `rest` holds the same values again plus everything else; its copies
 // of the leading arguments are never read.
 // tileWalk = xcdR | lastRows << 4 | fullGroups << 8.
+//
+// ANY == true (register staging only): operands at any element alignment, rows
+// of any length from 8 values up.  The hardware's 16-byte loads take any element
+// boundary, so the main loop is the same; what differs is confined to the slab
+// behind the full ones.  There a vector that would reach past the end of K (or,
+// row-major B, of N) is read ending at that end and shifted down, so that no
+// load ever leaves the tensor; and with a row-major B the last row of B is always
+// left to that slab, because a full slab's vectors may run past the end of
+// their row, which must not be the tensor's last.  1000 x 1001 x 1003: 135 us
+// with the scalar staging of gemm_staged.h, 9.9 us this way (1000 x 1000 x 1000
+// on the aligned kernel: 7.9 us; a misaligned vector touches two cache lines);
+// 16000 x 4095 x 1023 with bias and GELU 1432 -> 208 us.
 template <int BM, int BN, int WM, int WN, int DIST, int EPI, bool B_NK,
-          bool DMA = false>
+          bool DMA = false, bool ANY = false>
 __global__ __launch_bounds__(WM *WN *kWave) void gemmPipeKernel(
     const _Float16 *argA, const _Float16 *argB, int argM, int argN, int argK,
     int argLda, int argLdb, int argTilesN, int argXcdQ, uint32_t argTileWalk,
@@ -197,7 +209,8 @@ __global__ __launch_bounds__(WM *WN *kWave) void gemmPipeKernel(
   half8 regA[DMA ? 1 : DIST][A_PER_T], regB[DMA ? 1 : DIST][B_PER_T];
   // Slabs of this slice that lie inside [0, kEnd) entirely, and whether a
   // partial one follows them (only the last slice of a ragged K has one).
-  const int nkFull = (kEnd - ktBegin * BK) / BK;
+  const int kFullEnd = ANY && !B_NK && kEnd == p.K ? kEnd - 1 : kEnd;
+  const int nkFull = (kFullEnd - ktBegin * BK) / BK;
   const bool hasTail = kEnd - ktBegin * BK > nkFull * BK;
   const int ktLastFull = ktBegin + nkFull - 1;
   // Full slab kt (requests past the last full slab fetch that one again).
@@ -238,10 +251,54 @@ __global__ __launch_bounds__(WM *WN *kWave) void gemmPipeKernel(
             half8, __builtin_amdgcn_raw_buffer_load_b128(rsrcB, bOff[i], sB, 0));
     }
   };
+  // `count` values of a vector that was read ending at the last one: shifted to
+  // the front, zeros behind them.
+  auto shiftDown = [](half8 v, int count) {
+    typedef unsigned long long u64x2 __attribute__((ext_vector_type(2)));
+    u64x2 w = __builtin_bit_cast(u64x2, v);
+    const int bits = (8 - count) * 16;
+    if (bits >= 64) {
+      w[0] = w[1] >> (bits - 64);
+      w[1] = 0;
+    } else if (bits > 0) {
+      w[0] = (w[0] >> bits) | (w[1] << (64 - bits));
+      w[1] >>= bits;
+    }
+    return __builtin_bit_cast(half8, w);
+  };
   // Slab kt with a range test per vector (the partial slab).
   auto loadGlobalChecked = [&](int kt, auto setC) {
     constexpr int S = decltype(setC)::value;
     const int k0 = kt * BK;
+    if constexpr (ANY) {
+      // (elements of the vector inside the range: none, 8, or the last 1..7)
+      auto fetch = [&](auto rsrc, uint32_t off, int inside) {
+        const int back = inside > 0 && inside < 8 ? 8 - inside : 0;
+        const half8 v = __builtin_bit_cast(
+            half8, __builtin_amdgcn_raw_buffer_load_b128(
+                       rsrc, inside > 0 ? off - uint32_t(back) * 2u : kOob, 0, 0));
+        return back > 0 ? shiftDown(v, inside) : v;
+      };
+#pragma unroll
+      for (int i = 0; i < A_PER_T; i++)
+        regA[S][i] = fetch(rsrcA, aOff[i] + uint32_t(k0) * 2u, kEnd - (k0 + aK[i]));
+#pragma unroll
+      for (int i = 0; i < B_PER_T; i++) {
+        if constexpr (B_NK) {
+          regB[S][i] = fetch(rsrcB, bOff[i] + uint32_t(k0) * 2u, kEnd - (k0 + bK[i]));
+        } else {
+          // (from the matrix base: the vector may start ahead of this tile)
+          const auto rsrcAll = __builtin_amdgcn_make_buffer_rsrc(
+              const_cast<_Float16 *>(p.B), 0, clampBytes(int64_t(p.K) * p.ldb * 2),
+              0x00020000);
+          const uint32_t row = uint32_t(k0 + bK[i]) * uint32_t(p.ldb);
+          const int n = n0 + (tid + i * THREADS) % B_VPR * 8;
+          regB[S][i] = fetch(rsrcAll, (row + uint32_t(n)) * 2u,
+                             k0 + bK[i] < kEnd ? p.N - n : 0);
+        }
+      }
+      return;
+    }
     const uint32_t sA = uint32_t(k0) * 2u;
     const uint32_t sB = B_NK ? sA : uint32_t(k0) * uint32_t(p.ldb) * 2u;
 #pragma unroll
@@ -749,8 +806,9 @@ __global__ __launch_bounds__(WM *WN *kWave) void gemmPipeKernel(
 }
 
 template <int BM, int BN, int WM, int WN, int DIST, int EPI, bool B_NK,
-          bool DMA = false>
+          bool DMA = false, bool ANY = false>
 Status launchPipe(const GemmProblem &pr, hipStream_t s) {
+  static_assert(!ANY || !DMA, "DMA staging needs aligned rows");
   constexpr int SMEM = (DMA ? DIST + 1 : 2) * (BM + BN) * 64 * 2;
   static_assert(!DMA || ((BM * 8) % (WM * WN * kWave) == 0 &&
                          (BN * 8) % (WM * WN * kWave) == 0 &&
@@ -767,7 +825,7 @@ Status launchPipe(const GemmProblem &pr, hipStream_t s) {
   HOM_CHECK_RET((int64_t(BM) * pr.lda + pr.K) * 2 < (int64_t(1) << 31) &&
                     (int64_t(BN) * pr.ldb + pr.K) * 2 < (int64_t(1) << 31),
                 Status::kInvalidArgument, "gemm: leading dimension too large");
-  auto kernel = gemmPipeKernel<BM, BN, WM, WN, DIST, EPI, B_NK, DMA>;
+  auto kernel = gemmPipeKernel<BM, BN, WM, WN, DIST, EPI, B_NK, DMA, ANY>;
   static bool attrSet = false;
   st = allowLds(kernel, SMEM, &attrSet);
   if (st != Status::kSuccess)

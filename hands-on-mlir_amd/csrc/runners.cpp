@@ -186,21 +186,111 @@ bool kernelFits(const GemmKernelInfo &k, int cls) {
   return cls == 8 || (cls == 2 && k.alignmentN <= 2);
 }
 
-// What to run when the selected kernel does not fit the problem's alignment.
-int fallbackKernel(Epilogue epi, int cls) {
-  if (cls == 2) {
-    for (int i = 0; i < gemmKernelCount(); i++) {
-      const GemmKernelInfo &k = gemmKernelInfo(i);
-      if (k.epilogue == epi && k.alignment == 8 && k.alignmentN <= 2 &&
-          k.tileM == 128 && k.tileN == 128)
-        return i;
-    }
-  }
-  return findKernel(64, 64, 32, epi, 1);
-}
-
 // Kernel and split-K (stored into pr) the [N, K]-B path runs for a problem.
 int chooseNvteKernel(GemmProblem *pr, int64_t activation);
+
+// The class of a problem whose operands are all aligned as well as its sizes
+// allow.
+int naturalClass(int64_t N, int64_t K) {
+  return K % 8 != 0 ? 1 : (N % 8 == 0 ? 8 : (N % 2 == 0 ? 2 : 1));
+}
+
+// One tile of the register-staged family as the model below sees it: the
+// kernels per epilogue of the vector-aligned and the any-alignment form (-1:
+// there is none).
+struct TileModel {
+  int tileM, tileN, wavesM, wavesN, depth;
+  int aligned[3], any[3];
+};
+// (the manifest is looked through once per process, not once per call)
+const std::vector<TileModel> &tileModels() {
+  static const std::vector<TileModel> models = [] {
+    std::vector<TileModel> v = {
+        {64, 64, 2, 2, 2, {}, {}},   {128, 64, 2, 2, 2, {}, {}},
+        {64, 128, 2, 2, 2, {}, {}},  {128, 128, 2, 4, 2, {}, {}},
+        {128, 256, 2, 4, 2, {}, {}}, {256, 128, 4, 2, 2, {}, {}},
+        {256, 256, 2, 4, 1, {}, {}},
+    };
+    static const char *const epiName[3] = {"linear", "gelu", "gelutanh"};
+    for (TileModel &t : v)
+      for (int e = 0; e < 3; e++)
+        for (int any = 0; any < 2; any++) {
+          char name[160];
+          snprintf(name, sizeof(name),
+                   "hom_gfx950_mfma_f16_s32x32x16gemm_f16_%dx%d_64x2%c%d_w%dx%d_"
+                   "nn_align%d_%s",
+                   t.tileM, t.tileN, any ? 'u' : 'r', t.depth, t.wavesM,
+                   t.wavesN, any ? 1 : 8, epiName[e]);
+          (any ? t.any : t.aligned)[e] = kernelByName(name);
+        }
+    return v;
+  }();
+  return models;
+}
+
+// Kernel and split-K for an untuned shape of alignment class cls, from a timing
+// model of the register-staged kernels, fitted to measurements of every tile
+// over BERT-base / BERT-large sized problems (it reproduces them within 10 %):
+//   t = launch + max(slabs * floor, compute + traffic) + epilogue
+// compute = 64-wide K slabs x workgroups on the fullest CU x tile area x
+// kUsPerOutputSlab (matrix cores and LDS of a CU are shared by its
+// workgroups); traffic = bytes all tiles pull from L2, tiles x (BM + BN) x K
+// x 2, at kL2BytesPerUs; floor = the load -> LDS -> MFMA latency chain of a
+// lone workgroup; the epilogue costs per output; split-K adds a second kernel
+// that moves the fp32 partial tiles through memory.
+void modelGemm(int64_t M, int64_t N, int64_t K, Epilogue epi, int cls,
+               int64_t *idx, int32_t *splitK) {
+  const int cus = deviceInfo().computeUnits > 0 ? deviceInfo().computeUnits : 256;
+  constexpr double kLaunchUs = 3.0, kReduceLaunchUs = 2.5, kInKernelSumUs = 1.0;
+  constexpr double kUsPerOutputSlab = 2.234e-5;
+  constexpr double kL2BytesPerUs = 24.0e6;
+  constexpr double kSlabFloorUs = 0.17;
+  constexpr double kReduceBytesPerUs = 3.0e6; // partial tiles, written + read
+  constexpr double kInKernelBytesPerUs = 9.0e6; // the same, staying in one L2
+  const double epiNsPerOutput = epi == Epilogue::kLinear ? 0.045 : 0.12;
+  double bestCost = 1e300;
+  *idx = findKernel(64, 64, 32, epi, 1); // (rows shorter than a vector)
+  *splitK = 1;
+  if (cls == 1 && (K < 8 || N < 8))
+    return;
+  const int slabs = int((K + 63) / 64);
+  for (const TileModel &t : tileModels()) {
+    const int kernel = (cls == 1 ? t.any : t.aligned)[int(epi)];
+    if (kernel < 0)
+      continue;
+    const int64_t tiles =
+        ((M + t.tileM - 1) / t.tileM) * ((N + t.tileN - 1) / t.tileN);
+    const double area = double(t.tileM) * t.tileN;
+    const double traffic = double(tiles) * (t.tileM + t.tileN) * double(K) *
+                           2.0 / kL2BytesPerUs;
+    const int maxSplit = std::max(1, std::min(16, int(K / 128)));
+    for (int sp = 1; sp <= maxSplit; sp++) {
+      const int perSlice = (slabs + sp - 1) / sp;
+      if (sp > 1 && perSlice < 4)
+        break;
+      const double perCu = std::ceil(double(tiles) * sp / cus);
+      const double compute = perSlice * perCu * area * kUsPerOutputSlab;
+      double cost = kLaunchUs +
+                    std::max(perSlice * kSlabFloorUs, compute + traffic) +
+                    std::ceil(double(tiles) / cus) * area * epiNsPerOutput * 1e-3;
+      if (sp > 1) {
+        // (the in-kernel sum saves most of the second launch where the
+        // launcher will take it: same conditions as launchPipe)
+        const bool inKernel = splitKInKernelMode() != 0 && tiles % 8 == 0 &&
+                              (splitKInKernelMode() != 3 ||
+                               splitKInKernelPays(t.tileM * t.tileN, sp, tiles));
+        cost += (inKernel ? kInKernelSumUs : kReduceLaunchUs) +
+                double(tiles) * sp * area * 8.0 /
+                    (inKernel ? kInKernelBytesPerUs : kReduceBytesPerUs);
+      }
+      if (cost < bestCost) {
+        bestCost = cost;
+        *idx = kernel;
+        *splitK = sp;
+      }
+    }
+  }
+}
 
 } // namespace
 
@@ -221,91 +311,7 @@ bool selectGemm(int64_t M, int64_t N, int64_t K, int64_t activation,
       return true;
     }
   }
-  // Untuned shapes: a timing model of the register-staged kernels, fitted to
-  // measurements of every tile over BERT-base / BERT-large sized problems
-  // (it reproduces them within 10 %):
-  //   t = launch + max(slabs * floor, compute + traffic) + epilogue
-  // compute = 64-wide K slabs x workgroups on the fullest CU x tile area x
-  // kUsPerOutputSlab (matrix cores and LDS of a CU are shared by its
-  // workgroups); traffic = bytes all tiles pull from L2, tiles x (BM + BN) x K
-  // x 2, at kL2BytesPerUs; floor = the load -> LDS -> MFMA latency chain of a
-  // lone workgroup; the epilogue costs per output; split-K adds a second kernel
-  // that moves the fp32 partial tiles through memory.
-  const int cls = K % 8 != 0 ? 1 : (N % 8 == 0 ? 8 : (N % 2 == 0 ? 2 : 1));
-  const int cus = deviceInfo().computeUnits > 0 ? deviceInfo().computeUnits : 256;
-  struct TileModel {
-    int tileM, tileN, wavesM, wavesN, depth;
-  };
-  static const TileModel kModels[] = {
-      {64, 64, 2, 2, 2},   {128, 64, 2, 2, 2},  {64, 128, 2, 2, 2},
-      {128, 128, 2, 4, 2}, {128, 256, 2, 4, 2}, {256, 128, 4, 2, 2},
-      {256, 256, 2, 4, 1},
-  };
-  constexpr double kLaunchUs = 3.0, kReduceLaunchUs = 2.5, kInKernelSumUs = 1.0;
-  constexpr double kUsPerOutputSlab = 2.234e-5;
-  constexpr double kL2BytesPerUs = 24.0e6;
-  constexpr double kSlabFloorUs = 0.17;
-  constexpr double kReduceBytesPerUs = 3.0e6; // partial tiles, written + read
-  constexpr double kInKernelBytesPerUs = 9.0e6; // the same, staying in one L2
-  const double epiNsPerOutput = epi == Epilogue::kLinear ? 0.045 : 0.12;
-  const char *epiName = epi == Epilogue::kLinear
-                            ? "linear"
-                            : (epi == Epilogue::kGeluErf ? "gelu" : "gelutanh");
-  double bestCost = 1e300;
-  int best = -1, bestSplit = 1;
-  if (cls != 1) {
-    const int slabs = int((K + 63) / 64);
-    for (const TileModel &t : kModels) {
-      char name[160];
-      snprintf(name, sizeof(name),
-               "hom_gfx950_mfma_f16_s32x32x16gemm_f16_%dx%d_64x2r%d_w%dx%d_nn_"
-               "align8_%s",
-               t.tileM, t.tileN, t.depth, t.wavesM, t.wavesN, epiName);
-      int idxOf = -1;
-      for (int i = 0; i < gemmKernelCount(); i++)
-        if (strcmp(gemmKernelInfo(i).name, name) == 0)
-          idxOf = i;
-      if (idxOf < 0 || !kernelFits(gemmKernelInfo(idxOf), cls))
-        continue;
-      const int64_t tiles =
-          ((M + t.tileM - 1) / t.tileM) * ((N + t.tileN - 1) / t.tileN);
-      const double area = double(t.tileM) * t.tileN;
-      const double traffic = double(tiles) * (t.tileM + t.tileN) * double(K) *
-                             2.0 / kL2BytesPerUs;
-      const int maxSplit = std::max(1, std::min(16, int(K / 128)));
-      for (int sp = 1; sp <= maxSplit; sp++) {
-        const int perSlice = (slabs + sp - 1) / sp;
-        if (sp > 1 && perSlice < 4)
-          break;
-        const double perCu = std::ceil(double(tiles) * sp / cus);
-        const double compute = perSlice * perCu * area * kUsPerOutputSlab;
-        double cost = kLaunchUs +
-                      std::max(perSlice * kSlabFloorUs, compute + traffic) +
-                      std::ceil(double(tiles) / cus) * area * epiNsPerOutput * 1e-3;
-        if (sp > 1) {
-          // (the in-kernel sum saves most of the second launch where the
-          // launcher will take it: same conditions as launchPipe)
-          const bool inKernel = splitKInKernelMode() != 0 && tiles % 8 == 0 &&
-                                (splitKInKernelMode() != 3 ||
-                                 splitKInKernelPays(t.tileM * t.tileN, sp, tiles));
-          cost += (inKernel ? kInKernelSumUs : kReduceLaunchUs) +
-                  double(tiles) * sp * area * 8.0 /
-                      (inKernel ? kInKernelBytesPerUs : kReduceBytesPerUs);
-        }
-        if (cost < bestCost) {
-          bestCost = cost;
-          best = idxOf;
-          bestSplit = sp;
-        }
-      }
-    }
-  }
-  if (best < 0) {
-    best = findKernel(64, 64, 32, epi, 1);
-    bestSplit = 1;
-  }
-  *idx = best;
-  *splitK = bestSplit;
+  modelGemm(M, N, K, epi, naturalClass(N, K), idx, splitK);
   return false;
 }
 
@@ -345,13 +351,12 @@ Status runGemmManifest(int64_t rankA, void *dstA, int64_t rankB, void *dstB,
     int64_t sel;
     int32_t sk;
     selectGemm(pr.M, pr.N, pr.K, activation, &sel, &sk);
+    const int cls = alignmentClass(pr);
+    if (!kernelFits(gemmKernelInfo(int(sel)), cls))
+      modelGemm(pr.M, pr.N, pr.K, gemmKernelInfo(int(sel)).epilogue, cls, &sel,
+                &sk);
     idx = int(sel);
     pr.splitK = sk;
-    const int cls = alignmentClass(pr);
-    if (!kernelFits(gemmKernelInfo(idx), cls)) {
-      idx = fallbackKernel(gemmKernelInfo(idx).epilogue, cls);
-      pr.splitK = 1;
-    }
     if (noAlloc) {
       // The caller did not ask for split-K: a factor the library chose itself
       // shrinks until its partial tiles fit the fixed array (1 needs none).
@@ -396,8 +401,9 @@ int chooseNvteKernel(GemmProblem *pr, int64_t activation) {
   }
   const int cls = alignmentClass(*pr);
   if (!kernelFits(gemmKernelInfo(idx), cls)) {
-    idx = fallbackKernel(epi, cls);
-    pr->splitK = 1;
+    modelGemm(pr->M, pr->N, pr->K, epi, cls, &sel, &sk);
+    idx = int(sel);
+    pr->splitK = sk;
   }
   return idx;
 }
@@ -724,7 +730,7 @@ void GemmProfiler::sweep(bool bIsNK, int64_t *bestIdx, int32_t *bestSplit,
   // Alignment class (the reference walks {8,4,2,1} over M, N, K:
   // lib/NVGPUKernels/GemmProfiler.cu:170-180; here K must be a multiple of 8
   // for the vector kernels, N of 8 or 2, and the row count is free).
-  const int cls = K_ % 8 != 0 ? 1 : (N_ % 8 == 0 ? 8 : (N_ % 2 == 0 ? 2 : 1));
+  const int cls = naturalClass(N_, K_);
   const int maxSplit = std::max(1, std::min<int>(16, int(K_ / 128)));
   const int cus = deviceInfo().computeUnits > 0 ? deviceInfo().computeUnits : 256;
   for (int idx = 0; idx < gemmKernelCount(); idx++) {

@@ -129,3 +129,39 @@ def test_results_kept_by_the_caller_stay_apart(synth):
         np.testing.assert_array_equal(a, c)
     enc.close()
     np.testing.assert_array_equal(again, copies[0])  # outlives the encoder
+
+
+# the any-alignment GEMM tiles: K and N around whole slabs, vectors and tiles, remainders that a shifted last vector
+# serves, split-K whose last slice is all remainder, and operands that start at odd elements
+@pytest.mark.parametrize("tile", ["64x64_64x2u2_w2x2", "128x128_64x2u2_w2x4", "256x256_64x2u1_w2x4"])
+@pytest.mark.parametrize("M,N,K", [(5, 9, 8), (64, 65, 9), (70, 127, 63), (130, 71, 64), (65, 1001, 65), (33, 64, 127),
+                                   (257, 259, 128), (100, 513, 129), (3, 8, 200), (260, 77, 321)])
+def test_gemm_any_alignment(gpu, rt, oracle, tile, M, N, K):
+    g = np.random.default_rng(M + N + K)
+    num = {n.rsplit("_", 1)[1]: i + 1 for i, n, _, _ in rt.manifest() if f"_{tile}_" in n}
+    A, B = g.standard_normal((1, M, K)).astype(np.float16), (g.standard_normal((1, K, N)) * 0.1).astype(np.float16)
+    R, bias = g.standard_normal((1, M, N)).astype(np.float16), g.standard_normal((1, 1, N)).astype(np.float16)
+    Mr = rt.MemRef.from_tensor
+
+    def odd(a):  # on the device, one element off any alignment
+        t = torch.zeros(a.size + 1, dtype=torch.float16, device="cuda")[1:].view(a.shape)
+        t.copy_(torch.from_numpy(a))
+        return t
+
+    for place in (dev, odd):
+        ta, tb, tr, tbias = place(A), place(B), place(R), place(bias)
+        for sk in (1, 2, 5):
+            td = place(np.zeros((1, M, N), np.float16))
+            gpu.cutlassGemmF16(*Mr(ta).args(), False, *Mr(tb).args(), False, *Mr(tr).args(), *Mr(td).args(), 0, 1.0,
+                               0.5, num["linear"], sk)
+            want = oracle.gemm(A[0], B[0], R[0], beta=0.5)
+            np.testing.assert_allclose(host(td)[0].astype(np.float64), want, rtol=1e-3, atol=1e-2)
+            gpu.cutlassGemmF16(*Mr(ta).args(), False, *Mr(tb).args(), False, *Mr(tbias).args(), *Mr(td).args(), 0, 1.0,
+                               1.0, num["gelu"], sk)
+            want = oracle.gemm(A[0], B[0], bias[0], beta=1.0, act="gelu_erf")
+            np.testing.assert_allclose(host(td)[0].astype(np.float64), want, rtol=1e-3, atol=1e-2)
+    # [N, K] weights, the library's own choice
+    Bt = np.ascontiguousarray(B[0].T)[None]
+    tb, td = odd(Bt), odd(np.zeros((1, M, N), np.float16))
+    gpu.nvteGemmF16(*Mr(odd(A)).args(), False, *Mr(tb).args(), True, *Mr(td).args(), *Mr(td).args(), 0, 1.0, 0.0, 0, 0)
+    np.testing.assert_allclose(host(td)[0].astype(np.float64), oracle.gemm(A[0], B[0]), rtol=1e-3, atol=1e-2)
