@@ -85,7 +85,7 @@ __global__ __launch_bounds__(NW *kWave)
 __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1, D == 64 && KS == 1 ? 4 : (D <= 128 ? 2 : 1)))) void bertAttentionKernel(
     const _Float16 *__restrict__ qkv, const int32_t *__restrict__ cu,
     _Float16 *__restrict__ out, int seq, int heads, int numQTiles, int pairs,
-    float scale) {
+    float scale, int packedOut) {
   static_assert(D == 64 || D == 128 || D == 192 || D == 256, "head size");
   static_assert(D <= 128 || KS == 1, "the key-split variant stages 128 keys per chunk");
   constexpr int kChunk = Chunk<D>::value;
@@ -142,6 +142,11 @@ __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1, D == 64 && KS == 1 ? 4 : (D 
   const _Float16 *vBase = base + (2 * heads + head) * kHeadDim;
   const int64_t outStride = int64_t(heads) * kHeadDim;
   _Float16 *oBase = out + int64_t(b) * seq * outStride + head * kHeadDim;
+  // 4 output columns from column c of query q (packedOut: fragment order)
+  auto outAt = [&](int q, int c) {
+    return packedOut ? out + packedOffset(int64_t(b) * seq + q, head * kHeadDim + c, outStride)
+                     : oBase + int64_t(q) * outStride + c;
+  };
 
   // Key-split variant (short sequences, few workgroups: latency is what
   // counts): K and V rows of a 128-key chunk travel global -> registers -> LDS,
@@ -198,8 +203,7 @@ __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1, D == 64 && KS == 1 ? 4 : (D 
         z[e] = _Float16(0);
 #pragma unroll
       for (int c = 0; c < CPR; c++)
-        *reinterpret_cast<half4 *>(oBase + int64_t(q) * outStride + c * 8 +
-                                   hb * 4) = z;
+        *reinterpret_cast<half4 *>(outAt(q, c * 8 + hb * 4)) = z;
     }
     return;
   }
@@ -517,8 +521,7 @@ __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1, D == 64 && KS == 1 ? 4 : (D 
 #pragma unroll
         for (int e = 0; e < 4; e++)
           o[e] = valid ? _Float16(accO[d][g * 4 + e] * inv) : _Float16(0);
-        *reinterpret_cast<half4 *>(oBase + int64_t(q) * outStride + d * 32 +
-                                   g * 8 + hb * 4) = o;
+        *reinterpret_cast<half4 *>(outAt(q, d * 32 + g * 8 + hb * 4)) = o;
       }
   }
 }
@@ -528,7 +531,7 @@ __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1, D == 64 && KS == 1 ? 4 : (D 
 Status launchBertAttentionF16(const _Float16 *qkv, const int32_t *cuSeqlens,
                               _Float16 *out, int64_t bs, int64_t seq,
                               int64_t heads, int64_t headDim, float scale,
-                              hipStream_t s) {
+                              hipStream_t s, bool packedOut) {
   // (the reference's contract is head size % 64 == 0, README.md:11; the
   // sizes with kernels here are 64, 128, 192 and 256)
   HOM_CHECK_RET(headDim == 64 || headDim == 128 || headDim == 192 || headDim == 256,
@@ -568,16 +571,20 @@ Status launchBertAttentionF16(const _Float16 *qkv, const int32_t *cuSeqlens,
     const dim3 grid((unsigned)(nq * pairs));
     if (headDim == 64)
       bertAttentionKernel<4, 1, 64><<<grid, dim3(256), 0, s>>>(
-          qkv, cuSeqlens, out, int(seq), int(heads), nq, int(pairs), scale);
+          qkv, cuSeqlens, out, int(seq), int(heads), nq, int(pairs), scale,
+          packedOut);
     else if (headDim == 128)
       bertAttentionKernel<4, 1, 128><<<grid, dim3(256), 0, s>>>(
-          qkv, cuSeqlens, out, int(seq), int(heads), nq, int(pairs), scale);
+          qkv, cuSeqlens, out, int(seq), int(heads), nq, int(pairs), scale,
+          packedOut);
     else if (headDim == 192)
       bertAttentionKernel<4, 1, 192><<<grid, dim3(256), 0, s>>>(
-          qkv, cuSeqlens, out, int(seq), int(heads), nq, int(pairs), scale);
+          qkv, cuSeqlens, out, int(seq), int(heads), nq, int(pairs), scale,
+          packedOut);
     else
       bertAttentionKernel<4, 1, 256><<<grid, dim3(256), 0, s>>>(
-          qkv, cuSeqlens, out, int(seq), int(heads), nq, int(pairs), scale);
+          qkv, cuSeqlens, out, int(seq), int(heads), nq, int(pairs), scale,
+          packedOut);
   } else {
     const int nq = int((seq + 63) / 64);
     HOM_CHECK_RET(heads < 65536 && bs < 65536, Status::kInvalidArgument,
@@ -585,10 +592,12 @@ Status launchBertAttentionF16(const _Float16 *qkv, const int32_t *cuSeqlens,
     const dim3 grid((unsigned)nq, (unsigned)heads, (unsigned)bs);
     if (headDim == 64)
       bertAttentionKernel<4, 2, 64><<<grid, dim3(256), 0, s>>>(
-          qkv, cuSeqlens, out, int(seq), int(heads), nq, int(pairs), scale);
+          qkv, cuSeqlens, out, int(seq), int(heads), nq, int(pairs), scale,
+          packedOut);
     else
       bertAttentionKernel<4, 2, 128><<<grid, dim3(256), 0, s>>>(
-          qkv, cuSeqlens, out, int(seq), int(heads), nq, int(pairs), scale);
+          qkv, cuSeqlens, out, int(seq), int(heads), nq, int(pairs), scale,
+          packedOut);
   }
   HOM_HIP_RET(hipGetLastError(), Status::kInternal);
   return Status::kSuccess;

@@ -95,6 +95,16 @@ struct HomBertEncoder {
   std::vector<float *> colSumQkv, colSumW1;
   float *rowSums[2] = {nullptr, nullptr};
   int32_t foldPieces = 0;
+  // Few rows (usesPacked): every layer GEMM runs on weights in fragment order,
+  // with the layer norms folded into the GEMMs around them.  One arena holds
+  // the packed weights in the order the forward reads them, one the column
+  // sums of Wqkv and W1; both are made from the uploaded weights before the
+  // next forward or capture (packWeights).
+  bool packed = false, packedReady = false;
+  char *packedArena = nullptr;
+  float *packedColSums = nullptr;
+  float *packedStats[2] = {nullptr, nullptr}; // rows of h entering QKV / FFN1
+  Tensor hPacked, attnPacked, fPacked;        // activations in fragment order
   hipStream_t stream = nullptr;
   hipGraph_t graph = nullptr;
   hipGraphExec_t graphExec = nullptr;
@@ -269,18 +279,138 @@ bool chooseGemm(HomBertEncoder *e, int64_t M, int64_t N, int64_t K, int64_t act,
   return true;
 }
 
+// The packed form serves few rows: beyond them a workgroup of the tiled
+// kernels, which shares operands through LDS, reads less per output.  us per
+// request, tiled -> packed: BERT-base with 64 rows 494 -> 296, 256 rows 515 ->
+// 403, 512 rows 630 -> 513, 768 rows 688 -> 650, 1024 rows 691 -> 769;
+// BERT-large with 16 rows 1006 -> 542, 256 rows 1106 -> 1061, 512 rows 1378 ->
+// 1527.  The line between them moves with the cube of the hidden size.
+bool usesPacked(const HomBertEncoder *e) {
+  const int64_t M = int64_t(e->batch) * e->seq;
+  bool pinned = false;
+  for (int r = 0; r < 4; r++)
+    pinned = pinned || e->roleLayout[r] != -1;
+  const double H = e->hidden;
+  return double(M) * H * H * H <= 3.7e11 && e->gemmMode == 1 && !pinned &&
+         e->hidden % 32 == 0 && e->ffn % 32 == 0 && e->hidden <= 2048;
+}
+
+struct PackedLayer { // byte offsets into the arena
+  int64_t qkv, out, ffn1, ffn2, end;
+};
+PackedLayer packedLayer(const HomBertEncoder *e, int l) {
+  const int64_t H = e->hidden, F = e->ffn;
+  PackedLayer p;
+  p.qkv = int64_t(l) * (4 * H * H + 2 * H * F) * 2;
+  p.out = p.qkv + 3 * H * H * 2;
+  p.ffn1 = p.out + H * H * 2;
+  p.ffn2 = p.ffn1 + H * F * 2;
+  p.end = p.ffn2 + H * F * 2;
+  return p;
+}
+float *packedColSum(const HomBertEncoder *e, int l, bool ffn1) {
+  return e->packedColSums + int64_t(l) * (3 * e->hidden + e->ffn) +
+         (ffn1 ? 3 * e->hidden : 0);
+}
+
+bool packWeights(HomBertEncoder *e) {
+  if (!e->packed || e->packedReady)
+    return true;
+  const int64_t H = e->hidden, F = e->ffn;
+  const int rows = (e->batch * e->seq + 15) / 16 * 16;
+  if (!e->packedArena) {
+    const size_t bytes = size_t(packedLayer(e, e->layers).qkv);
+    if (!hipOk(hipMalloc(reinterpret_cast<void **>(&e->packedArena), bytes), "hipMalloc") ||
+        !hipOk(hipMalloc(reinterpret_cast<void **>(&e->packedColSums),
+                         size_t(e->layers) * size_t(3 * H + F) * 4),
+               "hipMalloc"))
+      return false;
+    for (float *&q : e->packedStats)
+      if (!hipOk(hipMalloc(reinterpret_cast<void **>(&q), size_t(rows) * 8), "hipMalloc"))
+        return false;
+    // (the logical shape is [batch, seq, .]: the padding rows lie behind it)
+    auto padded = [&](Tensor &t, int cols) {
+      t.m = alloc3DMemRefNVGPUF16(1, rows, cols);
+      int64_t *sz = hom_memref_sizes(t.m.descriptor);
+      int64_t *st = hom_memref_strides(t.m.descriptor, 3);
+      sz[0] = e->batch;
+      sz[1] = e->seq;
+      st[0] = int64_t(e->seq) * cols;
+    };
+    padded(e->hPacked, int(H));
+    padded(e->attnPacked, int(H));
+    padded(e->fPacked, int(F));
+  }
+  void *prev = homGetStream();
+  homSetStream(e->stream);
+  for (int l = 0; l < e->layers; l++) {
+    const LayerWeights &w = e->w[size_t(l)];
+    const PackedLayer at = packedLayer(e, l);
+    homPackWeightF16(w.wqkv.m.rank, w.wqkv.m.descriptor, e->packedArena + at.qkv);
+    homPackWeightF16(w.wo.m.rank, w.wo.m.descriptor, e->packedArena + at.out);
+    homPackWeightF16(w.w1.m.rank, w.w1.m.descriptor, e->packedArena + at.ffn1);
+    homPackWeightF16(w.w2.m.rank, w.w2.m.descriptor, e->packedArena + at.ffn2);
+    homColumnSumsF16(w.wqkv.m.rank, w.wqkv.m.descriptor, packedColSum(e, l, false));
+    homColumnSumsF16(w.w1.m.rank, w.w1.m.descriptor, packedColSum(e, l, true));
+  }
+  homSetStream(prev);
+  e->packedReady = true;
+  return true;
+}
+
+// The layers on packed weights: 5 launches each.  h travels un-normalised
+// between the GEMMs that add to it (out-projection, FFN2); QKV and FFN1
+// normalise it on the way in and leave its row statistics for the residual of
+// the GEMM after next.
+void packedLayers(HomBertEncoder *e, int64_t geluAct, float scale) {
+  const int kAll = HOM_PACKED_A | HOM_PACKED_C | HOM_PACKED_D;
+  auto gemm = [&](const Tensor &a, int64_t weight, const Tensor *c, const Tensor &d, int64_t act,
+                  bool norm, const float *colSum, const float *statsIn, float *statsOut,
+                  int packing, int64_t ahead, int64_t aheadEnd) {
+    homPackedGemmF16(a.m.rank, a.m.descriptor, e->packedArena + weight, c ? c->m.rank : 0,
+                     c ? c->m.descriptor : nullptr, d.m.rank, d.m.descriptor, act, norm, e->eps,
+                     colSum, statsIn, statsOut, packing,
+                     e->packedArena + ahead, aheadEnd - ahead);
+  };
+  for (int l = 0; l < e->layers; l++) {
+    const PackedLayer at = packedLayer(e, l);
+    const bool last = l + 1 == e->layers;
+    // (the embeddings arrive normalised)
+    const bool norm = l > 0;
+    gemm(e->hPacked, at.qkv, nullptr, e->qkv, 0, norm, norm ? packedColSum(e, l, false) : nullptr,
+         nullptr, norm ? e->packedStats[0] : nullptr, HOM_PACKED_A, at.out, at.ffn1);
+    homBertAttentionF16(e->qkv.m.rank, e->qkv.m.descriptor, e->cu.m.rank, e->cu.m.descriptor,
+                        e->attnPacked.m.rank, e->attnPacked.m.descriptor, scale, e->heads,
+                        HOM_PACKED_D);
+    gemm(e->attnPacked, at.out, &e->hPacked, e->hPacked, 0, false, nullptr,
+         norm ? e->packedStats[0] : nullptr, nullptr, kAll, at.ffn1, at.ffn2);
+    gemm(e->hPacked, at.ffn1, nullptr, e->fPacked, geluAct, true, packedColSum(e, l, true), nullptr,
+         e->packedStats[1], HOM_PACKED_A | HOM_PACKED_D, at.ffn2, at.end);
+    gemm(e->fPacked, at.ffn2, &e->hPacked, last ? e->h : e->hPacked, 0, false, nullptr,
+         e->packedStats[1], nullptr, last ? HOM_PACKED_A | HOM_PACKED_C : kAll, at.end,
+         last ? at.end : at.end + (at.out - at.qkv));
+  }
+  nvteLayernormF16(e->h.m.rank, e->h.m.descriptor, e->eps);
+}
+
 void callList(HomBertEncoder *e, int fromIds) {
+  // (a forward from given hidden states has them row-major in h)
+  const bool packed = e->packed && fromIds;
+  const Tensor &front = packed ? e->hPacked : e->h;
   if (fromIds)
     homEmbedF16(e->ids.m.rank, e->ids.m.descriptor, e->mask.m.rank,
                 e->mask.m.descriptor, e->wordEmb.m.rank, e->wordEmb.m.descriptor,
-                e->posType.m.rank, e->posType.m.descriptor, e->h.m.rank,
-                e->h.m.descriptor, e->cu.m.rank, e->cu.m.descriptor, e->eps);
+                e->posType.m.rank, e->posType.m.descriptor, front.m.rank,
+                front.m.descriptor, e->cu.m.rank, e->cu.m.descriptor, e->eps,
+                packed ? HOM_PACKED_D : 0);
   else
     thrustCuSeqLenI64(e->mask.m.rank, e->mask.m.descriptor, e->cu.m.rank,
                       e->cu.m.descriptor);
   const float scale = 1.0f / sqrtf(float(e->hidden / e->heads));
   const int64_t geluAct = e->gemmMode == 0 ? 1 : (e->geluForm == 1 ? 2 : 1);
-  if (e->foldLn) {
+  if (packed) {
+    packedLayers(e, geluAct, scale);
+  } else if (e->foldLn) {
     // The same graph with the two layer norms of every layer folded into the
     // GEMMs around them: the residual GEMMs (out-projection, FFN2) leave the
     // un-normalised sum in h together with the partial row sums of it, and
@@ -367,6 +497,10 @@ homBertCreateWithLayout(int layers, int hidden, int heads, int ffn, int batch,
     // a bad pin fails at creation, not at homBertEnableLmHead
     const bool transformOk =
         !(e->roleLayout[4] == 1 && geluForm == 0 && gemmMode != 0);
+    // Row-major weights for the packed form to start from.
+    e->packed = usesPacked(e);
+    for (int r = 0; r < 4 && e->packed; r++)
+      e->roleLayout[r] = 0;
     if (!chooseGemm(e, M, 3 * hidden, hidden, 0, 0.0f, e->roleLayout[0], &e->cQkv) ||
         !chooseGemm(e, M, hidden, hidden, 0, 1.0f, e->roleLayout[1], &e->cOut) ||
         !chooseGemm(e, M, ffn, hidden, gelu, 0.0f, e->roleLayout[2], &e->cFfn1) ||
@@ -500,6 +634,7 @@ DRV_EXPORT int homBertFoldLayernorm(HomBertEncoder *e) {
   if (!ok)
     return -1;
   e->foldPieces = pOut;
+  e->packed = false;
   e->foldLn = true;
   return 0;
 }
@@ -536,6 +671,13 @@ DRV_EXPORT void homBertDestroy(HomBertEncoder *e) {
   for (Tensor *t : {&e->wordEmb, &e->posType, &e->cu, &e->h, &e->qkv, &e->attn,
                     &e->f, &e->wTransform, &e->wDecoder, &e->t, &e->logits})
     t->release();
+  e->hPacked.release();
+  e->attnPacked.release();
+  e->fPacked.release();
+  (void)hipFree(e->packedArena);
+  (void)hipFree(e->packedColSums);
+  for (float *q : e->packedStats)
+    (void)hipFree(q);
   releasePinned(e->ids);
   releasePinned(e->mask);
   pinnedPool().dropUser();
@@ -549,6 +691,7 @@ DRV_EXPORT void homBertDestroy(HomBertEncoder *e) {
 DRV_EXPORT int homBertUpload(HomBertEncoder *e, int layer, int which,
                              const void *host, int64_t numel) {
   Tensor *t = nullptr;
+  e->packedReady = false;
   if (which <= 3) {
     if (layer < 0 || layer >= e->layers)
       return -1;
@@ -602,7 +745,8 @@ DRV_EXPORT void homBertForward(HomBertEncoder *e, int fromIds) {
   void *prev = homGetStream();
   homSetStream(e->stream);
   e->inFlight = true;
-  callList(e, fromIds);
+  if (packWeights(e))
+    callList(e, fromIds);
   homSetStream(prev);
 }
 
@@ -638,7 +782,7 @@ DRV_EXPORT int homBertCapture(HomBertEncoder *e, int fromIds) {
 }
 
 DRV_EXPORT int homBertReplay(HomBertEncoder *e) {
-  if (!e->graphExec)
+  if (!e->graphExec || !packWeights(e)) // (weights uploaded since the capture)
     return -1;
   e->inFlight = true;
   return hipOk(hipGraphLaunch(e->graphExec, e->stream), "hipGraphLaunch") ? 0
@@ -741,6 +885,7 @@ DRV_EXPORT int homBertSetGemmChoice(HomBertEncoder *e, int role,
     return -2; // the role's weight is [N, K]: it runs through nvteGemmF16
   c[role]->gemmNum = gemmNum;
   c[role]->splitK = splitK;
+  e->packed = false; // a pinned kernel is what runs
   return 0;
 }
 

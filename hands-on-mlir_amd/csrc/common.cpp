@@ -121,7 +121,10 @@ void *libraryScratch(ScratchSlot slot, size_t bytes, bool zero) {
     g_scratchGeneration++;
   }
   if (zero) {
+    // (the memset may still be running when the call returns, and a stream
+    // that does not synchronise with the null stream would overtake it)
     HOM_HIP_RET(hipMemset(p, 0, want), nullptr);
+    HOM_HIP_RET(hipStreamSynchronize(nullptr), nullptr);
   }
   b.ptr = p;
   b.bytes = want;

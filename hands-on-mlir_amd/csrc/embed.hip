@@ -32,7 +32,7 @@ __global__ __launch_bounds__(kThreads) void embedKernel(
     const int64_t *__restrict__ ids, const int64_t *__restrict__ mask,
     const _Float16 *__restrict__ word, const _Float16 *__restrict__ pos,
     _Float16 *__restrict__ out, int32_t *__restrict__ cu, int bs, int seq,
-    int hidden, int vocab, uint32_t seqMagic, float eps) {
+    int hidden, int vocab, uint32_t seqMagic, float eps, bool packedOut) {
   __shared__ int32_t rowSum[256];
   const int lane = threadIdx.x % kWave;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
@@ -97,7 +97,10 @@ __global__ __launch_bounds__(kThreads) void embedKernel(
       for (int e = 0; e < 8; e++)
         o[e] = _Float16((v[i][e] - mean) * rstd);
       if (row0 + r < rows && lane + i * kWave < nvec)
-        storeWriteThrough(out + int64_t(row0 + r) * hidden + (lane + i * kWave) * 8, o);
+        storeWriteThrough(
+            out + (packedOut ? packedOffset(row0 + r, (lane + i * kWave) * 8, hidden)
+                             : int64_t(row0 + r) * hidden + (lane + i * kWave) * 8),
+            o);
     }
   }
 }
@@ -115,7 +118,7 @@ bool embedFits(const _Float16 *word, const _Float16 *pos, const _Float16 *out,
 Status launchEmbed(const int64_t *ids, const int64_t *mask, const _Float16 *word,
                    const _Float16 *pos, _Float16 *out, int32_t *cu, int64_t bs,
                    int64_t seq, int64_t hidden, int64_t vocab, float eps,
-                   hipStream_t s) {
+                   bool packedOut, hipStream_t s) {
   const int64_t rows = bs * seq, perBlock = kWaves * kRows;
   const dim3 grid((unsigned)(1 + (rows + perBlock - 1) / perBlock)), block(kThreads);
   const uint32_t magic = magicFor(uint32_t(seq));
@@ -124,7 +127,7 @@ Status launchEmbed(const int64_t *ids, const int64_t *mask, const _Float16 *word
                 : nvec <= 2 * kWave ? embedKernel<2>
                                     : embedKernel<4>;
   kernel<<<grid, block, 0, s>>>(ids, mask, word, pos, out, cu, int(bs), int(seq),
-                                int(hidden), int(vocab), magic, eps);
+                                int(hidden), int(vocab), magic, eps, packedOut);
   HOM_HIP_RET(hipGetLastError(), Status::kInternal);
   return Status::kSuccess;
 }

@@ -1,0 +1,423 @@
+// GEMMs of a few dozen to a few hundred rows against weights laid out for them.
+//
+//   D = act(A . B) or act(LN(A) . B), linear results also + C or + LN(C)
+//
+// At these sizes a GEMM is a weight matrix passing once through the chip and a
+// chain of latencies: launch, first load, K loop, epilogue.  The tiled kernels
+// (gemm_pipe.h) walk K in slabs of 64 through LDS, 12 to 48 barriers one after
+// the other; here the wavefronts of a workgroup split K between them, every
+// wavefront requests all of its operands at once, straight into registers in
+// the layout the MFMA takes them, and the partial sums meet in LDS once:
+//   - B is packed when it is loaded: the fragment of 16 columns x 32 k that one
+//     v_mfma_f32_16x16x32_f16 takes is 1 KiB in lane order, so a wavefront
+//     streams its part of B with fully coalesced 16-byte loads, no LDS and no
+//     transposition;
+//   - A may come in the same order (packedOffset() in kernels.h), which is how
+//     these kernels, the attention and the embedding kernel can leave their
+//     results; from a row-major A a fragment load touches 16 half-used lines.
+// A layer norm without affine parameters in front of the GEMM costs no kernel:
+// the wavefronts have whole rows of A in registers between them, so they form
+// sum and sum of squares on the way and the epilogue applies
+//   LN(A) . B = rstd (A . B) - mu rstd colsum(B)
+// with colsum(B) from packing time; the statistics are written for the later
+// GEMM whose residual source is the same tensor, LN(C) = rstd c - mu rstd.
+#include "cross_lane.h"
+#include "fast_div.h"
+#include "kernels.h"
+#include "store_policy.h"
+
+#include <algorithm>
+
+namespace hom {
+namespace {
+
+typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+typedef _Float16 half4 __attribute__((ext_vector_type(4)));
+typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+typedef float float4v __attribute__((ext_vector_type(4)));
+typedef float float2v __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+constexpr int kWave = 64, kWaves = 8, kThreads = kWave * kWaves;
+constexpr uint32_t kOob = 0x80000000u;
+
+// GELU as the tiled kernels' epilogues compute it (gemm_device.h).
+__device__ __forceinline__ float geluErf(float x) {
+  const float ax = fabsf(x);
+  const float a = fminf(ax, 8.0f);
+  float P = fmaf(3.448796997e-05f, a, -7.812886615e-04f);
+  P = fmaf(P, a, 8.119936101e-03f);
+  P = fmaf(P, a, -5.347220227e-02f);
+  P = fmaf(P, a, -4.587264359e-01f);
+  P = fmaf(P, a, -1.151216269e+00f);
+  P = fmaf(P, a, 8.451195754e-06f);
+  return fmaf(-0.5f * ax, __builtin_amdgcn_exp2f(P), fmaxf(x, 0.0f));
+}
+__device__ __forceinline__ float geluTanh(float x) {
+  const float w = fmaf(x * x, -0.1029432397f, -2.3022081983f);
+  return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x * w));
+}
+
+struct PackedArgs {
+  const _Float16 *C; // residual source [M, N] or null
+  _Float16 *D;
+  const float *colSum;  // [N], read when A is normalised
+  const float *statsIn; // (rstd, -mu rstd) per row of C, or null: C as it is
+  float *statsOut;      // (rstd, -mu rstd) per row of A, or null
+  const char *ahead;    // weights of the kernels behind this one
+  int64_t aheadBytes;
+  int M, N;
+  int activation; // 0, 1 erf GELU, 2 tanh GELU
+  int cPacked, dPacked; // in fragment order
+  float invK, eps;
+};
+
+// MB x NB blocks of 16 x 16 per workgroup; CH k steps of a wavefront in flight
+// at once (ONCE: that is all of them).  The leading scalars arrive
+// in registers with the wavefront (kernel-argument preload, see the Makefile),
+// so the operands are requested before anything is fetched; `rest` is read
+// behind those requests.
+template <int MB, int NB, int CH, bool ONCE, bool NORM_A, bool A_PACKED>
+__global__ __launch_bounds__(kThreads, (MB + NB) * CH <= 20 && (ONCE || !NORM_A) ? 4 : 2) void packedGemmKernel(
+    const _Float16 *A, const _Float16 *B, int M, int K, int steps, int perWave,
+    int tilesM, int tilesN, uint32_t tilesMMagic, int tiles, PackedArgs rest) {
+  (void)rest; // (through the argument pointer, see below)
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const int tid = threadIdx.x, lane = tid % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int id = blockIdx.x;
+  // Tiles of one column block lie on one XCD (ids 8 apart), whose L2 then
+  // fetches that part of B once.
+  int tileM, tileN;
+  if (tilesN % 8 == 0) {
+    const int loc = id / 8;
+    const int q = int(divByMagic(uint32_t(loc), uint32_t(tilesM), tilesMMagic));
+    tileM = loc - q * tilesM;
+    tileN = q * 8 + id % 8;
+  } else {
+    tileN = int(divByMagic(uint32_t(id), uint32_t(tilesM), tilesMMagic));
+    tileM = id - tileN * tilesM;
+  }
+  const int m0 = tileM * (MB * 16), n0 = tileN * (NB * 16);
+  const int stepBegin = wave * perWave;
+  const int stepEnd = stepBegin + perWave < steps ? stepBegin + perWave : steps;
+  auto clampBytes = [](int64_t b) -> int32_t {
+    return b > 0x7fffffffLL ? 0x7fffffff : (b < 0 ? 0 : int32_t(b));
+  };
+  const bool isTile = id < tiles;
+  const auto rsrcA = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<_Float16 *>(A) + int64_t(m0) * K, 0,
+      isTile ? clampBytes(int64_t(A_PACKED ? (M - m0 + 15) / 16 * 16 : M - m0) * K * 2) : 0,
+      0x00020000);
+  const auto rsrcB = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<_Float16 *>(B) + int64_t(n0) * K, 0, isTile ? NB * 16 * K * 2 : 0,
+      0x00020000);
+  const uint32_t aLane = A_PACKED ? uint32_t(lane) * 16u
+                                  : (uint32_t(lane % 16) * uint32_t(K) + uint32_t(lane / 16) * 8u) * 2u;
+  const uint32_t aStep = A_PACKED ? 1024u : 64u;
+  const uint32_t aBlock = 16u * uint32_t(K) * 2u;
+  const uint32_t bBlock = uint32_t(steps) * 1024u;
+  half8 fa[CH][MB], fb[CH][NB];
+  // (steps past the wavefront's last one: an offset outside the descriptors
+  // reads as zero without touching memory)
+  auto request = [&](int s0) {
+#pragma unroll
+    for (int c = 0; c < CH; c++) {
+      const bool in = s0 + c < stepEnd;
+      const uint32_t step = uint32_t(s0 + c);
+#pragma unroll
+      for (int j = 0; j < NB; j++)
+        fb[c][j] = __builtin_bit_cast(
+            half8, __builtin_amdgcn_raw_buffer_load_b128(
+                       rsrcB, in ? uint32_t(lane) * 16u + step * 1024u + uint32_t(j) * bBlock : kOob, 0, 0));
+#pragma unroll
+      for (int i = 0; i < MB; i++)
+        fa[c][i] = __builtin_bit_cast(
+            half8, __builtin_amdgcn_raw_buffer_load_b128(
+                       rsrcA, in ? aLane + step * aStep + uint32_t(i) * aBlock : kOob, 0, 0));
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  request(stepBegin);
+  PackedArgs p = {};
+#if defined(__HIP_DEVICE_COMPILE__) // (the host pass only needs the kernel's stub)
+  {
+    typedef const __attribute__((address_space(4))) PackedArgs *RestPtr;
+    constexpr int kRestOffset = 2 * 8 + 8 * 4; // bytes of the leading arguments
+    static_assert(kRestOffset % alignof(PackedArgs) == 0, "argument layout");
+    RestPtr late = (RestPtr)((const __attribute__((address_space(4))) char *)
+                                 __builtin_amdgcn_kernarg_segment_ptr() +
+                             kRestOffset);
+    asm volatile("" : "+s"(late));
+    p = *late;
+  }
+#endif
+  if (!isTile) {
+    // Workgroups behind the tiles read weights that the next kernels need, so
+    // that those find them in the last-level cache: a lone small GEMM leaves
+    // CUs and most of the memory system idle.
+    constexpr int kLoads = 8;
+    const int64_t step = int64_t(gridDim.x - tiles) * (kThreads * 16 * kLoads);
+    for (int64_t at = int64_t(id - tiles) * (kThreads * 16 * kLoads); at < p.aheadBytes;
+         at += step) {
+      u32x4 v[kLoads];
+#pragma unroll
+      for (int i = 0; i < kLoads; i++) {
+        const int64_t o = at + (i * kThreads + tid) * 16;
+        v[i] = *reinterpret_cast<const u32x4 *>(p.ahead + (o < p.aheadBytes ? o : 0));
+      }
+#pragma unroll
+      for (int i = 0; i < kLoads; i++)
+        asm volatile("" ::"v"(v[i])); // (nothing else uses the values)
+    }
+    return;
+  }
+  // What the epilogue reads: thread t < MB * NB * 64 finishes 4 consecutive
+  // columns of one row.
+  constexpr int kOutThreads = MB * NB * kWave;
+  const int outBlock = tid / kWave; // (mb, nb) = (outBlock / NB, outBlock % NB)
+  const int m = m0 + (outBlock / NB) * 16 + lane % 16;
+  const int n = n0 + (outBlock % NB) * 16 + (lane / 16) * 4;
+  const bool mine = tid < kOutThreads && m < p.M;
+  const int64_t plain = int64_t(m) * p.N + n, packed = packedOffset(m, n, p.N);
+  half4 cv = {};
+  float2v cStat{1.f, 0.f};
+  float4v cSum = {};
+  if (mine) {
+    if (p.C)
+      cv = *reinterpret_cast<const half4 *>(p.C + (p.cPacked ? packed : plain));
+    if (p.statsIn)
+      cStat = *reinterpret_cast<const float2v *>(p.statsIn + int64_t(m) * 2);
+    if (NORM_A)
+      cSum = *reinterpret_cast<const float4v *>(p.colSum + n);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+
+  float4v acc[MB][NB];
+#pragma unroll
+  for (int i = 0; i < MB; i++)
+#pragma unroll
+    for (int j = 0; j < NB; j++)
+      acc[i][j] = float4v{0.f, 0.f, 0.f, 0.f};
+  float sum[MB], sq[MB];
+#pragma unroll
+  for (int i = 0; i < MB; i++)
+    sum[i] = sq[i] = 0.f;
+  for (int s0 = stepBegin;;) {
+#pragma unroll
+    for (int c = 0; c < CH; c++) {
+#pragma unroll
+      for (int i = 0; i < MB; i++) {
+        if (NORM_A) {
+          const half2v one = {_Float16(1), _Float16(1)};
+#pragma unroll
+          for (int e = 0; e < 4; e++) {
+            const half2v x = {fa[c][i][2 * e], fa[c][i][2 * e + 1]};
+            sum[i] = __builtin_amdgcn_fdot2(x, one, sum[i], false);
+            sq[i] = __builtin_amdgcn_fdot2(x, x, sq[i], false);
+          }
+        }
+#pragma unroll
+        for (int j = 0; j < NB; j++)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fb[c][j], fa[c][i], acc[i][j], 0, 0, 0);
+        // (in the order of arrival: reordered, the operands of several steps
+        // get second copies and the workgroup no longer fits a CU twice)
+        if (NORM_A)
+          __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    if constexpr (ONCE)
+      break;
+    s0 += CH;
+    if (s0 >= stepEnd)
+      break;
+    request(s0);
+  }
+
+  // The wavefronts' partial sums meet: [wave][block][lane] and, of the row
+  // statistics, [wave][row].
+  float4v *part = reinterpret_cast<float4v *>(smem);
+  float2v *stat = reinterpret_cast<float2v *>(smem + kWaves * MB * NB * kWave * 16);
+#pragma unroll
+  for (int i = 0; i < MB; i++) {
+#pragma unroll
+    for (int j = 0; j < NB; j++)
+      part[(wave * MB * NB + i * NB + j) * kWave + lane] = acc[i][j];
+    if (NORM_A) {
+      const float s = pairSum(rowPairSum(sum[i])), q = pairSum(rowPairSum(sq[i]));
+      if (lane < 16)
+        stat[wave * MB * 16 + i * 16 + lane] = float2v{s, q};
+    }
+  }
+  __syncthreads();
+  if (!mine)
+    return;
+  float4v v = part[outBlock * kWave + lane];
+#pragma unroll
+  for (int w = 1; w < kWaves; w++)
+    v += part[(w * MB * NB + outBlock) * kWave + lane];
+  if (NORM_A) {
+    float2v st{0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < kWaves; w++)
+      st += stat[w * MB * 16 + (outBlock / NB) * 16 + lane % 16];
+    const float mu = st[0] * p.invK;
+    // the difference cancels to a small negative number for near-constant
+    // rows; clamped so that a tiny eps cannot turn it into a NaN
+    const float rstd = 1.0f / sqrtf(fmaxf(st[1] * p.invK - mu * mu, 0.f) + p.eps);
+    const float shift = -mu * rstd;
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+      v[e] = fmaf(rstd, v[e], shift * cSum[e]);
+    if (p.statsOut && tileN == 0 && outBlock % NB == 0 && lane < 16)
+      storeWriteThrough(p.statsOut + int64_t(m) * 2, float2v{rstd, shift});
+  }
+  half4 o;
+#pragma unroll
+  for (int e = 0; e < 4; e++) {
+    float x = v[e];
+    if (p.activation == 1)
+      x = geluErf(x);
+    else if (p.activation == 2)
+      x = geluTanh(x);
+    if (p.C)
+      x += fmaf(float(cv[e]), cStat[0], cStat[1]);
+    o[e] = _Float16(x);
+  }
+  storeWriteThrough(p.D + (p.dPacked ? packed : plain), o);
+}
+
+// B [K, N] row-major -> fragments: block (column block j, k step s) is 1 KiB,
+// lane l of it holds B[32 s + 8 (l / 16) + e][16 j + l % 16], e = 0..7.
+__global__ __launch_bounds__(256) void packWeightKernel(const _Float16 *__restrict__ B,
+                                                        _Float16 *__restrict__ out,
+                                                        int K, int N) {
+  const int64_t v = int64_t(blockIdx.x) * 256 + threadIdx.x; // 16-byte vector of the output
+  const int steps = K / 32;
+  if (v >= int64_t(N / 16) * steps * kWave)
+    return;
+  const int l = int(v % kWave);
+  const int64_t block = v / kWave;
+  const int s = int(block % steps), j = int(block / steps);
+  half8 o;
+#pragma unroll
+  for (int e = 0; e < 8; e++)
+    o[e] = B[int64_t(32 * s + 8 * (l / 16) + e) * N + 16 * j + l % 16];
+  reinterpret_cast<half8 *>(out)[v] = o;
+}
+
+template <int MB, int NB, int CH, bool ONCE>
+Status launchVariant(const PackedGemm &g, const PackedArgs &p, int aheadGroups, hipStream_t s) {
+  const int steps = int(g.K / 32), perWave = (steps + kWaves - 1) / kWaves;
+  const int tilesM = int((g.M + MB * 16 - 1) / (MB * 16)), tilesN = int(g.N / (NB * 16));
+  constexpr int kLds = kWaves * MB * NB * kWave * 16 + kWaves * MB * 16 * 8;
+  const dim3 grid((unsigned)(tilesM * tilesN + aheadGroups)), block(kThreads);
+  auto kernel = g.aPacked ? (g.normA ? packedGemmKernel<MB, NB, CH, ONCE, true, true>
+                                     : packedGemmKernel<MB, NB, CH, ONCE, false, true>)
+                          : (g.normA ? packedGemmKernel<MB, NB, CH, ONCE, true, false>
+                                     : packedGemmKernel<MB, NB, CH, ONCE, false, false>);
+  if (kLds > 48 * 1024) {
+    static bool done[4] = {};
+    bool &set = done[2 * g.aPacked + g.normA];
+    if (!set)
+      HOM_HIP_RET(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
+                                      hipFuncAttributeMaxDynamicSharedMemorySize, kLds),
+                  Status::kInternal);
+    set = true;
+  }
+  kernel<<<grid, block, kLds, s>>>(g.A, g.packedB, int(g.M), int(g.K), steps, perWave, tilesM,
+                                   tilesN, magicFor(uint32_t(tilesM)), tilesM * tilesN, p);
+  HOM_HIP_RET(hipGetLastError(), Status::kInternal);
+  return Status::kSuccess;
+}
+
+} // namespace
+
+Status launchPackWeight(const _Float16 *B, _Float16 *packed, int64_t K, int64_t N,
+                        hipStream_t s) {
+  const int64_t vecs = K * N / 8;
+  packWeightKernel<<<dim3((unsigned)((vecs + 255) / 256)), dim3(256), 0, s>>>(B, packed, int(K),
+                                                                              int(N));
+  HOM_HIP_RET(hipGetLastError(), Status::kInternal);
+  return Status::kSuccess;
+}
+
+Status launchPackedGemm(const PackedGemm &g, hipStream_t s) {
+  PackedArgs p{};
+  p.C = g.C;
+  p.D = g.D;
+  p.colSum = g.colSum;
+  p.statsIn = g.statsIn;
+  p.statsOut = g.statsOut;
+  p.M = int(g.M);
+  p.N = int(g.N);
+  p.activation = g.activation;
+  p.cPacked = g.cPacked;
+  p.dPacked = g.dPacked;
+  p.invK = 1.0f / float(g.K);
+  p.eps = g.eps;
+  p.ahead = static_cast<const char *>(g.ahead);
+  p.aheadBytes = g.ahead ? g.aheadBytes : 0;
+  // k steps per wavefront, all in flight at once where the registers allow
+  const int perWave = int((g.K / 32 + kWaves - 1) / kWaves);
+  // The tile by a model of its time in a chain of launches, fitted to M = 16 ..
+  // 384 x the shapes of BERT-base and -large (within 10 %): launch, latency and
+  // the meeting of the partial sums, then what the fullest CU pulls through its
+  // L1; workgroups of a CU beyond those that fit its registers at once start a
+  // second chain of latencies.
+  const int cus = deviceInfo().computeUnits > 0 ? deviceInfo().computeUnits : 256;
+  struct Shape {
+    int mb, nb, resident;
+  };
+  const Shape shapes[4] = {{1, 1, perWave <= 4 ? 3 : 1},
+                           {2, 1, 2},
+                           {4, 1, 2},
+                           {4, 2, perWave == 4 ? 1 : 2}};
+  const double usPerKb = perWave <= 4 ? 0.0088 : 0.0062;
+  int best = 0;
+  double bestCost = 1e300;
+  int64_t bestTiles = 0;
+  for (int i = 0; i < 4; i++) {
+    const Shape &t = shapes[i];
+    if (g.N % (t.nb * 16) != 0)
+      continue;
+    const int64_t tiles = ((g.M + t.mb * 16 - 1) / (t.mb * 16)) * (g.N / (t.nb * 16));
+    const int64_t perCu = (tiles + cus - 1) / cus;
+    const double kb = double(t.mb + t.nb) * 16 * double(g.K) * 2 / 1024;
+    const double cost = 2.1 + 0.1 * t.mb * t.nb + usPerKb * kb * double(perCu) +
+                        0.8 * double((perCu - 1) / t.resident);
+    if (cost < bestCost) {
+      bestCost = cost;
+      best = i;
+      bestTiles = tiles;
+    }
+  }
+  // (64 KiB per workgroup that reads ahead; half the CUs when the tiles take
+  // all of them)
+  constexpr int64_t kAheadBytes = kThreads * 16 * 8;
+  const int groups =
+      int(std::min<int64_t>((p.aheadBytes + kAheadBytes - 1) / kAheadBytes,
+                            std::max<int64_t>(cus - bestTiles, cus / 2)));
+  switch (best) {
+  case 0:
+    return perWave <= 3    ? launchVariant<1, 1, 3, true>(g, p, groups, s)
+           : perWave <= 4  ? launchVariant<1, 1, 4, true>(g, p, groups, s)
+           : perWave <= 12 ? launchVariant<1, 1, 12, true>(g, p, groups, s)
+           : perWave <= 16 ? launchVariant<1, 1, 16, true>(g, p, groups, s)
+                           : launchVariant<1, 1, 12, false>(g, p, groups, s);
+  case 1:
+    return perWave <= 3   ? launchVariant<2, 1, 3, true>(g, p, groups, s)
+           : perWave <= 4 ? launchVariant<2, 1, 4, true>(g, p, groups, s)
+                          : launchVariant<2, 1, 6, false>(g, p, groups, s);
+  case 2:
+    return perWave <= 3   ? launchVariant<4, 1, 3, true>(g, p, groups, s)
+           : perWave <= 4 ? launchVariant<4, 1, 4, true>(g, p, groups, s)
+                          : launchVariant<4, 1, 4, false>(g, p, groups, s);
+  default:
+    return perWave <= 3   ? launchVariant<4, 2, 3, true>(g, p, groups, s)
+           : perWave <= 4 ? launchVariant<4, 2, 4, true>(g, p, groups, s)
+                          : launchVariant<4, 2, 3, false>(g, p, groups, s);
+  }
+}
+
+} // namespace hom

@@ -59,7 +59,7 @@ bool embedFits(const _Float16 *word, const _Float16 *pos, const _Float16 *out,
 Status launchEmbed(const int64_t *ids, const int64_t *mask, const _Float16 *word,
                    const _Float16 *pos, _Float16 *out, int32_t *cu, int64_t bs,
                    int64_t seq, int64_t hidden, int64_t vocab, float eps,
-                   hipStream_t s);
+                   bool packedOut, hipStream_t s);
 
 // ------------------------------------------------------------- attention --
 // qkv [bs, seq, 3*heads*headDim] fp16, cu int32[bs+1], out [bs, seq,
@@ -67,7 +67,7 @@ Status launchEmbed(const int64_t *ids, const int64_t *mask, const _Float16 *word
 Status launchBertAttentionF16(const _Float16 *qkv, const int32_t *cuSeqlens,
                               _Float16 *out, int64_t bs, int64_t seq,
                               int64_t heads, int64_t headDim, float scale,
-                              hipStream_t s);
+                              hipStream_t s, bool packedOut = false);
 
 // ------------------------------------------------------------------ gemm --
 enum class Epilogue : int { kLinear = 0, kGeluErf = 1, kGeluTanh = 2 };
@@ -166,6 +166,37 @@ Status launchGemmRowAffine(int likeKernel, const GemmProblem &p,
 Status launchGemmFolded(int likeKernel, const GemmProblem &p, int mode,
                         int activation, float *statsOut, hipStream_t s);
 int foldedPieces(int likeKernel, int64_t N);
+// GEMM of few rows against a packed weight (gemm_packed.hip):
+//   D = act(A . B) or, normA, act(LN(A) . B); activation 0 (then + C, or + LN(C)
+//   when statsIn is given), 1 erf GELU, 2 tanh GELU.
+// A [M, K], C and D [M, N] row-major and dense or in fragment order; K % 32 == 0,
+// N % 16 == 0 (N % 32 == 0 when C or D is packed).
+// Element (row, col) of a matrix in fragment order: blocks of 16 rows x 32
+// columns, 1 KiB each and in row-block order, hold lane l = 16 q + r of row r,
+// columns 8 q .. 8 q + 7.  (A packed weight is the same with B's columns as
+// rows and k as columns.)  The last row block is whole.
+__host__ __device__ inline int64_t packedOffset(int64_t row, int64_t col, int64_t cols) {
+  return ((row / 16) * (cols / 32) + col / 32) * 512 + (col % 32) / 8 * 128 +
+         row % 16 * 8 + col % 8;
+}
+struct PackedGemm {
+  bool aPacked, cPacked, dPacked; // in fragment order
+  const _Float16 *A, *packedB, *C;
+  _Float16 *D;
+  const float *colSum;  // [N] column sums of B (normA)
+  const float *statsIn; // [M][2] (rstd, -mean * rstd) of C's rows
+  float *statsOut;      // the same of A's rows, written when normA; may be null
+  int64_t M, N, K;
+  int activation;
+  bool normA;
+  float eps;
+  const void *ahead; // device memory that later kernels read first (may be null)
+  int64_t aheadBytes;
+};
+Status launchPackedGemm(const PackedGemm &g, hipStream_t s);
+// B [K, N] row-major, dense -> the layout above, K * N values.
+Status launchPackWeight(const _Float16 *B, _Float16 *packed, int64_t K, int64_t N,
+                        hipStream_t s);
 // out[n] = sum over k of B[k, n] (fp32), B row-major [K, N], N % 8 == 0.
 Status launchColumnSums(const _Float16 *B, int64_t ldb, int64_t K, int64_t N,
                         float *out, hipStream_t s);

@@ -111,6 +111,12 @@ void nvteBertAttentionF16(int64_t rankA, void *dstA, int64_t rankSeqlen,
   (void)runBertAttentionF16(rankA, dstA, rankSeqlen, dstSeqlen, rankOut, dstOut,
                             scale, headNum);
 }
+void homBertAttentionF16(int64_t rankA, void *dstA, int64_t rankSeqlen,
+                         void *dstSeqlen, int64_t rankOut, void *dstOut,
+                         float scale, int64_t headNum, int32_t packing) {
+  (void)runBertAttentionF16(rankA, dstA, rankSeqlen, dstSeqlen, rankOut, dstOut,
+                            scale, headNum, (packing & HOM_PACKED_D) != 0);
+}
 void nvteBertAttentionF32(int64_t, void *, int64_t, void *, int64_t, void *,
                           float, int64_t) {
   // The reference instantiates BertAttentionRunner<float>, which the fused
@@ -223,6 +229,21 @@ int32_t homFoldedLayernormPieces(int64_t M, int64_t N, int64_t K,
   return foldedLayernormPieces(M, N, K, activation, likeGemmNum);
 }
 
+void homPackWeightF16(int64_t rankB, void *dstB, void *packed) {
+  (void)runPackWeight(rankB, dstB, packed);
+}
+
+void homPackedGemmF16(int64_t rankA, void *dstA, const void *packedB,
+                      int64_t rankC, void *dstC, int64_t rankD, void *dstD,
+                      int64_t activation, int32_t normA, float eps,
+                      const float *colSumB, const float *statsIn,
+                      float *statsOut, int32_t packing, const void *ahead,
+                      int64_t aheadBytes) {
+  (void)runPackedGemm(rankA, dstA, packedB, rankC, dstC, rankD, dstD, activation,
+                      normA, eps, colSumB, statsIn, statsOut, packing, ahead,
+                      aheadBytes);
+}
+
 void homColumnSumsF16(int64_t rankB, void *dstB, float *out) {
   (void)runColumnSums(rankB, dstB, out);
 }
@@ -230,9 +251,9 @@ void homColumnSumsF16(int64_t rankB, void *dstB, float *out) {
 void homEmbedF16(int64_t rankIds, void *desIds, int64_t rankMask, void *desMask,
                  int64_t rankWord, void *desWord, int64_t rankPos, void *desPos,
                  int64_t rankOut, void *desOut, int64_t rankCu, void *desCu,
-                 float eps) {
+                 float eps, int32_t packing) {
   (void)runEmbed(rankIds, desIds, rankMask, desMask, rankWord, desWord, rankPos,
-                 desPos, rankOut, desOut, rankCu, desCu, eps);
+                 desPos, rankOut, desOut, rankCu, desCu, eps, packing);
 }
 
 void homGeluF16(int64_t rankA, void *dstA, int64_t rankOut, void *dstOut,

@@ -1,5 +1,7 @@
 #include "runners.h"
 
+#include "hom_amdgpu_runner_utils.h"
+
 #include <cerrno>
 #include <cmath>
 #include <cstring>
@@ -552,6 +554,86 @@ Status runColumnSums(int64_t rankB, void *dstB, float *out) {
                           stream());
 }
 
+Status runPackWeight(int64_t rankB, void *dstB, void *packed) {
+  View<_Float16> B(rankB, dstB);
+  HOM_CHECK_RET(B.sizes && rankB == 3 && B.sizes[0] == 1 && B.contiguous() &&
+                    B.sizes[1] % 32 == 0 && B.sizes[2] % 16 == 0 &&
+                    B.numel() * 2 < (int64_t(1) << 31),
+                Status::kInvalidArgument,
+                "pack weight: B must be a contiguous [1, K, N] tensor below 2 GiB "
+                "with K a multiple of 32 and N of 16");
+  HOM_CHECK_RET(packed && (reinterpret_cast<uintptr_t>(packed) & 15) == 0,
+                Status::kInvalidArgument, "pack weight: misaligned destination");
+  if (B.numel() == 0)
+    return Status::kSuccess;
+  return launchPackWeight(B.data, static_cast<_Float16 *>(packed), B.sizes[1],
+                          B.sizes[2], stream());
+}
+
+Status runPackedGemm(int64_t rankA, void *dstA, const void *packedB, int64_t rankC,
+                     void *dstC, int64_t rankD, void *dstD, int64_t activation,
+                     int32_t normA, float eps, const float *colSumB,
+                     const float *statsIn, float *statsOut, int32_t packing,
+                     const void *ahead, int64_t aheadBytes) {
+  View<_Float16> A(rankA, dstA), C(rankC, dstC), D(rankD, dstD);
+  HOM_CHECK_RET(A.rank == 3 && D.rank == 3 && A.sizes && D.sizes &&
+                    A.contiguous() && D.contiguous() &&
+                    A.sizes[0] == D.sizes[0] && A.sizes[1] == D.sizes[1],
+                Status::kInvalidArgument,
+                "packed gemm: A and D must be contiguous [b, M', K] and [b, M', N]");
+  PackedGemm g{};
+  g.M = A.sizes[0] * A.sizes[1];
+  g.K = A.sizes[2];
+  g.N = D.sizes[2];
+  HOM_CHECK_RET(g.K % 32 == 0 && g.N % 16 == 0 && g.K > 0 &&
+                    g.M * std::max(g.K, g.N) < (int64_t(1) << 30) &&
+                    g.K * g.N < (int64_t(1) << 30),
+                Status::kInvalidArgument,
+                "packed gemm: K must be a multiple of 32, N of 16, and the "
+                "operands below 2 GiB (M=%lld N=%lld K=%lld)",
+                (long long)g.M, (long long)g.N, (long long)g.K);
+  g.aPacked = (packing & HOM_PACKED_A) != 0;
+  g.cPacked = (packing & HOM_PACKED_C) != 0;
+  g.dPacked = (packing & HOM_PACKED_D) != 0;
+  HOM_CHECK_RET(g.N % 32 == 0 || !(g.cPacked || g.dPacked),
+                Status::kInvalidArgument,
+                "packed gemm: C or D in fragment order need N a multiple of 32");
+  HOM_CHECK_RET(activation >= 0 && activation <= 2, Status::kInvalidArgument,
+                "packed gemm: unknown activation %lld", (long long)activation);
+  if (dstC) {
+    HOM_CHECK_RET(C.rank == 3 && C.contiguous() && C.numel() == g.M * g.N &&
+                      C.sizes[2] == g.N && activation == 0,
+                  Status::kInvalidArgument,
+                  "packed gemm: C must be a contiguous tensor of D's shape, and "
+                  "the activation linear");
+    g.C = C.data;
+  }
+  HOM_CHECK_RET(!normA || colSumB, Status::kInvalidArgument,
+                "packed gemm: a normalised A needs the column sums of B");
+  HOM_CHECK_RET(!statsOut || normA, Status::kInvalidArgument,
+                "packed gemm: statistics are written for a normalised A only");
+  HOM_CHECK_RET(!statsIn || dstC, Status::kInvalidArgument,
+                "packed gemm: row statistics without a source");
+  auto al16 = [](const void *q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
+  HOM_CHECK_RET(al16(A.data) && al16(packedB) && al16(D.data) && al16(g.C) &&
+                    al16(colSumB) && al16(ahead),
+                Status::kInvalidArgument, "packed gemm: misaligned operands");
+  if (g.M == 0 || g.N == 0)
+    return Status::kSuccess;
+  g.A = A.data;
+  g.packedB = static_cast<const _Float16 *>(packedB);
+  g.D = D.data;
+  g.colSum = colSumB;
+  g.statsIn = statsIn;
+  g.statsOut = statsOut;
+  g.activation = int(activation);
+  g.normA = normA != 0;
+  g.eps = eps;
+  g.ahead = ahead;
+  g.aheadBytes = aheadBytes;
+  return launchPackedGemm(g, stream());
+}
+
 Status runLayernormGemm(int64_t rankA, void *dstA, int64_t rankB, void *dstB,
                         int64_t rankC, void *dstC, int64_t rankD, void *dstD,
                         int64_t rankVar, void *dstVar, int64_t rankMean,
@@ -889,7 +971,7 @@ Status runAddLayernormF16(int64_t rankX, void *dstX, int64_t rankRes,
 // --------------------------------------------------------------- attention --
 Status runBertAttentionF16(int64_t rankA, void *dstA, int64_t rankSeqlen,
                            void *dstSeqlen, int64_t rankOut, void *dstOut,
-                           float scale, int64_t headNum) {
+                           float scale, int64_t headNum, bool packedOut) {
   View<_Float16> A(rankA, dstA), Out(rankOut, dstOut);
   View<int32_t> Seq(rankSeqlen, dstSeqlen);
   // BertAttentionRunner::construct_tensors (BertAttentionRunner.h:61-73)
@@ -917,7 +999,7 @@ Status runBertAttentionF16(int64_t rankA, void *dstA, int64_t rankSeqlen,
   HOM_CHECK_RET(A.contiguous() && Out.contiguous(), Status::kInvalidArgument,
                 "attention: tensors must be contiguous");
   return launchBertAttentionF16(A.data, Seq.data, Out.data, bs, seq, headNum,
-                                headDim, scale, stream());
+                                headDim, scale, stream(), packedOut);
 }
 
 // ------------------------------------------------------------- elementwise --
@@ -1013,7 +1095,7 @@ template Status runCuSeqLen<int32_t>(int64_t, void *, int64_t, void *);
 Status runEmbed(int64_t rankIds, void *desIds, int64_t rankMask, void *desMask,
                 int64_t rankWord, void *desWord, int64_t rankPos, void *desPos,
                 int64_t rankOut, void *desOut, int64_t rankCu, void *desCu,
-                float eps) {
+                float eps, int32_t packing) {
   View<int64_t> I(rankIds, desIds), Mk(rankMask, desMask);
   View<_Float16> W(rankWord, desWord), P(rankPos, desPos), O(rankOut, desOut);
   View<int32_t> Cu(rankCu, desCu);
@@ -1037,9 +1119,14 @@ Status runEmbed(int64_t rankIds, void *desIds, int64_t rankMask, void *desMask,
   HOM_CHECK_RET(I.contiguous() && Mk.contiguous() && W.contiguous() &&
                     P.contiguous() && O.contiguous(),
                 Status::kInvalidArgument, "embed: tensors must be contiguous");
+  const bool packedOut = (packing & HOM_PACKED_D) != 0;
+  HOM_CHECK_RET(!packedOut || hidden % 32 == 0, Status::kInvalidArgument,
+                "embed: fragment order needs H a multiple of 32");
   if (embedFits(W.data, P.data, O.data, bs, seq, hidden, vocab))
     return launchEmbed(I.data, Mk.data, W.data, P.data, O.data, Cu.data, bs, seq,
-                       hidden, vocab, eps, stream());
+                       hidden, vocab, eps, packedOut, stream());
+  HOM_CHECK_RET(!packedOut, Status::kInvalidArgument,
+                "embed: fragment order needs H of at most 2048");
   // rows off the vector width or beyond a wavefront's registers: step by step
   Status st = launchCuSeqLen<int64_t>(Mk.data, Cu.data, bs, seq, stream());
   if (st == Status::kSuccess)

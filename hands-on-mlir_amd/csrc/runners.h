@@ -45,6 +45,12 @@ Status runGemmFoldedLayernorm(int64_t rankA, void *dstA, int64_t rankB,
                               int32_t likeGemmNum);
 int32_t foldedLayernormPieces(int64_t M, int64_t N, int64_t K, int64_t activation,
                               int32_t likeGemmNum);
+Status runPackWeight(int64_t rankB, void *dstB, void *packed);
+Status runPackedGemm(int64_t rankA, void *dstA, const void *packedB, int64_t rankC,
+                     void *dstC, int64_t rankD, void *dstD, int64_t activation,
+                     int32_t normA, float eps, const float *colSumB,
+                     const float *statsIn, float *statsOut, int32_t packing,
+                     const void *ahead, int64_t aheadBytes);
 Status runColumnSums(int64_t rankB, void *dstB, float *out);
 
 // Kernel choice without timing: tuned table first, heuristic otherwise.
@@ -115,7 +121,7 @@ Status runAddLayernormF16(int64_t rankX, void *dstX, int64_t rankRes,
                           void *dstOut, float eps);
 Status runBertAttentionF16(int64_t rankA, void *dstA, int64_t rankSeqlen,
                            void *dstSeqlen, int64_t rankOut, void *dstOut,
-                           float scale, int64_t headNum);
+                           float scale, int64_t headNum, bool packedOut = false);
 template <typename T>
 Status runElementwise(BinOp op, int64_t rankA, void *dstA, int64_t rankB,
                       void *dstB, int64_t rankOut, void *dstOut);
@@ -127,7 +133,7 @@ Status runCuSeqLen(int64_t rankIn, void *desIn, int64_t rankOut, void *desOut);
 Status runEmbed(int64_t rankIds, void *desIds, int64_t rankMask, void *desMask,
                 int64_t rankWord, void *desWord, int64_t rankPos, void *desPos,
                 int64_t rankOut, void *desOut, int64_t rankCu, void *desCu,
-                float eps);
+                float eps, int32_t packing);
 Status runGeluF16(int64_t rankA, void *dstA, int64_t rankOut, void *dstOut,
                   int32_t form);
 

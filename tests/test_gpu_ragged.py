@@ -95,7 +95,7 @@ def test_embed_equals_its_steps(gpu, rt, b, s, H, pinned):
     M = rt.MemRef.from_tensor
     new = lambda *shape, dt=torch.float16: torch.zeros(shape, dtype=dt, device="cuda")  # noqa: E731
     out, cu = new(b, s, H), new(b + 1, dt=torch.int32)
-    gpu.homEmbedF16(*M(ti).args(), *M(tm).args(), *M(tw).args(), *M(tp).args(), *M(out).args(), *M(cu).args(), 1e-12)
+    gpu.homEmbedF16(*M(ti).args(), *M(tm).args(), *M(tw).args(), *M(tp).args(), *M(out).args(), *M(cu).args(), 1e-12, 0)
     rows, want, wantCu = new(b, s, H), new(b, s, H), new(b + 1, dt=torch.int32)
     gpu.thrustCuSeqLenI64(*M(dev(mask)).args(), *M(wantCu).args())
     gpu.thrustGatherF16(*M(dev(ids)).args(), *M(tw).args(), *M(rows).args())
@@ -165,3 +165,65 @@ def test_gemm_any_alignment(gpu, rt, oracle, tile, M, N, K):
     tb, td = odd(Bt), odd(np.zeros((1, M, N), np.float16))
     gpu.nvteGemmF16(*Mr(odd(A)).args(), False, *Mr(tb).args(), True, *Mr(td).args(), *Mr(td).args(), 0, 1.0, 0.0, 0, 0)
     np.testing.assert_allclose(host(td)[0].astype(np.float64), oracle.gemm(A[0], B[0]), rtol=1e-3, atol=1e-2)
+
+
+def fragment_order(a):
+    """[rows, cols] -> blocks of 16 rows x 32 columns as the packed GEMM takes them (rows padded to 16)."""
+    rows, cols = a.shape
+    p = np.zeros((-(-rows // 16) * 16, cols), a.dtype)
+    p[:rows] = a
+    return np.ascontiguousarray(p.reshape(-1, 16, cols // 32, 4, 8).transpose(0, 2, 3, 1, 4)).reshape(-1)
+
+
+# row counts around the 16 / 32 / 64-row tiles, one k step per wavefront and several rounds of them, few and many
+# column blocks, both orders of every operand
+@pytest.mark.parametrize("M,N,K", [(1, 32, 32), (16, 96, 256), (17, 768, 768), (33, 2304, 768), (64, 3072, 768),
+                                   (65, 768, 3072), (130, 1024, 1024), (200, 1024, 4096), (300, 4096, 1056),
+                                   (257, 320, 5120)])
+@pytest.mark.parametrize("packing", [0, 7, 3, 5])
+def test_packed_gemm(gpu, rt, oracle, M, N, K, packing):
+    g = np.random.default_rng(M + N + K + packing)
+    A = (g.standard_normal((M, K)) + 0.3).astype(np.float16)
+    B, C = (g.standard_normal((K, N)) * 0.03).astype(np.float16), g.standard_normal((M, N)).astype(np.float16)
+    stats = np.stack([0.5 + g.random(M), g.standard_normal(M)], 1).astype(np.float32)
+    Mr, R = rt.MemRef, -(-M // 16) * 16
+
+    def place(a, flag):
+        t = dev(fragment_order(a) if packing & flag else np.concatenate([a, np.zeros((R - M, a.shape[1]), a.dtype)]))
+        return t, Mr(t.data_ptr(), [1, M, a.shape[1]])
+
+    def result(t):
+        v = host(t)
+        if not packing & 4:
+            return v.reshape(R, N)[:M]
+        return v.reshape(-1, N // 32, 4, 16, 8).transpose(0, 3, 1, 2, 4).reshape(R, N)[:M]
+
+    tb = dev(B[None])
+    packed = torch.zeros(K * N, dtype=torch.float16, device="cuda")
+    gpu.homPackWeightF16(*Mr.from_tensor(tb).args(), packed.data_ptr())
+    np.testing.assert_array_equal(host(packed), fragment_order(np.ascontiguousarray(B.T)))
+    colsum = dev(B.astype(np.float32).sum(0))
+    (ta, ma), (tc, mc), ts = place(A, 1), place(C, 2), dev(stats)
+    td, out = torch.zeros(R * N, dtype=torch.float16, device="cuda"), torch.zeros((M, 2), device="cuda")
+    md = Mr(td.data_ptr(), [1, M, N])
+    x = A.astype(np.float64)
+    rstd = 1 / np.sqrt(x.var(1) + 1e-6)
+    ln = (x - x.mean(1, keepdims=True)) * rstd[:, None]
+    # residual of normalised rows
+    gpu.homPackedGemmF16(*ma.args(), packed.data_ptr(), *mc.args(), *md.args(), 0, 0, 1e-6, None, ts.data_ptr(), None,
+                         packing, None, 0)
+    want = x @ B.astype(np.float64) + C.astype(np.float64) * stats[:, :1] + stats[:, 1:]
+    np.testing.assert_allclose(result(td).astype(np.float64), want, rtol=1e-3, atol=1e-2)
+    # plain residual, reading ahead
+    gpu.homPackedGemmF16(*ma.args(), packed.data_ptr(), *mc.args(), *md.args(), 0, 0, 1e-6, None, None, None, packing,
+                         packed.data_ptr(), 2 * K * N)
+    want = x @ B.astype(np.float64) + C.astype(np.float64)
+    np.testing.assert_allclose(result(td).astype(np.float64), want, rtol=1e-3, atol=1e-2)
+    # normalised A with both activations, and the row statistics
+    for act, name in ((1, "gelu_erf"), (2, "gelu_tanh"), (0, "linear")):
+        gpu.homPackedGemmF16(*ma.args(), packed.data_ptr(), 0, None, *md.args(), act, 1, 1e-6, colsum.data_ptr(), None,
+                             out.data_ptr(), packing & ~2, None, 0)
+        z = oracle.gemm(ln.astype(np.float32).astype(np.float16), B, act=name)  # (A rounded: within the tolerance)
+        np.testing.assert_allclose(result(td).astype(np.float64), z, rtol=2e-3, atol=1e-2)
+        np.testing.assert_allclose(host(out)[:, 0], rstd, rtol=1e-4)
+        np.testing.assert_allclose(host(out)[:, 1], -x.mean(1) * rstd, rtol=1e-3, atol=1e-4)
