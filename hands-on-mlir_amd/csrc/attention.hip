@@ -30,7 +30,7 @@
 // LDS rows are 128 bytes, unpadded; 16-byte chunks (K) / 64-byte groups (V) are
 // XOR-permuted by row so that the fragment reads are bank-conflict free.
 #include "cross_lane.h"
-#include "kernels.h"
+#include "packed_args.h"
 
 #include <cstring>
 
@@ -80,14 +80,18 @@ template <int D> __device__ __forceinline__ int swzV(int k, int group) {
 // keys of its own 32 rows; KS = 2: half the serial work per wavefront, for
 // short sequences where there are fewer workgroups than CUs and the key walk
 // of one wavefront is the critical path; the halves are merged through LDS).
-template <int NW, int KS, int D>
+// PACKED_IN: QKV in fragment order (packedOffset() in kernels.h): the 8 values of
+// a token row that a vector takes are contiguous there as well, only the address
+// of a row differs.
+template <int NW, int KS, int D, bool PACKED_IN = false>
 __global__ __launch_bounds__(NW *kWave)
 __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1, D == 64 && KS == 1 ? 4 : (D <= 128 ? 2 : 1)))) void bertAttentionKernel(
     const _Float16 *__restrict__ qkv, const int32_t *__restrict__ cu,
     _Float16 *__restrict__ out, int seq, int heads, int numQTiles, int pairs,
-    float scale, int packedOut) {
+    float scale, int packedOut, const char *ahead, int64_t aheadBytes) {
   static_assert(D == 64 || D == 128 || D == 192 || D == 256, "head size");
   static_assert(D <= 128 || KS == 1, "the key-split variant stages 128 keys per chunk");
+  static_assert(!PACKED_IN || D == 64, "fragment order is read at head size 64");
   constexpr int kChunk = Chunk<D>::value;
   constexpr int kHeadDim = D;
   constexpr int kRowB = D * 2;               // bytes of a K or V row
@@ -115,6 +119,13 @@ __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1, D == 64 && KS == 1 ? 4 : (D 
   int qTile, head, b;
   if (KS == 1) {
     const int id = blockIdx.x;
+    if constexpr (PACKED_IN) {
+      if (id >= numQTiles * pairs) {
+        readAhead<kThreads>(ahead, aheadBytes, id - numQTiles * pairs,
+                            int(gridDim.x) - numQTiles * pairs, tid);
+        return;
+      }
+    }
     int pair;
     if (pairs % 8 == 0) {
       const int t = id / 8;
@@ -130,6 +141,14 @@ __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1, D == 64 && KS == 1 ? 4 : (D 
     qTile = blockIdx.x;
     head = blockIdx.y;
     b = blockIdx.z;
+    if constexpr (PACKED_IN) {
+      const int plane = numQTiles * heads; // workgroups of a batch entry
+      if (b * heads >= pairs) {
+        readAhead<kThreads>(ahead, aheadBytes, b * plane + head * numQTiles + qTile - numQTiles * pairs,
+                            int(gridDim.z) * plane - numQTiles * pairs, tid);
+        return;
+      }
+    }
   }
   const int q0 = qTile * (QG * 32) + qg * 32;
   const int cuLo = cu[b], cuHi = cu[b + 1]; // consumed after the first loads are out
@@ -159,6 +178,14 @@ __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1, D == 64 && KS == 1 ? 4 : (D 
   // registers measured 3-8 % slower than loading each chunk when it is due
   // (also with barriers that do not wait for the prefetch).
   // (D = 128: the prefetched rows would take 64 more registers than there are)
+  // PACKED_IN: 8 values from column 8 * c8 of part `part` (0 Q, 1 K, 2 V) of token
+  // row `row`, as an offset in halves
+  const int wide = 3 * heads * (kHeadDim / 32); // 32-column blocks of QKV
+  auto packedAt = [&](int row, int part, int c8) {
+    const int t = b * seq + row;
+    return (int64_t(t / 16) * wide + (part * heads + head) * (kHeadDim / 32) + c8 / 4) * 512 +
+           (c8 % 4) * 128 + (t % 16) * 8;
+  };
   constexpr bool kPrefetch = KS == 2 && D == 64;
   constexpr int VPT = kChunk * CPR / kThreads; // vectors of K (and of V) per thread
   half8 rk[VPT], rv[VPT];
@@ -168,8 +195,10 @@ __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1, D == 64 && KS == 1 ? 4 : (D 
       const int v = tid + i * kThreads;
       const int r = v / CPR, c = v % CPR;
       const int row = key0 + r < seq ? key0 + r : seq - 1;
-      rk[i] = *reinterpret_cast<const half8 *>(kBase + int64_t(row) * tokStride + c * 8);
-      rv[i] = *reinterpret_cast<const half8 *>(vBase + int64_t(row) * tokStride + c * 8);
+      rk[i] = *reinterpret_cast<const half8 *>(
+          PACKED_IN ? qkv + packedAt(row, 1, c) : kBase + int64_t(row) * tokStride + c * 8);
+      rv[i] = *reinterpret_cast<const half8 *>(
+          PACKED_IN ? qkv + packedAt(row, 2, c) : vBase + int64_t(row) * tokStride + c * 8);
     }
   };
   if (kPrefetch)
@@ -183,8 +212,9 @@ __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1, D == 64 && KS == 1 ? 4 : (D 
     const int q = q0 + l32 < seq ? q0 + l32 : seq - 1;
 #pragma unroll
     for (int kk = 0; kk < kHeadDim / 16; kk++)
-      fq[kk] = *reinterpret_cast<const half8 *>(qBase + int64_t(q) * tokStride +
-                                                kk * 16 + hb * 8);
+      fq[kk] = *reinterpret_cast<const half8 *>(
+          PACKED_IN ? qkv + packedAt(q, 0, kk * 2 + hb)
+                    : qBase + int64_t(q) * tokStride + kk * 16 + hb * 8);
   }
 
   int len = cuHi - cuLo;
@@ -233,17 +263,23 @@ __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1, D == 64 && KS == 1 ? 4 : (D 
   // whole number; those compute every vector's addresses, see below.)
   constexpr bool kFastStage = kThreads % CPR == 0 && (kThreads / CPR) % 16 == 0;
   static_assert(kFastStage || D > 128, "row step per vector must leave the swizzles alone");
-  const uint32_t rowBytes = uint32_t(tokStride) * 2u;
-  const uint32_t stageOff = uint32_t(tid / CPR) * rowBytes + uint32_t(tid % CPR) * 16u;
+  // (fragment order: 16 rows further on is one row of blocks further on; the
+  // descriptors cannot end at row `len` there, so rows past it are aimed outside)
+  const uint32_t rowBytes = PACKED_IN ? uint32_t(wide) * 64u : uint32_t(tokStride) * 2u;
+  const uint32_t stageOff =
+      PACKED_IN ? uint32_t(packedAt(tid / CPR, 1, tid % CPR)) * 2u
+                : uint32_t(tid / CPR) * rowBytes + uint32_t(tid % CPR) * 16u;
+  const uint32_t vFromK = PACKED_IN ? uint32_t(heads * (kHeadDim / 32)) * 1024u : 0u;
   const int stageK = (tid / CPR) * kRowB + swzK<D>(tid / CPR, tid % CPR) * 16;
   const int stageV = (tid / CPR) * kRowB + swzV<D>(tid / CPR, (tid % CPR) / 4) * 64 +
                      ((tid % CPR) % 4) * 16;
+  const int32_t stageBytes = PACKED_IN ? int32_t(uint32_t((pairs / heads * seq + 15) / 16) *
+                                                 uint32_t(wide) * 1024u)
+                                       : int32_t(uint32_t(len) * rowBytes);
   const auto rsrcK = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<_Float16 *>(kBase), 0, int32_t(uint32_t(len) * rowBytes),
-      0x00020000);
+      const_cast<_Float16 *>(PACKED_IN ? qkv : kBase), 0, stageBytes, 0x00020000);
   const auto rsrcV = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<_Float16 *>(vBase), 0, int32_t(uint32_t(len) * rowBytes),
-      0x00020000);
+      const_cast<_Float16 *>(PACKED_IN ? qkv : vBase), 0, stageBytes, 0x00020000);
 
   // uniform over the workgroup; at least one round in the key-split variant,
   // whose first chunk is already on its way
@@ -286,11 +322,13 @@ __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1, D == 64 && KS == 1 ? 4 : (D 
         const uint32_t chunkOff = stageOff + uint32_t(key0) * rowBytes;
 #pragma unroll
         for (int i = 0; i < VPT; i++) {
-          const uint32_t off = chunkOff + uint32_t(i * (kThreads / CPR)) * rowBytes;
+          uint32_t off = chunkOff + uint32_t(i * (kThreads / CPR)) * rowBytes;
+          if (PACKED_IN && key0 + tid / CPR + i * (kThreads / CPR) >= len)
+            off = 0x80000000u - vFromK;
           kv[i] = __builtin_bit_cast(
               half8, __builtin_amdgcn_raw_buffer_load_b128(rsrcK, off, 0, 0));
           vv[i] = __builtin_bit_cast(
-              half8, __builtin_amdgcn_raw_buffer_load_b128(rsrcV, off, 0, 0));
+              half8, __builtin_amdgcn_raw_buffer_load_b128(rsrcV, off + vFromK, 0, 0));
         }
 #pragma unroll
         for (int i = 0; i < VPT; i++) {
@@ -531,7 +569,12 @@ __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1, D == 64 && KS == 1 ? 4 : (D 
 Status launchBertAttentionF16(const _Float16 *qkv, const int32_t *cuSeqlens,
                               _Float16 *out, int64_t bs, int64_t seq,
                               int64_t heads, int64_t headDim, float scale,
-                              hipStream_t s, bool packedOut) {
+                              hipStream_t s, bool packedOut, bool packedIn,
+                              const void *ahead, int64_t aheadBytes) {
+  HOM_CHECK_RET(!packedIn || (headDim == 64 && ((bs * seq + 15) / 16) * 96 * heads * 64 <
+                                                   (int64_t(1) << 30)),
+                Status::kInvalidArgument,
+                "attention: QKV in fragment order needs head size 64 and less than 1 GiB");
   // (the reference's contract is head size % 64 == 0, README.md:11; the
   // sizes with kernels here are 64, 128, 192 and 256)
   HOM_CHECK_RET(headDim == 64 || headDim == 128 || headDim == 192 || headDim == 256,
@@ -566,38 +609,52 @@ Status launchBertAttentionF16(const _Float16 *qkv, const int32_t *cuSeqlens,
     wide = true; // (the key-split variant exists for 64 and 128 only)
   HOM_CHECK_RET(pairs * ((seq + 63) / 64) < (int64_t(1) << 31),
                 Status::kInvalidArgument, "attention: too many workgroups");
+  // Workgroups that read weights ahead (readAhead() in packed_args.h), while the
+  // attention itself leaves room: two workgroups of it per CU or fewer.
+  const unsigned extra =
+      ahead && pairs * ((seq + 127) / 128) <= 2 * cus ? aheadGroups<256>(aheadBytes, cus) : 0;
   if (wide) {
     const int nq = int((seq + 127) / 128);
     const dim3 grid((unsigned)(nq * pairs));
-    if (headDim == 64)
+    if (packedIn)
+      bertAttentionKernel<4, 1, 64, true><<<dim3(grid.x + extra), dim3(256), 0, s>>>(
+          qkv, cuSeqlens, out, int(seq), int(heads), nq, int(pairs), scale,
+          packedOut, static_cast<const char *>(ahead), aheadBytes);
+    else if (headDim == 64)
       bertAttentionKernel<4, 1, 64><<<grid, dim3(256), 0, s>>>(
           qkv, cuSeqlens, out, int(seq), int(heads), nq, int(pairs), scale,
-          packedOut);
+          packedOut, nullptr, 0);
     else if (headDim == 128)
       bertAttentionKernel<4, 1, 128><<<grid, dim3(256), 0, s>>>(
           qkv, cuSeqlens, out, int(seq), int(heads), nq, int(pairs), scale,
-          packedOut);
+          packedOut, nullptr, 0);
     else if (headDim == 192)
       bertAttentionKernel<4, 1, 192><<<grid, dim3(256), 0, s>>>(
           qkv, cuSeqlens, out, int(seq), int(heads), nq, int(pairs), scale,
-          packedOut);
+          packedOut, nullptr, 0);
     else
       bertAttentionKernel<4, 1, 256><<<grid, dim3(256), 0, s>>>(
           qkv, cuSeqlens, out, int(seq), int(heads), nq, int(pairs), scale,
-          packedOut);
+          packedOut, nullptr, 0);
   } else {
     const int nq = int((seq + 63) / 64);
     HOM_CHECK_RET(heads < 65536 && bs < 65536, Status::kInvalidArgument,
                   "attention: heads and batch size must be below 65536");
     const dim3 grid((unsigned)nq, (unsigned)heads, (unsigned)bs);
-    if (headDim == 64)
+    const unsigned plane = unsigned(nq) * unsigned(heads);
+    if (packedIn)
+      bertAttentionKernel<4, 2, 64, true>
+          <<<dim3(grid.x, grid.y, grid.z + (extra + plane - 1) / plane), dim3(256), 0, s>>>(
+              qkv, cuSeqlens, out, int(seq), int(heads), nq, int(pairs), scale, packedOut,
+              static_cast<const char *>(ahead), aheadBytes);
+    else if (headDim == 64)
       bertAttentionKernel<4, 2, 64><<<grid, dim3(256), 0, s>>>(
           qkv, cuSeqlens, out, int(seq), int(heads), nq, int(pairs), scale,
-          packedOut);
+          packedOut, nullptr, 0);
     else
       bertAttentionKernel<4, 2, 128><<<grid, dim3(256), 0, s>>>(
           qkv, cuSeqlens, out, int(seq), int(heads), nq, int(pairs), scale,
-          packedOut);
+          packedOut, nullptr, 0);
   }
   HOM_HIP_RET(hipGetLastError(), Status::kInternal);
   return Status::kSuccess;

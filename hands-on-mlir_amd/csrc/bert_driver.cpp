@@ -95,8 +95,9 @@ struct HomBertEncoder {
   std::vector<float *> colSumQkv, colSumW1;
   float *rowSums[2] = {nullptr, nullptr};
   int32_t foldPieces = 0;
-  // Few rows (usesPacked): every layer GEMM runs on weights in fragment order,
-  // with the layer norms folded into the GEMMs around them.  One arena holds
+  // usesPacked: every layer GEMM runs on weights in fragment order; up to a few
+  // thousand rows (foldsPacked) with the layer norms folded into the GEMMs around
+  // them.  One arena holds
   // the packed weights in the order the forward reads them, one the column
   // sums of Wqkv and W1; both are made from the uploaded weights before the
   // next forward or capture (packWeights).
@@ -104,7 +105,7 @@ struct HomBertEncoder {
   char *packedArena = nullptr;
   float *packedColSums = nullptr;
   float *packedStats[2] = {nullptr, nullptr}; // rows of h entering QKV / FFN1
-  Tensor hPacked, attnPacked, fPacked;        // activations in fragment order
+  Tensor hPacked, qkvPacked, attnPacked, fPacked; // activations in fragment order
   hipStream_t stream = nullptr;
   hipGraph_t graph = nullptr;
   hipGraphExec_t graphExec = nullptr;
@@ -279,20 +280,30 @@ bool chooseGemm(HomBertEncoder *e, int64_t M, int64_t N, int64_t K, int64_t act,
   return true;
 }
 
-// The packed form serves few rows: beyond them a workgroup of the tiled
-// kernels, which shares operands through LDS, reads less per output.  us per
-// request, tiled -> packed: BERT-base with 64 rows 494 -> 296, 256 rows 515 ->
-// 403, 512 rows 630 -> 513, 768 rows 688 -> 650, 1024 rows 691 -> 769;
-// BERT-large with 16 rows 1006 -> 542, 256 rows 1106 -> 1061, 512 rows 1378 ->
-// 1527.  The line between them moves with the cube of the hidden size.
+// Packed weights wherever their kernels take the shapes (head size 64, whole
+// 64-k slabs, operands within 32-bit byte offsets) and the caller has not pinned
+// a weight layout.  Row-major -> packed, us: BERT-base 64 rows 491 -> 284, 1024 rows
+// 685 -> 618, 2048 rows 977 -> 876, 16384 rows 4437 -> 4095; BERT-large 495 rows
+// 1336 -> 1244, 4096 rows 3862 -> 3406, 8192 rows (the tiles do not come out even)
+// 6301 -> 6327, 16384 rows 12482 -> 11495.
 bool usesPacked(const HomBertEncoder *e) {
-  const int64_t M = int64_t(e->batch) * e->seq;
   bool pinned = false;
   for (int r = 0; r < 4; r++)
     pinned = pinned || e->roleLayout[r] != -1;
-  const double H = e->hidden;
-  return double(M) * H * H * H <= 3.7e11 && e->gemmMode == 1 && !pinned &&
-         e->hidden % 32 == 0 && e->ffn % 32 == 0 && e->hidden <= 2048;
+  const int64_t rows = (int64_t(e->batch) * e->seq + 15) / 16 * 16;
+  return e->gemmMode == 1 && !pinned && e->hidden % 64 == 0 && e->ffn % 64 == 0 &&
+         e->hidden <= 2048 && e->hidden == e->heads * 64 &&
+         rows * std::max<int64_t>(6 * e->hidden, e->ffn) < (int64_t(1) << 30) &&
+         int64_t(e->hidden) * e->ffn < (int64_t(1) << 30);
+}
+// Two launches a layer less against row sums taken inside the GEMMs, which slow
+// a GEMM down that fills the chip several times over (in front of the 256 x 256
+// tiles by 10 - 13 %).  Folded against explicit layer norms, us: BERT-large 1024
+// rows 1534 / 1600, 4096 rows 3406 / 3479, 6144 rows 5446 / 5344, 16384 rows
+// 11880 / 11495; BERT-base 1024 rows 618 / 642, 8192 rows 2423 / 2435, 16384 rows
+// 4110 / 4095.
+bool foldsPacked(const HomBertEncoder *e) {
+  return int64_t(e->batch) * e->seq * e->hidden <= 5500000;
 }
 
 struct PackedLayer { // byte offsets into the arena
@@ -338,6 +349,7 @@ bool packWeights(HomBertEncoder *e) {
       st[0] = int64_t(e->seq) * cols;
     };
     padded(e->hPacked, int(H));
+    padded(e->qkvPacked, int(3 * H));
     padded(e->attnPacked, int(H));
     padded(e->fPacked, int(F));
   }
@@ -372,25 +384,37 @@ void packedLayers(HomBertEncoder *e, int64_t geluAct, float scale) {
                      colSum, statsIn, statsOut, packing,
                      e->packedArena + ahead, aheadEnd - ahead);
   };
+  const bool fold = foldsPacked(e);
   for (int l = 0; l < e->layers; l++) {
     const PackedLayer at = packedLayer(e, l);
     const bool last = l + 1 == e->layers;
+    const int64_t nextQkv = last ? at.end : at.end + (at.out - at.qkv);
     // (the embeddings arrive normalised)
-    const bool norm = l > 0;
-    gemm(e->hPacked, at.qkv, nullptr, e->qkv, 0, norm, norm ? packedColSum(e, l, false) : nullptr,
-         nullptr, norm ? e->packedStats[0] : nullptr, HOM_PACKED_A, at.out, at.ffn1);
-    homBertAttentionF16(e->qkv.m.rank, e->qkv.m.descriptor, e->cu.m.rank, e->cu.m.descriptor,
-                        e->attnPacked.m.rank, e->attnPacked.m.descriptor, scale, e->heads,
-                        HOM_PACKED_D);
+    const bool norm = fold && l > 0;
+    gemm(e->hPacked, at.qkv, nullptr, e->qkvPacked, 0, norm,
+         norm ? packedColSum(e, l, false) : nullptr, nullptr, norm ? e->packedStats[0] : nullptr,
+         HOM_PACKED_A | HOM_PACKED_D, at.out, at.ffn1);
+    homBertAttentionF16(e->qkvPacked.m.rank, e->qkvPacked.m.descriptor, e->cu.m.rank,
+                        e->cu.m.descriptor, e->attnPacked.m.rank, e->attnPacked.m.descriptor,
+                        scale, e->heads, HOM_PACKED_A | HOM_PACKED_D,
+                        e->packedArena + at.ffn1, at.ffn2 - at.ffn1);
     gemm(e->attnPacked, at.out, &e->hPacked, e->hPacked, 0, false, nullptr,
-         norm ? e->packedStats[0] : nullptr, nullptr, kAll, at.ffn1, at.ffn2);
-    gemm(e->hPacked, at.ffn1, nullptr, e->fPacked, geluAct, true, packedColSum(e, l, true), nullptr,
-         e->packedStats[1], HOM_PACKED_A | HOM_PACKED_D, at.ffn2, at.end);
-    gemm(e->fPacked, at.ffn2, &e->hPacked, last ? e->h : e->hPacked, 0, false, nullptr,
-         e->packedStats[1], nullptr, last ? HOM_PACKED_A | HOM_PACKED_C : kAll, at.end,
-         last ? at.end : at.end + (at.out - at.qkv));
+         norm ? e->packedStats[0] : nullptr, nullptr, kAll, at.ffn2, at.end);
+    if (!fold)
+      homPackedLayernormF16(e->hPacked.m.rank, e->hPacked.m.descriptor, e->hPacked.m.rank,
+                            e->hPacked.m.descriptor, e->eps, HOM_PACKED_A | HOM_PACKED_D);
+    gemm(e->hPacked, at.ffn1, nullptr, e->fPacked, geluAct, fold,
+         fold ? packedColSum(e, l, true) : nullptr, nullptr, fold ? e->packedStats[1] : nullptr,
+         HOM_PACKED_A | HOM_PACKED_D, at.end, nextQkv);
+    gemm(e->fPacked, at.ffn2, &e->hPacked, e->hPacked, 0, false, nullptr,
+         fold ? e->packedStats[1] : nullptr, nullptr, kAll, at.end, nextQkv);
+    if (!fold || last) {
+      const Tensor &out = last ? e->h : e->hPacked;
+      homPackedLayernormF16(e->hPacked.m.rank, e->hPacked.m.descriptor, out.m.rank,
+                            out.m.descriptor, e->eps,
+                            last ? HOM_PACKED_A : HOM_PACKED_A | HOM_PACKED_D);
+    }
   }
-  nvteLayernormF16(e->h.m.rank, e->h.m.descriptor, e->eps);
 }
 
 void callList(HomBertEncoder *e, int fromIds) {
@@ -672,6 +696,7 @@ DRV_EXPORT void homBertDestroy(HomBertEncoder *e) {
                     &e->f, &e->wTransform, &e->wDecoder, &e->t, &e->logits})
     t->release();
   e->hPacked.release();
+  e->qkvPacked.release();
   e->attnPacked.release();
   e->fPacked.release();
   (void)hipFree(e->packedArena);

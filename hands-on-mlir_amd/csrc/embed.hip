@@ -23,11 +23,11 @@ constexpr int kWave = 64;
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 
 constexpr int kThreads = 1024, kWaves = kThreads / kWave;
-// Token rows of a wavefront, consecutive: their ids arrive with one request.
-constexpr int kRows = 4;
 
-// VPL: 16-byte vectors of a row per lane.
-template <int VPL>
+// VPL: 16-byte vectors of a row per lane; kRows: token rows of a wavefront,
+// consecutive, whose ids arrive with one request: 4 where there are enough rows
+// to fill the chip, 1 where the chain of latencies (id, row, result) counts.
+template <int VPL, int kRows>
 __global__ __launch_bounds__(kThreads) void embedKernel(
     const int64_t *__restrict__ ids, const int64_t *__restrict__ mask,
     const _Float16 *__restrict__ word, const _Float16 *__restrict__ pos,
@@ -44,9 +44,11 @@ __global__ __launch_bounds__(kThreads) void embedKernel(
   const int row0 = (int(blockIdx.x - 1) * kWaves + wave) * kRows;
   if (row0 >= rows)
     return;
-  // lane l holds the id of row l % kRows
-  const int idRow = row0 + lane % kRows < rows ? row0 + lane % kRows : rows - 1;
-  const int64_t idWant = ids[idRow];
+  // Lane l < kRows holds the id of row row0 + l.  (The other lanes ask for
+  // nothing: every lane's request of uncached host memory is one of its own.)
+  int64_t idWant = 0;
+  if (lane < kRows)
+    idWant = ids[row0 + lane < rows ? row0 + lane : rows - 1];
   // An index outside the table would read foreign memory; clamp it.
   const int id = idWant < 0 ? 0 : (idWant >= vocab ? vocab - 1 : int(idWant));
   const int nvec = hidden / 8;
@@ -96,11 +98,15 @@ __global__ __launch_bounds__(kThreads) void embedKernel(
 #pragma unroll
       for (int e = 0; e < 8; e++)
         o[e] = _Float16((v[i][e] - mean) * rstd);
-      if (row0 + r < rows && lane + i * kWave < nvec)
-        storeWriteThrough(
-            out + (packedOut ? packedOffset(row0 + r, (lane + i * kWave) * 8, hidden)
-                             : int64_t(row0 + r) * hidden + (lane + i * kWave) * 8),
-            o);
+      if (row0 + r < rows && lane + i * kWave < nvec) {
+        // (fragment order: 16 bytes of a line that the rows next to this one
+        // complete, which is for the L2 to put together)
+        if (packedOut)
+          *reinterpret_cast<half8 *>(
+              out + packedOffset(row0 + r, (lane + i * kWave) * 8, hidden)) = o;
+        else
+          storeWriteThrough(out + int64_t(row0 + r) * hidden + (lane + i * kWave) * 8, o);
+      }
     }
   }
 }
@@ -111,7 +117,7 @@ bool embedFits(const _Float16 *word, const _Float16 *pos, const _Float16 *out,
                int64_t bs, int64_t seq, int64_t hidden, int64_t vocab) {
   auto al16 = [](const void *q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
   return hidden % 8 == 0 && hidden <= 4 * kWave * 8 && al16(word) && al16(pos) &&
-         al16(out) && bs * seq < (int64_t(1) << 31) - kWaves * kRows &&
+         al16(out) && bs * seq < (int64_t(1) << 31) - kWaves * 4 &&
          vocab < (int64_t(1) << 31);
 }
 
@@ -119,13 +125,15 @@ Status launchEmbed(const int64_t *ids, const int64_t *mask, const _Float16 *word
                    const _Float16 *pos, _Float16 *out, int32_t *cu, int64_t bs,
                    int64_t seq, int64_t hidden, int64_t vocab, float eps,
                    bool packedOut, hipStream_t s) {
-  const int64_t rows = bs * seq, perBlock = kWaves * kRows;
+  const int64_t rows = bs * seq;
+  const bool few = rows <= 4096;
+  const int64_t perBlock = kWaves * (few ? 1 : 4);
   const dim3 grid((unsigned)(1 + (rows + perBlock - 1) / perBlock)), block(kThreads);
   const uint32_t magic = magicFor(uint32_t(seq));
   const int nvec = int(hidden / 8);
-  auto kernel = nvec <= kWave       ? embedKernel<1>
-                : nvec <= 2 * kWave ? embedKernel<2>
-                                    : embedKernel<4>;
+  auto kernel = nvec <= kWave       ? (few ? embedKernel<1, 1> : embedKernel<1, 4>)
+                : nvec <= 2 * kWave ? (few ? embedKernel<2, 1> : embedKernel<2, 4>)
+                                    : (few ? embedKernel<4, 1> : embedKernel<4, 4>);
   kernel<<<grid, block, 0, s>>>(ids, mask, word, pos, out, cu, int(bs), int(seq),
                                 int(hidden), int(vocab), magic, eps, packedOut);
   HOM_HIP_RET(hipGetLastError(), Status::kInternal);

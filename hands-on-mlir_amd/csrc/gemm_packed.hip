@@ -20,10 +20,14 @@
 // sum and sum of squares on the way and the epilogue applies
 //   LN(A) . B = rstd (A . B) - mu rstd colsum(B)
 // with colsum(B) from packing time; the statistics are written for the later
-// GEMM whose residual source is the same tensor, LN(C) = rstd c - mu rstd.
+// GEMM whose residual source is the same tensor, LN(C) = rstd c - mu rstd,
+// rounded to fp16 where the graph stores it: the residual is what carries rounding
+// from layer to layer, and without that point 12 layers come out 1.74e-3 instead
+// of 1.28e-3 (in norm) from a pipeline with separate layer norms (1.23e-3 apart
+// from itself in another summation order; 1.41e-3 against 1.44e-3 from fp32).
 #include "cross_lane.h"
 #include "fast_div.h"
-#include "kernels.h"
+#include "packed_args.h"
 #include "store_policy.h"
 
 #include <algorithm>
@@ -40,37 +44,6 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kWave = 64, kWaves = 8, kThreads = kWave * kWaves;
 constexpr uint32_t kOob = 0x80000000u;
-
-// GELU as the tiled kernels' epilogues compute it (gemm_device.h).
-__device__ __forceinline__ float geluErf(float x) {
-  const float ax = fabsf(x);
-  const float a = fminf(ax, 8.0f);
-  float P = fmaf(3.448796997e-05f, a, -7.812886615e-04f);
-  P = fmaf(P, a, 8.119936101e-03f);
-  P = fmaf(P, a, -5.347220227e-02f);
-  P = fmaf(P, a, -4.587264359e-01f);
-  P = fmaf(P, a, -1.151216269e+00f);
-  P = fmaf(P, a, 8.451195754e-06f);
-  return fmaf(-0.5f * ax, __builtin_amdgcn_exp2f(P), fmaxf(x, 0.0f));
-}
-__device__ __forceinline__ float geluTanh(float x) {
-  const float w = fmaf(x * x, -0.1029432397f, -2.3022081983f);
-  return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x * w));
-}
-
-struct PackedArgs {
-  const _Float16 *C; // residual source [M, N] or null
-  _Float16 *D;
-  const float *colSum;  // [N], read when A is normalised
-  const float *statsIn; // (rstd, -mu rstd) per row of C, or null: C as it is
-  float *statsOut;      // (rstd, -mu rstd) per row of A, or null
-  const char *ahead;    // weights of the kernels behind this one
-  int64_t aheadBytes;
-  int M, N;
-  int activation; // 0, 1 erf GELU, 2 tanh GELU
-  int cPacked, dPacked; // in fragment order
-  float invK, eps;
-};
 
 // MB x NB blocks of 16 x 16 per workgroup; CH k steps of a wavefront in flight
 // at once (ONCE: that is all of them).  The leading scalars arrive
@@ -153,23 +126,7 @@ __global__ __launch_bounds__(kThreads, (MB + NB) * CH <= 20 && (ONCE || !NORM_A)
   }
 #endif
   if (!isTile) {
-    // Workgroups behind the tiles read weights that the next kernels need, so
-    // that those find them in the last-level cache: a lone small GEMM leaves
-    // CUs and most of the memory system idle.
-    constexpr int kLoads = 8;
-    const int64_t step = int64_t(gridDim.x - tiles) * (kThreads * 16 * kLoads);
-    for (int64_t at = int64_t(id - tiles) * (kThreads * 16 * kLoads); at < p.aheadBytes;
-         at += step) {
-      u32x4 v[kLoads];
-#pragma unroll
-      for (int i = 0; i < kLoads; i++) {
-        const int64_t o = at + (i * kThreads + tid) * 16;
-        v[i] = *reinterpret_cast<const u32x4 *>(p.ahead + (o < p.aheadBytes ? o : 0));
-      }
-#pragma unroll
-      for (int i = 0; i < kLoads; i++)
-        asm volatile("" ::"v"(v[i])); // (nothing else uses the values)
-    }
+    readAhead<kThreads>(p.ahead, p.aheadBytes, id - tiles, int(gridDim.x) - tiles, tid);
     return;
   }
   // What the epilogue reads: thread t < MB * NB * 64 finishes 4 consecutive
@@ -277,14 +234,78 @@ __global__ __launch_bounds__(kThreads, (MB + NB) * CH <= 20 && (ONCE || !NORM_A)
   for (int e = 0; e < 4; e++) {
     float x = v[e];
     if (p.activation == 1)
-      x = geluErf(x);
+      x = packedGeluErf(x);
     else if (p.activation == 2)
-      x = geluTanh(x);
+      x = packedGeluTanh(x);
     if (p.C)
-      x += fmaf(float(cv[e]), cStat[0], cStat[1]);
+      x += float(_Float16(fmaf(float(cv[e]), cStat[0], cStat[1])));
     o[e] = _Float16(x);
   }
   storeWriteThrough(p.D + (p.dPacked ? packed : plain), o);
+}
+
+// Layer norm without affine parameters of rows in fragment order; the result in
+// the same order (out may be in) or row-major.  A workgroup owns a block of 16
+// rows, its wavefronts every eighth kilobyte of it, the row in registers for
+// both passes: whole cache lines, where a wavefront per row would touch eight
+// rows' lines for its own 16 bytes of each.
+template <int VPW> // kilobytes per wavefront
+__global__ __launch_bounds__(kThreads) void packedLayernormKernel(const _Float16 *in, _Float16 *out,
+                                                                  int M, int N, bool outPacked,
+                                                                  float eps) {
+  __shared__ float part[2][kWaves][16];
+  const int lane = threadIdx.x % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int blocks = N / 32, r = lane % 16;
+  const half8 *src = reinterpret_cast<const half8 *>(in) + int64_t(blockIdx.x) * blocks * kWave;
+  half8 raw[VPW];
+#pragma unroll
+  for (int i = 0; i < VPW; i++) {
+    const int j = i * kWaves + wave;
+    raw[i] = src[(j < blocks ? j : 0) * kWave + lane];
+  }
+  __builtin_amdgcn_sched_barrier(0); // every request is out
+  auto rowTotal = [&](float v, int which) { // over the row's lanes and wavefronts
+    v = pairSum(rowPairSum(v));
+    if (lane < 16)
+      part[which][wave][lane] = v;
+    __syncthreads();
+    v = 0.f;
+#pragma unroll
+    for (int w = 0; w < kWaves; w++)
+      v += part[which][w][r];
+    return v;
+  };
+  float sum = 0.f;
+#pragma unroll
+  for (int i = 0; i < VPW; i++)
+#pragma unroll
+    for (int e = 0; e < 8; e++)
+      sum += i * kWaves + wave < blocks ? float(raw[i][e]) : 0.f;
+  const float invN = 1.0f / float(N);
+  const float mean = rowTotal(sum, 0) * invN;
+  float sq = 0.f;
+#pragma unroll
+  for (int i = 0; i < VPW; i++)
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+      const float d = i * kWaves + wave < blocks ? float(raw[i][e]) - mean : 0.f;
+      sq += d * d;
+    }
+  const float rstd = 1.0f / sqrtf(rowTotal(sq, 1) * invN + eps);
+  const int64_t row = int64_t(blockIdx.x) * 16 + r;
+#pragma unroll
+  for (int i = 0; i < VPW; i++) {
+    const int j = i * kWaves + wave;
+    half8 o;
+#pragma unroll
+    for (int e = 0; e < 8; e++)
+      o[e] = _Float16((float(raw[i][e]) - mean) * rstd);
+    if (j < blocks && (outPacked || row < M))
+      storeWriteThrough(outPacked ? out + (int64_t(blockIdx.x) * blocks + j) * 512 + lane * 8
+                                  : out + row * N + j * 32 + (lane / 16) * 8,
+                        o);
+  }
 }
 
 // B [K, N] row-major -> fragments: block (column block j, k step s) is 1 KiB,
@@ -342,6 +363,18 @@ Status launchPackWeight(const _Float16 *B, _Float16 *packed, int64_t K, int64_t 
   return Status::kSuccess;
 }
 
+Status launchPackedLayernorm(const _Float16 *in, _Float16 *out, int64_t M, int64_t N, float eps,
+                             bool outPacked, hipStream_t s) {
+  const dim3 grid((unsigned)((M + 15) / 16)), block(kThreads);
+  const int perWave = int((N / 32 + kWaves - 1) / kWaves);
+  auto kernel = perWave <= 3   ? packedLayernormKernel<3>
+                : perWave <= 4 ? packedLayernormKernel<4>
+                               : packedLayernormKernel<8>;
+  kernel<<<grid, block, 0, s>>>(in, out, int(M), int(N), outPacked, eps);
+  HOM_HIP_RET(hipGetLastError(), Status::kInternal);
+  return Status::kSuccess;
+}
+
 Status launchPackedGemm(const PackedGemm &g, hipStream_t s) {
   PackedArgs p{};
   p.C = g.C;
@@ -358,13 +391,15 @@ Status launchPackedGemm(const PackedGemm &g, hipStream_t s) {
   p.eps = g.eps;
   p.ahead = static_cast<const char *>(g.ahead);
   p.aheadBytes = g.ahead ? g.aheadBytes : 0;
+  const PackedTileChoice tiled = choosePackedTile(g);
   // k steps per wavefront, all in flight at once where the registers allow
   const int perWave = int((g.K / 32 + kWaves - 1) / kWaves);
   // The tile by a model of its time in a chain of launches, fitted to M = 16 ..
-  // 384 x the shapes of BERT-base and -large (within 10 %): launch, latency and
+  // 2048 x the shapes of BERT-base and -large (within 10 %): launch, latency and
   // the meeting of the partial sums, then what the fullest CU pulls through its
   // L1; workgroups of a CU beyond those that fit its registers at once start a
-  // second chain of latencies.
+  // second chain of latencies.  (Those of the tile kernels that fill the chip do
+  // not read ahead, which is worth most of a microsecond to the launch behind.)
   const int cus = deviceInfo().computeUnits > 0 ? deviceInfo().computeUnits : 256;
   struct Shape {
     int mb, nb, resident;
@@ -373,7 +408,6 @@ Status launchPackedGemm(const PackedGemm &g, hipStream_t s) {
                            {2, 1, 2},
                            {4, 1, 2},
                            {4, 2, perWave == 4 ? 1 : 2}};
-  const double usPerKb = perWave <= 4 ? 0.0088 : 0.0062;
   int best = 0;
   double bestCost = 1e300;
   int64_t bestTiles = 0;
@@ -384,20 +418,22 @@ Status launchPackedGemm(const PackedGemm &g, hipStream_t s) {
     const int64_t tiles = ((g.M + t.mb * 16 - 1) / (t.mb * 16)) * (g.N / (t.nb * 16));
     const int64_t perCu = (tiles + cus - 1) / cus;
     const double kb = double(t.mb + t.nb) * 16 * double(g.K) * 2 / 1024;
-    const double cost = 2.1 + 0.1 * t.mb * t.nb + usPerKb * kb * double(perCu) +
-                        0.8 * double((perCu - 1) / t.resident);
+    // (deep K: rounds of two workgroups, since one alone fetches half as fast, and
+    // the matrix cores have their say in the largest tile)
+    const double usPerKb = perWave <= 4 ? 0.0088 : t.mb * t.nb == 8 ? 0.0104 : 0.0062;
+    const int64_t paired = perWave <= 4 || perCu == 1 ? perCu : (perCu + 1) / 2 * 2;
+    const double cost = 2.1 + 0.1 * t.mb * t.nb + usPerKb * kb * double(paired) +
+                        (t.resident == 1 ? 1.8 : 1.0) * double((perCu - 1) / t.resident);
     if (cost < bestCost) {
       bestCost = cost;
       best = i;
       bestTiles = tiles;
     }
   }
-  // (64 KiB per workgroup that reads ahead; half the CUs when the tiles take
-  // all of them)
-  constexpr int64_t kAheadBytes = kThreads * 16 * 8;
-  const int groups =
-      int(std::min<int64_t>((p.aheadBytes + kAheadBytes - 1) / kAheadBytes,
-                            std::max<int64_t>(cus - bestTiles, cus / 2)));
+  if (tiled.us + (g.ahead ? 0.7 : 0.0) < bestCost)
+    return launchPackedTile(tiled.tile, g, p, s);
+  // (half the CUs read ahead when the tiles take all of them)
+  const int groups = aheadGroups<kThreads>(p.aheadBytes, std::max<int64_t>(cus - bestTiles, cus / 2));
   switch (best) {
   case 0:
     return perWave <= 3    ? launchVariant<1, 1, 3, true>(g, p, groups, s)

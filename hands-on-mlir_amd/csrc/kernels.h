@@ -67,7 +67,9 @@ Status launchEmbed(const int64_t *ids, const int64_t *mask, const _Float16 *word
 Status launchBertAttentionF16(const _Float16 *qkv, const int32_t *cuSeqlens,
                               _Float16 *out, int64_t bs, int64_t seq,
                               int64_t heads, int64_t headDim, float scale,
-                              hipStream_t s, bool packedOut = false);
+                              hipStream_t s, bool packedOut = false,
+                              bool packedIn = false, const void *ahead = nullptr,
+                              int64_t aheadBytes = 0);
 
 // ------------------------------------------------------------------ gemm --
 enum class Epilogue : int { kLinear = 0, kGeluErf = 1, kGeluTanh = 2 };
@@ -194,6 +196,10 @@ struct PackedGemm {
   int64_t aheadBytes;
 };
 Status launchPackedGemm(const PackedGemm &g, hipStream_t s);
+// Layer norm (no affine parameters) of M rows of N <= 2048 values in fragment
+// order; out: the same order (may be in) or row-major.
+Status launchPackedLayernorm(const _Float16 *in, _Float16 *out, int64_t M, int64_t N, float eps,
+                             bool outPacked, hipStream_t s);
 // B [K, N] row-major, dense -> the layout above, K * N values.
 Status launchPackWeight(const _Float16 *B, _Float16 *packed, int64_t K, int64_t N,
                         hipStream_t s);

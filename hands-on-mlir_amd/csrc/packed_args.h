@@ -1,0 +1,76 @@
+// What the two packed GEMM kernels (gemm_packed.hip, gemm_packed_tile.hip) share.
+#pragma once
+
+#include "kernels.h"
+
+namespace hom {
+
+struct PackedArgs {
+  const _Float16 *C; // residual source [M, N] or null
+  _Float16 *D;
+  const float *colSum;  // [N], read when A is normalised
+  const float *statsIn; // (rstd, -mu rstd) per row of C, or null: C as it is
+  float *statsOut;      // (rstd, -mu rstd) per row of A, or null
+  const char *ahead;    // weights of the kernels behind this one
+  int64_t aheadBytes;
+  int M, N;
+  int activation;       // 0, 1 erf GELU, 2 tanh GELU
+  int cPacked, dPacked; // in fragment order
+  float invK, eps;
+};
+
+// A workgroup behind those with work of their own reads weights that the next
+// kernels need, so that those find them in the last-level cache: a lone small
+// kernel leaves CUs and most of the memory system idle.  Group `group` of
+// `groups` takes its runs of kAheadBytes<THREADS>.
+constexpr int kAheadLoads = 8;
+template <int THREADS> constexpr int64_t kAheadBytes = int64_t(THREADS) * 16 * kAheadLoads;
+template <int THREADS>
+__device__ __forceinline__ void readAhead(const char *ahead, int64_t bytes, int group, int groups,
+                                          int tid) {
+  typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+  for (int64_t at = group * kAheadBytes<THREADS>; at < bytes;
+       at += groups * kAheadBytes<THREADS>) {
+    u32x4 v[kAheadLoads];
+#pragma unroll
+    for (int i = 0; i < kAheadLoads; i++) {
+      const int64_t o = at + (i * THREADS + tid) * 16;
+      v[i] = *reinterpret_cast<const u32x4 *>(ahead + (o < bytes ? o : 0));
+    }
+#pragma unroll
+    for (int i = 0; i < kAheadLoads; i++)
+      asm volatile("" ::"v"(v[i])); // (nothing else uses the values)
+  }
+}
+// Workgroups to add for that: one for each run, up to `most`.
+template <int THREADS> inline int aheadGroups(int64_t bytes, int64_t most) {
+  const int64_t runs = (bytes + kAheadBytes<THREADS> - 1) / kAheadBytes<THREADS>;
+  return int(runs < most ? runs : most < 0 ? 0 : most);
+}
+
+// GELU as the tiled kernels' epilogues compute it (gemm_device.h).
+__device__ __forceinline__ float packedGeluErf(float x) {
+  const float ax = fabsf(x);
+  const float a = fminf(ax, 8.0f);
+  float P = fmaf(3.448796997e-05f, a, -7.812886615e-04f);
+  P = fmaf(P, a, 8.119936101e-03f);
+  P = fmaf(P, a, -5.347220227e-02f);
+  P = fmaf(P, a, -4.587264359e-01f);
+  P = fmaf(P, a, -1.151216269e+00f);
+  P = fmaf(P, a, 8.451195754e-06f);
+  return fmaf(-0.5f * ax, __builtin_amdgcn_exp2f(P), fmaxf(x, 0.0f));
+}
+__device__ __forceinline__ float packedGeluTanh(float x) {
+  const float w = fmaf(x * x, -0.1029432397f, -2.3022081983f);
+  return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x * w));
+}
+
+// The tiled kernel (A packed); false: no tile of it suits the problem.
+struct PackedTileChoice {
+  int tile;
+  double us; // modelled time
+};
+PackedTileChoice choosePackedTile(const PackedGemm &g);
+Status launchPackedTile(int tile, const PackedGemm &g, const PackedArgs &p, hipStream_t s);
+
+} // namespace hom

@@ -113,9 +113,10 @@ void nvteBertAttentionF16(int64_t rankA, void *dstA, int64_t rankSeqlen,
 }
 void homBertAttentionF16(int64_t rankA, void *dstA, int64_t rankSeqlen,
                          void *dstSeqlen, int64_t rankOut, void *dstOut,
-                         float scale, int64_t headNum, int32_t packing) {
+                         float scale, int64_t headNum, int32_t packing,
+                         const void *ahead, int64_t aheadBytes) {
   (void)runBertAttentionF16(rankA, dstA, rankSeqlen, dstSeqlen, rankOut, dstOut,
-                            scale, headNum, (packing & HOM_PACKED_D) != 0);
+                            scale, headNum, packing, ahead, aheadBytes);
 }
 void nvteBertAttentionF32(int64_t, void *, int64_t, void *, int64_t, void *,
                           float, int64_t) {
@@ -231,6 +232,11 @@ int32_t homFoldedLayernormPieces(int64_t M, int64_t N, int64_t K,
 
 void homPackWeightF16(int64_t rankB, void *dstB, void *packed) {
   (void)runPackWeight(rankB, dstB, packed);
+}
+
+void homPackedLayernormF16(int64_t rankA, void *dstA, int64_t rankOut,
+                           void *dstOut, float eps, int32_t packing) {
+  (void)runPackedLayernorm(rankA, dstA, rankOut, dstOut, eps, packing);
 }
 
 void homPackedGemmF16(int64_t rankA, void *dstA, const void *packedB,

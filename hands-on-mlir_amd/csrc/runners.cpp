@@ -570,6 +570,31 @@ Status runPackWeight(int64_t rankB, void *dstB, void *packed) {
                           B.sizes[2], stream());
 }
 
+Status runPackedLayernorm(int64_t rankA, void *dstA, int64_t rankOut, void *dstOut,
+                          float eps, int32_t packing) {
+  View<_Float16> A(rankA, dstA), O(rankOut, dstOut);
+  HOM_CHECK_RET(A.rank == 3 && O.rank == 3 && A.sizes && O.sizes &&
+                    A.contiguous() && O.contiguous() &&
+                    A.sizes[0] == O.sizes[0] && A.sizes[1] == O.sizes[1] &&
+                    A.sizes[2] == O.sizes[2],
+                Status::kInvalidArgument,
+                "packed layer norm: A and Out must be contiguous tensors of one "
+                "[b, s, H] shape");
+  const int64_t M = A.sizes[0] * A.sizes[1], N = A.sizes[2];
+  HOM_CHECK_RET((packing & HOM_PACKED_A) && N % 32 == 0 && N <= 2048 &&
+                    M < (int64_t(1) << 31) - 16,
+                Status::kInvalidArgument,
+                "packed layer norm: A must be in fragment order with H a multiple "
+                "of 32, at most 2048");
+  HOM_CHECK_RET(A.data != O.data || (packing & HOM_PACKED_D),
+                Status::kInvalidArgument,
+                "packed layer norm: a row-major result cannot replace A");
+  if (M == 0 || N == 0)
+    return Status::kSuccess;
+  return launchPackedLayernorm(A.data, O.data, M, N, eps,
+                               (packing & HOM_PACKED_D) != 0, stream());
+}
+
 Status runPackedGemm(int64_t rankA, void *dstA, const void *packedB, int64_t rankC,
                      void *dstC, int64_t rankD, void *dstD, int64_t activation,
                      int32_t normA, float eps, const float *colSumB,
@@ -630,7 +655,7 @@ Status runPackedGemm(int64_t rankA, void *dstA, const void *packedB, int64_t ran
   g.normA = normA != 0;
   g.eps = eps;
   g.ahead = ahead;
-  g.aheadBytes = aheadBytes;
+  g.aheadBytes = aheadBytes & ~int64_t(15);
   return launchPackedGemm(g, stream());
 }
 
@@ -971,7 +996,8 @@ Status runAddLayernormF16(int64_t rankX, void *dstX, int64_t rankRes,
 // --------------------------------------------------------------- attention --
 Status runBertAttentionF16(int64_t rankA, void *dstA, int64_t rankSeqlen,
                            void *dstSeqlen, int64_t rankOut, void *dstOut,
-                           float scale, int64_t headNum, bool packedOut) {
+                           float scale, int64_t headNum, int32_t packing,
+                           const void *ahead, int64_t aheadBytes) {
   View<_Float16> A(rankA, dstA), Out(rankOut, dstOut);
   View<int32_t> Seq(rankSeqlen, dstSeqlen);
   // BertAttentionRunner::construct_tensors (BertAttentionRunner.h:61-73)
@@ -998,8 +1024,12 @@ Status runBertAttentionF16(int64_t rankA, void *dstA, int64_t rankSeqlen,
                 "attention: cu_seqlens must be int32[%lld]", (long long)bs + 1);
   HOM_CHECK_RET(A.contiguous() && Out.contiguous(), Status::kInvalidArgument,
                 "attention: tensors must be contiguous");
+  HOM_CHECK_RET((reinterpret_cast<uintptr_t>(ahead) & 15) == 0,
+                Status::kInvalidArgument, "attention: misaligned memory to read ahead");
   return launchBertAttentionF16(A.data, Seq.data, Out.data, bs, seq, headNum,
-                                headDim, scale, stream(), packedOut);
+                                headDim, scale, stream(),
+                                (packing & HOM_PACKED_D) != 0,
+                                (packing & HOM_PACKED_A) != 0, ahead, ahead ? aheadBytes & ~int64_t(15) : 0);
 }
 
 // ------------------------------------------------------------- elementwise --

@@ -46,6 +46,8 @@ Status runGemmFoldedLayernorm(int64_t rankA, void *dstA, int64_t rankB,
 int32_t foldedLayernormPieces(int64_t M, int64_t N, int64_t K, int64_t activation,
                               int32_t likeGemmNum);
 Status runPackWeight(int64_t rankB, void *dstB, void *packed);
+Status runPackedLayernorm(int64_t rankA, void *dstA, int64_t rankOut, void *dstOut,
+                          float eps, int32_t packing);
 Status runPackedGemm(int64_t rankA, void *dstA, const void *packedB, int64_t rankC,
                      void *dstC, int64_t rankD, void *dstD, int64_t activation,
                      int32_t normA, float eps, const float *colSumB,
@@ -121,7 +123,8 @@ Status runAddLayernormF16(int64_t rankX, void *dstX, int64_t rankRes,
                           void *dstOut, float eps);
 Status runBertAttentionF16(int64_t rankA, void *dstA, int64_t rankSeqlen,
                            void *dstSeqlen, int64_t rankOut, void *dstOut,
-                           float scale, int64_t headNum, bool packedOut = false);
+                           float scale, int64_t headNum, int32_t packing = 0,
+                           const void *ahead = nullptr, int64_t aheadBytes = 0);
 template <typename T>
 Status runElementwise(BinOp op, int64_t rankA, void *dstA, int64_t rankB,
                       void *dstB, int64_t rankOut, void *dstOut);

@@ -227,3 +227,102 @@ def test_packed_gemm(gpu, rt, oracle, M, N, K, packing):
         np.testing.assert_allclose(result(td).astype(np.float64), z, rtol=2e-3, atol=1e-2)
         np.testing.assert_allclose(host(out)[:, 0], rstd, rtol=1e-4)
         np.testing.assert_allclose(host(out)[:, 1], -x.mean(1) * rstd, rtol=1e-3, atol=1e-4)
+
+
+# every tile of the packed GEMM for many rows, with one tile and with several of them per workgroup; partial row
+# blocks and column tiles
+@pytest.mark.parametrize("M,N,K", [(392, 1184, 64), (524, 1856, 64), (583, 3296, 64), (1476, 2976, 448),
+                                   (16439, 160, 64), (10970, 352, 192), (17111, 288, 64), (16546, 672, 128),
+                                   (16388, 1696, 128)])
+def test_packed_gemm_many_rows(gpu, rt, M, N, K):
+    g = torch.Generator("cuda").manual_seed(M)
+    Mr, R = rt.MemRef, -(-M // 16) * 16
+
+    def rand(*shape, std=1.0):
+        return (torch.randn(shape, device="cuda", generator=g) * std).half()
+
+    def order(a):
+        p = torch.zeros(R, a.shape[1], dtype=a.dtype, device="cuda")
+        p[:M] = a
+        return p.view(-1, 16, a.shape[1] // 32, 4, 8).permute(0, 2, 3, 1, 4).contiguous().view(-1)
+
+    A, B, C = rand(M, K) + 0.3, rand(K, N, std=0.05), rand(M, N)
+    packed, stats = torch.zeros(K * N, dtype=torch.float16, device="cuda"), torch.rand(M, 2, device="cuda", generator=g)
+    gpu.homPackWeightF16(*Mr(B.data_ptr(), [1, K, N]).args(), packed.data_ptr())
+    ta, tc, td = order(A), order(C), torch.zeros(R * N, dtype=torch.float16, device="cuda")
+    ma, mc, md = (Mr(t.data_ptr(), [1, M, w]) for t, w in ((ta, K), (tc, N), (td, N)))
+    out, colsum = torch.zeros(M, 2, device="cuda"), B.float().sum(0)
+
+    def check(want, rtol):
+        got = td.view(-1, N // 32, 4, 16, 8).permute(0, 3, 1, 2, 4).reshape(R, N)[:M].double()
+        torch.testing.assert_close(got, want, rtol=rtol, atol=1e-2)
+
+    x, w = A.double(), B.double()
+    gpu.homPackedGemmF16(*ma.args(), packed.data_ptr(), *mc.args(), *md.args(), 0, 0, 1e-6, None, stats.data_ptr(), None,
+                         7, packed.data_ptr(), 2 * K * N)
+    check(x @ w + C.double() * stats[:, :1].double() + stats[:, 1:].double(), 1e-3)
+    rstd = (x.var(1, unbiased=False) + 1e-6).rsqrt()
+    z = ((x - x.mean(1, keepdim=True)) * rstd[:, None]) @ w
+    for act, fn in ((0, lambda v: v), (1, torch.nn.functional.gelu), (2, lambda v: torch.nn.functional.gelu(v, approximate="tanh"))):
+        gpu.homPackedGemmF16(*ma.args(), packed.data_ptr(), 0, None, *md.args(), act, 1, 1e-6, colsum.data_ptr(), None,
+                             out.data_ptr(), 5, None, 0)
+        check(fn(z), 2e-3)
+        torch.testing.assert_close(out[:, 0].double(), rstd, rtol=1e-4, atol=0)
+        gpu.homPackedGemmF16(*ma.args(), packed.data_ptr(), 0, None, *md.args(), act, 0, 1e-6, None, None, None, 5, None, 0)
+        check(fn(x @ w), 1e-3)
+
+
+@pytest.mark.parametrize("M,H", [(1, 32), (17, 96), (33, 768), (16, 800), (50, 1024), (15, 1056), (100, 2048)])
+def test_packed_layernorm(gpu, rt, M, H):
+    x = (np.random.default_rng(M + H).standard_normal((M, H)) * 2 + 0.5).astype(np.float16)
+    Mr, R = rt.MemRef, -(-M // 16) * 16
+    t, rows = dev(fragment_order(x)), torch.zeros((M, H), dtype=torch.float16, device="cuda")
+    m = Mr(t.data_ptr(), [1, M, H])
+    want = torch.nn.functional.layer_norm(torch.from_numpy(x).double(), (H,), eps=1e-6).numpy()
+    gpu.homPackedLayernormF16(*m.args(), *Mr(rows.data_ptr(), [1, M, H]).args(), 1e-6, 1)
+    np.testing.assert_allclose(host(rows), want, rtol=1e-3, atol=2e-3)
+    gpu.homPackedLayernormF16(*m.args(), *m.args(), 1e-6, 5)
+    got = host(t).reshape(-1, H // 32, 4, 16, 8).transpose(0, 3, 1, 2, 4).reshape(R, H)[:M]
+    np.testing.assert_array_equal(got, host(rows))
+
+
+# both variants of the attention kernel; batch entries that start inside a row block, chunk ends inside one
+@pytest.mark.parametrize("bs,seq,heads", [(1, 1, 1), (3, 33, 2), (2, 64, 12), (5, 99, 16), (2, 300, 4), (24, 128, 12),
+                                          (40, 200, 8), (257, 17, 3)])
+def test_attention_in_fragment_order(gpu, rt, bs, seq, heads):
+    g, H = np.random.default_rng(bs + seq), heads * 64
+    rows, Mr = bs * seq, rt.MemRef
+    R = -(-rows // 16) * 16
+    qkv = g.standard_normal((rows, 3 * H)).astype(np.float16)
+    lens = g.integers(1, seq + 1, bs)
+    cu = dev(np.concatenate([[0], np.cumsum(lens)]).astype(np.int32))
+    a, out = dev(qkv.reshape(bs, seq, 3 * H)), torch.zeros((bs, seq, H), dtype=torch.float16, device="cuda")
+    gpu.nvteBertAttentionF16(*Mr.from_tensor(a).args(), *Mr.from_tensor(cu).args(), *Mr.from_tensor(out).args(), 0.125, heads)
+    p, packed = dev(fragment_order(qkv)), torch.zeros(R * H, dtype=torch.float16, device="cuda")
+    gpu.homBertAttentionF16(*Mr(p.data_ptr(), [bs, seq, 3 * H]).args(), *Mr.from_tensor(cu).args(),
+                            *Mr(packed.data_ptr(), [bs, seq, H]).args(), 0.125, heads, 5, p.data_ptr(), 6 * rows * H)
+    got = host(packed).reshape(-1, H // 32, 4, 16, 8).transpose(0, 3, 1, 2, 4).reshape(R, H)[:rows].reshape(bs, seq, H)
+    want = host(out)
+    for b in range(bs):
+        np.testing.assert_allclose(got[b, :lens[b]].astype(np.float32), want[b, :lens[b]].astype(np.float32), rtol=2e-3,
+                                   atol=1e-3)
+
+
+@pytest.mark.parametrize("bs,seq", [(300, 128), (340, 127)])
+def test_encoder_many_rows_equals_row_major(synth, bs, seq):
+    """Enough rows for packed layer norms of their own, against the same weights on the row-major path."""
+    import importlib
+    bert = importlib.import_module("hands-on-mlir_amd.bert")
+    model = synth.bert_encoder(layers=2, hidden=128, heads=2, ffn=512, bs=bs, seq=seq, vocab=1000, config=40)
+    got = []
+    for layout in (None, {"qkv": "kn"}):
+        enc = bert.BertEncoder(2, 128, 2, 512, bs, seq, 1000, gemm_mode=1, gelu_form="erf", role_layout=layout)
+        try:
+            enc.load(model)
+            enc.set_inputs(ids=model["ids"], mask=model["mask"])
+            enc.forward()
+            got.append(enc.output().astype(np.float32))
+        finally:
+            enc.close()
+    live = np.asarray(model["mask"]).astype(bool)
+    np.testing.assert_allclose(got[0][live], got[1][live], rtol=1e-2, atol=1e-2)
