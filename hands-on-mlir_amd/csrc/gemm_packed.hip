@@ -52,32 +52,24 @@ constexpr uint32_t kOob = 0x80000000u;
 // behind those requests.
 template <int MB, int NB, int CH, bool ONCE, bool NORM_A, bool A_PACKED>
 __global__ __launch_bounds__(kThreads, (MB + NB) * CH <= 20 && (ONCE || !NORM_A) ? 4 : 2) void packedGemmKernel(
-    const _Float16 *A, const _Float16 *B, int M, int K, int steps, int perWave,
-    int tilesM, int tilesN, uint32_t tilesMMagic, int tiles, PackedArgs rest) {
+    const _Float16 *A, const _Float16 *B, int M, int N, int K, int steps, int perWave,
+    int chunkM, uint32_t chunkMMagic, int chunkN, int xmLog, PackedArgs rest) {
   (void)rest; // (through the argument pointer, see below)
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int tid = threadIdx.x, lane = tid % kWave;
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int id = blockIdx.x;
-  // Tiles of one column block lie on one XCD (ids 8 apart), whose L2 then
-  // fetches that part of B once.
-  int tileM, tileN;
-  if (tilesN % 8 == 0) {
-    const int loc = id / 8;
-    const int q = int(divByMagic(uint32_t(loc), uint32_t(tilesM), tilesMMagic));
-    tileM = loc - q * tilesM;
-    tileN = q * 8 + id % 8;
-  } else {
-    tileN = int(divByMagic(uint32_t(id), uint32_t(tilesM), tilesMMagic));
-    tileM = id - tileN * tilesM;
-  }
+  // XCD id % 8 owns a rectangle of chunkM x chunkN tiles (chooseRectangles()).
+  const int xcd = id % 8, loc = id / 8, xm = xcd & ((1 << xmLog) - 1), xn = xcd >> xmLog;
+  const int ln = int(divByMagic(uint32_t(loc), uint32_t(chunkM), chunkMMagic));
+  const int tileM = xm * chunkM + loc - ln * chunkM, tileN = xn * chunkN + ln;
   const int m0 = tileM * (MB * 16), n0 = tileN * (NB * 16);
   const int stepBegin = wave * perWave;
   const int stepEnd = stepBegin + perWave < steps ? stepBegin + perWave : steps;
   auto clampBytes = [](int64_t b) -> int32_t {
     return b > 0x7fffffffLL ? 0x7fffffff : (b < 0 ? 0 : int32_t(b));
   };
-  const bool isTile = id < tiles;
+  const bool isTile = ln < chunkN && m0 < M && n0 < N;
   const auto rsrcA = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<_Float16 *>(A) + int64_t(m0) * K, 0,
       isTile ? clampBytes(int64_t(A_PACKED ? (M - m0 + 15) / 16 * 16 : M - m0) * K * 2) : 0,
@@ -93,30 +85,29 @@ __global__ __launch_bounds__(kThreads, (MB + NB) * CH <= 20 && (ONCE || !NORM_A)
   half8 fa[CH][MB], fb[CH][NB];
   // (steps past the wavefront's last one: an offset outside the descriptors
   // reads as zero without touching memory)
-  auto request = [&](int s0) {
+  auto requestStep = [&](int c, int s) {
+    const bool in = s < stepEnd;
+    const uint32_t step = uint32_t(s);
 #pragma unroll
-    for (int c = 0; c < CH; c++) {
-      const bool in = s0 + c < stepEnd;
-      const uint32_t step = uint32_t(s0 + c);
+    for (int j = 0; j < NB; j++)
+      fb[c][j] = __builtin_bit_cast(
+          half8, __builtin_amdgcn_raw_buffer_load_b128(
+                     rsrcB, in ? uint32_t(lane) * 16u + step * 1024u + uint32_t(j) * bBlock : kOob, 0, 0));
 #pragma unroll
-      for (int j = 0; j < NB; j++)
-        fb[c][j] = __builtin_bit_cast(
-            half8, __builtin_amdgcn_raw_buffer_load_b128(
-                       rsrcB, in ? uint32_t(lane) * 16u + step * 1024u + uint32_t(j) * bBlock : kOob, 0, 0));
-#pragma unroll
-      for (int i = 0; i < MB; i++)
-        fa[c][i] = __builtin_bit_cast(
-            half8, __builtin_amdgcn_raw_buffer_load_b128(
-                       rsrcA, in ? aLane + step * aStep + uint32_t(i) * aBlock : kOob, 0, 0));
-    }
-    __builtin_amdgcn_sched_barrier(0);
+    for (int i = 0; i < MB; i++)
+      fa[c][i] = __builtin_bit_cast(
+          half8, __builtin_amdgcn_raw_buffer_load_b128(
+                     rsrcA, in ? aLane + step * aStep + uint32_t(i) * aBlock : kOob, 0, 0));
   };
-  request(stepBegin);
+#pragma unroll
+  for (int c = 0; c < CH; c++)
+    requestStep(c, stepBegin + c);
+  __builtin_amdgcn_sched_barrier(0);
   PackedArgs p = {};
 #if defined(__HIP_DEVICE_COMPILE__) // (the host pass only needs the kernel's stub)
   {
     typedef const __attribute__((address_space(4))) PackedArgs *RestPtr;
-    constexpr int kRestOffset = 2 * 8 + 8 * 4; // bytes of the leading arguments
+    constexpr int kRestOffset = 2 * 8 + 10 * 4; // bytes of the leading arguments
     static_assert(kRestOffset % alignof(PackedArgs) == 0, "argument layout");
     RestPtr late = (RestPtr)((const __attribute__((address_space(4))) char *)
                                  __builtin_amdgcn_kernarg_segment_ptr() +
@@ -126,27 +117,34 @@ __global__ __launch_bounds__(kThreads, (MB + NB) * CH <= 20 && (ONCE || !NORM_A)
   }
 #endif
   if (!isTile) {
-    readAhead<kThreads>(p.ahead, p.aheadBytes, id - tiles, int(gridDim.x) - tiles, tid);
+    const int tiles = 8 * chunkM * chunkN;
+    if (id >= tiles)
+      readAhead<kThreads>(p.ahead, p.aheadBytes, id - tiles, int(gridDim.x) - tiles, tid);
     return;
   }
-  // What the epilogue reads: thread t < MB * NB * 64 finishes 4 consecutive
-  // columns of one row.
-  constexpr int kOutThreads = MB * NB * kWave;
-  const int outBlock = tid / kWave; // (mb, nb) = (outBlock / NB, outBlock % NB)
-  const int m = m0 + (outBlock / NB) * 16 + lane % 16;
-  const int n = n0 + (outBlock % NB) * 16 + (lane / 16) * 4;
-  const bool mine = tid < kOutThreads && m < p.M;
-  const int64_t plain = int64_t(m) * p.N + n, packed = packedOffset(m, n, p.N);
-  half4 cv = {};
-  float2v cStat{1.f, 0.f};
-  float4v cSum = {};
-  if (mine) {
-    if (p.C)
-      cv = *reinterpret_cast<const half4 *>(p.C + (p.cPacked ? packed : plain));
-    if (p.statsIn)
-      cStat = *reinterpret_cast<const float2v *>(p.statsIn + int64_t(m) * 2);
-    if (NORM_A)
-      cSum = *reinterpret_cast<const float4v *>(p.colSum + n);
+  // What the epilogue reads: wavefront w finishes 16 x 16 blocks w, w + 8, .. of
+  // the tile, a lane 4 consecutive columns of one row of each.
+  constexpr int OUTS = (MB * NB + kWaves - 1) / kWaves;
+  half4 cv[OUTS] = {};
+  float2v cStat[OUTS];
+  float4v cSum[OUTS] = {};
+  auto blockOf = [&](int q) { return wave + q * kWaves; }; // (mb, nb) = (/ NB, % NB)
+  auto rowOf = [&](int q) { return m0 + blockOf(q) / NB * 16 + lane % 16; };
+  auto colOf = [&](int q) { return n0 + blockOf(q) % NB * 16 + lane / 16 * 4; };
+  auto mine = [&](int q) { return blockOf(q) < MB * NB && rowOf(q) < p.M; };
+#pragma unroll
+  for (int q = 0; q < OUTS; q++) {
+    cStat[q] = float2v{1.f, 0.f};
+    if (mine(q)) {
+      const int m = rowOf(q), n = colOf(q);
+      if (p.C)
+        cv[q] = *reinterpret_cast<const half4 *>(
+            p.C + (p.cPacked ? packedOffset(m, n, p.N) : int64_t(m) * p.N + n));
+      if (p.statsIn)
+        cStat[q] = *reinterpret_cast<const float2v *>(p.statsIn + int64_t(m) * 2);
+      if (NORM_A)
+        cSum[q] = *reinterpret_cast<const float4v *>(p.colSum + n);
+    }
   }
   __builtin_amdgcn_sched_barrier(0);
 
@@ -160,36 +158,44 @@ __global__ __launch_bounds__(kThreads, (MB + NB) * CH <= 20 && (ONCE || !NORM_A)
 #pragma unroll
   for (int i = 0; i < MB; i++)
     sum[i] = sq[i] = 0.f;
-  for (int s0 = stepBegin;;) {
+  auto multiply = [&](int c) {
 #pragma unroll
-    for (int c = 0; c < CH; c++) {
+    for (int i = 0; i < MB; i++) {
+      if (NORM_A) {
+        const half2v one = {_Float16(1), _Float16(1)};
 #pragma unroll
-      for (int i = 0; i < MB; i++) {
-        if (NORM_A) {
-          const half2v one = {_Float16(1), _Float16(1)};
-#pragma unroll
-          for (int e = 0; e < 4; e++) {
-            const half2v x = {fa[c][i][2 * e], fa[c][i][2 * e + 1]};
-            sum[i] = __builtin_amdgcn_fdot2(x, one, sum[i], false);
-            sq[i] = __builtin_amdgcn_fdot2(x, x, sq[i], false);
-          }
+        for (int e = 0; e < 4; e++) {
+          const half2v x = {fa[c][i][2 * e], fa[c][i][2 * e + 1]};
+          sum[i] = __builtin_amdgcn_fdot2(x, one, sum[i], false);
+          sq[i] = __builtin_amdgcn_fdot2(x, x, sq[i], false);
         }
+      }
 #pragma unroll
-        for (int j = 0; j < NB; j++)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fb[c][j], fa[c][i], acc[i][j], 0, 0, 0);
-        // (in the order of arrival: reordered, the operands of several steps
-        // get second copies and the workgroup no longer fits a CU twice)
-        if (NORM_A)
-          __builtin_amdgcn_sched_barrier(0);
+      for (int j = 0; j < NB; j++)
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fb[c][j], fa[c][i], acc[i][j], 0, 0, 0);
+      // (in the order of arrival: reordered, the operands of several steps
+      // get second copies and the workgroup no longer fits a CU twice)
+      if (NORM_A)
+        __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  // Behind its MFMAs a step's registers are asked to hold the one CH further on.
+  int s0 = stepBegin;
+  if constexpr (!ONCE) {
+#pragma unroll 1
+    for (; s0 + CH < stepEnd; s0 += CH) {
+#pragma unroll
+      for (int c = 0; c < CH; c++) {
+        multiply(c);
+        __builtin_amdgcn_sched_barrier(0);
+        requestStep(c, s0 + CH + c);
+        __builtin_amdgcn_sched_barrier(0);
       }
     }
-    if constexpr (ONCE)
-      break;
-    s0 += CH;
-    if (s0 >= stepEnd)
-      break;
-    request(s0);
   }
+#pragma unroll
+  for (int c = 0; c < CH; c++)
+    multiply(c);
 
   // The wavefronts' partial sums meet: [wave][block][lane] and, of the row
   // statistics, [wave][row].
@@ -207,41 +213,45 @@ __global__ __launch_bounds__(kThreads, (MB + NB) * CH <= 20 && (ONCE || !NORM_A)
     }
   }
   __syncthreads();
-  if (!mine)
-    return;
-  float4v v = part[outBlock * kWave + lane];
 #pragma unroll
-  for (int w = 1; w < kWaves; w++)
-    v += part[(w * MB * NB + outBlock) * kWave + lane];
-  if (NORM_A) {
-    float2v st{0.f, 0.f};
+  for (int q = 0; q < OUTS; q++) {
+    if (!mine(q))
+      continue;
+    const int block = blockOf(q), m = rowOf(q), n = colOf(q);
+    float4v v = part[block * kWave + lane];
 #pragma unroll
-    for (int w = 0; w < kWaves; w++)
-      st += stat[w * MB * 16 + (outBlock / NB) * 16 + lane % 16];
-    const float mu = st[0] * p.invK;
-    // the difference cancels to a small negative number for near-constant
-    // rows; clamped so that a tiny eps cannot turn it into a NaN
-    const float rstd = 1.0f / sqrtf(fmaxf(st[1] * p.invK - mu * mu, 0.f) + p.eps);
-    const float shift = -mu * rstd;
+    for (int w = 1; w < kWaves; w++)
+      v += part[(w * MB * NB + block) * kWave + lane];
+    if (NORM_A) {
+      float2v st{0.f, 0.f};
 #pragma unroll
-    for (int e = 0; e < 4; e++)
-      v[e] = fmaf(rstd, v[e], shift * cSum[e]);
-    if (p.statsOut && tileN == 0 && outBlock % NB == 0 && lane < 16)
-      storeWriteThrough(p.statsOut + int64_t(m) * 2, float2v{rstd, shift});
+      for (int w = 0; w < kWaves; w++)
+        st += stat[w * MB * 16 + (block / NB) * 16 + lane % 16];
+      const float mu = st[0] * p.invK;
+      // the difference cancels to a small negative number for near-constant
+      // rows; clamped so that a tiny eps cannot turn it into a NaN
+      const float rstd = 1.0f / sqrtf(fmaxf(st[1] * p.invK - mu * mu, 0.f) + p.eps);
+      const float shift = -mu * rstd;
+#pragma unroll
+      for (int e = 0; e < 4; e++)
+        v[e] = fmaf(rstd, v[e], shift * cSum[q][e]);
+      if (p.statsOut && tileN == 0 && block % NB == 0 && lane < 16)
+        storeWriteThrough(p.statsOut + int64_t(m) * 2, float2v{rstd, shift});
+    }
+    half4 o;
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      float x = v[e];
+      if (p.activation == 1)
+        x = packedGeluErf(x);
+      else if (p.activation == 2)
+        x = packedGeluTanh(x);
+      if (p.C)
+        x += float(_Float16(fmaf(float(cv[q][e]), cStat[q][0], cStat[q][1])));
+      o[e] = _Float16(x);
+    }
+    storeWriteThrough(p.D + (p.dPacked ? packedOffset(m, n, p.N) : int64_t(m) * p.N + n), o);
   }
-  half4 o;
-#pragma unroll
-  for (int e = 0; e < 4; e++) {
-    float x = v[e];
-    if (p.activation == 1)
-      x = packedGeluErf(x);
-    else if (p.activation == 2)
-      x = packedGeluTanh(x);
-    if (p.C)
-      x += float(_Float16(fmaf(float(cv[e]), cStat[0], cStat[1])));
-    o[e] = _Float16(x);
-  }
-  storeWriteThrough(p.D + (p.dPacked ? packed : plain), o);
 }
 
 // Layer norm without affine parameters of rows in fragment order; the result in
@@ -327,16 +337,42 @@ __global__ __launch_bounds__(256) void packWeightKernel(const _Float16 *__restri
   reinterpret_cast<half8 *>(out)[v] = o;
 }
 
+// What an XCD works on: chunkM x chunkN tiles, 2^xmLog XCDs along M.  Its L2 fetches
+// the operands of the rectangle once, at about 0.7 TB/s per XCD from the last-level
+// cache, which from some 500 rows on is what bounds these kernels (512 x 1024 x
+// 4096 moved 42 MB so in 7.2 us); among the splits that leave the fullest CU the
+// fewest tiles, the one that fetches least.
+struct Rectangles {
+  int xmLog, chunkM, chunkN;
+  int64_t perCu;    // tiles of the fullest CU
+  double fillBytes; // all XCDs
+};
+Rectangles chooseRectangles(int64_t M, int64_t N, int64_t K, int mb, int nb, int cus) {
+  const int64_t tilesM = (M + mb * 16 - 1) / (mb * 16), tilesN = N / (nb * 16);
+  const int64_t perXcd = std::max(1, cus / 8);
+  Rectangles best{};
+  for (int x = 0; x <= 3; x++) {
+    const int64_t cm = (tilesM + (1 << x) - 1) >> x, cn = (tilesN + (8 >> x) - 1) / (8 >> x);
+    const int64_t perCu = (cm * cn + perXcd - 1) / perXcd;
+    const double fill = 8.0 * double(cm * mb + cn * nb) * 16 * double(K) * 2;
+    if (x == 0 || perCu < best.perCu || (perCu == best.perCu && fill < best.fillBytes))
+      best = {x, int(cm), int(cn), perCu, fill};
+  }
+  return best;
+}
+
 template <int MB, int NB, int CH, bool ONCE>
-Status launchVariant(const PackedGemm &g, const PackedArgs &p, int aheadGroups, hipStream_t s) {
+Status launchVariant(const PackedGemm &g, const PackedArgs &p, const Rectangles &r,
+                     int aheadGroups, hipStream_t s) {
   const int steps = int(g.K / 32), perWave = (steps + kWaves - 1) / kWaves;
-  const int tilesM = int((g.M + MB * 16 - 1) / (MB * 16)), tilesN = int(g.N / (NB * 16));
   constexpr int kLds = kWaves * MB * NB * kWave * 16 + kWaves * MB * 16 * 8;
-  const dim3 grid((unsigned)(tilesM * tilesN + aheadGroups)), block(kThreads);
-  auto kernel = g.aPacked ? (g.normA ? packedGemmKernel<MB, NB, CH, ONCE, true, true>
-                                     : packedGemmKernel<MB, NB, CH, ONCE, false, true>)
-                          : (g.normA ? packedGemmKernel<MB, NB, CH, ONCE, true, false>
-                                     : packedGemmKernel<MB, NB, CH, ONCE, false, false>);
+  const dim3 grid((unsigned)(8 * r.chunkM * r.chunkN + aheadGroups)), block(kThreads);
+  constexpr bool kRowMajorA = MB * NB < 16; // (an A of so many rows arrives packed)
+  auto kernel = g.aPacked || !kRowMajorA
+                    ? (g.normA ? packedGemmKernel<MB, NB, CH, ONCE, true, true>
+                               : packedGemmKernel<MB, NB, CH, ONCE, false, true>)
+                    : (g.normA ? packedGemmKernel<MB, NB, CH, ONCE, true, !kRowMajorA>
+                               : packedGemmKernel<MB, NB, CH, ONCE, false, !kRowMajorA>);
   if (kLds > 48 * 1024) {
     static bool done[4] = {};
     bool &set = done[2 * g.aPacked + g.normA];
@@ -346,8 +382,8 @@ Status launchVariant(const PackedGemm &g, const PackedArgs &p, int aheadGroups, 
                   Status::kInternal);
     set = true;
   }
-  kernel<<<grid, block, kLds, s>>>(g.A, g.packedB, int(g.M), int(g.K), steps, perWave, tilesM,
-                                   tilesN, magicFor(uint32_t(tilesM)), tilesM * tilesN, p);
+  kernel<<<grid, block, kLds, s>>>(g.A, g.packedB, int(g.M), int(g.N), int(g.K), steps, perWave,
+                                   r.chunkM, magicFor(uint32_t(r.chunkM)), r.chunkN, r.xmLog, p);
   HOM_HIP_RET(hipGetLastError(), Status::kInternal);
   return Status::kSuccess;
 }
@@ -375,6 +411,46 @@ Status launchPackedLayernorm(const _Float16 *in, _Float16 *out, int64_t M, int64
   return Status::kSuccess;
 }
 
+namespace {
+// The steps in flight for a wavefront's share of K: all of it while that is 3 or 4
+// steps (for one block of 16 x 16 up to 16), else a count that goes into it and
+// fits the registers.
+Status launchShape(int mb, int nb, int perWave, const PackedGemm &g, const PackedArgs &p,
+                   const Rectangles &r, int groups, hipStream_t s) {
+  const bool byThree = perWave % 3 == 0;
+  switch (mb * 8 + nb) {
+  case 1 * 8 + 1:
+    return perWave <= 3    ? launchVariant<1, 1, 3, true>(g, p, r, groups, s)
+           : perWave <= 4  ? launchVariant<1, 1, 4, true>(g, p, r, groups, s)
+           : perWave <= 12 ? launchVariant<1, 1, 12, true>(g, p, r, groups, s)
+           : perWave <= 16 ? launchVariant<1, 1, 16, true>(g, p, r, groups, s)
+                           : launchVariant<1, 1, 12, false>(g, p, r, groups, s);
+  case 2 * 8 + 1:
+    return perWave <= 3   ? launchVariant<2, 1, 3, true>(g, p, r, groups, s)
+           : perWave <= 4 ? launchVariant<2, 1, 4, true>(g, p, r, groups, s)
+                          : launchVariant<2, 1, 6, false>(g, p, r, groups, s);
+  case 2 * 8 + 2:
+    return perWave <= 3   ? launchVariant<2, 2, 3, true>(g, p, r, groups, s)
+           : perWave <= 4 ? launchVariant<2, 2, 4, true>(g, p, r, groups, s)
+                          : launchVariant<2, 2, 4, false>(g, p, r, groups, s);
+  case 4 * 8 + 1:
+    return perWave <= 3   ? launchVariant<4, 1, 3, true>(g, p, r, groups, s)
+           : perWave <= 4 ? launchVariant<4, 1, 4, true>(g, p, r, groups, s)
+                          : launchVariant<4, 1, 4, false>(g, p, r, groups, s);
+  case 4 * 8 + 2:
+    return perWave <= 3   ? launchVariant<4, 2, 3, true>(g, p, r, groups, s)
+           : perWave <= 4 ? launchVariant<4, 2, 4, true>(g, p, r, groups, s)
+           : byThree      ? launchVariant<4, 2, 3, false>(g, p, r, groups, s)
+                          : launchVariant<4, 2, 4, false>(g, p, r, groups, s);
+  default:
+    return perWave <= 3   ? launchVariant<4, 4, 3, true>(g, p, r, groups, s)
+           : perWave <= 4 ? launchVariant<4, 4, 4, true>(g, p, r, groups, s)
+           : byThree      ? launchVariant<4, 4, 3, false>(g, p, r, groups, s)
+                          : launchVariant<4, 4, 4, false>(g, p, r, groups, s);
+  }
+}
+} // namespace
+
 Status launchPackedGemm(const PackedGemm &g, hipStream_t s) {
   PackedArgs p{};
   p.C = g.C;
@@ -395,65 +471,52 @@ Status launchPackedGemm(const PackedGemm &g, hipStream_t s) {
   // k steps per wavefront, all in flight at once where the registers allow
   const int perWave = int((g.K / 32 + kWaves - 1) / kWaves);
   // The tile by a model of its time in a chain of launches, fitted to M = 16 ..
-  // 2048 x the shapes of BERT-base and -large (within 10 %): launch, latency and
-  // the meeting of the partial sums, then what the fullest CU pulls through its
-  // L1; workgroups of a CU beyond those that fit its registers at once start a
-  // second chain of latencies.  (Those of the tile kernels that fill the chip do
-  // not read ahead, which is worth most of a microsecond to the launch behind.)
+  // 2048 x the shapes of BERT-base and -large (6 % off in the mean, the choice within
+  // 8 % of the best but for a few shapes): launch, latency and the meeting of
+  // the partial sums; then what the fullest CU pulls through its L1, no faster
+  // than its XCD fetches the rectangle's operands; and a chain of latencies more
+  // for every round of workgroups that do not fit a CU together.  (Those of the
+  // tile kernels that fill the chip do not read ahead, which is worth most of a
+  // microsecond to the launch behind.)
   const int cus = deviceInfo().computeUnits > 0 ? deviceInfo().computeUnits : 256;
   struct Shape {
     int mb, nb, resident;
   };
-  const Shape shapes[4] = {{1, 1, perWave <= 4 ? 3 : 1},
-                           {2, 1, 2},
-                           {4, 1, 2},
-                           {4, 2, perWave == 4 ? 1 : 2}};
-  int best = 0;
+  const Shape shapes[] = {{1, 1, perWave <= 4 ? 3 : 1},
+                          {2, 1, 2},
+                          {2, 2, 2},
+                          {4, 1, 2},
+                          {4, 2, perWave <= 3 || (perWave > 4 && perWave % 3 == 0) ? 2 : 1},
+                          {4, 4, 1}};
+  const Shape *best = nullptr;
   double bestCost = 1e300;
-  int64_t bestTiles = 0;
-  for (int i = 0; i < 4; i++) {
-    const Shape &t = shapes[i];
-    if (g.N % (t.nb * 16) != 0)
+  Rectangles rect{};
+  for (const Shape &t : shapes) {
+    if (g.N % (t.nb * 16) != 0 || (t.mb * t.nb == 16 && !g.aPacked))
       continue;
-    const int64_t tiles = ((g.M + t.mb * 16 - 1) / (t.mb * 16)) * (g.N / (t.nb * 16));
-    const int64_t perCu = (tiles + cus - 1) / cus;
+    const Rectangles r = chooseRectangles(g.M, g.N, g.K, t.mb, t.nb, cus);
     const double kb = double(t.mb + t.nb) * 16 * double(g.K) * 2 / 1024;
-    // (deep K: rounds of two workgroups, since one alone fetches half as fast, and
-    // the matrix cores have their say in the largest tile)
-    const double usPerKb = perWave <= 4 ? 0.0088 : t.mb * t.nb == 8 ? 0.0104 : 0.0062;
-    const int64_t paired = perWave <= 4 || perCu == 1 ? perCu : (perCu + 1) / 2 * 2;
-    const double cost = 2.1 + 0.1 * t.mb * t.nb + usPerKb * kb * double(paired) +
-                        (t.resident == 1 ? 1.8 : 1.0) * double((perCu - 1) / t.resident);
+    const int64_t rounds = (r.perCu + t.resident - 1) / t.resident;
+    // (a workgroup alone on its CU in the last round does not fetch twice as fast)
+    const double load = perWave <= 4 || r.perCu == 1
+                            ? double(r.perCu)
+                            : 0.5 * double(r.perCu + rounds * t.resident);
+    const double fetch =
+        std::max((perWave <= 4 ? 0.00915 : 0.0077) * kb * load, r.fillBytes / 5.3e6);
+    const double round = t.resident > 1 || t.mb == 1 ? 0.2 : perWave <= 4 ? 2.0 : 8.0;
+    const double cost = 1.7 + 0.08 * t.mb * t.nb + fetch * (g.normA ? 1.25 : 1.0) +
+                        round * double(rounds - 1);
     if (cost < bestCost) {
       bestCost = cost;
-      best = i;
-      bestTiles = tiles;
+      best = &t;
+      rect = r;
     }
   }
   if (tiled.us + (g.ahead ? 0.7 : 0.0) < bestCost)
     return launchPackedTile(tiled.tile, g, p, s);
   // (half the CUs read ahead when the tiles take all of them)
-  const int groups = aheadGroups<kThreads>(p.aheadBytes, std::max<int64_t>(cus - bestTiles, cus / 2));
-  switch (best) {
-  case 0:
-    return perWave <= 3    ? launchVariant<1, 1, 3, true>(g, p, groups, s)
-           : perWave <= 4  ? launchVariant<1, 1, 4, true>(g, p, groups, s)
-           : perWave <= 12 ? launchVariant<1, 1, 12, true>(g, p, groups, s)
-           : perWave <= 16 ? launchVariant<1, 1, 16, true>(g, p, groups, s)
-                           : launchVariant<1, 1, 12, false>(g, p, groups, s);
-  case 1:
-    return perWave <= 3   ? launchVariant<2, 1, 3, true>(g, p, groups, s)
-           : perWave <= 4 ? launchVariant<2, 1, 4, true>(g, p, groups, s)
-                          : launchVariant<2, 1, 6, false>(g, p, groups, s);
-  case 2:
-    return perWave <= 3   ? launchVariant<4, 1, 3, true>(g, p, groups, s)
-           : perWave <= 4 ? launchVariant<4, 1, 4, true>(g, p, groups, s)
-                          : launchVariant<4, 1, 4, false>(g, p, groups, s);
-  default:
-    return perWave <= 3   ? launchVariant<4, 2, 3, true>(g, p, groups, s)
-           : perWave <= 4 ? launchVariant<4, 2, 4, true>(g, p, groups, s)
-                          : launchVariant<4, 2, 3, false>(g, p, groups, s);
-  }
+  const int groups = aheadGroups<kThreads>(p.aheadBytes, std::max<int64_t>(cus - int64_t(rect.chunkM) * rect.chunkN * 8, cus / 2));
+  return launchShape(best->mb, best->nb, perWave, g, p, rect, groups, s);
 }
 
 } // namespace hom

@@ -51,7 +51,7 @@ template <int N, class F> __device__ __forceinline__ void unrolled(F &&f) {
 // BM x BN tile, WM x WN wavefronts, slabs of SB * 32 k in a ring of NBUF LDS
 // buffers.  ACT: 0 linear, 1 erf GELU, 2 tanh GELU; SRC: a residual source.
 template <int BM, int BN, int WM, int WN, int SB, int NBUF, bool NORM_A, int ACT, bool SRC>
-__global__ __launch_bounds__(WM *WN *kWave) void packedTileKernel(
+__global__ __launch_bounds__(WM *WN *kWave, NBUF *(BM + BN) * SB > 1280 ? 1 : WM *WN / 2) void packedTileKernel(
     const _Float16 *A, const _Float16 *B, int rowBlocks, int colBlocks, int slabs, int tilesN,
     int xcdQ, uint32_t groupMagic, int walk, int workers, int tiles, PackedArgs p) {
   constexpr int WAVES = WM * WN, WTM = BM / WM, WTN = BN / WN;
@@ -446,19 +446,28 @@ struct Tile {
   double fixedUs; // per tile of a CU: first slab, epilogue
   double slabUs;  // per 64 k, one tile per CU
   double rate;    // bytes per us that all tiles together load at most
+  // the same of workgroups that share a CU and fill each other's gaps
+  double sharedFactor, sharedRate;
 };
-constexpr Tile kTiles[] = {{256, 256, 4.5, 1.09, 11.5e6},
-                           {256, 128, 3.0, 0.57, 11.5e6},
-                           {128, 128, 0.9, 0.43, 14.5e6},
-                           {64, 128, 0.7, 0.27, 18.5e6},
-                           {64, 64, 0.4, 0.20, 22.5e6}};
+constexpr Tile kTiles[] = {{256, 256, 4.5, 1.09, 11.5e6, 1.0, 11.5e6},
+                           {256, 128, 2.5, 0.57, 11.5e6, 0.93, 14.5e6},
+                           {128, 128, 1.1, 0.43, 14.5e6, 0.88, 18.0e6},
+                           {64, 128, 0.7, 0.27, 18.5e6, 0.8, 18.5e6},
+                           {64, 64, 0.4, 0.20, 22.5e6, 0.8, 22.5e6}};
+
+// More tiles than CUs: slabs of 32 k, so that two rings fit a CU and one
+// workgroup's epilogue runs beside the other's main loop (128 x 128: 4096 x 3072 x 768
+// with GELU 27.7 -> 24.9 us; 256 x 128: 27.1 -> 25.4, 8192 rows 46.9 -> 44.0).
+// Otherwise 64 k per barrier (128 x 128: 4096 x 768 x 3072 28.1 -> 26.7), and also
+// with the row sums of a folded layer norm, which need the registers.
+bool sharesCu(const PackedGemm &g, int64_t tiles, int cus) { return tiles > cus && !g.normA; }
 } // namespace
 
 // Model of a tile's time in a chain of launches (us), fitted to M = 512 .. 16384
 // x the shapes of BERT-base and -large (most within 10 %): launch, then per tile of
-// the fullest CU a fixed part and its slabs, these no faster than the L2s
-// deliver all tiles' operands (13.5 TB/s) or the matrix cores multiply at the
-// clock the power allows (1.2 PFLOP/s).
+// the fullest CU a fixed part and its slabs, these no faster than all tiles'
+// operands arrive or the matrix cores multiply at the clock the power allows
+// (1.2 PFLOP/s).
 PackedTileChoice choosePackedTile(const PackedGemm &g) {
   PackedTileChoice best{-1, 1e300};
   if (!g.aPacked || !g.dPacked || (g.C && !g.cPacked) || g.K % 64 != 0 || g.N % 32 != 0 ||
@@ -469,11 +478,11 @@ PackedTileChoice choosePackedTile(const PackedGemm &g) {
     const Tile &t = kTiles[i];
     const int64_t tiles = ((g.M + t.bm - 1) / t.bm) * ((g.N + t.bn - 1) / t.bn);
     const double perCu = double((tiles + cus - 1) / cus);
-    // (workgroups of the small tiles share a CU and fill each other's gaps)
-    const double overlap = i >= 3 && perCu > 1 ? 0.8 : 1.0;
-    const double loop = std::max({perCu * double(g.K) / 64 * t.slabUs * overlap,
-                                  double(tiles) * (t.bm + t.bn) * double(g.K) * 2 / t.rate,
-                                  2.0 * double(g.M) * double(g.N) * double(g.K) / 1.2e9});
+    const bool shared = i >= 3 ? perCu > 1 : sharesCu(g, tiles, cus);
+    const double loop =
+        std::max({perCu * double(g.K) / 64 * t.slabUs * (shared ? t.sharedFactor : 1.0),
+                  double(tiles) * (t.bm + t.bn) * double(g.K) * 2 / (shared ? t.sharedRate : t.rate),
+                  2.0 * double(g.M) * double(g.N) * double(g.K) / 1.2e9});
     const double us = 2.2 + loop * (g.normA ? 1.25 : 1.0) +
                       perCu * (t.fixedUs + (g.activation ? 5e-5 * t.bm * t.bn : 0));
     if (us < best.us)
@@ -483,13 +492,22 @@ PackedTileChoice choosePackedTile(const PackedGemm &g) {
 }
 
 Status launchPackedTile(int tile, const PackedGemm &g, const PackedArgs &p, hipStream_t s) {
+  const int cus = deviceInfo().computeUnits > 0 ? deviceInfo().computeUnits : 256;
+  auto shared = [&](int bm, int bn) {
+    return sharesCu(g, ((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn), cus);
+  };
   switch (tile) {
   case 0:
     return launchTile<256, 256, 2, 4, 1, 4>(g, p, s);
   case 1:
-    return launchTile<256, 128, 4, 2, 2, 3>(g, p, s);
+    return shared(256, 128) ? launchTile<256, 128, 4, 2, 1, 3>(g, p, s)
+                            : launchTile<256, 128, 4, 2, 2, 3>(g, p, s);
   case 2:
-    return launchTile<128, 128, 2, 4, 2, 4>(g, p, s);
+    // (and not for so few slabs that the first one counts: 1024 x 3072 x 768 9.7 us
+    // against 10.3)
+    return shared(128, 128) || (g.K <= 1024 && !g.normA)
+               ? launchTile<128, 128, 2, 4, 1, 4>(g, p, s)
+               : launchTile<128, 128, 2, 4, 2, 4>(g, p, s);
   case 3:
     return launchTile<64, 128, 1, 4, 2, 4>(g, p, s);
   default:
