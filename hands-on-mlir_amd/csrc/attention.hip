@@ -30,9 +30,11 @@
 // LDS rows are 128 bytes, unpadded; 16-byte chunks (K) / 64-byte groups (V) are
 // XOR-permuted by row so that the fragment reads are bank-conflict free.
 #include "cross_lane.h"
+#include "fast_div.h"
 #include "packed_args.h"
 
 #include <cstring>
+#include <type_traits>
 
 namespace hom {
 namespace {
@@ -44,13 +46,13 @@ typedef short short4v __attribute__((ext_vector_type(4)));
 typedef short short8v __attribute__((ext_vector_type(8)));
 
 constexpr int kWave = 64;
+#define HOM_LDS_PTR(p) ((__attribute__((address_space(3))) void *)(p))
 // Head sizes 64, 128, 192 and 256 (template parameter D; the reference's
-// contract is head size % 64 == 0).  64 is what every BERT configuration has
-// and what the kernel is tuned for, 128 is the same code with twice the
-// registers, 192 and 256 are functional (one wavefront per SIMD, half the keys
-// per LDS chunk, staging addresses computed per vector).  A K or V row in LDS
-// is D halves: 128 bytes = 8 chunks of 16 bytes = 2 groups of 64 bytes for
-// D = 64.
+// contract is head size % 64 == 0).  A K or V row in LDS is D halves: 128 bytes = 8
+// chunks of 16 bytes = 2 groups of 64 bytes for D = 64.  Two wavefronts share a
+// SIMD up to head size 192: held to 256 registers, head size 128 went from 292
+// registers and one wavefront to 212 and two, 138 -> 82 us at 32 x 512 x 16 heads
+// and 24.6 -> 17.9 us at 8 x 384 x 16.
 //
 // Keys staged per barrier: 128, or 64 where two tiles of 128 rows would not fit
 // the 64 KB of static LDS.
@@ -83,24 +85,26 @@ template <int D> __device__ __forceinline__ int swzV(int k, int group) {
 // PACKED_IN: QKV in fragment order (packedOffset() in kernels.h): the 8 values of
 // a token row that a vector takes are contiguous there as well, only the address
 // of a row differs.
-template <int NW, int KS, int D, bool PACKED_IN = false>
+template <int NW, int KS, int D, bool PACKED_IN = false, bool DMA = false>
 __global__ __launch_bounds__(NW *kWave)
-__attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1, D == 64 && KS == 1 ? 4 : (D <= 128 ? 2 : 1)))) void bertAttentionKernel(
+__attribute__((amdgpu_waves_per_eu(D <= 128 || NW == 8 ? 2 : 1, D == 64 && KS == 1 ? 4 : (D <= 128 || NW == 8 ? 2 : 1)))) void bertAttentionKernel(
     const _Float16 *__restrict__ qkv, const int32_t *__restrict__ cu,
-    _Float16 *__restrict__ out, int seq, int heads, int numQTiles, int pairs,
-    float scale, int packedOut, const char *ahead, int64_t aheadBytes) {
+    _Float16 *__restrict__ out, int seq, int heads, int numQTiles, int bs,
+    float scale, int packedOut, uint32_t numQMagic, uint32_t headsMagic, const char *ahead,
+    int64_t aheadBytes) {
   static_assert(D == 64 || D == 128 || D == 192 || D == 256, "head size");
-  static_assert(D <= 128 || KS == 1, "the key-split variant stages 128 keys per chunk");
+  static_assert(D <= 128 || KS == 1 || DMA, "the key-split variant stages 128 keys per chunk");
   static_assert(!PACKED_IN || D == 64, "fragment order is read at head size 64");
-  constexpr int kChunk = Chunk<D>::value;
+  constexpr int kChunk = DMA ? 64 : Chunk<D>::value;
+  constexpr int SBW = DMA && KS == 2 ? 1 : 2; // 32-key sub-blocks a wavefront takes at a time
   constexpr int kHeadDim = D;
   constexpr int kRowB = D * 2;               // bytes of a K or V row
   constexpr int CPR = D / 8;                 // 16-byte chunks per row
   constexpr int kTileBytes = kChunk * kRowB; // one K or V chunk in LDS
   constexpr int kThreads = NW * kWave;
   constexpr int QG = NW / KS; // groups of 32 query rows per workgroup
-  __shared__ __attribute__((aligned(16))) unsigned char smem[2 * kTileBytes];
-  unsigned char *const sK = smem, *const sV = smem + kTileBytes;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  unsigned char *sK = smem, *sV = smem + kTileBytes;
 
   const int tid = threadIdx.x, lane = tid % kWave;
   // (the same for every lane: what depends on it stays in scalar registers)
@@ -116,8 +120,9 @@ __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1, D == 64 && KS == 1 ? 4 : (D 
   // The key-split variant is launched on a (query tile, head, batch) grid: the
   // same order of workgroups as a flat id, without the divisions that would
   // stand between the kernel's entry and its first loads.
+  const int pairs = bs * heads;
   int qTile, head, b;
-  if (KS == 1) {
+  if (KS == 1 || DMA) {
     const int id = blockIdx.x;
     if constexpr (PACKED_IN) {
       if (id >= numQTiles * pairs) {
@@ -128,15 +133,15 @@ __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1, D == 64 && KS == 1 ? 4 : (D 
     }
     int pair;
     if (pairs % 8 == 0) {
-      const int t = id / 8;
-      qTile = t % numQTiles;
-      pair = (t / numQTiles) * 8 + id % 8;
+      const uint32_t t = uint32_t(id) / 8, g = divByMagic(t, uint32_t(numQTiles), numQMagic);
+      qTile = int(t - g * uint32_t(numQTiles));
+      pair = int(g * 8 + uint32_t(id) % 8);
     } else {
-      qTile = id % numQTiles;
-      pair = id / numQTiles;
+      pair = int(divByMagic(uint32_t(id), uint32_t(numQTiles), numQMagic));
+      qTile = id - pair * numQTiles;
     }
-    head = pair % heads;
-    b = pair / heads;
+    b = int(divByMagic(uint32_t(pair), uint32_t(heads), headsMagic));
+    head = pair - b * heads;
   } else {
     qTile = blockIdx.x;
     head = blockIdx.y;
@@ -161,11 +166,13 @@ __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1, D == 64 && KS == 1 ? 4 : (D 
   const _Float16 *vBase = base + (2 * heads + head) * kHeadDim;
   const int64_t outStride = int64_t(heads) * kHeadDim;
   _Float16 *oBase = out + int64_t(b) * seq * outStride + head * kHeadDim;
-  // 4 output columns from column c of query q (packedOut: fragment order)
-  auto outAt = [&](int q, int c) {
-    return packedOut ? out + packedOffset(int64_t(b) * seq + q, head * kHeadDim + c, outStride)
-                     : oBase + int64_t(q) * outStride + c;
-  };
+  // Output columns 32 d + 8 g + 4 hb .. + 3 of this lane's query: oRow + d * oWide +
+  // g * oEight (packedOut: fragment order).
+  const int oWide = packedOut ? 512 : 32, oEight = packedOut ? 128 : 8;
+  _Float16 *const oRow =
+      (packedOut ? out + packedOffset(int64_t(b) * seq + q0 + l32, head * kHeadDim, outStride)
+                 : oBase + int64_t(q0 + l32) * outStride) +
+      hb * 4;
 
   // Key-split variant (short sequences, few workgroups: latency is what
   // counts): K and V rows of a 128-key chunk travel global -> registers -> LDS,
@@ -186,7 +193,7 @@ __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1, D == 64 && KS == 1 ? 4 : (D 
     return (int64_t(t / 16) * wide + (part * heads + head) * (kHeadDim / 32) + c8 / 4) * 512 +
            (c8 % 4) * 128 + (t % 16) * 8;
   };
-  constexpr bool kPrefetch = KS == 2 && D == 64;
+  constexpr bool kPrefetch = KS == 2 && D == 64 && !DMA;
   constexpr int VPT = kChunk * CPR / kThreads; // vectors of K (and of V) per thread
   half8 rk[VPT], rv[VPT];
   auto loadChunk = [&](int key0) {
@@ -224,7 +231,7 @@ __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1, D == 64 && KS == 1 ? 4 : (D 
   // prefetched rows lets the compiler move their loads behind the test, i.e.
   // behind the arrival of the sequence length.  Such a workgroup walks one
   // empty chunk there and stores zeros at the end.)
-  if (KS == 1 && qTile * (QG * 32) >= len) {
+  if ((KS == 1 || DMA) && qTile * (QG * 32) >= len) {
     const int q = q0 + l32;
     if (q < seq && kh == 0) {
       half4 z;
@@ -233,7 +240,7 @@ __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1, D == 64 && KS == 1 ? 4 : (D 
         z[e] = _Float16(0);
 #pragma unroll
       for (int c = 0; c < CPR; c++)
-        *reinterpret_cast<half4 *>(outAt(q, c * 8 + hb * 4)) = z;
+        *reinterpret_cast<half4 *>(oRow + c / 4 * oWide + c % 4 * oEight) = z;
     }
     return;
   }
@@ -273,7 +280,7 @@ __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1, D == 64 && KS == 1 ? 4 : (D 
   const int stageK = (tid / CPR) * kRowB + swzK<D>(tid / CPR, tid % CPR) * 16;
   const int stageV = (tid / CPR) * kRowB + swzV<D>(tid / CPR, (tid % CPR) / 4) * 64 +
                      ((tid % CPR) % 4) * 16;
-  const int32_t stageBytes = PACKED_IN ? int32_t(uint32_t((pairs / heads * seq + 15) / 16) *
+  const int32_t stageBytes = PACKED_IN ? int32_t(uint32_t((bs * seq + 15) / 16) *
                                                  uint32_t(wide) * 1024u)
                                        : int32_t(uint32_t(len) * rowBytes);
   const auto rsrcK = __builtin_amdgcn_make_buffer_rsrc(
@@ -285,19 +292,65 @@ __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1, D == 64 && KS == 1 ? 4 : (D 
   // whose first chunk is already on its way
   const int numChunks =
       KS == 2 && len <= kChunk ? 1 : (len + kChunk - 1) / kChunk;
+  // DMA: chunk ch travels global -> LDS (buffer_load ... lds) into buffer ch % 2
+  // while the chunk before it is worked on.  An instruction fills 1 KiB in lane
+  // order, so the swizzles are applied on the source side: vector v of a tile
+  // lies at byte 16 v, and the lane fetches the chunk that belongs there.  Rows past
+  // the sequence end are outside the descriptors and arrive as zeros.
+  uint32_t dmaK[DMA ? VPT : 1], dmaV[DMA ? VPT : 1];
+  if constexpr (DMA) {
+#pragma unroll
+    for (int i = 0; i < VPT; i++) {
+      const int v = tid + i * kThreads, r = v / CPR, pc = v % CPR;
+      const int cK = swzK<D>(r, pc), cV = swzV<D>(r, pc / 4) * 4 + pc % 4;
+      dmaK[i] = PACKED_IN ? uint32_t(packedAt(r, 1, cK)) * 2u
+                          : uint32_t(r) * rowBytes + uint32_t(cK) * 16u;
+      dmaV[i] = PACKED_IN ? uint32_t(packedAt(r, 2, cV)) * 2u
+                          : uint32_t(r) * rowBytes + uint32_t(cV) * 16u;
+    }
+  }
+  auto requestChunk = [&](int ch) {
+#if defined(__HIP_DEVICE_COMPILE__) // (the builtin's LDS pointer type exists only for the GPU target)
+    if constexpr (DMA) {
+      const uint32_t chunkOff = uint32_t(ch * kChunk) * rowBytes;
+      unsigned char *dst = smem + (ch % 2) * (2 * kTileBytes) + wave * 1024;
+#pragma unroll
+      for (int i = 0; i < VPT; i++) {
+        const bool out = PACKED_IN && ch * kChunk + (tid + i * kThreads) / CPR >= len;
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(
+            rsrcK, HOM_LDS_PTR(dst + i * (kThreads * 16)), 16,
+            out ? 0x80000000u : dmaK[i] + chunkOff, 0, 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(
+            rsrcV, HOM_LDS_PTR(dst + kTileBytes + i * (kThreads * 16)), 16,
+            out ? 0x80000000u : dmaV[i] + chunkOff, 0, 0, 0);
+      }
+    }
+#endif
+  };
+  requestChunk(0);
   // (at least one round in either variant: a loop that may run zero times
   // would put a test of the sequence length ahead of the prefetched loads)
   int ch = 0;
   do {
     const int key0 = ch * kChunk;
     // keys of this chunk that any wavefront will touch, rounded up to a block
-    const int live = (len - key0 < kChunk ? ((len - key0 + 63) / 64) * 64 : kChunk);
-    if (ch > 0)
+    constexpr int kRound = SBW * 32;
+    const int live =
+        len - key0 < kChunk ? ((len - key0 + kRound - 1) / kRound) * kRound : kChunk;
+    if (ch > 0 && !DMA)
       __syncthreads(); // previous chunk fully consumed
     // ---- stage K and V rows [key0, key0 + live): 8 vectors of 16 bytes per row.
     // Rows past the sequence end are zero-filled: masked scores ignore K, but a
     // masked probability (0) times a non-finite V would poison the output.
-    if (kPrefetch) {
+    if constexpr (DMA) {
+      // this chunk has landed and every wavefront is done with the one before it,
+      // whose buffer takes the next
+      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      if (ch + 1 < numChunks)
+        requestChunk(ch + 1);
+      sK = smem + (ch % 2) * (2 * kTileBytes);
+      sV = sK + kTileBytes;
+    } else if (kPrefetch) {
 #pragma unroll
       for (int i = 0; i < VPT; i++) {
         const int v = tid + i * kThreads;
@@ -358,40 +411,48 @@ __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1, D == 64 && KS == 1 ? 4 : (D 
         }
       }
     }
-    if (kPrefetch && ch + 1 < numChunks)
-      loadChunk(key0 + kChunk);
-    __syncthreads();
+    if constexpr (!DMA) {
+      if (kPrefetch && ch + 1 < numChunks)
+        loadChunk(key0 + kChunk);
+      __syncthreads();
+    }
 
-    for (int blk = kh * 64; blk < live; blk += 64 * KS) {
+    for (int blk = kh * (SBW * 32); blk < live; blk += SBW * 32 * KS) {
       // ---- S^T = K Q^T for two 32-key sub-blocks ----
       // All eight K fragments are requested before the first MFMA: read one
       // at a time, each MFMA would wait out a full LDS round trip.
       // accS[sb][e] is the raw score (before scaling) of query l32 against key
       //   key0 + blk + sb*32 + 8*(e/4) + 4*hb + e%4.
       // Only a block that reaches past the sequence end pays for the key mask.
-      float16v accS[2];
+      float16v accS[SBW];
       auto scores = [&]() {
-        half8 fk[2][kHeadDim / 16];
+        constexpr int kSteps = kHeadDim / 16;
+        constexpr int kBatch = D <= 128 ? kSteps : kSteps / 2; // fragments read at a time
 #pragma unroll
-        for (int sb = 0; sb < 2; sb++)
-#pragma unroll
-          for (int kk = 0; kk < kHeadDim / 16; kk++)
-            fk[sb][kk] = *reinterpret_cast<const half8 *>(
-                sK + (blk + sb * 32 + l32) * kRowB + ((kk * 2 + hb) ^ swzLane) * 16);
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int sb = 0; sb < 2; sb++) {
+        for (int sb = 0; sb < SBW; sb++)
 #pragma unroll
           for (int e = 0; e < 16; e++)
             accS[sb][e] = 0.f;
 #pragma unroll
-          for (int kk = 0; kk < kHeadDim / 16; kk++)
-            accS[sb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fk[sb][kk], fq[kk],
-                                                              accS[sb], 0, 0, 0);
-        }
-        if (key0 + blk + 64 > len) {
+        for (int k0 = 0; k0 < kSteps; k0 += kBatch) {
+          half8 fk[SBW][kBatch];
 #pragma unroll
-          for (int sb = 0; sb < 2; sb++)
+          for (int sb = 0; sb < SBW; sb++)
+#pragma unroll
+            for (int kk = 0; kk < kBatch; kk++)
+              fk[sb][kk] = *reinterpret_cast<const half8 *>(
+                  sK + (blk + sb * 32 + l32) * kRowB + (((k0 + kk) * 2 + hb) ^ swzLane) * 16);
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int sb = 0; sb < SBW; sb++)
+#pragma unroll
+            for (int kk = 0; kk < kBatch; kk++)
+              accS[sb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fk[sb][kk], fq[k0 + kk],
+                                                                accS[sb], 0, 0, 0);
+        }
+        if (key0 + blk + SBW * 32 > len) {
+#pragma unroll
+          for (int sb = 0; sb < SBW; sb++)
 #pragma unroll
             for (int e = 0; e < 16; e++) {
               const int key = key0 + blk + sb * 32 + 8 * (e / 4) + 4 * hb + (e % 4);
@@ -420,13 +481,13 @@ __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1, D == 64 && KS == 1 ? 4 : (D 
       // Every block that is visited has at least one valid key, so blockMax
       // is finite and the differences below are never inf - inf.
       constexpr float kSumLimit = 4096.0f;
-      const bool first = ch == 0 && blk == kh * 64;
+      const bool first = ch == 0 && blk == kh * (SBW * 32);
       float blockSum = 0.f;
       bool slow = first;
       if (!first) {
         const float negMax = -rowMax * scaleLog2e;
 #pragma unroll
-        for (int sb = 0; sb < 2; sb++)
+        for (int sb = 0; sb < SBW; sb++)
 #pragma unroll
           for (int e = 0; e < 16; e++) {
             const float pv =
@@ -442,7 +503,7 @@ __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1, D == 64 && KS == 1 ? 4 : (D 
       if (slow) {
         float blockMax = -INFINITY;
 #pragma unroll
-        for (int sb = 0; sb < 2; sb++)
+        for (int sb = 0; sb < SBW; sb++)
 #pragma unroll
           for (int e = 0; e < 16; e++)
             blockMax = fmaxf(blockMax, accS[sb][e]);
@@ -460,7 +521,7 @@ __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1, D == 64 && KS == 1 ? 4 : (D 
         const float negMax = -rowMax * scaleLog2e;
         blockSum = 0.f;
 #pragma unroll
-        for (int sb = 0; sb < 2; sb++)
+        for (int sb = 0; sb < SBW; sb++)
 #pragma unroll
           for (int e = 0; e < 16; e++) {
             const float pv =
@@ -473,8 +534,70 @@ __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1, D == 64 && KS == 1 ? 4 : (D 
       rowSum += blockSum;
 
       // ---- O^T += V^T P^T ----
+      if constexpr (DMA) {
+        // The same reads as below, issued and waited for by hand: in front of its
+        // own transposing reads the compiler would wait for every copy into LDS
+        // that is on its way, i.e. for the whole next chunk.
+        // INVARIANT: what an asm read writes is not valid until the wait; the
+        // values pass through an empty asm behind it so that nothing moves ahead.
+        constexpr int kGroups = SBW * 2, kSets = D <= 128 ? 2 : 1;
+        const uint32_t vLane = uint32_t(uintptr_t(HOM_LDS_PTR(sV))) +
+                               uint32_t((blk + 4 * hb + trRow) * kRowB + trCol * 2);
+        short4v run[kSets][DB][2];
+        auto readGroup = [&](auto gC) {
+          constexpr int g = decltype(gC)::value;
 #pragma unroll
-      for (int sb = 0; sb < 2; sb++) {
+          for (int d = 0; d < DB; d++) {
+            const uint32_t at = vLane + uint32_t((d ^ vSwz) * 64);
+            asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2"
+                         : "=v"(run[g % kSets][d][0])
+                         : "v"(at), "i"(g * 16 * kRowB));
+            asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2"
+                         : "=v"(run[g % kSets][d][1])
+                         : "v"(at), "i"((g * 16 + 8) * kRowB));
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        };
+        __builtin_amdgcn_sched_barrier(0);
+        readGroup(std::integral_constant<int, 0>{});
+        auto pvGroup = [&](auto gC) {
+          constexpr int g = decltype(gC)::value;
+          constexpr bool kMore = g + 1 < kGroups;
+          using Next = std::integral_constant<int, kMore ? g + 1 : 0>;
+          half8 fp;
+#pragma unroll
+          for (int e = 0; e < 8; e++)
+            fp[e] = _Float16(accS[g / 2][8 * (g % 2) + e]);
+          __builtin_amdgcn_sched_barrier(0);
+          if constexpr (kMore && kSets == 2)
+            readGroup(Next{});
+          asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(kMore && kSets == 2 ? DB * 2 : 0) : "memory");
+#pragma unroll
+          for (int d = 0; d < DB; d++) {
+            short4v lo = run[g % kSets][d][0], hi = run[g % kSets][d][1];
+            asm volatile("" : "+v"(lo), "+v"(hi)); // not before the wait
+            short8v both;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+              both[e] = lo[e];
+              both[4 + e] = hi[e];
+            }
+            accO[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+                __builtin_bit_cast(half8, both), fp, accO[d], 0, 0, 0);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+          if constexpr (kMore && kSets == 1)
+            readGroup(Next{});
+        };
+        pvGroup(std::integral_constant<int, 0>{});
+        pvGroup(std::integral_constant<int, 1>{});
+        if constexpr (kGroups == 4) {
+          pvGroup(std::integral_constant<int, 2>{});
+          pvGroup(std::integral_constant<int, 3>{});
+        }
+      } else {
+#pragma unroll
+      for (int sb = 0; sb < SBW; sb++) {
 #pragma unroll
         for (int t = 0; t < 2; t++) {
           // B operand: P[q][key(hb, e)], key(hb, e) = sb*32 + 8*(2t + e/4) + 4*hb
@@ -506,6 +629,7 @@ __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1, D == 64 && KS == 1 ? 4 : (D 
           }
         }
       }
+      }
     }
   } while (++ch < numChunks);
 
@@ -518,7 +642,7 @@ __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1, D == 64 && KS == 1 ? 4 : (D 
   // always owns the first block, which has one.
   if constexpr (KS == 2) {
     constexpr int XV = DB * 16; // accumulator values per lane
-    static_assert(QG * (XV + 2) * kWave * 4 <= 2 * kTileBytes, "exchange fits the K/V tiles");
+    static_assert(DMA || QG * (XV + 2) * kWave * 4 <= 2 * kTileBytes, "exchange fits the K/V tiles");
     float *xch = reinterpret_cast<float *>(smem) + qg * ((XV + 2) * kWave) + lane;
     __syncthreads(); // every wavefront is done with K and V
     if (kh == 1) {
@@ -559,9 +683,51 @@ __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1, D == 64 && KS == 1 ? 4 : (D 
 #pragma unroll
         for (int e = 0; e < 4; e++)
           o[e] = valid ? _Float16(accO[d][g * 4 + e] * inv) : _Float16(0);
-        *reinterpret_cast<half4 *>(outAt(q, d * 32 + g * 8 + hb * 4)) = o;
+        *reinterpret_cast<half4 *>(oRow + d * oWide + g * oEight) = o;
       }
   }
+}
+
+struct Launch {
+  const _Float16 *qkv;
+  const int32_t *cu;
+  _Float16 *out;
+  int64_t bs, seq, heads;
+  float scale;
+  int packedOut;
+  const char *ahead;
+  int64_t aheadBytes;
+  unsigned extra; // workgroups that read ahead
+  hipStream_t stream;
+};
+template <int NW, int KS, int D, bool PACKED_IN, bool DMA> Status launchVariant(const Launch &l) {
+  constexpr int QG = NW / KS;
+  constexpr int kTileBytes = (DMA ? 64 : Chunk<D>::value) * D * 2;
+  constexpr int kExchange = KS == 2 ? QG * (D / 2 + 2) * kWave * 4 : 0;
+  constexpr int kTiles = (DMA ? 4 : 2) * kTileBytes;
+  constexpr int kLds = kTiles > kExchange ? kTiles : kExchange;
+  auto kernel = bertAttentionKernel<NW, KS, D, PACKED_IN, DMA>;
+  if (kLds > 64 * 1024) {
+    static bool done = false;
+    if (!done)
+      HOM_HIP_RET(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
+                                      hipFuncAttributeMaxDynamicSharedMemorySize, kLds),
+                  Status::kInternal);
+    done = true;
+  }
+  const unsigned nq = unsigned((l.seq + QG * 32 - 1) / (QG * 32));
+  const int64_t pairs = l.bs * l.heads;
+  dim3 grid(unsigned(nq * pairs) + l.extra);
+  if (KS == 2 && !DMA) {
+    const unsigned plane = nq * unsigned(l.heads);
+    grid = dim3(nq, unsigned(l.heads), unsigned(l.bs) + (l.extra + plane - 1) / plane);
+  }
+  kernel<<<grid, dim3(NW * kWave), kLds, l.stream>>>(l.qkv, l.cu, l.out, int(l.seq), int(l.heads),
+                                                     int(nq), int(l.bs), l.scale, l.packedOut,
+                                                     magicFor(nq), magicFor(uint32_t(l.heads)),
+                                                     l.ahead, l.aheadBytes);
+  HOM_HIP_RET(hipGetLastError(), Status::kInternal);
+  return Status::kSuccess;
 }
 
 } // namespace
@@ -596,68 +762,72 @@ Status launchBertAttentionF16(const _Float16 *qkv, const int32_t *cuSeqlens,
                 Status::kInvalidArgument, "attention: misaligned operands");
   if (bs == 0 || seq == 0 || heads == 0)
     return Status::kSuccess;
-  // 128 query rows per workgroup (one wavefront per 32 rows) when that still
-  // gives every CU work, otherwise 64 with the keys split over two wavefronts
-  // per 32 rows (K/V of a (batch, head) are then staged by two workgroups).
-  const int cus = deviceInfo().computeUnits;
+  const int cus = deviceInfo().computeUnits > 0 ? deviceInfo().computeUnits : 256;
   const int64_t pairs = bs * heads;
-  bool wide = pairs * ((seq + 127) / 128) >= int64_t(cus) || seq <= 32;
-  // profiling knob: HOM_ATTENTION_VARIANT=wide | split
-  if (const char *force = getenv("HOM_ATTENTION_VARIANT"))
-    wide = strcmp(force, "wide") == 0;
-  if (headDim > 128)
-    wide = true; // (the key-split variant exists for 64 and 128 only)
   HOM_CHECK_RET(pairs * ((seq + 63) / 64) < (int64_t(1) << 31),
                 Status::kInvalidArgument, "attention: too many workgroups");
   // Workgroups that read weights ahead (readAhead() in packed_args.h), while the
   // attention itself leaves room: two workgroups of it per CU or fewer.
   const unsigned extra =
       ahead && pairs * ((seq + 127) / 128) <= 2 * cus ? aheadGroups<256>(aheadBytes, cus) : 0;
-  if (wide) {
-    const int nq = int((seq + 127) / 128);
-    const dim3 grid((unsigned)(nq * pairs));
-    if (packedIn)
-      bertAttentionKernel<4, 1, 64, true><<<dim3(grid.x + extra), dim3(256), 0, s>>>(
-          qkv, cuSeqlens, out, int(seq), int(heads), nq, int(pairs), scale,
-          packedOut, static_cast<const char *>(ahead), aheadBytes);
-    else if (headDim == 64)
-      bertAttentionKernel<4, 1, 64><<<grid, dim3(256), 0, s>>>(
-          qkv, cuSeqlens, out, int(seq), int(heads), nq, int(pairs), scale,
-          packedOut, nullptr, 0);
-    else if (headDim == 128)
-      bertAttentionKernel<4, 1, 128><<<grid, dim3(256), 0, s>>>(
-          qkv, cuSeqlens, out, int(seq), int(heads), nq, int(pairs), scale,
-          packedOut, nullptr, 0);
-    else if (headDim == 192)
-      bertAttentionKernel<4, 1, 192><<<grid, dim3(256), 0, s>>>(
-          qkv, cuSeqlens, out, int(seq), int(heads), nq, int(pairs), scale,
-          packedOut, nullptr, 0);
-    else
-      bertAttentionKernel<4, 1, 256><<<grid, dim3(256), 0, s>>>(
-          qkv, cuSeqlens, out, int(seq), int(heads), nq, int(pairs), scale,
-          packedOut, nullptr, 0);
-  } else {
-    const int nq = int((seq + 63) / 64);
-    HOM_CHECK_RET(heads < 65536 && bs < 65536, Status::kInvalidArgument,
-                  "attention: heads and batch size must be below 65536");
-    const dim3 grid((unsigned)nq, (unsigned)heads, (unsigned)bs);
-    const unsigned plane = unsigned(nq) * unsigned(heads);
-    if (packedIn)
-      bertAttentionKernel<4, 2, 64, true>
-          <<<dim3(grid.x, grid.y, grid.z + (extra + plane - 1) / plane), dim3(256), 0, s>>>(
-              qkv, cuSeqlens, out, int(seq), int(heads), nq, int(pairs), scale, packedOut,
-              static_cast<const char *>(ahead), aheadBytes);
-    else if (headDim == 64)
-      bertAttentionKernel<4, 2, 64><<<grid, dim3(256), 0, s>>>(
-          qkv, cuSeqlens, out, int(seq), int(heads), nq, int(pairs), scale,
-          packedOut, nullptr, 0);
-    else
-      bertAttentionKernel<4, 2, 128><<<grid, dim3(256), 0, s>>>(
-          qkv, cuSeqlens, out, int(seq), int(heads), nq, int(pairs), scale,
-          packedOut, nullptr, 0);
+  const Launch l{qkv, cuSeqlens, out, bs, seq, heads, scale, packedOut,
+                 static_cast<const char *>(ahead), aheadBytes, packedIn ? extra : 0, s};
+  // Four ways, all with the same arithmetic per 32 query rows (us, lengths uniform
+  // in [seq / 4, seq], batch : seq : heads):
+  //  - Prefetch: 64 rows per workgroup with the keys split over two wavefronts per
+  //    32 rows, K and V of the first 128 keys requested before anything else is
+  //    known.  The fastest while that is all of them and workgroups are few
+  //    (head size 64, 8:128:12 4.2, against 5.0 - 5.3).
+  //  - Wide: 128 rows, chunks of 128 keys through registers; head size 64 for so
+  //    many short sequences that the workgroups of a CU cover each other
+  //    (64:128:12 10.5 against 10.8), and 256, whose chunks by DMA would leave too
+  //    few registers (8:384:16 42 against 47).
+  //  - Dma: 128 rows, chunks of 64 keys straight into LDS while the one before is
+  //    worked on (head size 64, 32:512:16 41.8 -> 40.6, 1:64:12 4.0 -> 3.6; 128,
+  //    32:512:16 66.9 -> 60.9).  Head size 192: 8 wavefronts, two per 32 rows, which
+  //    then fit two to a SIMD (32:512:12 117 -> 97).
+  //  - DmaSplit: the same with 64 rows and two wavefronts per 32 rows, for fewer
+  //    workgroups than fill the chip twice (head size 64, 2:700:16 13.1 -> 10.8;
+  //    128, 2:700:12 21.2 -> 17.6; 192, 2:100:8 10.0 -> 8.5; 256 12.5 -> 10.5).
+  enum { Prefetch, Wide, Dma, DmaSplit } way;
+  const int64_t tiles = pairs * ((seq + 127) / 128);
+  if (headDim == 64)
+    way = seq <= 64    ? Dma
+          : seq <= 128 ? (tiles < cus ? Prefetch : Wide)
+                       : (tiles < 2 * cus ? DmaSplit : Dma);
+  else if (headDim == 128)
+    way = seq > 64 && (tiles < cus / 2 || (seq > 128 && tiles < 2 * cus)) ? DmaSplit : Dma;
+  else
+    way = tiles < cus / 2 ? DmaSplit : headDim == 192 ? Dma : Wide;
+  // profiling knob: HOM_ATTENTION_VARIANT=wide | split
+  if (const char *force = getenv("HOM_ATTENTION_VARIANT"))
+    way = strcmp(force, "wide") == 0 ? (headDim == 256 ? Wide : Dma) : DmaSplit;
+  switch (headDim) {
+  case 64:
+    switch (way) {
+    case Prefetch:
+      return packedIn ? launchVariant<4, 2, 64, true, false>(l)
+                      : launchVariant<4, 2, 64, false, false>(l);
+    case Wide:
+      return packedIn ? launchVariant<4, 1, 64, true, false>(l)
+                      : launchVariant<4, 1, 64, false, false>(l);
+    case Dma:
+      return packedIn ? launchVariant<4, 1, 64, true, true>(l)
+                      : launchVariant<4, 1, 64, false, true>(l);
+    default:
+      return packedIn ? launchVariant<4, 2, 64, true, true>(l)
+                      : launchVariant<4, 2, 64, false, true>(l);
+    }
+  case 128:
+    return way == Dma ? launchVariant<4, 1, 128, false, true>(l)
+                      : launchVariant<4, 2, 128, false, true>(l);
+  case 192:
+    return way == Dma ? launchVariant<8, 2, 192, false, true>(l)
+                      : launchVariant<4, 2, 192, false, true>(l);
+  default:
+    return way == Wide ? launchVariant<4, 1, 256, false, false>(l)
+                       : launchVariant<4, 2, 256, false, true>(l);
   }
-  HOM_HIP_RET(hipGetLastError(), Status::kInternal);
-  return Status::kSuccess;
 }
 
 } // namespace hom

@@ -327,3 +327,28 @@ def test_encoder_many_rows_equals_row_major(synth, bs, seq):
             enc.close()
     live = np.asarray(model["mask"]).astype(bool)
     np.testing.assert_allclose(got[0][live], got[1][live], rtol=1e-2, atol=1e-2)
+
+
+# every way the attention is split, lengths around its chunk ends; what lies behind a sequence must not matter
+@pytest.mark.parametrize("bs,seq,heads,d", [(2, 60, 4, 64), (3, 100, 4, 64), (30, 128, 12, 64), (2, 300, 4, 64),
+                                            (40, 200, 8, 64), (2, 64, 4, 128), (3, 130, 4, 128), (40, 256, 8, 128),
+                                            (2, 70, 3, 192), (16, 129, 9, 192), (2, 70, 3, 256), (16, 129, 9, 256),
+                                            (5, 193, 2, 256)])
+def test_attention_splits(gpu, rt, bs, seq, heads, d):
+    g = torch.Generator("cuda").manual_seed(seq + d)
+    qkv = torch.randn(bs, seq, 3, heads, d, device="cuda", generator=g).half()
+    lens = torch.randint(1, seq + 1, (bs,), device="cuda", generator=g)
+    lens[0], lens[-1] = seq, min(seq, 65)
+    live = torch.arange(seq, device="cuda")[None, :] < lens[:, None]
+    q, k, v = qkv.float().permute(2, 0, 3, 1, 4).contiguous()
+    s = torch.matmul(q, k.transpose(2, 3).contiguous()) / d ** 0.5
+    want = torch.matmul(s.masked_fill(~live[:, None, None, :], float("-inf")).softmax(-1), v).permute(0, 2, 1, 3)
+    want = want.reshape(bs, seq, heads * d) * live[:, :, None]
+    qkv[~live] = float("nan")
+    cu = torch.zeros(bs + 1, dtype=torch.int32, device="cuda")
+    cu[1:] = lens.cumsum(0)
+    out = torch.full((bs, seq, heads * d), 7.0, dtype=torch.float16, device="cuda")
+    Mr = rt.MemRef
+    gpu.nvteBertAttentionF16(*Mr.from_tensor(qkv.view(bs, seq, -1)).args(), *Mr.from_tensor(cu).args(),
+                             *Mr.from_tensor(out).args(), d ** -0.5, heads)
+    torch.testing.assert_close(out.float(), want, rtol=2e-3, atol=2e-3)
