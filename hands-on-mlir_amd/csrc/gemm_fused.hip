@@ -13,28 +13,29 @@ using namespace gemmk;
 // ------------------------------------------------------- layer-norm pair --
 // Row-statistic partials [pieces][M] (sum, sum of squares) -> var / mean in the
 // form the pair exchanges (Layernorm.h:166-192 of the reference: the second
-// moment minus the squared mean, no shift).  Four lanes per row, 16 apart in
-// the wavefront so that 16 neighbouring lanes read 16 neighbouring rows; each
-// takes every fourth piece, four loads in flight.
-__global__ __launch_bounds__(256) void rowStatsFinalizeKernel(
+// moment minus the squared mean, no shift).  A chain of latencies: a wavefront
+// has 16 rows, four lanes each, 16 apart so that 16 neighbouring lanes read 16
+// neighbouring rows; a lane asks for every fourth piece, eight at a time (32 pieces
+// in one go), and a workgroup is one wavefront, so that all CUs take part.
+__global__ __launch_bounds__(kWave) void rowStatsFinalizeKernel(
     const float *__restrict__ partials, int pieces, int M, int N, float eps,
     _Float16 *__restrict__ var, _Float16 *__restrict__ mean) {
-  const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
-  const int q = lane / 16;
-  const int m = (blockIdx.x * 4 + wave) * 16 + lane % 16;
+  const int lane = threadIdx.x, q = lane / 16;
+  const int m = blockIdx.x * 16 + lane % 16;
   const int mc = m < M ? m : M - 1;
+  constexpr int kLoads = 8;
   float s = 0.f, sq = 0.f;
-  for (int pc = q; pc < pieces; pc += 16) {
-    float2v v[4];
+  for (int pc = q; pc < pieces; pc += 4 * kLoads) {
+    float2v v[kLoads];
 #pragma unroll
-    for (int u = 0; u < 4; u++) {
+    for (int u = 0; u < kLoads; u++) {
       const int pu = pc + 4 * u;
       v[u] = pu < pieces ? *reinterpret_cast<const float2v *>(
                                partials + (int64_t(pu) * M + mc) * 2)
                          : float2v{0.f, 0.f};
     }
 #pragma unroll
-    for (int u = 0; u < 4; u++) {
+    for (int u = 0; u < kLoads; u++) {
       s += v[u][0];
       sq += v[u][1];
     }
@@ -52,49 +53,45 @@ __global__ __launch_bounds__(256) void rowStatsFinalizeKernel(
 }
 
 // Partial column sums of row-major B [K, N]: workgroup (x, y) sums rows
-// [y * kPer, (y + 1) * kPer) of columns [32 x, 32 x + 32) into out[y][n].  A
-// thread reads 8 columns of every 64th row; the 64 row phases meet in LDS.
+// [y * kPer, (y + 1) * kPer) of columns [64 x, 64 x + 64) into out[y][n]: whole
+// cache lines, 8 columns of every 32nd row per thread, four rows asked for at a
+// time; the row phases of a wavefront meet in registers, the wavefronts in LDS.
 __global__ __launch_bounds__(256) void colSumKernel(
     const _Float16 *__restrict__ B, int64_t ldb, int K, int N, int kPer,
     float *__restrict__ out) {
-  __shared__ float part[64][33];
-  const int tid = threadIdx.x;
-  const int cg = tid % 4, ph = tid / 4;
-  const int n = blockIdx.x * 32 + cg * 8;
+  __shared__ float part[4][64];
+  const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
+  const int cg = tid % 8, ph = tid / 8;
+  const int n = blockIdx.x * 64 + cg * 8;
   const int kBegin = blockIdx.y * kPer;
   const int kEnd = kBegin + kPer < K ? kBegin + kPer : K;
   float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   if (n < N) {
-#pragma unroll 4
-    for (int k = kBegin + ph; k < kEnd; k += 64) {
-      const half8 v = *reinterpret_cast<const half8 *>(B + int64_t(k) * ldb + n);
+    for (int k = kBegin + ph; k < kEnd; k += 128) {
+      half8 v[4];
 #pragma unroll
-      for (int e = 0; e < 8; e++)
-        acc[e] += float(v[e]);
+      for (int u = 0; u < 4; u++) {
+        const int ku = k + 32 * u;
+        v[u] = *reinterpret_cast<const half8 *>(B + int64_t(ku < kEnd ? ku : k) * ldb + n);
+      }
+#pragma unroll
+      for (int u = 0; u < 4; u++)
+#pragma unroll
+        for (int e = 0; e < 8; e++)
+          acc[e] += k + 32 * u < kEnd ? float(v[u][e]) : 0.f;
     }
   }
+  // (lanes 8 apart hold the same columns)
 #pragma unroll
-  for (int e = 0; e < 8; e++)
-    part[ph][cg * 8 + e] = acc[e];
-  __syncthreads();
-  // 64 phases -> 8 -> 1, every thread busy in the first step
-  {
-    const int c = tid % 32, grp = tid / 32;
-    float sum = 0.f;
-#pragma unroll
-    for (int r = 0; r < 8; r++)
-      sum += part[grp * 8 + r][c];
-    __syncthreads();
-    part[grp][c] = sum;
+  for (int e = 0; e < 8; e++) {
+    const float s = pairSum(rowPairSum(acc[e] + __shfl_xor(acc[e], 8, kWave)));
+    if (lane < 8)
+      part[wave][lane * 8 + e] = s;
   }
   __syncthreads();
-  if (tid < 32 && blockIdx.x * 32 + tid < N) {
-    float sum = 0.f;
-#pragma unroll
-    for (int r = 0; r < 8; r++)
-      sum += part[r][tid];
-    out[int64_t(blockIdx.y) * N + blockIdx.x * 32 + tid] = sum;
-  }
+  if (tid < 64 && blockIdx.x * 64 + tid < N)
+    out[int64_t(blockIdx.y) * N + blockIdx.x * 64 + tid] =
+        (part[0][tid] + part[1][tid]) + (part[2][tid] + part[3][tid]);
 }
 
 // Tiles the layer-norm pair kernels exist in (square, `edge` on a side, a
@@ -161,7 +158,7 @@ Status launchGemmRowStats(int likeKernel, const GemmProblem &p, _Float16 *var,
   Status st = launchFusedTile<kEpiRowStats>(likeKernel, q, s);
   if (st != Status::kSuccess)
     return st;
-  rowStatsFinalizeKernel<<<dim3((unsigned)((p.M + 63) / 64)), dim3(256), 0,
+  rowStatsFinalizeKernel<<<dim3((unsigned)((p.M + 15) / 16)), dim3(kWave), 0,
                            s>>>(partials, pieces, int(p.M), int(p.N), eps, var,
                                 mean);
   HOM_HIP_RET(hipGetLastError(), Status::kInternal);
@@ -174,7 +171,7 @@ Status launchGemmRowAffine(int likeKernel, const GemmProblem &p,
   HOM_CHECK_RET(likeKernel >= 0 && likeKernel < gemmKernelCount() && fusedGemmFits(p),
                 Status::kInvalidArgument,
                 "layernorm + gemm: problem does not fit the fused kernels");
-  // 128 rows of B per column-sum workgroup (two 16-byte loads per lane), at
+  // 128 rows of B per column-sum workgroup (four 16-byte loads per lane), at
   // most 16 slices
   int slices = int((p.K + 127) / 128);
   if (slices > 16)
@@ -184,7 +181,7 @@ Status launchGemmRowAffine(int likeKernel, const GemmProblem &p,
       libraryScratch(kTemp, size_t(slices) * size_t(p.N) * sizeof(float), false));
   if (!colSum)
     return Status::kInternal;
-  colSumKernel<<<dim3((unsigned)((p.N + 31) / 32), (unsigned)slices), dim3(256),
+  colSumKernel<<<dim3((unsigned)((p.N + 63) / 64), (unsigned)slices), dim3(256),
                  0, s>>>(p.B, p.ldb, int(p.K), int(p.N), kPer, colSum);
   HOM_HIP_RET(hipGetLastError(), Status::kInternal);
   GemmProblem q = p;
@@ -210,7 +207,7 @@ Status launchColumnSums(const _Float16 *B, int64_t ldb, int64_t K, int64_t N,
                     aligned16(B),
                 Status::kInvalidArgument,
                 "column sums: N and the leading dimension must be multiples of 8");
-  colSumKernel<<<dim3((unsigned)((N + 31) / 32), 1), dim3(256), 0, s>>>(
+  colSumKernel<<<dim3((unsigned)((N + 63) / 64), 1), dim3(256), 0, s>>>(
       B, ldb, int(K), int(N), int(K), out);
   HOM_HIP_RET(hipGetLastError(), Status::kInternal);
   return Status::kSuccess;
