@@ -453,7 +453,11 @@ constexpr Tile kTiles[] = {{256, 256, 4.5, 1.09, 11.5e6, 1.0, 11.5e6},
                            {256, 128, 2.5, 0.57, 11.5e6, 0.93, 14.5e6},
                            {128, 128, 1.1, 0.43, 14.5e6, 0.88, 18.0e6},
                            {64, 128, 0.7, 0.27, 18.5e6, 0.8, 18.5e6},
-                           {64, 64, 0.4, 0.20, 22.5e6, 0.8, 22.5e6}};
+                           {64, 64, 0.4, 0.20, 22.5e6, 0.8, 22.5e6},
+                           {64, 192, 0.9, 0.40, 14.5e6, 1.0, 14.5e6}};
+// (Row sums between the MFMAs cost a quarter of the main loop; least where a
+// wavefront has three MFMAs to a fragment of A.)
+constexpr double kRowSumFactor[] = {1.25, 1.25, 1.25, 1.25, 1.25, 1.1};
 
 // More tiles than CUs: slabs of 32 k, so that two rings fit a CU and one
 // workgroup's epilogue runs beside the other's main loop (128 x 128: 4096 x 3072 x 768
@@ -478,12 +482,12 @@ PackedTileChoice choosePackedTile(const PackedGemm &g) {
     const Tile &t = kTiles[i];
     const int64_t tiles = ((g.M + t.bm - 1) / t.bm) * ((g.N + t.bn - 1) / t.bn);
     const double perCu = double((tiles + cus - 1) / cus);
-    const bool shared = i >= 3 ? perCu > 1 : sharesCu(g, tiles, cus);
+    const bool shared = i == 3 || i == 4 ? perCu > 1 : sharesCu(g, tiles, cus);
     const double loop =
         std::max({perCu * double(g.K) / 64 * t.slabUs * (shared ? t.sharedFactor : 1.0),
                   double(tiles) * (t.bm + t.bn) * double(g.K) * 2 / (shared ? t.sharedRate : t.rate),
                   2.0 * double(g.M) * double(g.N) * double(g.K) / 1.2e9});
-    const double us = 2.2 + loop * (g.normA ? 1.25 : 1.0) +
+    const double us = 2.2 + loop * (g.normA ? kRowSumFactor[i] : 1.0) +
                       perCu * (t.fixedUs + (g.activation ? 5e-5 * t.bm * t.bn : 0));
     if (us < best.us)
       best = {i, us};
@@ -510,8 +514,10 @@ Status launchPackedTile(int tile, const PackedGemm &g, const PackedArgs &p, hipS
                : launchTile<128, 128, 2, 4, 2, 4>(g, p, s);
   case 3:
     return launchTile<64, 128, 1, 4, 2, 4>(g, p, s);
-  default:
+  case 4:
     return launchTile<64, 64, 2, 2, 2, 4>(g, p, s);
+  default: // (between 128 x 128 and 64 x 128: 1024 x 3072 x 768 11.5 -> 10.4 us, 2304 columns 10.0 -> 8.9)
+    return launchTile<64, 192, 2, 2, 2, 3>(g, p, s);
   }
 }
 

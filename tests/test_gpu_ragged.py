@@ -231,7 +231,7 @@ def test_packed_gemm(gpu, rt, oracle, M, N, K, packing):
 
 # every tile of the packed GEMM for many rows, with one tile and with several of them per workgroup; partial row
 # blocks and column tiles, and rectangles of an XCD that the tiles do not fill
-@pytest.mark.parametrize("M,N,K", [(192, 768, 3072), (250, 1088, 2080), (1000, 768, 3072), (760, 1088, 2048),
+@pytest.mark.parametrize("M,N,K", [(1000, 3072, 768), (192, 768, 3072), (250, 1088, 2080), (1000, 768, 3072), (760, 1088, 2048),
                                    (1000, 1024, 1024), (8000, 3072, 768), (392, 1184, 64), (524, 1856, 64), (583, 3296, 64), (1476, 2976, 448),
                                    (16439, 160, 64), (10970, 352, 192), (17111, 288, 64), (16546, 672, 128),
                                    (16388, 1696, 128)])
