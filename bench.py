@@ -141,6 +141,7 @@ def main():
     layouts = {r: ("[N,K] via nvteGemmF16" if enc.role_is_nk(r) else "[K,N] via cutlassGemmF16")
                for r in ("qkv", "out", "ffn1", "ffn2")}
     names = {i + 1: n for i, n, _, _ in rt.manifest()}
+    packed = enc.uses_packed()
     enc.close()
     # a [N, K] role goes through nvteGemmF16, which picks the kernel per call: ask the library which
     M_rows = d["bs"] * d["seq"]
@@ -279,7 +280,7 @@ def main():
             "call_list": "optional: homGemmFoldedLayernormF16 in place of GEMM + nvteLayernormF16"}
 
     # Several independent forwards in flight: one encoder instance (its own buffers, stream and captured graph) per
-    # forward, replays issued round-robin.  A b8 x s128 forward is 88 dependent launches of a few microseconds that
+    # forward, replays issued round-robin.  A b8 x s128 forward is 62 dependent launches of a few microseconds that
     # leave the chip idle between and partly inside them (192 tiles on 256 CUs); a second and third stream fill that.
     # Timed with the host clock around issue + synchronisation of every stream (there is no single stream to put
     # events on); every instance's output is compared with the single-stream one.
@@ -317,15 +318,17 @@ def main():
             "note": "throughput of independent batches on separate streams; the headline value is one forward "
                     "after the other, the reference's protocol"}
 
-    # What the chain of launches itself costs: 88 empty kernels as the nodes of one replayed graph.  A forward is 88
-    # dependent kernels, so this times 88 is the part of ms_per_step no kernel can win back.
+    # What the chain of launches itself costs: as many empty kernels as a forward has dependent ones (embedding, 5 a
+    # layer on packed weights or else 7, and a final or an initial pair) as the nodes of one replayed graph; the part
+    # of ms_per_step no kernel can win back.
     # (left out under a tracer: its ~20 000 empty dispatches would only pad the trace)
     if not args.eager and not traced:
-        node_ms = drv.homTimeEmptyGraphNodes(88, 256, 200)
+        nodes = 62 if packed else 88
+        node_ms = drv.homTimeEmptyGraphNodes(nodes, 256, 200)
         if node_ms > 0:
-            kernels["graph_of_88_empty_kernels"] = {
-                "us_per_node": node_ms * 1e3, "us_per_graph": node_ms * 88e3,
-                "note": "floor under the 88 dependent kernel nodes of the b8 x s128 forward"}
+            kernels["graph_of_empty_kernels"] = {
+                "nodes": nodes, "us_per_node": node_ms * 1e3, "us_per_graph": node_ms * nodes * 1e3,
+                "note": "floor under the dependent kernel nodes of the b8 x s128 forward"}
 
     # the reference's whole BertForMaskedLM graph: encoder + LM head to logits [8, 128, 30522]
     enc = bert.BertEncoder(d["layers"], d["hidden"], d["heads"], d["ffn"], d["bs"], d["seq"], d["vocab"],
@@ -352,7 +355,8 @@ def main():
                                "batch 8 x seq 128, padding mask (configs[3])",
                    "launch": "eager C-ABI calls" if args.eager else "HIP graph replay of the C-ABI call list",
                    "gemm_mode": args.gemm_mode,
-                   "gemm_kernels": {k: {"kernel": names.get(v[0], "library-selected"), "splitK": v[1],
+                   "gemm_kernels": "homPackedGemmF16 on weights in fragment order, tile chosen by size" if packed else
+                                   {k: {"kernel": names.get(v[0], "library-selected"), "splitK": v[1],
                                         "weights": layouts[k]}
                                     for k, v in choices.items()}},
         "encoder_TFLOP/s": flops_forward / (ms * 1e-3) / 1e12,

@@ -130,6 +130,10 @@ class BertEncoder:
     def role_is_nk(self, role):
         return bool(self.drv.homBertRoleIsNK(self.h, self.ROLES.index(role)))
 
+    def uses_packed(self):
+        """Whether the layer GEMMs run on packed weights (homPackedGemmF16) instead of gemm_choices()."""
+        return bool(self.drv.homBertUsesPacked(self.h))
+
     def gemm_choices(self):
         buf = (ctypes.c_int32 * 8)()
         self.drv.homBertGetGemmChoices(self.h, buf)

@@ -941,6 +941,10 @@ DRV_EXPORT int homBertSetGemmChoice(HomBertEncoder *e, int role,
   return 0;
 }
 
+// Whether the layers run on packed weights (homPackedGemmF16) instead of the kernels
+// of homBertGetGemmChoices.
+DRV_EXPORT int homBertUsesPacked(HomBertEncoder *e) { return e->packed; }
+
 // ---- single-operator timing through the boundary -------------------------
 // Each helper enqueues `iters` back-to-back calls of one entry point between
 // two events on a private stream, behind a warm-up (Timer::warm), and returns
