@@ -41,7 +41,8 @@ class BertEncoder:
                                                   1 if gelu_form == "tanh" else 0, layout)
         if not self.h:
             raise ValueError("homBertCreateWithLayout refused the configuration (a GELU role of an erf-GELU "
-                             "graph pinned to [N, K] weights: nvteGemmF16 computes the tanh form only)")
+                             "graph pinned to [N, K] weights: nvteGemmF16 computes the tanh form only) or "
+                             "could not allocate the encoder; the message is on stderr")
         self.lm_head = lm_head
         if lm_head:
             assert self.drv.homBertEnableLmHead(self.h) == 0, "homBertEnableLmHead failed"

@@ -355,35 +355,37 @@ float *packedColSum(const HomBertEncoder *e, int l, bool ffn1) {
          (ffn1 ? 3 * e->hidden : 0);
 }
 
-bool packWeights(HomBertEncoder *e) {
-  if (!e->packed || e->packedReady)
-    return true;
+// What the packed list needs besides the row-major buffers.  All of it at
+// creation: a forward allocates nothing and cannot fail for want of memory.
+bool allocPacked(HomBertEncoder *e) {
   const int64_t H = e->hidden, F = e->ffn;
   const int rows = (e->batch * e->seq + 15) / 16 * 16;
-  if (!e->packedArena) {
-    const size_t bytes = size_t(packedLayer(e, e->layers).qkv);
-    if (!hipOk(hipMalloc(reinterpret_cast<void **>(&e->packedArena), bytes), "hipMalloc") ||
-        !hipOk(hipMalloc(reinterpret_cast<void **>(&e->packedColSums),
-                         size_t(e->layers) * size_t(3 * H + F) * 4),
-               "hipMalloc"))
+  auto alloc = [](auto *&p, size_t bytes) {
+    return hipOk(hipMalloc(reinterpret_cast<void **>(&p), bytes), "hipMalloc of packed weights");
+  };
+  if (!alloc(e->packedArena, size_t(packedLayer(e, e->layers).qkv)) ||
+      !alloc(e->packedColSums, size_t(e->layers) * size_t(3 * H + F) * 4) ||
+      !alloc(e->packedStats[0], size_t(rows) * 8) || !alloc(e->packedStats[1], size_t(rows) * 8))
+    return false;
+  // (the logical shape is [batch, seq, .]: the padding rows lie behind it)
+  auto padded = [&](Tensor &t, int64_t cols) {
+    t.m = alloc3DMemRefNVGPUF16(1, rows, int32_t(cols));
+    if (!t.m.descriptor)
       return false;
-    for (float *&q : e->packedStats)
-      if (!hipOk(hipMalloc(reinterpret_cast<void **>(&q), size_t(rows) * 8), "hipMalloc"))
-        return false;
-    // (the logical shape is [batch, seq, .]: the padding rows lie behind it)
-    auto padded = [&](Tensor &t, int cols) {
-      t.m = alloc3DMemRefNVGPUF16(1, rows, cols);
-      int64_t *sz = hom_memref_sizes(t.m.descriptor);
-      int64_t *st = hom_memref_strides(t.m.descriptor, 3);
-      sz[0] = e->batch;
-      sz[1] = e->seq;
-      st[0] = int64_t(e->seq) * cols;
-    };
-    padded(e->hPacked, int(H));
-    padded(e->qkvPacked, int(3 * H));
-    padded(e->attnPacked, int(H));
-    padded(e->fPacked, int(F));
-  }
+    int64_t *sz = hom_memref_sizes(t.m.descriptor);
+    int64_t *st = hom_memref_strides(t.m.descriptor, 3);
+    sz[0] = e->batch;
+    sz[1] = e->seq;
+    st[0] = int64_t(e->seq) * cols;
+    return true;
+  };
+  return padded(e->hPacked, H) && padded(e->qkvPacked, 3 * H) && padded(e->attnPacked, H) &&
+         padded(e->fPacked, F);
+}
+
+void packWeights(HomBertEncoder *e) {
+  if (!e->packed || e->packedReady)
+    return;
   void *prev = homGetStream();
   homSetStream(e->stream);
   for (int l = 0; l < e->layers; l++) {
@@ -398,7 +400,6 @@ bool packWeights(HomBertEncoder *e) {
   }
   homSetStream(prev);
   e->packedReady = true;
-  return true;
 }
 
 // The layers on packed weights: 5 launches each.  h travels un-normalised
@@ -526,7 +527,9 @@ void callList(HomBertEncoder *e, int fromIds) {
 // gemmMode / geluForm as documented on HomBertEncoder.  roleLayout: weight
 // layout per GEMM role (QKV, out-proj, FFN1, FFN2, LM transform, LM decoder):
 // 0 [K, N] + cutlassGemmF16, 1 [N, K] + nvteGemmF16, -1 (or a null pointer) the
-// driver decides, see chooseGemm.
+// driver decides, see chooseGemm.  Null when the layout is refused or something
+// cannot be allocated (the message is on stderr).
+DRV_EXPORT void homBertDestroy(HomBertEncoder *e);
 DRV_EXPORT HomBertEncoder *
 homBertCreateWithLayout(int layers, int hidden, int heads, int ffn, int batch,
                         int seq, int vocab, int gemmMode, int geluForm,
@@ -589,11 +592,21 @@ homBertCreateWithLayout(int layers, int hidden, int heads, int ffn, int batch,
   e->qkv.m = alloc3DMemRefNVGPUF16(batch, seq, 3 * hidden);
   e->attn.m = alloc3DMemRefNVGPUF16(batch, seq, hidden);
   e->f.m = alloc3DMemRefNVGPUF16(batch, seq, ffn);
-  if (!hipOk(hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking),
-             "hipStreamCreate") ||
-      !hipOk(hipEventCreate(&e->evStart), "hipEventCreate") ||
-      !hipOk(hipEventCreate(&e->evStop), "hipEventCreate"))
-    return e;
+  bool ok = true;
+  for (const auto &w : e->w)
+    for (const Tensor *t : {&w.wqkv, &w.wo, &w.w1, &w.w2})
+      ok = ok && t->m.descriptor;
+  for (const Tensor *t : {&e->wordEmb, &e->posType, &e->ids, &e->mask, &e->cu, &e->h, &e->qkv,
+                          &e->attn, &e->f})
+    ok = ok && t->m.descriptor;
+  ok = ok && (!e->packed || allocPacked(e)) &&
+       hipOk(hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking), "hipStreamCreate") &&
+       hipOk(hipEventCreate(&e->evStart), "hipEventCreate") &&
+       hipOk(hipEventCreate(&e->evStop), "hipEventCreate");
+  if (!ok) {
+    homBertDestroy(e);
+    return nullptr;
+  }
   return e;
 }
 
@@ -801,8 +814,8 @@ DRV_EXPORT void homBertForward(HomBertEncoder *e, int fromIds) {
   void *prev = homGetStream();
   homSetStream(e->stream);
   e->inFlight = true;
-  if (packWeights(e))
-    callList(e, fromIds);
+  packWeights(e);
+  callList(e, fromIds);
   homSetStream(prev);
 }
 
@@ -838,8 +851,9 @@ DRV_EXPORT int homBertCapture(HomBertEncoder *e, int fromIds) {
 }
 
 DRV_EXPORT int homBertReplay(HomBertEncoder *e) {
-  if (!e->graphExec || !packWeights(e)) // (weights uploaded since the capture)
+  if (!e->graphExec)
     return -1;
+  packWeights(e); // (weights uploaded since the capture)
   e->inFlight = true;
   return hipOk(hipGraphLaunch(e->graphExec, e->stream), "hipGraphLaunch") ? 0
                                                                           : -1;

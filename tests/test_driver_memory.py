@@ -1,0 +1,79 @@
+"""The BERT driver's allocations, on host memory: the driver and the library run on a HIP runtime without kernels
+(modules/host_hip.cpp) that counts allocations and refuses the one it is told to."""
+import json
+import os
+import subprocess
+import sys
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+PRELUDE = r"""
+import ctypes, importlib, json, sys
+import numpy as np
+sys.path.insert(0, {root!r})
+hip = ctypes.CDLL({shim!r}, mode=ctypes.RTLD_GLOBAL)   # in front of the real runtime
+hip.hostHipLiveBytes.restype = ctypes.c_size_t
+hip.hostHipFailAt.argtypes = [ctypes.c_long]
+hip.hostHipAllocations.restype = hip.hostHipLaunches.restype = ctypes.c_long
+rt = importlib.import_module("hands-on-mlir_amd.hom_runtime")
+drv, lib = rt.load_driver(), rt.load_runtime()
+L, H, HEADS, F, B, S, V = 3, 128, 2, 256, 2, 33, 50
+def create():
+    return drv.homBertCreate(L, H, HEADS, F, B, S, V, 1, 0)
+def upload(e):
+    for l in range(L):
+        for which, n in enumerate((3 * H * H, H * H, H * F, H * F)):
+            assert drv.homBertUpload(e, l, which, np.zeros(n, np.float16).ctypes.data, n) == 0
+    for which, n in ((4, V * H), (5, S * H)):
+        assert drv.homBertUpload(e, 0, which, np.zeros(n, np.float16).ctypes.data, n) == 0
+"""
+
+
+@pytest.fixture(scope="module")
+def on_host(tmp_path_factory):
+    shim = str(tmp_path_factory.mktemp("hip") / "libhost_hip.so")
+    res = subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                          os.path.join(ROOT, "tests", "modules", "host_hip.cpp"), "-o", shim],
+                         capture_output=True, text=True, timeout=300)
+    assert res.returncode == 0, res.stderr
+
+    def run(code):
+        p = subprocess.run([sys.executable, "-c", PRELUDE.format(root=ROOT, shim=shim) + code], capture_output=True,
+                           text=True, timeout=300)
+        assert p.returncode == 0, p.stderr
+        return json.loads(p.stdout.strip().splitlines()[-1])
+    return run
+
+
+def test_failed_allocation_is_reported_at_creation(on_host):
+    """Whichever allocation fails, the encoder is not handed out and nothing is left behind; an encoder that was
+    handed out allocates nothing in its forwards."""
+    out = on_host(r"""
+lib.homSetErrorMode(1)
+hip.hostHipFailAt(-1)
+e = create()
+n = hip.hostHipAllocations()
+upload(e)
+hip.hostHipFailAt(-1)
+drv.homBertForward(e, 1)
+later, launches = hip.hostHipAllocations(), hip.hostHipLaunches()
+packed = drv.homBertUsesPacked(e)
+drv.homBertDestroy(e)
+left = hip.hostHipLiveBytes()
+refused, leaks = [], []
+for k in range(n):
+    hip.hostHipFailAt(k)
+    e = create()
+    refused.append(not e)
+    if e:
+        drv.homBertDestroy(e)
+    leaks.append(hip.hostHipLiveBytes())
+print(json.dumps(dict(n=n, later=later, launches=launches, packed=packed, left=left, refused=refused, leaks=leaks)))
+""")
+    assert out["packed"] == 1 and out["launches"] >= 5 * 3 and out["n"] > 20
+    assert out["later"] == 0, "a forward allocates"
+    assert out["left"] == 0 and not any(out["leaks"]), "memory left behind"
+    # (one allocation is the first buffer of the pool of results, without which results take pageable memory)
+    assert out["refused"].count(False) == 1
