@@ -41,10 +41,12 @@ namespace {
 
 struct Tensor {
   C_UnrankedMemRefType m{0, nullptr};
+  bool view = false; // the data is another tensor's
   void *data() const { return m.descriptor ? hom_memref_data(m.descriptor) : nullptr; }
   void release() {
     if (m.descriptor) {
-      deallocNVGPUF16(m.rank, m.descriptor);
+      if (!view)
+        deallocNVGPUF16(m.rank, m.descriptor);
       free(m.descriptor);
       m.descriptor = nullptr;
     }
@@ -52,7 +54,9 @@ struct Tensor {
 };
 
 struct LayerWeights {
-  Tensor wqkv, wo, w1, w2; // [1,K,N] (manifest path) or [1,N,K] (nvte path)
+  // [1,K,N] (manifest path) or [1,N,K] (nvte path); [1,K,N] with the data in
+  // fragment order while the encoder runs on packed weights
+  Tensor wqkv, wo, w1, w2;
 };
 
 // How one GEMM role of the graph is called.  nk: the weight is stored as
@@ -97,15 +101,17 @@ struct HomBertEncoder {
   int32_t foldPieces = 0;
   // usesPacked: every layer GEMM runs on weights in fragment order; up to a few
   // thousand rows (foldsPacked) with the layer norms folded into the GEMMs around
-  // them.  One arena holds
-  // the packed weights in the order the forward reads them, one the column
-  // sums of Wqkv and W1; both are made from the uploaded weights before the
-  // next forward or capture (packWeights).
-  bool packed = false, packedReady = false;
-  char *packedArena = nullptr;
+  // them.  The layers' weights lie in packedArena in the order a forward reads them.
+  // An upload passes through `staging` (the largest weight, row-major) into
+  // the layer's weight and, of Wqkv and W1, into packedColSums; qkv, attn and f are
+  // in fragment order as well, and so is hPacked, what h is between the layers.
+  // A call that pins the row-major list lays all of that out anew (leavePacked);
+  // graphs captured before it still hold the arena and what is in `retired`.
+  bool packed = false;
+  Tensor packedArena, staging, hPacked;
   float *packedColSums = nullptr;
   float *packedStats[2] = {nullptr, nullptr}; // rows of h entering QKV / FFN1
-  Tensor hPacked, qkvPacked, attnPacked, fPacked; // activations in fragment order
+  std::vector<Tensor> retired;
   hipStream_t stream = nullptr;
   hipGraph_t graph = nullptr;
   hipGraphExec_t graphExec = nullptr;
@@ -337,109 +343,158 @@ bool foldsPacked(const HomBertEncoder *e) {
   return int64_t(e->batch) * e->seq * e->hidden <= 5500000;
 }
 
-struct PackedLayer { // byte offsets into the arena
-  int64_t qkv, out, ffn1, ffn2, end;
-};
-PackedLayer packedLayer(const HomBertEncoder *e, int l) {
-  const int64_t H = e->hidden, F = e->ffn;
-  PackedLayer p;
-  p.qkv = int64_t(l) * (4 * H * H + 2 * H * F) * 2;
-  p.out = p.qkv + 3 * H * H * 2;
-  p.ffn1 = p.out + H * H * 2;
-  p.ffn2 = p.ffn1 + H * F * 2;
-  p.end = p.ffn2 + H * F * 2;
-  return p;
-}
 float *packedColSum(const HomBertEncoder *e, int l, bool ffn1) {
   return e->packedColSums + int64_t(l) * (3 * e->hidden + e->ffn) +
          (ffn1 ? 3 * e->hidden : 0);
 }
 
-// What the packed list needs besides the row-major buffers.  All of it at
-// creation: a forward allocates nothing and cannot fail for want of memory.
-bool allocPacked(HomBertEncoder *e) {
-  const int64_t H = e->hidden, F = e->ffn;
-  const int rows = (e->batch * e->seq + 15) / 16 * 16;
-  auto alloc = [](auto *&p, size_t bytes) {
-    return hipOk(hipMalloc(reinterpret_cast<void **>(&p), bytes), "hipMalloc of packed weights");
-  };
-  if (!alloc(e->packedArena, size_t(packedLayer(e, e->layers).qkv)) ||
-      !alloc(e->packedColSums, size_t(e->layers) * size_t(3 * H + F) * 4) ||
-      !alloc(e->packedStats[0], size_t(rows) * 8) || !alloc(e->packedStats[1], size_t(rows) * 8))
-    return false;
-  // (the logical shape is [batch, seq, .]: the padding rows lie behind it)
-  auto padded = [&](Tensor &t, int64_t cols) {
-    t.m = alloc3DMemRefNVGPUF16(1, rows, int32_t(cols));
-    if (!t.m.descriptor)
-      return false;
+// [batch, seq, cols], with the rows that whole row blocks need behind it
+Tensor allocPadded(const HomBertEncoder *e, int cols) {
+  Tensor t;
+  t.m = alloc3DMemRefNVGPUF16(1, (e->batch * e->seq + 15) / 16 * 16, cols);
+  if (t.m.descriptor) {
     int64_t *sz = hom_memref_sizes(t.m.descriptor);
     int64_t *st = hom_memref_strides(t.m.descriptor, 3);
     sz[0] = e->batch;
     sz[1] = e->seq;
     st[0] = int64_t(e->seq) * cols;
-    return true;
+  }
+  return t;
+}
+// All of it at creation: a forward allocates nothing and cannot fail for want
+// of memory.
+bool allocPacked(HomBertEncoder *e) {
+  const int H = e->hidden, F = e->ffn;
+  auto alloc = [](float *&p, size_t floats) {
+    return hipOk(hipMalloc(reinterpret_cast<void **>(&p), floats * 4), "hipMalloc for packed weights");
   };
-  return padded(e->hPacked, H) && padded(e->qkvPacked, 3 * H) && padded(e->attnPacked, H) &&
-         padded(e->fPacked, F);
+  const size_t rows = (size_t(e->batch) * e->seq + 15) / 16 * 16;
+  e->packedArena.m = alloc3DMemRefNVGPUF16(e->layers, H, 4 * H + 2 * F);
+  if (!e->packedArena.m.descriptor)
+    return false;
+  _Float16 *at = static_cast<_Float16 *>(e->packedArena.data());
+  auto weight = [&](Tensor &t, int K, int N) {
+    auto *d = static_cast<HomStridedMemRef3 *>(malloc(sizeof(HomStridedMemRef3)));
+    *d = HomStridedMemRef3{};
+    d->basePtr = d->data = at;
+    d->sizes[0] = 1;
+    d->sizes[1] = K;
+    d->sizes[2] = N;
+    d->strides[0] = int64_t(K) * N;
+    d->strides[1] = N;
+    d->strides[2] = 1;
+    t.m = C_UnrankedMemRefType{3, d};
+    t.view = true;
+    at += d->strides[0];
+  };
+  for (LayerWeights &w : e->w) {
+    weight(w.wqkv, H, 3 * H);
+    weight(w.wo, H, H);
+    weight(w.w1, H, F);
+    weight(w.w2, F, H);
+  }
+  e->staging.m = alloc3DMemRefNVGPUF16(1, H, std::max(3 * H, F));
+  e->hPacked = allocPadded(e, H);
+  return e->staging.m.descriptor && e->hPacked.m.descriptor &&
+         alloc(e->packedColSums, size_t(e->layers) * size_t(3 * H + F)) &&
+         alloc(e->packedStats[0], rows * 2) && alloc(e->packedStats[1], rows * 2);
 }
 
-void packWeights(HomBertEncoder *e) {
-  if (!e->packed || e->packedReady)
-    return;
+// The row-major values in e->staging become weight `which` (0 Wqkv, 1 Wo, 2 W1,
+// 3 W2) of a layer.  Queued behind what runs on the stream and waited for: the
+// staging buffer is free again.
+bool packUploaded(HomBertEncoder *e, int layer, int which, const Tensor &w) {
+  HomStridedMemRef3 from = *static_cast<const HomStridedMemRef3 *>(w.m.descriptor);
+  from.basePtr = from.data = e->staging.data();
   void *prev = homGetStream();
   homSetStream(e->stream);
-  for (int l = 0; l < e->layers; l++) {
-    const LayerWeights &w = e->w[size_t(l)];
-    const PackedLayer at = packedLayer(e, l);
-    homPackWeightF16(w.wqkv.m.rank, w.wqkv.m.descriptor, e->packedArena + at.qkv);
-    homPackWeightF16(w.wo.m.rank, w.wo.m.descriptor, e->packedArena + at.out);
-    homPackWeightF16(w.w1.m.rank, w.w1.m.descriptor, e->packedArena + at.ffn1);
-    homPackWeightF16(w.w2.m.rank, w.w2.m.descriptor, e->packedArena + at.ffn2);
-    homColumnSumsF16(w.wqkv.m.rank, w.wqkv.m.descriptor, packedColSum(e, l, false));
-    homColumnSumsF16(w.w1.m.rank, w.w1.m.descriptor, packedColSum(e, l, true));
-  }
+  homPackWeightF16(3, &from, w.data());
+  if (which == 0 || which == 2)
+    homColumnSumsF16(3, &from, packedColSum(e, layer, which == 2));
   homSetStream(prev);
-  e->packedReady = true;
+  return hipOk(hipStreamSynchronize(e->stream), "hipStreamSynchronize");
+}
+
+// From packed weights to the row-major list: the weights' values unpacked into
+// tensors of their own, and row-major activations.  False, with nothing changed,
+// if there is no memory for them.
+bool leavePacked(HomBertEncoder *e) {
+  if (!e->packed)
+    return true;
+  std::vector<Tensor *> old;
+  for (auto &w : e->w)
+    for (Tensor *t : {&w.wqkv, &w.wo, &w.w1, &w.w2})
+      old.push_back(t);
+  const size_t weights = old.size();
+  for (Tensor *t : {&e->qkv, &e->attn, &e->f})
+    old.push_back(t);
+  std::vector<Tensor> fresh(old.size());
+  for (size_t i = 0; i < old.size(); i++) {
+    const int64_t *sz = hom_memref_sizes(old[i]->m.descriptor);
+    fresh[i].m = alloc3DMemRefNVGPUF16(int32_t(sz[0]), int32_t(sz[1]), int32_t(sz[2]));
+    if (!fresh[i].m.descriptor) {
+      for (Tensor &t : fresh)
+        t.release();
+      return false;
+    }
+  }
+  void *prev = homGetStream();
+  homSetStream(e->stream);
+  for (size_t i = 0; i < weights; i++)
+    homUnpackWeightF16(old[i]->data(), fresh[i].m.rank, fresh[i].m.descriptor);
+  homSetStream(prev);
+  (void)hipOk(hipStreamSynchronize(e->stream), "hipStreamSynchronize");
+  for (size_t i = 0; i < old.size(); i++) {
+    if (!old[i]->view)
+      e->retired.push_back(*old[i]);
+    else
+      old[i]->release();
+    *old[i] = fresh[i];
+  }
+  e->packed = false;
+  return true;
 }
 
 // The layers on packed weights: 5 launches each.  h travels un-normalised
 // between the GEMMs that add to it (out-projection, FFN2); QKV and FFN1
 // normalise it on the way in and leave its row statistics for the residual of
 // the GEMM after next.
+// Every launch is told which weight comes after the next one (`ahead`).
 void packedLayers(HomBertEncoder *e, int64_t geluAct, float scale) {
   const int kAll = HOM_PACKED_A | HOM_PACKED_C | HOM_PACKED_D;
-  auto gemm = [&](const Tensor &a, int64_t weight, const Tensor *c, const Tensor &d, int64_t act,
-                  bool norm, const float *colSum, const float *statsIn, float *statsOut,
-                  int packing, int64_t ahead, int64_t aheadEnd) {
-    homPackedGemmF16(a.m.rank, a.m.descriptor, e->packedArena + weight, c ? c->m.rank : 0,
+  auto bytes = [](const Tensor *t) -> int64_t {
+    const int64_t *sz = t ? hom_memref_sizes(t->m.descriptor) : nullptr;
+    return sz ? sz[1] * sz[2] * 2 : 0;
+  };
+  auto gemm = [&](const Tensor &a, const Tensor &weight, const Tensor *c, const Tensor &d,
+                  int64_t act, bool norm, const float *colSum, const float *statsIn,
+                  float *statsOut, int packing, const Tensor *ahead) {
+    homPackedGemmF16(a.m.rank, a.m.descriptor, weight.data(), c ? c->m.rank : 0,
                      c ? c->m.descriptor : nullptr, d.m.rank, d.m.descriptor, act, norm, e->eps,
-                     colSum, statsIn, statsOut, packing,
-                     e->packedArena + ahead, aheadEnd - ahead);
+                     colSum, statsIn, statsOut, packing, ahead ? ahead->data() : nullptr,
+                     bytes(ahead));
   };
   const bool fold = foldsPacked(e);
   for (int l = 0; l < e->layers; l++) {
-    const PackedLayer at = packedLayer(e, l);
+    const LayerWeights &w = e->w[size_t(l)];
     const bool last = l + 1 == e->layers;
-    const int64_t nextQkv = last ? at.end : at.end + (at.out - at.qkv);
+    const Tensor *nextQkv = last ? nullptr : &e->w[size_t(l) + 1].wqkv;
     // (the embeddings arrive normalised)
     const bool norm = fold && l > 0;
-    gemm(e->hPacked, at.qkv, nullptr, e->qkvPacked, 0, norm,
-         norm ? packedColSum(e, l, false) : nullptr, nullptr, norm ? e->packedStats[0] : nullptr,
-         HOM_PACKED_A | HOM_PACKED_D, at.out, at.ffn1);
-    homBertAttentionF16(e->qkvPacked.m.rank, e->qkvPacked.m.descriptor, e->cu.m.rank,
-                        e->cu.m.descriptor, e->attnPacked.m.rank, e->attnPacked.m.descriptor,
-                        scale, e->heads, HOM_PACKED_A | HOM_PACKED_D,
-                        e->packedArena + at.ffn1, at.ffn2 - at.ffn1);
-    gemm(e->attnPacked, at.out, &e->hPacked, e->hPacked, 0, false, nullptr,
-         norm ? e->packedStats[0] : nullptr, nullptr, kAll, at.ffn2, at.end);
+    gemm(e->hPacked, w.wqkv, nullptr, e->qkv, 0, norm, norm ? packedColSum(e, l, false) : nullptr,
+         nullptr, norm ? e->packedStats[0] : nullptr, HOM_PACKED_A | HOM_PACKED_D, &w.wo);
+    homBertAttentionF16(e->qkv.m.rank, e->qkv.m.descriptor, e->cu.m.rank, e->cu.m.descriptor,
+                        e->attn.m.rank, e->attn.m.descriptor, scale, e->heads,
+                        HOM_PACKED_A | HOM_PACKED_D, w.w1.data(), bytes(&w.w1));
+    gemm(e->attn, w.wo, &e->hPacked, e->hPacked, 0, false, nullptr,
+         norm ? e->packedStats[0] : nullptr, nullptr, kAll, &w.w2);
     if (!fold)
       homPackedLayernormF16(e->hPacked.m.rank, e->hPacked.m.descriptor, e->hPacked.m.rank,
                             e->hPacked.m.descriptor, e->eps, HOM_PACKED_A | HOM_PACKED_D);
-    gemm(e->hPacked, at.ffn1, nullptr, e->fPacked, geluAct, fold,
-         fold ? packedColSum(e, l, true) : nullptr, nullptr, fold ? e->packedStats[1] : nullptr,
-         HOM_PACKED_A | HOM_PACKED_D, at.end, nextQkv);
-    gemm(e->fPacked, at.ffn2, &e->hPacked, e->hPacked, 0, false, nullptr,
-         fold ? e->packedStats[1] : nullptr, nullptr, kAll, at.end, nextQkv);
+    gemm(e->hPacked, w.w1, nullptr, e->f, geluAct, fold, fold ? packedColSum(e, l, true) : nullptr,
+         nullptr, fold ? e->packedStats[1] : nullptr, HOM_PACKED_A | HOM_PACKED_D, nextQkv);
+    gemm(e->f, w.w2, &e->hPacked, e->hPacked, 0, false, nullptr,
+         fold ? e->packedStats[1] : nullptr, nullptr, kAll, nextQkv);
     if (!fold || last) {
       const Tensor &out = last ? e->h : e->hPacked;
       homPackedLayernormF16(e->hPacked.m.rank, e->hPacked.m.descriptor, out.m.rank,
@@ -450,8 +505,7 @@ void packedLayers(HomBertEncoder *e, int64_t geluAct, float scale) {
 }
 
 void callList(HomBertEncoder *e, int fromIds) {
-  // (a forward from given hidden states has them row-major in h)
-  const bool packed = e->packed && fromIds;
+  const bool packed = e->packed;
   const Tensor &front = packed ? e->hPacked : e->h;
   if (fromIds)
     homEmbedF16(e->ids.m.rank, e->ids.m.descriptor, e->mask.m.rank,
@@ -465,6 +519,8 @@ void callList(HomBertEncoder *e, int fromIds) {
   const float scale = 1.0f / sqrtf(float(e->hidden / e->heads));
   const int64_t geluAct = e->gemmMode == 0 ? 1 : (e->geluForm == 1 ? 2 : 1);
   if (packed) {
+    if (!fromIds) // (given hidden states are row-major in h)
+      homPackRowsF16(e->h.m.rank, e->h.m.descriptor, e->hPacked.m.rank, e->hPacked.m.descriptor);
     packedLayers(e, geluAct, scale);
   } else if (e->foldLn) {
     // The same graph with the two layer norms of every layer folded into the
@@ -555,7 +611,7 @@ homBertCreateWithLayout(int layers, int hidden, int heads, int ffn, int batch,
     // a bad pin fails at creation, not at homBertEnableLmHead
     const bool transformOk =
         !(e->roleLayout[4] == 1 && geluForm == 0 && gemmMode != 0);
-    // Row-major weights for the packed form to start from.
+    // (packed weights are made from row-major ones)
     e->packed = usesPacked(e);
     for (int r = 0; r < 4 && e->packed; r++)
       e->roleLayout[r] = 0;
@@ -572,6 +628,8 @@ homBertCreateWithLayout(int layers, int hidden, int heads, int ffn, int batch,
     }
   }
   for (auto &w : e->w) {
+    if (e->packed)
+      break; // (views, see allocPacked)
     w.wqkv.m = e->cQkv.nk ? alloc3DMemRefNVGPUF16(1, 3 * hidden, hidden)
                           : alloc3DMemRefNVGPUF16(1, hidden, 3 * hidden);
     w.wo.m = alloc3DMemRefNVGPUF16(1, hidden, hidden);
@@ -589,17 +647,23 @@ homBertCreateWithLayout(int layers, int hidden, int heads, int ffn, int batch,
   pinnedPool().release(pinnedPool().acquire(size_t(batch) * seq * hidden * 2));
   e->cu.m = alloc1DMemRefNVGPUI32(batch + 1);
   e->h.m = alloc3DMemRefNVGPUF16(batch, seq, hidden);
-  e->qkv.m = alloc3DMemRefNVGPUF16(batch, seq, 3 * hidden);
-  e->attn.m = alloc3DMemRefNVGPUF16(batch, seq, hidden);
-  e->f.m = alloc3DMemRefNVGPUF16(batch, seq, ffn);
-  bool ok = true;
+  auto activation = [&](Tensor &t, int cols) {
+    if (e->packed)
+      t = allocPadded(e, cols);
+    else
+      t.m = alloc3DMemRefNVGPUF16(batch, seq, cols);
+  };
+  activation(e->qkv, 3 * hidden);
+  activation(e->attn, hidden);
+  activation(e->f, ffn);
+  bool ok = !e->packed || allocPacked(e);
   for (const auto &w : e->w)
     for (const Tensor *t : {&w.wqkv, &w.wo, &w.w1, &w.w2})
       ok = ok && t->m.descriptor;
   for (const Tensor *t : {&e->wordEmb, &e->posType, &e->ids, &e->mask, &e->cu, &e->h, &e->qkv,
                           &e->attn, &e->f})
     ok = ok && t->m.descriptor;
-  ok = ok && (!e->packed || allocPacked(e)) &&
+  ok = ok &&
        hipOk(hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking), "hipStreamCreate") &&
        hipOk(hipEventCreate(&e->evStart), "hipEventCreate") &&
        hipOk(hipEventCreate(&e->evStop), "hipEventCreate");
@@ -676,6 +740,8 @@ DRV_EXPORT int homBertFoldLayernorm(HomBertEncoder *e) {
   const int32_t pFfn2 = homFoldedLayernormPieces(M, e->hidden, e->ffn, 0, 0);
   if (pOut != pFfn2 || pOut < 1)
     return -1; // (both depend on M and N only)
+  if (!leavePacked(e))
+    return -1;
   bool ok = true;
   for (float *&q : e->rowSums)
     ok = ok && hipOk(hipMalloc(reinterpret_cast<void **>(&q),
@@ -702,7 +768,6 @@ DRV_EXPORT int homBertFoldLayernorm(HomBertEncoder *e) {
   if (!ok)
     return -1;
   e->foldPieces = pOut;
-  e->packed = false;
   e->foldLn = true;
   return 0;
 }
@@ -739,11 +804,11 @@ DRV_EXPORT void homBertDestroy(HomBertEncoder *e) {
   for (Tensor *t : {&e->wordEmb, &e->posType, &e->cu, &e->h, &e->qkv, &e->attn,
                     &e->f, &e->wTransform, &e->wDecoder, &e->t, &e->logits})
     t->release();
+  for (Tensor &t : e->retired)
+    t.release();
+  e->packedArena.release();
   e->hPacked.release();
-  e->qkvPacked.release();
-  e->attnPacked.release();
-  e->fPacked.release();
-  (void)hipFree(e->packedArena);
+  e->staging.release();
   (void)hipFree(e->packedColSums);
   for (float *q : e->packedStats)
     (void)hipFree(q);
@@ -760,7 +825,6 @@ DRV_EXPORT void homBertDestroy(HomBertEncoder *e) {
 DRV_EXPORT int homBertUpload(HomBertEncoder *e, int layer, int which,
                              const void *host, int64_t numel) {
   Tensor *t = nullptr;
-  e->packedReady = false;
   if (which <= 3) {
     if (layer < 0 || layer >= e->layers)
       return -1;
@@ -781,9 +845,11 @@ DRV_EXPORT int homBertUpload(HomBertEncoder *e, int layer, int which,
                     "%lld\n", (long long)numel, (long long)expect);
     return -2;
   }
-  return hipOk(hipMemcpy(t->data(), host, size_t(numel) * 2,
+  const bool pack = which <= 3 && e->packed;
+  return hipOk(hipMemcpy(pack ? e->staging.data() : t->data(), host, size_t(numel) * 2,
                          hipMemcpyHostToDevice),
-               "hipMemcpy")
+               "hipMemcpy") &&
+                 (!pack || packUploaded(e, layer, which, *t))
              ? 0
              : -3;
 }
@@ -814,7 +880,6 @@ DRV_EXPORT void homBertForward(HomBertEncoder *e, int fromIds) {
   void *prev = homGetStream();
   homSetStream(e->stream);
   e->inFlight = true;
-  packWeights(e);
   callList(e, fromIds);
   homSetStream(prev);
 }
@@ -853,7 +918,6 @@ DRV_EXPORT int homBertCapture(HomBertEncoder *e, int fromIds) {
 DRV_EXPORT int homBertReplay(HomBertEncoder *e) {
   if (!e->graphExec)
     return -1;
-  packWeights(e); // (weights uploaded since the capture)
   e->inFlight = true;
   return hipOk(hipGraphLaunch(e->graphExec, e->stream), "hipGraphLaunch") ? 0
                                                                           : -1;
@@ -949,9 +1013,10 @@ DRV_EXPORT int homBertSetGemmChoice(HomBertEncoder *e, int role,
     return -1;
   if (c[role]->nk)
     return -2; // the role's weight is [N, K]: it runs through nvteGemmF16
+  if (!leavePacked(e)) // a pinned kernel is what runs
+    return -3;
   c[role]->gemmNum = gemmNum;
   c[role]->splitK = splitK;
-  e->packed = false; // a pinned kernel is what runs
   return 0;
 }
 

@@ -337,6 +337,39 @@ __global__ __launch_bounds__(256) void packWeightKernel(const _Float16 *__restri
   reinterpret_cast<half8 *>(out)[v] = o;
 }
 
+// The way back: fragments -> B [K, N] row-major.
+__global__ __launch_bounds__(256) void unpackWeightKernel(const _Float16 *__restrict__ packed,
+                                                          _Float16 *__restrict__ B, int K, int N) {
+  const int64_t v = int64_t(blockIdx.x) * 256 + threadIdx.x; // 16-byte vector of the input
+  const int steps = K / 32;
+  if (v >= int64_t(N / 16) * steps * kWave)
+    return;
+  const int l = int(v % kWave);
+  const int64_t block = v / kWave;
+  const int s = int(block % steps), j = int(block / steps);
+  const half8 x = reinterpret_cast<const half8 *>(packed)[v];
+#pragma unroll
+  for (int e = 0; e < 8; e++)
+    B[int64_t(32 * s + 8 * (l / 16) + e) * N + 16 * j + l % 16] = x[e];
+}
+
+// Rows [M, C] row-major -> fragment order, zeros in the rows that fill the last
+// block.  A copy, 16 bytes per thread: whole kilobytes out, 64 bytes of 16 rows in.
+__global__ __launch_bounds__(256) void packRowsKernel(const _Float16 *__restrict__ in,
+                                                      _Float16 *__restrict__ out, int64_t M, int C,
+                                                      int64_t vecs) {
+  const int64_t v = int64_t(blockIdx.x) * 256 + threadIdx.x; // 16-byte vector of the output
+  if (v >= vecs)
+    return;
+  const int l = int(v % kWave), wide = C / 32;
+  const int64_t block = v / kWave, row = block / wide * 16 + l % 16;
+  const int col = int(block % wide) * 32 + l / 16 * 8;
+  half8 x = {};
+  if (row < M)
+    x = *reinterpret_cast<const half8 *>(in + row * C + col);
+  storeWriteThrough(out + v * 8, x);
+}
+
 // What an XCD works on: chunkM x chunkN tiles, 2^xmLog XCDs along M.  Its L2 fetches
 // the operands of the rectangle once, at about 0.7 TB/s per XCD from the last-level
 // cache, which from some 500 rows on is what bounds these kernels (512 x 1024 x
@@ -395,6 +428,23 @@ Status launchPackWeight(const _Float16 *B, _Float16 *packed, int64_t K, int64_t 
   const int64_t vecs = K * N / 8;
   packWeightKernel<<<dim3((unsigned)((vecs + 255) / 256)), dim3(256), 0, s>>>(B, packed, int(K),
                                                                               int(N));
+  HOM_HIP_RET(hipGetLastError(), Status::kInternal);
+  return Status::kSuccess;
+}
+
+Status launchUnpackWeight(const _Float16 *packed, _Float16 *B, int64_t K, int64_t N,
+                          hipStream_t s) {
+  const int64_t vecs = K * N / 8;
+  unpackWeightKernel<<<dim3((unsigned)((vecs + 255) / 256)), dim3(256), 0, s>>>(packed, B, int(K),
+                                                                                int(N));
+  HOM_HIP_RET(hipGetLastError(), Status::kInternal);
+  return Status::kSuccess;
+}
+
+Status launchPackRows(const _Float16 *in, _Float16 *out, int64_t M, int64_t C, hipStream_t s) {
+  const int64_t vecs = (M + 15) / 16 * 16 * C / 8;
+  packRowsKernel<<<dim3((unsigned)((vecs + 255) / 256)), dim3(256), 0, s>>>(in, out, M, int(C),
+                                                                            vecs);
   HOM_HIP_RET(hipGetLastError(), Status::kInternal);
   return Status::kSuccess;
 }

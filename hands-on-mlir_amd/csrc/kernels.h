@@ -203,6 +203,11 @@ Status launchPackedLayernorm(const _Float16 *in, _Float16 *out, int64_t M, int64
 // B [K, N] row-major, dense -> the layout above, K * N values.
 Status launchPackWeight(const _Float16 *B, _Float16 *packed, int64_t K, int64_t N,
                         hipStream_t s);
+// ... and back.
+Status launchUnpackWeight(const _Float16 *packed, _Float16 *B, int64_t K, int64_t N,
+                          hipStream_t s);
+// [M, C] row-major, dense -> fragment order, zeros up to whole row blocks; C % 32 == 0.
+Status launchPackRows(const _Float16 *in, _Float16 *out, int64_t M, int64_t C, hipStream_t s);
 // out[n] = sum over k of B[k, n] (fp32), B row-major [K, N], N % 8 == 0.
 Status launchColumnSums(const _Float16 *B, int64_t ldb, int64_t K, int64_t N,
                         float *out, hipStream_t s);

@@ -234,6 +234,14 @@ void homPackWeightF16(int64_t rankB, void *dstB, void *packed) {
   (void)runPackWeight(rankB, dstB, packed);
 }
 
+void homUnpackWeightF16(const void *packed, int64_t rankB, void *dstB) {
+  (void)runUnpackWeight(packed, rankB, dstB);
+}
+
+void homPackRowsF16(int64_t rankA, void *dstA, int64_t rankOut, void *dstOut) {
+  (void)runPackRows(rankA, dstA, rankOut, dstOut);
+}
+
 void homPackedLayernormF16(int64_t rankA, void *dstA, int64_t rankOut,
                            void *dstOut, float eps, int32_t packing) {
   (void)runPackedLayernorm(rankA, dstA, rankOut, dstOut, eps, packing);

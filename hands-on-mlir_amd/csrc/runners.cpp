@@ -554,20 +554,55 @@ Status runColumnSums(int64_t rankB, void *dstB, float *out) {
                           stream());
 }
 
-Status runPackWeight(int64_t rankB, void *dstB, void *packed) {
-  View<_Float16> B(rankB, dstB);
-  HOM_CHECK_RET(B.sizes && rankB == 3 && B.sizes[0] == 1 && B.contiguous() &&
+// B [1, K, N] as the packed form takes it, and where that lies
+static Status checkPackWeight(const char *what, const View<_Float16> &B, const void *packed) {
+  HOM_CHECK_RET(B.sizes && B.rank == 3 && B.sizes[0] == 1 && B.contiguous() &&
                     B.sizes[1] % 32 == 0 && B.sizes[2] % 16 == 0 &&
                     B.numel() * 2 < (int64_t(1) << 31),
                 Status::kInvalidArgument,
-                "pack weight: B must be a contiguous [1, K, N] tensor below 2 GiB "
-                "with K a multiple of 32 and N of 16");
+                "%s: B must be a contiguous [1, K, N] tensor below 2 GiB "
+                "with K a multiple of 32 and N of 16", what);
   HOM_CHECK_RET(packed && (reinterpret_cast<uintptr_t>(packed) & 15) == 0,
-                Status::kInvalidArgument, "pack weight: misaligned destination");
-  if (B.numel() == 0)
-    return Status::kSuccess;
+                Status::kInvalidArgument, "%s: misaligned packed weight", what);
+  return Status::kSuccess;
+}
+
+Status runPackWeight(int64_t rankB, void *dstB, void *packed) {
+  View<_Float16> B(rankB, dstB);
+  const Status st = checkPackWeight("pack weight", B, packed);
+  if (st != Status::kSuccess || B.numel() == 0)
+    return st;
   return launchPackWeight(B.data, static_cast<_Float16 *>(packed), B.sizes[1],
                           B.sizes[2], stream());
+}
+
+Status runUnpackWeight(const void *packed, int64_t rankB, void *dstB) {
+  View<_Float16> B(rankB, dstB);
+  const Status st = checkPackWeight("unpack weight", B, packed);
+  if (st != Status::kSuccess || B.numel() == 0)
+    return st;
+  return launchUnpackWeight(static_cast<const _Float16 *>(packed), B.data, B.sizes[1],
+                            B.sizes[2], stream());
+}
+
+Status runPackRows(int64_t rankA, void *dstA, int64_t rankOut, void *dstOut) {
+  View<_Float16> A(rankA, dstA), O(rankOut, dstOut);
+  HOM_CHECK_RET(A.rank == 3 && O.rank == 3 && A.sizes && O.sizes &&
+                    A.contiguous() && O.contiguous() &&
+                    A.sizes[0] == O.sizes[0] && A.sizes[1] == O.sizes[1] &&
+                    A.sizes[2] == O.sizes[2] && A.sizes[2] % 32 == 0 &&
+                    A.data != O.data,
+                Status::kInvalidArgument,
+                "pack rows: A and Out must be two contiguous tensors of one "
+                "[b, s, H] shape with H a multiple of 32");
+  const int64_t M = A.sizes[0] * A.sizes[1], C = A.sizes[2];
+  HOM_CHECK_RET(M < (int64_t(1) << 31) && (M + 15) / 16 * 16 * C < (int64_t(1) << 37),
+                Status::kInvalidArgument, "pack rows: tensor too large");
+  HOM_CHECK_RET(((reinterpret_cast<uintptr_t>(A.data) | reinterpret_cast<uintptr_t>(O.data)) & 15) == 0,
+                Status::kInvalidArgument, "pack rows: misaligned operands");
+  if (M == 0 || C == 0)
+    return Status::kSuccess;
+  return launchPackRows(A.data, O.data, M, C, stream());
 }
 
 Status runPackedLayernorm(int64_t rankA, void *dstA, int64_t rankOut, void *dstOut,

@@ -46,6 +46,8 @@ Status runGemmFoldedLayernorm(int64_t rankA, void *dstA, int64_t rankB,
 int32_t foldedLayernormPieces(int64_t M, int64_t N, int64_t K, int64_t activation,
                               int32_t likeGemmNum);
 Status runPackWeight(int64_t rankB, void *dstB, void *packed);
+Status runUnpackWeight(const void *packed, int64_t rankB, void *dstB);
+Status runPackRows(int64_t rankA, void *dstA, int64_t rankOut, void *dstOut);
 Status runPackedLayernorm(int64_t rankA, void *dstA, int64_t rankOut, void *dstOut,
                           float eps, int32_t packing);
 Status runPackedGemm(int64_t rankA, void *dstA, const void *packedB, int64_t rankC,

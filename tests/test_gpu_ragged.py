@@ -352,3 +352,104 @@ def test_attention_splits(gpu, rt, bs, seq, heads, d):
     gpu.nvteBertAttentionF16(*Mr.from_tensor(qkv.view(bs, seq, -1)).args(), *Mr.from_tensor(cu).args(),
                              *Mr.from_tensor(out).args(), d ** -0.5, heads)
     torch.testing.assert_close(out.float(), want, rtol=2e-3, atol=2e-3)
+
+
+@pytest.mark.parametrize("K,N", [(32, 16), (96, 48), (768, 2304), (1056, 320)])
+def test_pack_weight_and_back(gpu, rt, K, N):
+    B = np.random.default_rng(K + N).standard_normal((1, K, N)).astype(np.float16)
+    Mr, tb = rt.MemRef, dev(B)
+    packed, back = (torch.zeros(K * N, dtype=torch.float16, device="cuda") for _ in range(2))
+    gpu.homPackWeightF16(*Mr.from_tensor(tb).args(), packed.data_ptr())
+    gpu.homUnpackWeightF16(packed.data_ptr(), *Mr(back.data_ptr(), [1, K, N]).args())
+    np.testing.assert_array_equal(host(back).reshape(1, K, N), B)
+
+
+@pytest.mark.parametrize("b,s,H", [(1, 1, 32), (1, 16, 64), (3, 11, 96), (5, 33, 768), (2, 100, 2048)])
+def test_pack_rows(gpu, rt, b, s, H):
+    a = np.random.default_rng(s + H).standard_normal((b, s, H)).astype(np.float16)
+    Mr, R = rt.MemRef, -(-b * s // 16) * 16
+    ta, out = dev(a), torch.full((R * H + 8,), 7.0, dtype=torch.float16, device="cuda")
+    gpu.homPackRowsF16(*Mr.from_tensor(ta).args(), *Mr(out.data_ptr(), [b, s, H]).args())
+    np.testing.assert_array_equal(host(out)[:R * H], fragment_order(a.reshape(b * s, H)))
+    assert (host(out)[R * H:] == 7).all()
+
+
+# few rows, the tile kernels with folded layer norms, and layer norms of their own
+@pytest.mark.parametrize("bs,seq", [(1, 16), (3, 33), (8, 128), (340, 127)])
+def test_encoder_from_hidden_states_equals_from_ids(gpu, rt, synth, bs, seq):
+    """Hidden states given to the encoder take the same kernels as those its embedding front makes: the same bits."""
+    import importlib
+    bert = importlib.import_module("hands-on-mlir_amd.bert")
+    m = synth.bert_encoder(layers=2, hidden=128, heads=2, ffn=512, bs=bs, seq=seq, vocab=100, config=43)
+    enc = bert.BertEncoder(2, 128, 2, 512, bs, seq, 100, gemm_mode=1, gelu_form="erf")
+    try:
+        enc.load(m)
+        assert enc.uses_packed()
+        Mr = rt.MemRef.from_tensor
+        ids, mask, word, pos = dev(m["ids"].astype(np.int64)), dev(m["mask"].astype(np.int64)), dev(m["word"][None]), dev(m["pos_type"][None])
+        h, cu = torch.zeros(bs, seq, 128, dtype=torch.float16, device="cuda"), torch.zeros(bs + 1, dtype=torch.int32, device="cuda")
+        gpu.homEmbedF16(*Mr(ids).args(), *Mr(mask).args(), *Mr(word).args(), *Mr(pos).args(), *Mr(h).args(),
+                        *Mr(cu).args(), 1e-12, 0)
+        hidden = host(h)
+        enc.set_inputs(ids=m["ids"], mask=m["mask"])
+        enc.forward()
+        want = enc.output()
+        enc.set_inputs(hidden=hidden)
+        enc.forward(from_ids=False)
+        np.testing.assert_array_equal(enc.output(), want)
+        enc.set_inputs(hidden=hidden)
+        enc.capture(from_ids=False)
+        for _ in range(3):
+            enc.set_inputs(hidden=hidden)
+            enc.replay()
+            np.testing.assert_array_equal(enc.output(), want)
+            enc.forward()
+            np.testing.assert_array_equal(enc.output(), want)
+    finally:
+        enc.close()
+
+
+@pytest.mark.parametrize("pin", [False, True])
+def test_weights_uploaded_again(gpu, rt, synth, pin):
+    """Weights uploaded between a capture and its replays take effect, on packed weights and after a pinned kernel
+    has taken the encoder off them; a graph captured on packed weights still runs then."""
+    import importlib
+    bert = importlib.import_module("hands-on-mlir_amd.bert")
+    a, b = (synth.bert_encoder(layers=2, hidden=128, heads=2, ffn=512, bs=3, seq=33, vocab=100, config=c) for c in (50, 51))
+    number = {n: i + 1 for i, n, _, _ in rt.manifest()}
+    tile = "hom_gfx950_mfma_f16_s32x32x16gemm_f16_128x64_64x2r2_w2x2_nn_align8_linear"
+
+    def make(m):
+        enc = bert.BertEncoder(2, 128, 2, 512, 3, 33, 100, gemm_mode=1, gelu_form="erf")
+        enc.load(m)
+        enc.set_inputs(ids=a["ids"], mask=a["mask"])
+        return enc
+
+    def result(enc):
+        enc.replay()
+        return enc.output()
+
+    want = []
+    for m in (a, b):  # encoders that never saw other weights
+        enc = make(m)
+        if pin:
+            enc.set_gemm_choice("out", number[tile])
+        enc.capture()
+        want.append(result(enc))
+        enc.close()
+    assert not np.array_equal(*want)
+    enc = make(a)
+    try:
+        enc.capture()
+        if pin:
+            packed = result(enc)
+            enc.set_gemm_choice("out", number[tile])
+            np.testing.assert_array_equal(result(enc), packed)  # the graph from before
+            enc.capture()
+        np.testing.assert_array_equal(result(enc), want[0])  # (unpacked weights are the uploaded ones)
+        for m, w in ((b, want[1]), (a, want[0])):
+            enc.load(m)
+            for _ in range(2):
+                np.testing.assert_array_equal(result(enc), w)
+    finally:
+        enc.close()
