@@ -19,7 +19,8 @@
 // the wavefronts have whole rows of A in registers between them, so they form
 // sum and sum of squares on the way and the epilogue applies
 //   LN(A) . B = rstd (A . B) - mu rstd colsum(B)
-// with colsum(B) from packing time; the statistics are written for the later
+// with colsum(B) from packing time (rows whose mean is many times their spread get
+// a second, centred pass, see meanDominates()); the statistics are written for the later
 // GEMM whose residual source is the same tensor, LN(C) = rstd c - mu rstd,
 // rounded to fp16 where the graph stores it: the residual is what carries rounding
 // from layer to layer, and without that point 12 layers come out 1.74e-3 instead
@@ -45,13 +46,15 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 constexpr int kWave = 64, kWaves = 8, kThreads = kWave * kWaves;
 constexpr uint32_t kOob = 0x80000000u;
 
+// (1 x 1 x 3: four workgroups to a CU, so that one that reads ahead fits beside
+// three with a tile.)
 // MB x NB blocks of 16 x 16 per workgroup; CH k steps of a wavefront in flight
 // at once (ONCE: that is all of them).  The leading scalars arrive
 // in registers with the wavefront (kernel-argument preload, see the Makefile),
 // so the operands are requested before anything is fetched; `rest` is read
 // behind those requests.
 template <int MB, int NB, int CH, bool ONCE, bool NORM_A, bool A_PACKED>
-__global__ __launch_bounds__(kThreads, (MB + NB) * CH <= 20 && (ONCE || !NORM_A) ? 4 : 2) void packedGemmKernel(
+__global__ __launch_bounds__(kThreads, A_PACKED && (MB + NB) * CH <= 6 ? 8 : (MB + NB) * CH <= 20 && (ONCE || !NORM_A) ? 4 : 2) void packedGemmKernel(
     const _Float16 *A, const _Float16 *B, int M, int N, int K, int steps, int perWave,
     int chunkM, uint32_t chunkMMagic, int chunkN, int xmLog, PackedArgs rest) {
   (void)rest; // (through the argument pointer, see below)
@@ -213,24 +216,24 @@ __global__ __launch_bounds__(kThreads, (MB + NB) * CH <= 20 && (ONCE || !NORM_A)
     }
   }
   __syncthreads();
-#pragma unroll
-  for (int q = 0; q < OUTS; q++) {
-    if (!mine(q))
-      continue;
-    const int block = blockOf(q), m = rowOf(q), n = colOf(q);
-    float4v v = part[block * kWave + lane];
+  auto total = [&](int q) {
+    float4v v = part[blockOf(q) * kWave + lane];
 #pragma unroll
     for (int w = 1; w < kWaves; w++)
-      v += part[(w * MB * NB + block) * kWave + lane];
-    if (NORM_A) {
-      float2v st{0.f, 0.f};
+      v += part[(w * MB * NB + blockOf(q)) * kWave + lane];
+    return v;
+  };
+  auto rowSums = [&](int q) {
+    float2v st{0.f, 0.f};
 #pragma unroll
-      for (int w = 0; w < kWaves; w++)
-        st += stat[w * MB * 16 + (block / NB) * 16 + lane % 16];
-      const float mu = st[0] * p.invK;
-      // the difference cancels to a small negative number for near-constant
-      // rows; clamped so that a tiny eps cannot turn it into a NaN
-      const float rstd = 1.0f / sqrtf(fmaxf(st[1] * p.invK - mu * mu, 0.f) + p.eps);
+    for (int w = 0; w < kWaves; w++)
+      st += stat[w * MB * 16 + (blockOf(q) / NB) * 16 + lane % 16];
+    return st;
+  };
+  auto finish = [&](int q, float4v v, float mu, float var) {
+    const int block = blockOf(q), m = rowOf(q), n = colOf(q);
+    if (NORM_A) {
+      const float rstd = 1.0f / sqrtf(var + p.eps);
       const float shift = -mu * rstd;
 #pragma unroll
       for (int e = 0; e < 4; e++)
@@ -251,6 +254,50 @@ __global__ __launch_bounds__(kThreads, (MB + NB) * CH <= 20 && (ONCE || !NORM_A)
       o[e] = _Float16(x);
     }
     storeWriteThrough(p.D + (p.dPacked ? packedOffset(m, n, p.N) : int64_t(m) * p.N + n), o);
+  };
+  bool again[OUTS], any = false;
+#pragma unroll
+  for (int q = 0; q < OUTS; q++) {
+    again[q] = false;
+    if (!mine(q))
+      continue;
+    const float4v v = total(q);
+    float mu = 0.f, var = 0.f;
+    if (NORM_A) {
+      const float2v st = rowSums(q);
+      mu = st[0] * p.invK;
+      // the difference cancels to a small negative number for near-constant
+      // rows; clamped so that a tiny eps cannot turn it into a NaN
+      var = fmaxf(st[1] * p.invK - mu * mu, 0.f);
+      again[q] = meanDominates(mu, var);
+      any = any || again[q];
+    }
+    finish(q, v, mu, var);
+  }
+  // Rows far from zero once more, centred.  (Behind the other rows' stores: in
+  // front of them the test alone costs 0.1 us a launch.)
+  if (NORM_A && __builtin_expect(__any(any), 0)) {
+#pragma unroll
+    for (int q = 0; q < OUTS; q++) {
+      if (blockOf(q) >= MB * NB)
+        continue; // (the same for the whole wavefront)
+      const float mu = rowSums(q)[0] * p.invK;
+      float d2 = 0.f;
+#pragma unroll 2
+      for (int s = 0; s < steps; s++) { // the block's rows as their fragments lie
+        const half8 x = __builtin_bit_cast(
+            half8, __builtin_amdgcn_raw_buffer_load_b128(
+                       rsrcA, aLane + uint32_t(s) * aStep + uint32_t(blockOf(q) / NB) * aBlock, 0, 0));
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+          const float d = float(x[e]) - mu;
+          d2 = fmaf(d, d, d2);
+        }
+      }
+      d2 = pairSum(rowPairSum(d2));
+      if (again[q])
+        finish(q, total(q), mu, d2 * p.invK);
+    }
   }
 }
 

@@ -351,11 +351,31 @@ __global__ __launch_bounds__(WM *WN *kWave, NBUF *(BM + BN) * SB > 1280 ? 1 : WM
         for (int w = i; w < WN; w += MI)
           t += stat[w * BM + waveM * WTM + i * 32 + l32];
         const float mu = t[0] * p.invK;
+        const int m = (block0 + 2 * i) * 16 + lane % 16;
         // the difference cancels to a small negative number for near-constant
         // rows; clamped so that a tiny eps cannot turn it into a NaN
-        const float rstd = 1.0f / sqrtf(fmaxf(t[1] * p.invK - mu * mu, 0.f) + p.eps);
+        float var = fmaxf(t[1] * p.invK - mu * mu, 0.f);
+        const bool again = m < p.M && meanDominates(mu, var);
+        if (__builtin_expect(__any(again), 0)) { // the 32 rows once more, the two halves of the wavefront in turn
+          float d2 = 0.f;
+          const uint32_t row = uint32_t((block0 + 2 * i) * steps) * 1024u +
+                               uint32_t(lane % 16) * 16u + uint32_t(kb) * 256u;
+#pragma unroll 2
+          for (int s = 0; s < 2 * steps; s++) { // 16 k each
+            const half8 x = __builtin_bit_cast(
+                half8,
+                __builtin_amdgcn_raw_buffer_load_b128(rsrcA, row + uint32_t(s) * 512u, 0, 0));
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+              const float d = float(x[e]) - mu;
+              d2 = fmaf(d, d, d2);
+            }
+          }
+          d2 = pairSum(d2);
+          var = again ? d2 * p.invK : var;
+        }
+        const float rstd = 1.0f / sqrtf(var + p.eps);
         rowStat[i] = float2v{rstd, -mu * rstd};
-        const int m = (block0 + 2 * i) * 16 + lane % 16;
         if (p.statsOut && tn == 0 && waveN == 0 && kb == 0 && m < p.M)
           *reinterpret_cast<float2v *>(p.statsOut + int64_t(m) * 2) = rowStat[i];
       }

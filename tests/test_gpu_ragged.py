@@ -453,3 +453,50 @@ def test_weights_uploaded_again(gpu, rt, synth, pin):
                 np.testing.assert_array_equal(result(enc), w)
     finally:
         enc.close()
+
+
+# few rows (both orders of A, all of K at once and in rounds) and every size of tile that folds a layer norm
+@pytest.mark.parametrize("M,N,K,packing", [(33, 2304, 768, 0), (33, 2304, 768, 5), (16, 32, 32, 5), (70, 96, 4096, 0),
+                                           (250, 1088, 2048, 5), (1000, 3072, 768, 5), (600, 768, 768, 5),
+                                           (4000, 3072, 768, 5), (1400, 2304, 768, 5), (8000, 4096, 1024, 5)])
+@pytest.mark.parametrize("sigmas", [0, 3, 5, 60, 300])
+def test_packed_gemm_of_rows_far_from_zero(gpu, rt, M, N, K, packing, sigmas):
+    """A folded layer norm on rows whose mean is `sigmas` times their spread, mixed with rows around zero, constant
+    rows and rows of one value among zeros: the statistics as close to 64 bits as sums of 32 allow, the result as
+    close as its rounding to fp16 and the sum that cancels (sigmas x 2^-24 x some ten) allow."""
+    g = torch.Generator("cuda").manual_seed(M + sigmas)
+    Mr, R = rt.MemRef, -(-M // 16) * 16
+    A = torch.randn(M, K, device="cuda", generator=g)
+    A[::3] += sigmas
+    A[1::5] -= sigmas
+    A[2::16] = 0
+    A[2::16, 1] = 5
+    if sigmas:
+        A[3::16] = 0.1  # constant
+    A, B = A.half(), (torch.randn(K, N, device="cuda", generator=g) * 0.05).half()
+    ta = torch.full((R, K), 3.0, device="cuda").half()  # (what fills the last row block is not a row)
+    ta[:M] = A
+    if packing & 1:
+        ta = ta.view(R // 16, 16, K // 32, 4, 8).permute(0, 2, 3, 1, 4).contiguous()
+    packed, td = torch.zeros(K * N, dtype=torch.float16, device="cuda"), torch.zeros(R * N, dtype=torch.float16, device="cuda")
+    out, colsum = torch.full((M + 1, 2), 7.0, device="cuda"), B.double().sum(0).float()
+    gpu.homPackWeightF16(*Mr(B.data_ptr(), [1, K, N]).args(), packed.data_ptr())
+    gpu.homPackedGemmF16(*Mr(ta.data_ptr(), [1, M, K]).args(), packed.data_ptr(), 0, None,
+                         *Mr(td.data_ptr(), [1, M, N]).args(), 0, 1, 1e-6, colsum.data_ptr(), None, out.data_ptr(), packing,
+                         None, 0)
+    got = td.view(R, N) if not packing & 4 else td.view(-1, N // 32, 4, 16, 8).permute(0, 3, 1, 2, 4).reshape(R, N)
+    x = A.double()
+    mean = x.mean(1, keepdim=True)
+    rstd = (((x - mean) ** 2).mean(1, keepdim=True) + 1e-6).rsqrt()
+    keep = torch.ones(M, dtype=torch.bool, device="cuda")
+    if sigmas:
+        keep[3::16] = False  # (there eps alone is left, and the mean's last place divided by it)
+        assert torch.isfinite(got[:M]).all()
+    # one pass serves up to 4 sigma: there (1 + 16) / 2 times what a sum of 256 terms in a row loses, sqrt(256) x 2^-24
+    # and for the worst of thousands of rows at most twice that, 1.6e-5
+    torch.testing.assert_close(out[:M][keep][:, :1].double(), rstd[keep], rtol=2e-5, atol=0)
+    torch.testing.assert_close(out[:M][keep][:, 1:].double(), (-mean * rstd)[keep], rtol=2e-5, atol=1e-5)
+    assert (out[M] == 7).all()
+    want = ((x - mean) * rstd) @ B.double()
+    rel = ((got[:M].double() - want)[keep].norm() / want[keep].norm()).item()
+    assert rel <= 3.5e-4 + 1e-6 * sigmas, rel
