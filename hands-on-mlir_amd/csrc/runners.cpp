@@ -678,6 +678,21 @@ Status runPackedGemm(int64_t rankA, void *dstA, const void *packedB, int64_t ran
   HOM_CHECK_RET(al16(A.data) && al16(packedB) && al16(D.data) && al16(g.C) &&
                     al16(colSumB) && al16(ahead),
                 Status::kInvalidArgument, "packed gemm: misaligned operands");
+  HOM_CHECK_RET(aheadBytes >= 0, Status::kInvalidArgument,
+                "packed gemm: aheadBytes must not be negative (%lld)", (long long)aheadBytes);
+  // D may take the place of C (same order: every value is read by the lane that
+  // replaces it), of nothing else that other workgroups may still read
+  auto overlaps = [&](const void *q, int64_t cols, bool packed) {
+    auto rows = [&](bool whole) { return whole ? (g.M + 15) / 16 * 16 : g.M; };
+    const uintptr_t d = reinterpret_cast<uintptr_t>(D.data), x = reinterpret_cast<uintptr_t>(q);
+    return x < d + uintptr_t(rows(g.dPacked) * g.N * 2) && d < x + uintptr_t(rows(packed) * cols * 2);
+  };
+  HOM_CHECK_RET(!overlaps(A.data, g.K, g.aPacked), Status::kInvalidArgument,
+                "packed gemm: D overlaps A");
+  HOM_CHECK_RET(!dstC || (g.C == D.data && g.cPacked == g.dPacked) ||
+                    !overlaps(g.C, g.N, g.cPacked),
+                Status::kInvalidArgument,
+                "packed gemm: D overlaps C in another place or order");
   if (g.M == 0 || g.N == 0)
     return Status::kSuccess;
   g.A = A.data;
@@ -1061,6 +1076,8 @@ Status runBertAttentionF16(int64_t rankA, void *dstA, int64_t rankSeqlen,
                 "attention: tensors must be contiguous");
   HOM_CHECK_RET((reinterpret_cast<uintptr_t>(ahead) & 15) == 0,
                 Status::kInvalidArgument, "attention: misaligned memory to read ahead");
+  HOM_CHECK_RET(aheadBytes >= 0, Status::kInvalidArgument,
+                "attention: aheadBytes must not be negative (%lld)", (long long)aheadBytes);
   return launchBertAttentionF16(A.data, Seq.data, Out.data, bs, seq, headNum,
                                 headDim, scale, stream(),
                                 (packing & HOM_PACKED_D) != 0,

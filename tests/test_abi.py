@@ -282,3 +282,28 @@ def test_folded_layernorm_gemm_argument_checks(rt):
     for (m, n, k) in [(1024, 768, 768), (16384, 1024, 1024), (64, 64, 64)]:
         pieces = lib.homFoldedLayernormPieces(m, n, k, 0, 0)
         assert 1 <= pieces <= (n + 63) // 64 and pieces in {-(-n // e) for e in (64, 128, 256)}
+
+
+def test_packed_entry_points_argument_checks(rt):
+    """Negative sizes to read ahead (which would shrink a grid below its tiles) and results over operands that other
+    workgroups still read are refused before any launch."""
+    M = rt.MemRef
+    w, MB = ctypes.c_void_p(1 << 30), 1 << 20
+
+    def call(a=64 * MB, c=None, d=128 * MB, packing=7, ahead=None, n=0, rows=33):
+        C = M(c, [1, rows, 96]).args() if c is not None else (0, None)
+        return lambda lib: lib.homPackedGemmF16(*M(a, [1, rows, 64]).args(), w, *C, *M(d, [1, rows, 96]).args(), 0, 0,
+                                                1e-6, None, None, None, packing, ahead, n)
+    assert "negative" in _errors(rt, call(ahead=w, n=-1))
+    assert "negative" in _errors(rt, call(ahead=w, n=-(1 << 40)))
+    assert "overlaps C" in _errors(rt, call(c=128 * MB, packing=3))   # C in fragment order, D not
+    assert "overlaps C" in _errors(rt, call(c=128 * MB, packing=5))
+    assert "overlaps C" in _errors(rt, call(c=128 * MB + 1024))
+    assert "overlaps C" in _errors(rt, call(c=128 * MB - 48 * 96 * 2 + 16))  # the last row block is whole
+    assert "overlaps A" in _errors(rt, call(a=128 * MB))
+    assert "overlaps A" in _errors(rt, call(a=128 * MB + 48 * 96 * 2 - 16))
+    qkv, cu, out = M(64 * MB, [1, 33, 192]), M(256, [2]), M(128 * MB, [1, 33, 64])
+    att = lambda n: (lambda lib: lib.homBertAttentionF16(*qkv.args(), *cu.args(), *out.args(), 0.125, 1, 5, w, n))  # noqa: E731
+    assert "negative" in _errors(rt, att(-16))
+    assert "pack rows" in _errors(rt, lambda lib: lib.homPackRowsF16(*qkv.args(), *qkv.args()))
+    assert "unpack weight" in _errors(rt, lambda lib: lib.homUnpackWeightF16(w, *M(256, [1, 31, 16]).args()))
