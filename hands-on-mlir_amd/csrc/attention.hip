@@ -538,9 +538,13 @@ __attribute__((amdgpu_waves_per_eu(D <= 128 || NW == 8 ? 2 : 1, D == 64 && KS ==
         // The same reads as below, issued and waited for by hand: in front of its
         // own transposing reads the compiler would wait for every copy into LDS
         // that is on its way, i.e. for the whole next chunk.
-        // INVARIANT: what an asm read writes is not valid until the wait; the
-        // values pass through an empty asm behind it so that nothing moves ahead.
+        // INVARIANT: what an asm read writes is not valid until the wait.  Every
+        // destination is an in/out operand of a wait, so that no use of it can
+        // move ahead of that one; that the register allocator does not copy or
+        // spill one in between either is checked on the compiled kernels
+        // (tests/test_attention_assembly.py).
         constexpr int kGroups = SBW * 2, kSets = D <= 128 ? 2 : 1;
+        static_assert(DB % 2 == 0, "a wait takes the reads of two column blocks");
         const uint32_t vLane = uint32_t(uintptr_t(HOM_LDS_PTR(sV))) +
                                uint32_t((blk + 4 * hb + trRow) * kRowB + trCol * 2);
         short4v run[kSets][DB][2];
@@ -571,11 +575,16 @@ __attribute__((amdgpu_waves_per_eu(D <= 128 || NW == 8 ? 2 : 1, D == 64 && KS ==
           __builtin_amdgcn_sched_barrier(0);
           if constexpr (kMore && kSets == 2)
             readGroup(Next{});
-          asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(kMore && kSets == 2 ? DB * 2 : 0) : "memory");
+#pragma unroll
+          for (int d = 0; d < DB; d += 2) // (the first one waits for all of them)
+            asm volatile("s_waitcnt lgkmcnt(%4)"
+                         : "+v"(run[g % kSets][d][0]), "+v"(run[g % kSets][d][1]),
+                           "+v"(run[g % kSets][d + 1][0]), "+v"(run[g % kSets][d + 1][1])
+                         : "n"(kMore && kSets == 2 ? DB * 2 : 0)
+                         : "memory");
 #pragma unroll
           for (int d = 0; d < DB; d++) {
-            short4v lo = run[g % kSets][d][0], hi = run[g % kSets][d][1];
-            asm volatile("" : "+v"(lo), "+v"(hi)); // not before the wait
+            const short4v lo = run[g % kSets][d][0], hi = run[g % kSets][d][1];
             short8v both;
 #pragma unroll
             for (int e = 0; e < 4; e++) {
