@@ -415,7 +415,8 @@ __global__ __launch_bounds__(WM *WN *kWave, NBUF *(BM + BN) * SB > 1280 ? 1 : WM
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // (no request outlives the workgroup)
 }
 
-template <int BM, int BN, int WM, int WN, int SB, int NBUF>
+// NORMS: normalised A as well (tiles that only share a CU never get one).
+template <int BM, int BN, int WM, int WN, int SB, int NBUF, bool NORMS = true>
 Status launchTile(const PackedGemm &g, const PackedArgs &p, hipStream_t s) {
   constexpr int kLds = NBUF * (BM + BN) * 64 * SB + WN * BM * 8;
   const int tilesM = int((g.M + BM - 1) / BM), tilesN = int((g.N + BN - 1) / BN);
@@ -423,16 +424,23 @@ Status launchTile(const PackedGemm &g, const PackedArgs &p, hipStream_t s) {
   const int cus = deviceInfo().computeUnits > 0 ? deviceInfo().computeUnits : 256;
   using Kernel = void (*)(const _Float16 *, const _Float16 *, int, int, int, int, int, uint32_t,
                           int, int, int, PackedArgs);
+  constexpr auto normalised = [](auto act) -> Kernel {
+    if constexpr (NORMS)
+      return packedTileKernel<BM, BN, WM, WN, SB, NBUF, true, decltype(act)::value, false>;
+    else
+      return nullptr;
+  };
   // [normalised A][linear, erf GELU, tanh GELU, linear + source]
   static const Kernel kernels[2][4] = {
       {packedTileKernel<BM, BN, WM, WN, SB, NBUF, false, 0, false>,
        packedTileKernel<BM, BN, WM, WN, SB, NBUF, false, 1, false>,
        packedTileKernel<BM, BN, WM, WN, SB, NBUF, false, 2, false>,
        packedTileKernel<BM, BN, WM, WN, SB, NBUF, false, 0, true>},
-      {packedTileKernel<BM, BN, WM, WN, SB, NBUF, true, 0, false>,
-       packedTileKernel<BM, BN, WM, WN, SB, NBUF, true, 1, false>,
-       packedTileKernel<BM, BN, WM, WN, SB, NBUF, true, 2, false>, nullptr}};
+      {normalised(std::integral_constant<int, 0>{}), normalised(std::integral_constant<int, 1>{}),
+       normalised(std::integral_constant<int, 2>{}), nullptr}};
   const int kind = g.C ? 3 : g.activation;
+  HOM_CHECK_RET(kernels[g.normA][kind], Status::kInternal,
+                "packed gemm: no %d x %d kernel of this kind", BM, BN);
   const Kernel kernel = kernels[g.normA][kind];
   static int resident[2][4] = {};
   int &res = resident[g.normA][kind];
@@ -524,13 +532,13 @@ Status launchPackedTile(int tile, const PackedGemm &g, const PackedArgs &p, hipS
   case 0:
     return launchTile<256, 256, 2, 4, 1, 4>(g, p, s);
   case 1:
-    return shared(256, 128) ? launchTile<256, 128, 4, 2, 1, 3>(g, p, s)
+    return shared(256, 128) ? launchTile<256, 128, 4, 2, 1, 3, false>(g, p, s)
                             : launchTile<256, 128, 4, 2, 2, 3>(g, p, s);
   case 2:
     // (and not for so few slabs that the first one counts: 1024 x 3072 x 768 9.7 us
     // against 10.3)
     return shared(128, 128) || (g.K <= 1024 && !g.normA)
-               ? launchTile<128, 128, 2, 4, 1, 4>(g, p, s)
+               ? launchTile<128, 128, 2, 4, 1, 4, false>(g, p, s)
                : launchTile<128, 128, 2, 4, 2, 4>(g, p, s);
   case 3:
     return launchTile<64, 128, 1, 4, 2, 4>(g, p, s);
