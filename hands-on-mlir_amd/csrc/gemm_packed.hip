@@ -246,9 +246,9 @@ __global__ __launch_bounds__(kThreads, A_PACKED && (MB + NB) * CH <= 6 ? 8 : (MB
     for (int e = 0; e < 4; e++) {
       float x = v[e];
       if (p.activation == 1)
-        x = packedGeluErf(x);
+        x = geluErf(x);
       else if (p.activation == 2)
-        x = packedGeluTanh(x);
+        x = geluTanh(x);
       if (p.C)
         x += float(_Float16(fmaf(float(cv[q][e]), cStat[q][0], cStat[q][1])));
       o[e] = _Float16(x);

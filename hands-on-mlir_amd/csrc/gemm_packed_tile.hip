@@ -399,9 +399,9 @@ __global__ __launch_bounds__(WM *WN *kWave, NBUF *(BM + BN) * SB > 1280 ? 1 : WM
             if constexpr (NORM_A)
               x = fmaf(rowStat[i][0], x, rowStat[i][1] * cs[j][g][e]);
             if constexpr (ACT == 1)
-              x = packedGeluErf(x);
+              x = geluErf(x);
             if constexpr (ACT == 2)
-              x = packedGeluTanh(x);
+              x = geluTanh(x);
             if constexpr (SRC)
               x += float(_Float16(fmaf(float(cv[i][j][g][e]), rowStat[i][0], rowStat[i][1])));
             o[e] = _Float16(x);

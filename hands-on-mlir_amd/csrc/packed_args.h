@@ -1,6 +1,7 @@
 // What the two packed GEMM kernels (gemm_packed.hip, gemm_packed_tile.hip) share.
 #pragma once
 
+#include "gelu.h"
 #include "kernels.h"
 
 namespace hom {
@@ -56,23 +57,6 @@ template <int THREADS> inline int aheadGroups(int64_t bytes, int64_t most) {
 // costs, and no other row anything.
 __device__ __forceinline__ bool meanDominates(float mu, float var) {
   return var * 16.0f < mu * mu;
-}
-
-// GELU as the tiled kernels' epilogues compute it (gemm_device.h).
-__device__ __forceinline__ float packedGeluErf(float x) {
-  const float ax = fabsf(x);
-  const float a = fminf(ax, 8.0f);
-  float P = fmaf(3.448796997e-05f, a, -7.812886615e-04f);
-  P = fmaf(P, a, 8.119936101e-03f);
-  P = fmaf(P, a, -5.347220227e-02f);
-  P = fmaf(P, a, -4.587264359e-01f);
-  P = fmaf(P, a, -1.151216269e+00f);
-  P = fmaf(P, a, 8.451195754e-06f);
-  return fmaf(-0.5f * ax, __builtin_amdgcn_exp2f(P), fmaxf(x, 0.0f));
-}
-__device__ __forceinline__ float packedGeluTanh(float x) {
-  const float w = fmaf(x * x, -0.1029432397f, -2.3022081983f);
-  return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x * w));
 }
 
 // The tiled kernel (A packed); false: no tile of it suits the problem.
