@@ -106,3 +106,45 @@ print(json.dumps(dict(weights=weights, live=live, left=hip.hostHipLiveBytes(), r
     assert out["weights"] < out["live"] < 1.2 * out["weights"]
     assert out["left"] == 0
     assert out["refused"] == [-3, 1]
+
+
+def test_result_buffers_from_several_threads(on_host):
+    """The pool of result buffers: no two threads hold the same memory at a time, buffers given back serve others,
+    more than the pool hands out is refused, and nothing stays behind the last encoder."""
+    out = on_host(r"""
+import threading
+e = create()
+start, errors, seen = hip.hostHipLiveBytes(), [], set()
+hip.hostHipFailAt(-1)
+def work(t):
+    rng = np.random.default_rng(t)
+    held = []
+    for i in range(600):
+        if held and rng.random() < 0.5:
+            p, n, v = held.pop(int(rng.integers(len(held))))
+            if (np.ctypeslib.as_array((ctypes.c_ubyte * n).from_address(p)) != v).any():
+                errors.append((t, i))
+            drv.homHostBufferRelease(p)
+        elif len(held) < 6:
+            n, v = int(rng.integers(1, 300000)), int(rng.integers(256))
+            p = drv.homHostBufferAcquire(n)
+            ctypes.memset(p, v, n)
+            held.append((p, n, v))
+            seen.add(p)
+    for p, n, v in held:
+        drv.homHostBufferRelease(p)
+threads = [threading.Thread(target=work, args=(t,)) for t in range(8)]
+[t.start() for t in threads]; [t.join() for t in threads]
+allocated, idle = hip.hostHipAllocations(), hip.hostHipLiveBytes() - start
+kept = drv.homHostBufferAcquire(1000)
+drv.homHostBufferRelease(12345)                   # (not a buffer of the pool)
+big = drv.homHostBufferAcquire((1 << 30) + 1)
+drv.homBertDestroy(e)
+behind = hip.hostHipLiveBytes()
+drv.homHostBufferRelease(kept)
+print(json.dumps(dict(errors=errors, allocated=allocated, idle=idle, big=big, behind=behind, left=hip.hostHipLiveBytes())))
+""")
+    assert out["errors"] == [] and out["big"] is None
+    assert out["allocated"] <= 8 * 6 * 5, "buffers given back are not used again"   # (five sizes of 64 KiB steps)
+    assert 0 < out["idle"] <= 256 << 20
+    assert 0 < out["behind"] <= 1 << 19 and out["left"] == 0   # the buffer still held, then nothing
