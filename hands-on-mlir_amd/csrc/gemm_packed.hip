@@ -444,6 +444,10 @@ Rectangles chooseRectangles(int64_t M, int64_t N, int64_t K, int mb, int nb, int
 template <int MB, int NB, int CH, bool ONCE>
 Status launchVariant(const PackedGemm &g, const PackedArgs &p, const Rectangles &r,
                      int aheadGroups, hipStream_t s) {
+  if (g.only) {
+    *g.only = {false, MB * 16, NB * 16, CH * 32};
+    return Status::kSuccess;
+  }
   const int steps = int(g.K / 32), perWave = (steps + kWaves - 1) / kWaves;
   constexpr int kLds = kWaves * MB * NB * kWave * 16 + kWaves * MB * 16 * 8;
   const dim3 grid((unsigned)(8 * r.chunkM * r.chunkN + aheadGroups)), block(kThreads);

@@ -418,6 +418,10 @@ __global__ __launch_bounds__(WM *WN *kWave, NBUF *(BM + BN) * SB > 1280 ? 1 : WM
 // NORMS: normalised A as well (tiles that only share a CU never get one).
 template <int BM, int BN, int WM, int WN, int SB, int NBUF, bool NORMS = true>
 Status launchTile(const PackedGemm &g, const PackedArgs &p, hipStream_t s) {
+  if (g.only) {
+    *g.only = {true, BM, BN, SB * 32};
+    return Status::kSuccess;
+  }
   constexpr int kLds = NBUF * (BM + BN) * 64 * SB + WN * BM * 8;
   const int tilesM = int((g.M + BM - 1) / BM), tilesN = int((g.N + BN - 1) / BN);
   const int tiles = tilesM * tilesN;

@@ -181,6 +181,12 @@ __host__ __device__ inline int64_t packedOffset(int64_t row, int64_t col, int64_
   return ((row / 16) * (cols / 32) + col / 32) * 512 + (col % 32) / 8 * 128 +
          row % 16 * 8 + col % 8;
 }
+// Which kernel a problem takes: rows x cols of D per workgroup, through LDS in
+// slabs of k (tiled) or from registers, k of a wavefront's share of K in flight.
+struct PackedKernel {
+  bool tiled;
+  int rows, cols, k;
+};
 struct PackedGemm {
   bool aPacked, cPacked, dPacked; // in fragment order
   const _Float16 *A, *packedB, *C;
@@ -194,6 +200,7 @@ struct PackedGemm {
   float eps;
   const void *ahead; // device memory that later kernels read first (may be null)
   int64_t aheadBytes;
+  PackedKernel *only; // not null: say which kernel it would be and launch nothing
 };
 Status launchPackedGemm(const PackedGemm &g, hipStream_t s);
 // Layer norm (no affine parameters) of M rows of N <= 2048 values in fragment

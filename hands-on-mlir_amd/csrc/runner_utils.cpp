@@ -354,6 +354,22 @@ int32_t homGemmSelectNvte(int64_t M, int64_t N, int64_t K, int64_t activation,
   return tuned ? 1 : 0;
 }
 
+int32_t homPackedGemmSelect(int64_t M, int64_t N, int64_t K, int64_t activation,
+                            int32_t normA, int32_t source, int32_t packing,
+                            int32_t readsAhead, int32_t *rows, int32_t *cols,
+                            int32_t *k) {
+  PackedKernel sel{};
+  if (!selectPackedGemm(M, N, K, activation, normA, source, packing, readsAhead, &sel))
+    return -1;
+  if (rows)
+    *rows = sel.rows;
+  if (cols)
+    *cols = sel.cols;
+  if (k)
+    *k = sel.k;
+  return sel.tiled ? 1 : 0;
+}
+
 int32_t homGemmPrefersNvte(int64_t M, int64_t N, int64_t K, int64_t activation) {
   return gemmPrefersNvte(M, N, K, activation) ? 1 : 0;
 }

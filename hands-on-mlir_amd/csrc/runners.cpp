@@ -709,6 +709,30 @@ Status runPackedGemm(int64_t rankA, void *dstA, const void *packedB, int64_t ran
   return launchPackedGemm(g, stream());
 }
 
+bool selectPackedGemm(int64_t M, int64_t N, int64_t K, int64_t activation, int32_t normA,
+                      int32_t source, int32_t packing, int32_t readsAhead, PackedKernel *out) {
+  const bool wide = packing & (HOM_PACKED_C | HOM_PACKED_D);
+  if (M < 1 || N < 1 || K < 1 || K % 32 != 0 || N % (wide ? 32 : 16) != 0 ||
+      M * std::max(K, N) >= (int64_t(1) << 30) || K * N >= (int64_t(1) << 30) ||
+      activation < 0 || activation > 2 || (source && activation))
+    return false;
+  // (operands are told apart by being there or not)
+  static const _Float16 present = 0;
+  PackedGemm g{};
+  g.M = M;
+  g.N = N;
+  g.K = K;
+  g.aPacked = (packing & HOM_PACKED_A) != 0;
+  g.cPacked = (packing & HOM_PACKED_C) != 0;
+  g.dPacked = (packing & HOM_PACKED_D) != 0;
+  g.C = source ? &present : nullptr;
+  g.ahead = readsAhead ? &present : nullptr;
+  g.activation = int(activation);
+  g.normA = normA != 0;
+  g.only = out;
+  return launchPackedGemm(g, nullptr) == Status::kSuccess;
+}
+
 Status runLayernormGemm(int64_t rankA, void *dstA, int64_t rankB, void *dstB,
                         int64_t rankC, void *dstC, int64_t rankD, void *dstD,
                         int64_t rankVar, void *dstVar, int64_t rankMean,

@@ -47,6 +47,8 @@ int32_t foldedLayernormPieces(int64_t M, int64_t N, int64_t K, int64_t activatio
                               int32_t likeGemmNum);
 Status runPackWeight(int64_t rankB, void *dstB, void *packed);
 Status runUnpackWeight(const void *packed, int64_t rankB, void *dstB);
+bool selectPackedGemm(int64_t M, int64_t N, int64_t K, int64_t activation, int32_t normA,
+                      int32_t source, int32_t packing, int32_t readsAhead, PackedKernel *out);
 Status runPackRows(int64_t rankA, void *dstA, int64_t rankOut, void *dstOut);
 Status runPackedLayernorm(int64_t rankA, void *dstA, int64_t rankOut, void *dstOut,
                           float eps, int32_t packing);

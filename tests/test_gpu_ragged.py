@@ -2,6 +2,7 @@
 import numpy as np
 import pytest
 import torch
+from packed_shapes import FEW_ROWS, MANY_ROWS, NORMALISED_FEW, NORMALISED_MANY
 
 pytestmark = pytest.mark.gpu
 
@@ -175,11 +176,8 @@ def fragment_order(a):
     return np.ascontiguousarray(p.reshape(-1, 16, cols // 32, 4, 8).transpose(0, 2, 3, 1, 4)).reshape(-1)
 
 
-# row counts around the 16 / 32 / 64-row tiles, one k step per wavefront and several rounds of them, few and many
-# column blocks, both orders of every operand
-@pytest.mark.parametrize("M,N,K", [(1, 32, 32), (16, 96, 256), (17, 768, 768), (33, 2304, 768), (64, 3072, 768),
-                                   (65, 768, 3072), (130, 1024, 1024), (200, 1024, 4096), (300, 4096, 1056),
-                                   (257, 320, 5120)])
+# every kernel for few rows (test_packed_selection.py), both orders of every operand
+@pytest.mark.parametrize("M,N,K", FEW_ROWS)
 @pytest.mark.parametrize("packing", [0, 7, 3, 5])
 def test_packed_gemm(gpu, rt, oracle, M, N, K, packing):
     g = np.random.default_rng(M + N + K + packing)
@@ -229,12 +227,9 @@ def test_packed_gemm(gpu, rt, oracle, M, N, K, packing):
         np.testing.assert_allclose(host(out)[:, 1], -x.mean(1) * rstd, rtol=1e-3, atol=1e-4)
 
 
-# every tile of the packed GEMM for many rows, with one tile and with several of them per workgroup; partial row
-# blocks and column tiles, and rectangles of an XCD that the tiles do not fill
-@pytest.mark.parametrize("M,N,K", [(1000, 3072, 768), (192, 768, 3072), (250, 1088, 2080), (1000, 768, 3072), (760, 1088, 2048),
-                                   (1000, 1024, 1024), (8000, 3072, 768), (392, 1184, 64), (524, 1856, 64), (583, 3296, 64), (1476, 2976, 448),
-                                   (16439, 160, 64), (10970, 352, 192), (17111, 288, 64), (16546, 672, 128),
-                                   (16388, 1696, 128)])
+# every tile of the packed GEMM for many rows, with one tile and with several of them per workgroup
+# (test_packed_selection.py)
+@pytest.mark.parametrize("M,N,K", MANY_ROWS)
 def test_packed_gemm_many_rows(gpu, rt, M, N, K):
     g = torch.Generator("cuda").manual_seed(M)
     Mr, R = rt.MemRef, -(-M // 16) * 16
@@ -455,10 +450,9 @@ def test_weights_uploaded_again(gpu, rt, synth, pin):
         enc.close()
 
 
-# few rows (both orders of A, all of K at once and in rounds) and every size of tile that folds a layer norm
-@pytest.mark.parametrize("M,N,K,packing", [(33, 2304, 768, 0), (33, 2304, 768, 5), (16, 32, 32, 5), (70, 96, 4096, 0),
-                                           (250, 1088, 2048, 5), (1000, 3072, 768, 5), (600, 768, 768, 5),
-                                           (4000, 3072, 768, 5), (1400, 2304, 768, 5), (8000, 4096, 1024, 5)])
+# few rows (both orders of A, all of K at once and in rounds) and every tile that folds a layer norm
+@pytest.mark.parametrize("M,N,K,packing", [(*size, packing) for packing in (0, 5) for size in NORMALISED_FEW] +
+                         [(*size, 5) for size in NORMALISED_MANY])
 @pytest.mark.parametrize("sigmas", [0, 3, 5, 60, 300])
 def test_packed_gemm_of_rows_far_from_zero(gpu, rt, M, N, K, packing, sigmas):
     """A folded layer norm on rows whose mean is `sigmas` times their spread, mixed with rows around zero, constant
