@@ -240,7 +240,7 @@ def main():
                                  "residency": "B (8.4 MB) stays in the Infinity Cache between launches"})
 
     if not args.no_large:
-        # configs[4]: BERT-large encoder end to end (reported beside the headline, not as `value`)
+        # BERT-large encoder end to end (reported beside the headline, not as `value`)
         big = synth.bert_encoder(layers=24, hidden=1024, heads=16, ffn=4096, bs=32, seq=512, config=41)
         enc = bert.BertEncoder(24, 1024, 16, 4096, 32, 512, big["dims"]["vocab"],
                                gemm_mode=args.gemm_mode, gelu_form="erf")
@@ -352,7 +352,7 @@ def main():
         "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
         "dtype": "f16", "data": "synthetic",
         "config": {"workload": "BERT-base encoder fp16, 12 layers, hidden 768, 12 heads, FFN 3072, "
-                               "batch 8 x seq 128, padding mask (configs[3])",
+                               "batch 8 x seq 128, padding mask",
                    "launch": "eager C-ABI calls" if args.eager else "HIP graph replay of the C-ABI call list",
                    "gemm_mode": args.gemm_mode,
                    "gemm_kernels": "homPackedGemmF16 on weights in fragment order, tile chosen by size" if packed else

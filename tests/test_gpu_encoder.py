@@ -141,7 +141,7 @@ def test_masked_lm_small(gpu, oracle, synth, gemm_mode, gelu):
 
 
 def test_masked_lm_bert_base_b8_s128(gpu, oracle, synth):
-    """BASELINE config 4 with the LM head (the reference's BertForMaskedLM graph, logits [8, 128, 30522]):
+    """BERT-base b8 x s128 with the LM head (the reference's BertForMaskedLM graph, logits [8, 128, 30522]):
     the head is checked from the GPU's own hidden states on 96 sampled valid positions x all 30522
     columns (GEMM tolerance rtol 1e-3 / atol 1e-2); the encoder in front of it has its own test."""
     bert = importlib.import_module("hands-on-mlir_amd.bert")
