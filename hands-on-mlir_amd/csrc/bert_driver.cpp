@@ -57,6 +57,12 @@ struct LayerWeights {
   // [1,K,N] (manifest path) or [1,N,K] (nvte path); [1,K,N] with the data in
   // fragment order while the encoder runs on packed weights
   Tensor wqkv, wo, w1, w2;
+  Tensor &operator[](int which) { return which == 0 ? wqkv : which == 1 ? wo : which == 2 ? w1 : w2; }
+  // Of encoders created on packed weights, by `which`: where the packed weight
+  // lies, and what the next forward has to do first (prepareWeights): pack what
+  // was uploaded, unpack it into the tensor above.
+  _Float16 *packed[4] = {};
+  bool toPack[4] = {}, toUnpack[4] = {};
 };
 
 // How one GEMM role of the graph is called.  nk: the weight is stored as
@@ -102,13 +108,16 @@ struct HomBertEncoder {
   // usesPacked: every layer GEMM runs on weights in fragment order; up to a few
   // thousand rows (foldsPacked) with the layer norms folded into the GEMMs around
   // them.  The layers' weights lie in packedArena in the order a forward reads them.
-  // An upload passes through `staging` (the largest weight, row-major) into
-  // the layer's weight and, of Wqkv and W1, into packedColSums; qkv, attn and f are
-  // in fragment order as well, and so is hPacked, what h is between the layers.
-  // A call that pins the row-major list lays all of that out anew (leavePacked);
-  // graphs captured before it still hold the arena and what is in `retired`.
+  // An upload waits in `uploads`, row-major and at the same place, for the next forward,
+  // which packs it, takes the column sums of Wqkv and W1 and gives `uploads`
+  // back; qkv, attn and f are in fragment order as well, and so is hPacked, what h
+  // is between the layers.  A call that pins the row-major list lays all of that
+  // out anew (leavePacked); graphs captured before it still hold the arena and
+  // what is in `retired`.
   bool packed = false;
-  Tensor packedArena, staging, hPacked;
+  Tensor packedArena, hPacked;
+  _Float16 *uploads = nullptr;
+  bool weightsToDo = false; // some toPack or toUnpack
   float *packedColSums = nullptr;
   float *packedStats[2] = {nullptr, nullptr}; // rows of h entering QKV / FFN1
   std::vector<Tensor> retired;
@@ -392,40 +401,39 @@ bool allocPacked(HomBertEncoder *e) {
     weight(w.wo, H, H);
     weight(w.w1, H, F);
     weight(w.w2, F, H);
+    for (int i = 0; i < 4; i++)
+      w.packed[i] = static_cast<_Float16 *>(w[i].data());
   }
-  e->staging.m = alloc3DMemRefNVGPUF16(1, H, std::max(3 * H, F));
   e->hPacked = allocPadded(e, H);
-  return e->staging.m.descriptor && e->hPacked.m.descriptor &&
+  return e->hPacked.m.descriptor &&
          alloc(e->packedColSums, size_t(e->layers) * size_t(3 * H + F)) &&
          alloc(e->packedStats[0], rows * 2) && alloc(e->packedStats[1], rows * 2);
 }
 
-// The row-major values in e->staging become weight `which` (0 Wqkv, 1 Wo, 2 W1,
-// 3 W2) of a layer.  Queued behind what runs on the stream and waited for: the
-// staging buffer is free again.
-bool packUploaded(HomBertEncoder *e, int layer, int which, const Tensor &w) {
-  HomStridedMemRef3 from = *static_cast<const HomStridedMemRef3 *>(w.m.descriptor);
-  from.basePtr = from.data = e->staging.data();
-  void *prev = homGetStream();
-  homSetStream(e->stream);
-  homPackWeightF16(3, &from, w.data());
-  if (which == 0 || which == 2)
-    homColumnSumsF16(3, &from, packedColSum(e, layer, which == 2));
-  homSetStream(prev);
-  return hipOk(hipStreamSynchronize(e->stream), "hipStreamSynchronize");
+// Where weight `which` of a layer is uploaded to on packed weights; null if
+// there is no memory for it.  Nothing is launched: another thread may be using
+// the library's stream for an encoder of its own.
+_Float16 *uploadTo(HomBertEncoder *e, LayerWeights &w, int which) {
+  const _Float16 *arena = static_cast<const _Float16 *>(e->packedArena.data());
+  if (!e->uploads) {
+    const int64_t *sz = hom_memref_sizes(e->packedArena.m.descriptor);
+    if (!hipOk(hipMalloc(reinterpret_cast<void **>(&e->uploads), size_t(sz[0] * sz[1] * sz[2]) * 2),
+               "hipMalloc for uploaded weights"))
+      return nullptr;
+  }
+  return e->uploads + (w.packed[which] - arena);
 }
 
-// From packed weights to the row-major list: the weights' values unpacked into
-// tensors of their own, and row-major activations.  False, with nothing changed,
-// if there is no memory for them.
+// From packed weights to the row-major list: tensors for it.  The weights'
+// values follow with the next forward.  False, with nothing changed, if there
+// is no memory for them.
 bool leavePacked(HomBertEncoder *e) {
   if (!e->packed)
     return true;
   std::vector<Tensor *> old;
   for (auto &w : e->w)
-    for (Tensor *t : {&w.wqkv, &w.wo, &w.w1, &w.w2})
-      old.push_back(t);
-  const size_t weights = old.size();
+    for (int i = 0; i < 4; i++)
+      old.push_back(&w[i]);
   for (Tensor *t : {&e->qkv, &e->attn, &e->f})
     old.push_back(t);
   std::vector<Tensor> fresh(old.size());
@@ -438,12 +446,6 @@ bool leavePacked(HomBertEncoder *e) {
       return false;
     }
   }
-  void *prev = homGetStream();
-  homSetStream(e->stream);
-  for (size_t i = 0; i < weights; i++)
-    homUnpackWeightF16(old[i]->data(), fresh[i].m.rank, fresh[i].m.descriptor);
-  homSetStream(prev);
-  (void)hipOk(hipStreamSynchronize(e->stream), "hipStreamSynchronize");
   for (size_t i = 0; i < old.size(); i++) {
     if (!old[i]->view)
       e->retired.push_back(*old[i]);
@@ -451,8 +453,42 @@ bool leavePacked(HomBertEncoder *e) {
       old[i]->release();
     *old[i] = fresh[i];
   }
+  for (auto &w : e->w)
+    std::fill(w.toUnpack, w.toUnpack + 4, true);
+  e->weightsToDo = true;
   e->packed = false;
   return true;
+}
+
+// What uploads and leavePacked left to do, queued behind what runs on the
+// stream and waited for.
+bool prepareWeights(HomBertEncoder *e) {
+  if (!e->weightsToDo)
+    return true;
+  const _Float16 *arena = static_cast<const _Float16 *>(e->packedArena.data());
+  void *prev = homGetStream();
+  homSetStream(e->stream);
+  for (int l = 0; l < e->layers; l++) {
+    LayerWeights &w = e->w[size_t(l)];
+    for (int i = 0; i < 4; i++) {
+      if (w.toPack[i]) {
+        HomStridedMemRef3 from = *static_cast<const HomStridedMemRef3 *>(w[i].m.descriptor);
+        from.basePtr = from.data = e->uploads + (w.packed[i] - arena);
+        homPackWeightF16(3, &from, w.packed[i]);
+        if (i == 0 || i == 2)
+          homColumnSumsF16(3, &from, packedColSum(e, l, i == 2));
+      }
+      if (w.toUnpack[i])
+        homUnpackWeightF16(w.packed[i], w[i].m.rank, w[i].m.descriptor);
+      w.toPack[i] = w.toUnpack[i] = false;
+    }
+  }
+  homSetStream(prev);
+  const bool ok = hipOk(hipStreamSynchronize(e->stream), "hipStreamSynchronize");
+  (void)hipFree(e->uploads);
+  e->uploads = nullptr;
+  e->weightsToDo = false;
+  return ok;
 }
 
 // The layers on packed weights: 5 launches each.  h travels un-normalised
@@ -740,7 +776,7 @@ DRV_EXPORT int homBertFoldLayernorm(HomBertEncoder *e) {
   const int32_t pFfn2 = homFoldedLayernormPieces(M, e->hidden, e->ffn, 0, 0);
   if (pOut != pFfn2 || pOut < 1)
     return -1; // (both depend on M and N only)
-  if (!leavePacked(e))
+  if (!leavePacked(e) || !prepareWeights(e))
     return -1;
   bool ok = true;
   for (float *&q : e->rowSums)
@@ -808,7 +844,7 @@ DRV_EXPORT void homBertDestroy(HomBertEncoder *e) {
     t.release();
   e->packedArena.release();
   e->hPacked.release();
-  e->staging.release();
+  (void)hipFree(e->uploads);
   (void)hipFree(e->packedColSums);
   for (float *q : e->packedStats)
     (void)hipFree(q);
@@ -826,10 +862,9 @@ DRV_EXPORT int homBertUpload(HomBertEncoder *e, int layer, int which,
                              const void *host, int64_t numel) {
   Tensor *t = nullptr;
   if (which <= 3) {
-    if (layer < 0 || layer >= e->layers)
+    if (which < 0 || layer < 0 || layer >= e->layers)
       return -1;
-    LayerWeights &w = e->w[size_t(layer)];
-    t = which == 0 ? &w.wqkv : which == 1 ? &w.wo : which == 2 ? &w.w1 : &w.w2;
+    t = &e->w[size_t(layer)][which];
   } else if (which <= 5) {
     t = which == 4 ? &e->wordEmb : &e->posType;
   } else {
@@ -845,13 +880,18 @@ DRV_EXPORT int homBertUpload(HomBertEncoder *e, int layer, int which,
                     "%lld\n", (long long)numel, (long long)expect);
     return -2;
   }
-  const bool pack = which <= 3 && e->packed;
-  return hipOk(hipMemcpy(pack ? e->staging.data() : t->data(), host, size_t(numel) * 2,
-                         hipMemcpyHostToDevice),
-               "hipMemcpy") &&
-                 (!pack || packUploaded(e, layer, which, *t))
-             ? 0
-             : -3;
+  void *to = t->data();
+  if (which <= 3 && e->packed && !(to = uploadTo(e, e->w[size_t(layer)], which)))
+    return -3;
+  if (!hipOk(hipMemcpy(to, host, size_t(numel) * 2, hipMemcpyHostToDevice), "hipMemcpy"))
+    return -3;
+  if (which <= 3) {
+    LayerWeights &w = e->w[size_t(layer)];
+    w.toPack[which] = e->packed;
+    w.toUnpack[which] = false; // (what is there now is newer)
+    e->weightsToDo = e->weightsToDo || e->packed;
+  }
+  return 0;
 }
 
 DRV_EXPORT int homBertSync(HomBertEncoder *e);
@@ -880,6 +920,7 @@ DRV_EXPORT void homBertForward(HomBertEncoder *e, int fromIds) {
   void *prev = homGetStream();
   homSetStream(e->stream);
   e->inFlight = true;
+  (void)prepareWeights(e);
   callList(e, fromIds);
   homSetStream(prev);
 }
@@ -916,7 +957,7 @@ DRV_EXPORT int homBertCapture(HomBertEncoder *e, int fromIds) {
 }
 
 DRV_EXPORT int homBertReplay(HomBertEncoder *e) {
-  if (!e->graphExec)
+  if (!e->graphExec || !prepareWeights(e)) // (weights uploaded since the capture)
     return -1;
   e->inFlight = true;
   return hipOk(hipGraphLaunch(e->graphExec, e->stream), "hipGraphLaunch") ? 0

@@ -148,3 +148,42 @@ print(json.dumps(dict(errors=errors, allocated=allocated, idle=idle, big=big, be
     assert out["allocated"] <= 8 * 6 * 5, "buffers given back are not used again"   # (five sizes of 64 KiB steps)
     assert 0 < out["idle"] <= 256 << 20
     assert 0 < out["behind"] <= 1 << 19 and out["left"] == 0   # the buffer still held, then nothing
+
+
+def test_uploads_and_pins_leave_the_library_alone(on_host):
+    """Another thread may be enqueueing on the library's stream: uploading and pinning launch nothing and never set
+    it; an upload with no memory for it is refused; what they leave to do happens once, with the next forward."""
+    out = on_host(r"""
+e = create()
+marker = ctypes.c_void_p(77)
+lib.homSetStream(marker)
+upload(e)
+assert drv.homBertSetGemmChoice(e, 1, 10**6, 1) < 0   # (no such kernel: stays on packed weights)
+quiet = [hip.hostHipLaunches(), lib.homGetStream()]
+def forward():
+    before = hip.hostHipLaunches()
+    drv.homBertForward(e, 1)
+    return hip.hostHipLaunches() - before
+first, second = forward(), forward()
+upload(e)
+again = forward()
+hip.hostHipFailAt(0)
+refused = drv.homBertUpload(e, 0, 0, np.zeros(3 * H * H, np.float16).ctypes.data, 3 * H * H)
+hip.hostHipFailAt(-1)
+third = forward()
+before = hip.hostHipLaunches()
+assert drv.homBertSetGemmChoice(e, 1, 1, 1) == 0
+n = 3 * H * H
+assert drv.homBertUpload(e, 1, 0, np.zeros(n, np.float16).ctypes.data, n) == 0
+quiet.append(hip.hostHipLaunches() - before)
+left, pinned = forward(), forward()
+bad = drv.homBertUpload(e, 0, -1, np.zeros(1, np.float16).ctypes.data, 1)
+drv.homBertDestroy(e)
+print(json.dumps(dict(quiet=quiet, stream=lib.homGetStream(), first=first, second=second, again=again, refused=refused,
+                      third=third, left=left, pinned=pinned, bad=bad, live=hip.hostHipLiveBytes())))
+""")
+    assert out["quiet"] == [0, 77, 0] and out["stream"] == 77
+    assert out["first"] - out["second"] == 6 * 3 == out["again"] - out["second"]   # 4 to pack, 2 column sums a layer
+    assert out["refused"] == -3 and out["third"] == out["second"] and out["bad"] == -1
+    assert out["left"] - out["pinned"] == 4 * 3 - 1   # unpacked but for the one uploaded since
+    assert out["live"] == 0
