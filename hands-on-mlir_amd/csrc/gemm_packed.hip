@@ -106,9 +106,11 @@ __global__ __launch_bounds__(kThreads, A_PACKED && (MB + NB) * CH <= 6 ? 8 : (MB
   for (int c = 0; c < CH; c++)
     requestStep(c, stepBegin + c);
   __builtin_amdgcn_sched_barrier(0);
-  PackedArgs p = {};
+  // (fetched where they are used: together, the two sides' fields would be waited
+  // for one after the other)
+  auto restArgs = [] {
+    PackedArgs p = {};
 #if defined(__HIP_DEVICE_COMPILE__) // (the host pass only needs the kernel's stub)
-  {
     typedef const __attribute__((address_space(4))) PackedArgs *RestPtr;
     constexpr int kRestOffset = 2 * 8 + 10 * 4; // bytes of the leading arguments
     static_assert(kRestOffset % alignof(PackedArgs) == 0, "argument layout");
@@ -117,14 +119,18 @@ __global__ __launch_bounds__(kThreads, A_PACKED && (MB + NB) * CH <= 6 ? 8 : (MB
                              kRestOffset);
     asm volatile("" : "+s"(late));
     p = *late;
-  }
 #endif
+    return p;
+  };
   if (!isTile) {
     const int tiles = 8 * chunkM * chunkN;
-    if (id >= tiles)
+    if (id >= tiles) {
+      const PackedArgs p = restArgs();
       readAhead<kThreads>(p.ahead, p.aheadBytes, id - tiles, int(gridDim.x) - tiles, tid);
+    }
     return;
   }
+  const PackedArgs p = restArgs();
   // What the epilogue reads: wavefront w finishes 16 x 16 blocks w, w + 8, .. of
   // the tile, a lane 4 consecutive columns of one row of each.
   constexpr int OUTS = (MB * NB + kWaves - 1) / kWaves;
@@ -295,6 +301,9 @@ __global__ __launch_bounds__(kThreads, A_PACKED && (MB + NB) * CH <= 6 ? 8 : (MB
         }
       }
       d2 = pairSum(rowPairSum(d2));
+      // (nothing shared with the stores above: what is would move in front of the
+      // barrier, into every launch)
+      asm volatile("" : "+v"(cv[q]), "+v"(cStat[q]), "+v"(cSum[q]));
       if (again[q])
         finish(q, total(q), mu, d2 * p.invK);
     }
