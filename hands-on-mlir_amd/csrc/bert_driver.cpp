@@ -60,8 +60,10 @@ struct LayerWeights {
   Tensor &operator[](int which) { return which == 0 ? wqkv : which == 1 ? wo : which == 2 ? w1 : w2; }
   // Of encoders created on packed weights, by `which`: where the packed weight
   // lies, and what the next forward has to do first (prepareWeights): pack what
-  // was uploaded, unpack it into the tensor above.
+  // was uploaded (row-major, in the same order from `uploads` on), unpack it into the
+  // tensor above.
   _Float16 *packed[4] = {};
+  _Float16 *uploads = nullptr;
   bool toPack[4] = {}, toUnpack[4] = {};
 };
 
@@ -108,15 +110,13 @@ struct HomBertEncoder {
   // usesPacked: every layer GEMM runs on weights in fragment order; up to a few
   // thousand rows (foldsPacked) with the layer norms folded into the GEMMs around
   // them.  The layers' weights lie in packedArena in the order a forward reads them.
-  // An upload waits in `uploads`, row-major and at the same place, for the next forward,
-  // which packs it, takes the column sums of Wqkv and W1 and gives `uploads`
-  // back; qkv, attn and f are in fragment order as well, and so is hPacked, what h
+  // An upload waits row-major for the next forward, which packs it, takes the column
+  // sums of Wqkv and W1 and gives the row-major memory back; qkv, attn and f are in fragment order as well, and so is hPacked, what h
   // is between the layers.  A call that pins the row-major list lays all of that
   // out anew (leavePacked); graphs captured before it still hold the arena and
   // what is in `retired`.
   bool packed = false;
   Tensor packedArena, hPacked;
-  _Float16 *uploads = nullptr;
   bool weightsToDo = false; // some toPack or toUnpack
   float *packedColSums = nullptr;
   float *packedStats[2] = {nullptr, nullptr}; // rows of h entering QKV / FFN1
@@ -412,16 +412,16 @@ bool allocPacked(HomBertEncoder *e) {
 
 // Where weight `which` of a layer is uploaded to on packed weights; null if
 // there is no memory for it.  Nothing is launched: another thread may be using
-// the library's stream for an encoder of its own.
-_Float16 *uploadTo(HomBertEncoder *e, LayerWeights &w, int which) {
-  const _Float16 *arena = static_cast<const _Float16 *>(e->packedArena.data());
-  if (!e->uploads) {
-    const int64_t *sz = hom_memref_sizes(e->packedArena.m.descriptor);
-    if (!hipOk(hipMalloc(reinterpret_cast<void **>(&e->uploads), size_t(sz[0] * sz[1] * sz[2]) * 2),
-               "hipMalloc for uploaded weights"))
-      return nullptr;
-  }
-  return e->uploads + (w.packed[which] - arena);
+// the library's stream for an encoder of its own.  (A layer at a time: one
+// allocation as large as the arena, given back between encoders, left the next ones
+// with memory that cold weights come out of more slowly: 2 x 57 with the LM head 453 ->
+// 462 us a request.)
+_Float16 *uploadTo(const HomBertEncoder *e, LayerWeights &w, int which) {
+  const int64_t *sz = hom_memref_sizes(e->packedArena.m.descriptor);
+  if (!w.uploads && !hipOk(hipMalloc(reinterpret_cast<void **>(&w.uploads), size_t(sz[1] * sz[2]) * 2),
+                           "hipMalloc for uploaded weights"))
+    return nullptr;
+  return w.uploads + (w.packed[which] - w.packed[0]);
 }
 
 // From packed weights to the row-major list: tensors for it.  The weights'
@@ -465,7 +465,6 @@ bool leavePacked(HomBertEncoder *e) {
 bool prepareWeights(HomBertEncoder *e) {
   if (!e->weightsToDo)
     return true;
-  const _Float16 *arena = static_cast<const _Float16 *>(e->packedArena.data());
   void *prev = homGetStream();
   homSetStream(e->stream);
   for (int l = 0; l < e->layers; l++) {
@@ -473,7 +472,7 @@ bool prepareWeights(HomBertEncoder *e) {
     for (int i = 0; i < 4; i++) {
       if (w.toPack[i]) {
         HomStridedMemRef3 from = *static_cast<const HomStridedMemRef3 *>(w[i].m.descriptor);
-        from.basePtr = from.data = e->uploads + (w.packed[i] - arena);
+        from.basePtr = from.data = w.uploads + (w.packed[i] - w.packed[0]);
         homPackWeightF16(3, &from, w.packed[i]);
         if (i == 0 || i == 2)
           homColumnSumsF16(3, &from, packedColSum(e, l, i == 2));
@@ -485,8 +484,10 @@ bool prepareWeights(HomBertEncoder *e) {
   }
   homSetStream(prev);
   const bool ok = hipOk(hipStreamSynchronize(e->stream), "hipStreamSynchronize");
-  (void)hipFree(e->uploads);
-  e->uploads = nullptr;
+  for (LayerWeights &w : e->w) {
+    (void)hipFree(w.uploads);
+    w.uploads = nullptr;
+  }
   e->weightsToDo = false;
   return ok;
 }
@@ -829,6 +830,7 @@ DRV_EXPORT void homBertDestroy(HomBertEncoder *e) {
     w.wo.release();
     w.w1.release();
     w.w2.release();
+    (void)hipFree(w.uploads);
   }
   for (float *q : e->colSumQkv)
     (void)hipFree(q);
@@ -844,7 +846,6 @@ DRV_EXPORT void homBertDestroy(HomBertEncoder *e) {
     t.release();
   e->packedArena.release();
   e->hPacked.release();
-  (void)hipFree(e->uploads);
   (void)hipFree(e->packedColSums);
   for (float *q : e->packedStats)
     (void)hipFree(q);
