@@ -46,13 +46,12 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 constexpr int kWave = 64, kWaves = 8, kThreads = kWave * kWaves;
 constexpr uint32_t kOob = 0x80000000u;
 
-// (1 x 1 x 3: four workgroups to a CU, so that one that reads ahead fits beside
-// three with a tile.)
 // MB x NB blocks of 16 x 16 per workgroup; CH k steps of a wavefront in flight
 // at once (ONCE: that is all of them).  The leading scalars arrive
 // in registers with the wavefront (kernel-argument preload, see the Makefile),
 // so the operands are requested before anything is fetched; `rest` is read
-// behind those requests.
+// behind those requests.  1 x 1 x 3 is held to four workgroups to a CU, so that
+// one that reads ahead fits beside three with a tile.
 template <int MB, int NB, int CH, bool ONCE, bool NORM_A, bool A_PACKED>
 __global__ __launch_bounds__(kThreads, A_PACKED && (MB + NB) * CH <= 6 ? 8 : (MB + NB) * CH <= 20 && (ONCE || !NORM_A) ? 4 : 2) void packedGemmKernel(
     const _Float16 *A, const _Float16 *B, int M, int N, int K, int steps, int perWave,
