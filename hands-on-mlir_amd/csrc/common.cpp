@@ -85,6 +85,14 @@ void releaseStreamScratch(hipStream_t s) {
       e.inUse = false;
 }
 
+bool libraryScratchReady(ScratchSlot slot, size_t bytes) {
+  for (const StreamScratch &e : g_scratch)
+    if (e.inUse && e.stream == g_stream && e.slot[slot].bytes >= bytes)
+      return true;
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(g_stream, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone;
+}
+
 void *libraryScratch(ScratchSlot slot, size_t bytes, bool zero) {
   StreamScratch *mine = nullptr, *spare = nullptr;
   for (StreamScratch &s : g_scratch) {

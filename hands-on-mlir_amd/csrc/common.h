@@ -107,6 +107,9 @@ enum ScratchSlot { kWorkspace = 0, kCounters = 1, kTemp = 2, kNumSlots = 3 };
 // Returns nullptr (after recording an error) on allocation failure.  `zero`
 // clears newly allocated memory once, at allocation time.
 void *libraryScratch(ScratchSlot slot, size_t bytes, bool zero);
+// Whether libraryScratch() can hand out that much now: the slot holds it, or
+// memory may be allocated (the calling stream is not being captured).
+bool libraryScratchReady(ScratchSlot slot, size_t bytes);
 // Number of times any slot has been replaced by a larger buffer (tests).
 int libraryScratchGeneration();
 // The caller is done with stream `s` (everything enqueued on it has finished

@@ -5,6 +5,7 @@
 // gemm_dma.h / gemm_pipe.h / gemm_staged.h, instantiated in gemm_inst_*.hip.
 #include "gemm_dma.h"
 #include "gemm_fine.h"
+#include "gemm_ksplit.h"
 #include "gemm_pipe.h"
 #include "gemm_staged.h"
 
@@ -58,6 +59,8 @@ namespace gemmk {
   HOM_EXTERN_U(1, true, BM, BN, WM, WN, DIST)                                  \
   HOM_EXTERN_U(2, false, BM, BN, WM, WN, DIST)                                 \
   HOM_EXTERN_U(2, true, BM, BN, WM, WN, DIST)
+#define HOM_KSPLIT_TILE(BM, BN)                                                \
+  HOM_EXTERN_EPILOGUES(launchKsplitEntry, BM / 16, BN / 16)
 #define HOM_STAGED_TILE(BM, BN, BK, WM, WN, VEC)                               \
   HOM_EXTERN_STAGED(BM, BN, BK, WM, WN, 0, VEC)                                \
   HOM_EXTERN_STAGED(BM, BN, BK, WM, WN, 1, VEC)                                \
@@ -71,6 +74,7 @@ namespace gemmk {
 #undef HOM_FINE_TILE
 #undef HOM_PIPE_TILE_Q
 #undef HOM_PIPE_TILE_U
+#undef HOM_KSPLIT_TILE
 #undef HOM_STAGED_TILE
 } // namespace gemmk
 
@@ -185,6 +189,24 @@ Status launchAny(const GemmProblem &p, hipStream_t s) {
   HOM_FINE_ENTRY(BM, BN, WM, WN, DIST, Epilogue::kLinear, "linear", 0),        \
       HOM_FINE_ENTRY(BM, BN, WM, WN, DIST, Epilogue::kGeluErf, "gelu", 1),     \
       HOM_FINE_ENTRY(BM, BN, WM, WN, DIST, Epilogue::kGeluTanh, "gelutanh", 1),
+
+// "k8" behind the slabs in flight: eight wavefronts split K, each multiplies slabs of
+// 64 k of the whole tile.  One launch function serves every alignment; the entries
+// differ in what they ask for, as those of the register-staged pipeline do.
+#define HOM_KSPLIT_ENTRY(BM, BN, EPI_ENUM, EPI_STR, ACT, AL, AL_N)             \
+  {                                                                            \
+    {"hom_gfx950_mfma_f16_s16x16x32gemm_f16_" #BM "x" #BN                      \
+     "_64x2r2k8_w1x1_nn_align" #AL "_" EPI_STR,                                \
+     BM, BN, 64, 1, 1, AL, AL_N, ACT, EPI_ENUM},                               \
+        launchKsplitEntry<BM / 16, BN / 16, int(EPI_ENUM), false>,             \
+        launchKsplitEntry<BM / 16, BN / 16, int(EPI_ENUM), true>               \
+  }
+#define HOM_KSPLIT_ENTRIES(BM, BN, AL, AL_N)                                   \
+  HOM_KSPLIT_ENTRY(BM, BN, Epilogue::kLinear, "linear", 0, AL, AL_N),          \
+      HOM_KSPLIT_ENTRY(BM, BN, Epilogue::kGeluErf, "gelu", 1, AL, AL_N),       \
+      HOM_KSPLIT_ENTRY(BM, BN, Epilogue::kGeluTanh, "gelutanh", 1, AL, AL_N),
+#define HOM_KSPLIT_TILE(BM, BN)                                                \
+  HOM_KSPLIT_ENTRIES(BM, BN, 8, 2) HOM_KSPLIT_ENTRIES(BM, BN, 1, 1)
 
 // Manifest order is part of the ABI: compiled modules carry indices into it.
 // New entries go at the end of gemm_manifest.inc.

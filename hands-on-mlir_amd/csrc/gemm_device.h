@@ -1071,8 +1071,9 @@ struct LaunchPlan {
   bool callerWorkspace; // partial tiles go to a buffer the caller brought
 };
 
-template <int BM, int BN, int BK>
-Status planLaunch(const GemmProblem &pr, LaunchPlan *plan) {
+// Tiles of bm x bn, slabs of bk; a partial tile holds tileElems sums.
+inline Status planTiles(const GemmProblem &pr, int bm, int bn, int bk, int tileElems,
+                        LaunchPlan *plan) {
   GemmParams &p = plan->p;
   p.A = pr.A;
   p.B = pr.B;
@@ -1097,9 +1098,9 @@ Status planLaunch(const GemmProblem &pr, LaunchPlan *plan) {
   p.foldPieces = pr.foldPieces;
   p.foldInvN = pr.foldInvN;
   p.foldEps = pr.foldEps;
-  p.tilesM = int((pr.M + BM - 1) / BM);
-  p.tilesN = int((pr.N + BN - 1) / BN);
-  const int kTiles = int((pr.K + BK - 1) / BK);
+  p.tilesM = int((pr.M + bm - 1) / bm);
+  p.tilesN = int((pr.N + bn - 1) / bn);
+  const int kTiles = int((pr.K + bk - 1) / bk);
   int splitK = pr.splitK < 1 ? 1 : pr.splitK;
   if (splitK > kTiles)
     splitK = kTiles > 0 ? kTiles : 1;
@@ -1118,15 +1119,15 @@ Status planLaunch(const GemmProblem &pr, LaunchPlan *plan) {
   p.fullGroups = p.tilesM / kGroupM;
   p.lastRows = p.tilesM % kGroupM > 0 ? p.tilesM % kGroupM : kGroupM;
   p.cRowMagic = magicFor(uint32_t(p.cRowPeriod));
-  // (the row range a wavefront addresses with 32-bit offsets is at most BM rows)
-  p.epiMode = epilogueFastMode(p, BM);
+  // (the row range a wavefront addresses with 32-bit offsets is at most bm rows)
+  p.epiMode = epilogueFastMode(p, bm);
   p.workspace = nullptr;
   p.tileArrivals = nullptr;
   p.misplaced = nullptr;
   plan->callerWorkspace = pr.workspace != nullptr;
   if (splitK > 1) {
     const size_t wsBytes =
-        size_t(plan->nTiles) * splitK * size_t(BM) * BN * sizeof(float);
+        size_t(plan->nTiles) * splitK * size_t(tileElems) * sizeof(float);
     if (pr.workspace) {
       // caller-provided partial-tile buffer: nothing may be allocated here
       HOM_CHECK_RET(wsBytes <= pr.workspaceBytes, Status::kInvalidArgument,
@@ -1142,6 +1143,11 @@ Status planLaunch(const GemmProblem &pr, LaunchPlan *plan) {
     }
   }
   return Status::kSuccess;
+}
+
+template <int BM, int BN, int BK>
+Status planLaunch(const GemmProblem &pr, LaunchPlan *plan) {
+  return planTiles(pr, BM, BN, BK, BM * BN, plan);
 }
 
 template <typename K> Status allowLds(K kernel, int bytes, bool *done) {

@@ -51,3 +51,4 @@
 #define HOM_PIPE_TILE_D(...)
 #define HOM_FINE_TILE(...)
 #define HOM_STAGED_TILE(...)
+#define HOM_KSPLIT_TILE(...)

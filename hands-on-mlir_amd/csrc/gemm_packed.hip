@@ -29,6 +29,7 @@
 #include "cross_lane.h"
 #include "fast_div.h"
 #include "packed_args.h"
+#include "rectangles.h"
 #include "store_policy.h"
 
 #include <algorithm>
@@ -425,30 +426,6 @@ __global__ __launch_bounds__(256) void packRowsKernel(const _Float16 *__restrict
   storeWriteThrough(out + v * 8, x);
 }
 
-// What an XCD works on: chunkM x chunkN tiles, 2^xmLog XCDs along M.  Its L2 fetches
-// the operands of the rectangle once, at about 0.7 TB/s per XCD from the last-level
-// cache, which from some 500 rows on is what bounds these kernels (512 x 1024 x
-// 4096 moved 42 MB so in 7.2 us); among the splits that leave the fullest CU the
-// fewest tiles, the one that fetches least.
-struct Rectangles {
-  int xmLog, chunkM, chunkN;
-  int64_t perCu;    // tiles of the fullest CU
-  double fillBytes; // all XCDs
-};
-Rectangles chooseRectangles(int64_t M, int64_t N, int64_t K, int mb, int nb, int cus) {
-  const int64_t tilesM = (M + mb * 16 - 1) / (mb * 16), tilesN = N / (nb * 16);
-  const int64_t perXcd = std::max(1, cus / 8);
-  Rectangles best{};
-  for (int x = 0; x <= 3; x++) {
-    const int64_t cm = (tilesM + (1 << x) - 1) >> x, cn = (tilesN + (8 >> x) - 1) / (8 >> x);
-    const int64_t perCu = (cm * cn + perXcd - 1) / perXcd;
-    const double fill = 8.0 * double(cm * mb + cn * nb) * 16 * double(K) * 2;
-    if (x == 0 || perCu < best.perCu || (perCu == best.perCu && fill < best.fillBytes))
-      best = {x, int(cm), int(cn), perCu, fill};
-  }
-  return best;
-}
-
 template <int MB, int NB, int CH, bool ONCE>
 Status launchVariant(const PackedGemm &g, const PackedArgs &p, const Rectangles &r,
                      int aheadGroups, hipStream_t s) {
@@ -603,7 +580,8 @@ Status launchPackedGemm(const PackedGemm &g, hipStream_t s) {
   for (const Shape &t : shapes) {
     if (g.N % (t.nb * 16) != 0 || (t.mb * t.nb == 16 && !g.aPacked))
       continue;
-    const Rectangles r = chooseRectangles(g.M, g.N, g.K, t.mb, t.nb, cus);
+    const Rectangles r = chooseRectangles((g.M + t.mb * 16 - 1) / (t.mb * 16),
+                                          g.N / (t.nb * 16), t.mb, t.nb, g.K, cus);
     const double kb = double(t.mb + t.nb) * 16 * double(g.K) * 2 / 1024;
     const int64_t rounds = (r.perCu + t.resident - 1) / t.resident;
     // (a workgroup alone on its CU in the last round does not fetch twice as fast)

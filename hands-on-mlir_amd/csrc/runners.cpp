@@ -1,6 +1,7 @@
 #include "runners.h"
 
 #include "hom_amdgpu_runner_utils.h"
+#include "rectangles.h"
 
 #include <cerrno>
 #include <cmath>
@@ -188,6 +189,9 @@ bool kernelFits(const GemmKernelInfo &k, int cls) {
   return cls == 8 || (cls == 2 && k.alignmentN <= 2);
 }
 
+// The kernels of gemm_ksplit.h: one wavefront computes the whole tile.
+bool wavesSplitK(const GemmKernelInfo &k) { return k.wavesM * k.wavesN == 1; }
+
 // Kernel and split-K (stored into pr) the [N, K]-B path runs for a problem.
 int chooseNvteKernel(GemmProblem *pr, int64_t activation);
 
@@ -240,8 +244,8 @@ const std::vector<TileModel> &tileModels() {
 // x 2, at kL2BytesPerUs; floor = the load -> LDS -> MFMA latency chain of a
 // lone workgroup; the epilogue costs per output; split-K adds a second kernel
 // that moves the fp32 partial tiles through memory.
-void modelGemm(int64_t M, int64_t N, int64_t K, Epilogue epi, int cls,
-               int64_t *idx, int32_t *splitK) {
+double modelPipe(int64_t M, int64_t N, int64_t K, Epilogue epi, int cls,
+                 int64_t *idx, int32_t *splitK) {
   const int cus = deviceInfo().computeUnits > 0 ? deviceInfo().computeUnits : 256;
   constexpr double kLaunchUs = 3.0, kReduceLaunchUs = 2.5, kInKernelSumUs = 1.0;
   constexpr double kUsPerOutputSlab = 2.234e-5;
@@ -254,7 +258,7 @@ void modelGemm(int64_t M, int64_t N, int64_t K, Epilogue epi, int cls,
   *idx = findKernel(64, 64, 32, epi, 1); // (rows shorter than a vector)
   *splitK = 1;
   if (cls == 1 && (K < 8 || N < 8))
-    return;
+    return 0.0;
   const int slabs = int((K + 63) / 64);
   for (const TileModel &t : tileModels()) {
     const int kernel = (cls == 1 ? t.any : t.aligned)[int(epi)];
@@ -292,8 +296,110 @@ void modelGemm(int64_t M, int64_t N, int64_t K, Epilogue epi, int cls,
       }
     }
   }
+  return bestCost;
 }
 
+// The same for the kernels whose wavefronts split K (gemm_ksplit.h), as far as all
+// workgroups are resident at once; more rounds of them are never the better
+// choice.  t = first + n (slab + crowd x share of the CUs at work) + sum, n slabs
+// per workgroup, sum only with slices across workgroups; no faster than the weights
+// arrive, 57 GB/s for a CU and 6.5 TB/s for all.  Fitted to 670 timings, M = 16
+// .. 1000 x 18 pairs of N and K from 256 to 4096, launches one after the
+// other on three sets of operands in turn: 1.4 to 3.5 % off in the mean.
+double modelKsplit(int64_t M, int64_t N, int64_t K, Epilogue epi, int cls,
+                   int64_t *idx, int32_t *splitK) {
+  struct Fit {
+    double first[2], slab[2], crowd[2]; // tiles of 16 and of 32 rows
+    double sum, sumPerSlice;
+  };
+  static const Fit kVec = {{3.54, 3.95}, {0.088, 0.114}, {0.036, 0.054}, 1.35, 0.147};
+  static const Fit kDword = {{3.42, 3.55}, {0.094, 0.138}, {0.090, 0.136}, 1.05, 0.19};
+  static const Fit kOdd = {{3.15, 3.29}, {0.140, 0.194}, {0.094, 0.121}, 1.40, 0.21};
+  static const std::vector<int> kernels = [] { // (tile, alignment, epilogue)
+    std::vector<int> k;
+    for (int rows : {16, 32})
+      for (int al : {8, 1})
+        for (Epilogue e : {Epilogue::kLinear, Epilogue::kGeluErf, Epilogue::kGeluTanh})
+          k.push_back(findKernel(rows, 64, 64, e, al));
+    return k;
+  }();
+  double best = 1e300;
+  if (K < 8 || N < 8 || (K + 63) / 64 * 64 * N * 2 >= (int64_t(1) << 31))
+    return best;
+  const bool oddK = cls == 1 && K % 2 != 0, oddN = cls == 1 && N % 2 != 0;
+  const Fit &f = cls != 1 ? kVec : oddK || oddN ? kOdd : kDword;
+  const int cus = deviceInfo().computeUnits > 0 ? deviceInfo().computeUnits : 256;
+  const int64_t slabs = (K + (oddK ? 62 : 63)) / (oddK ? 63 : 64);
+  const int64_t cols = oddN ? 63 : 64;
+  for (int t = 0; t < 2; t++) {
+    const Rectangles r = chooseRectangles((M + 16 * (t + 1) - 1) / (16 * (t + 1)),
+                                          (N + cols - 1) / cols, t + 1, 4, K, cus);
+    const int64_t perXcd = int64_t(r.chunkM) * r.chunkN;
+    for (int64_t sp = 1; sp <= 16 && perXcd * sp <= cus / 8; sp++) {
+      const int64_t n = (slabs + sp - 1) / sp;
+      if (sp > 1 && n < 4)
+        break;
+      if ((slabs + n - 1) / n != sp)
+        continue;
+      const double share = double(perXcd * sp) / (cus / 8);
+      const double fetch = double(K * N + M * K) * 2 / std::min(6.5e6, 57e3 * cus * share);
+      const double cost = f.first[t] + std::max(double(n) * (f.slab[t] + f.crowd[t] * share), fetch) +
+                          (sp > 1 ? f.sum + f.sumPerSlice * double(sp) : 0.0);
+      if (cost < best) {
+        best = cost;
+        *idx = kernels[(t * 2 + (cls == 1)) * 3 + int(epi)];
+        *splitK = int32_t(sp);
+      }
+    }
+  }
+  return best;
+}
+
+// (a round of the larger tile on every CU: what modelKsplit() looks at at most)
+bool ksplitFits(int64_t M, int64_t N) {
+  const int cus = deviceInfo().computeUnits > 0 ? deviceInfo().computeUnits : 256;
+  return ((M + 31) / 32) * ((N + 63) / 64) <= cus;
+}
+
+// Which of the two: the timings of the slab pipelines in the same runs lay off
+// their model (fitted to one set of operands, aligned rows) by the lines below.
+bool ksplitPays(int64_t M, int64_t N, int64_t K, Epilogue epi, int cls,
+                double pipe, int32_t pipeSplitK, int64_t *idx, int32_t *splitK) {
+  int64_t i = -1;
+  int32_t sk = 1;
+  const double ksplit = modelKsplit(M, N, K, epi, cls, &i, &sk);
+  const double seen = cls != 1 ? (pipeSplitK == 1 ? 1.1 + 0.78 * pipe : 0.8 + pipe)
+                               : (pipeSplitK == 1 ? 1.5 * pipe - 0.3 : 1.3 * pipe + 0.6);
+  if (i < 0 || ksplit >= 0.97 * seen)
+    return false;
+  *idx = i;
+  *splitK = sk;
+  return true;
+}
+
+void modelGemm(int64_t M, int64_t N, int64_t K, Epilogue epi, int cls,
+               int64_t *idx, int32_t *splitK) {
+  const double pipe = modelPipe(M, N, K, epi, cls, idx, splitK);
+  if (ksplitFits(M, N))
+    ksplitPays(M, N, K, epi, cls, pipe, *splitK, idx, splitK);
+}
+
+} // namespace
+
+namespace {
+// A split that the library chose needs scratch memory, which a stream under capture
+// cannot allocate: in front of the first eager call, K is not split across
+// workgroups there.
+void unsplitWithoutScratch(int idx, GemmProblem *pr) {
+  const GemmKernelInfo &ki = gemmKernelInfo(idx);
+  if (pr->splitK <= 1 || pr->workspace || !wavesSplitK(ki))
+    return;
+  // (63 columns: see gemm_ksplit.h)
+  const size_t tiles = size_t((pr->M + ki.tileM - 1) / ki.tileM) *
+                       size_t((pr->N + ki.tileN - 2) / (ki.tileN - 1));
+  if (!libraryScratchReady(kWorkspace, tiles * size_t(pr->splitK) * ki.tileM * ki.tileN * sizeof(float)))
+    pr->splitK = 1;
+}
 } // namespace
 
 bool gemmPrefersNvte(int64_t M, int64_t N, int64_t K, int64_t activation) {
@@ -304,7 +410,14 @@ bool gemmPrefersNvte(int64_t M, int64_t N, int64_t K, int64_t activation) {
 bool selectGemm(int64_t M, int64_t N, int64_t K, int64_t activation,
                 int64_t *idx, int32_t *splitK, bool bIsNK) {
   const Epilogue epi = epilogueFor(activation, false);
-  if (const TunedEntry *t = findTuned(M, N, K, activation)) {
+  const TunedEntry *t = findTuned(M, N, K, activation);
+  // (the table holds kernels with slabs in sequence only)
+  if (t && ksplitFits(M, N)) {
+    modelGemm(M, N, K, epi, naturalClass(N, K), idx, splitK);
+    if (wavesSplitK(gemmKernelInfo(int(*idx))))
+      return false;
+  }
+  if (t) {
     const int nk = bIsNK ? kernelByName(t->nkKernel) : -1;
     const int i = nk >= 0 ? nk : kernelByName(t->kernel);
     if (i >= 0) {
@@ -371,6 +484,8 @@ Status runGemmManifest(int64_t rankA, void *dstA, int64_t rankB, void *dstB,
         pr.splitK--;
     }
   }
+  if (gemmNum == 0)
+    unsplitWithoutScratch(idx, &pr);
   return launchGemm(idx, pr, stream());
 }
 
@@ -440,7 +555,9 @@ Status runGemmNvte(int64_t rankA, void *dstA, bool transa, int64_t rankB,
   }
   pr.alpha = alpha;
   pr.beta = beta;
-  return launchGemm(chooseNvteKernel(&pr, activation), pr, stream());
+  const int idx = chooseNvteKernel(&pr, activation);
+  unsplitWithoutScratch(idx, &pr);
+  return launchGemm(idx, pr, stream());
 }
 
 // The two halves of the layer-norm pair (LayernormGemmRunner.h:17-361).  Both

@@ -1,4 +1,6 @@
 """Sizes off the vector width, broadcast forms and edges of the dispatch rules, against numpy and the oracle."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -166,6 +168,75 @@ def test_gemm_any_alignment(gpu, rt, oracle, tile, M, N, K):
     tb, td = odd(Bt), odd(np.zeros((1, M, N), np.float16))
     gpu.nvteGemmF16(*Mr(odd(A)).args(), False, *Mr(tb).args(), True, *Mr(td).args(), *Mr(td).args(), 0, 1.0, 0.0, 0, 0)
     np.testing.assert_allclose(host(td)[0].astype(np.float64), oracle.gemm(A[0], B[0]), rtol=1e-3, atol=1e-2)
+
+
+# the kernels whose wavefronts split K: tiles and slabs of 64 and, rows at odd elements, of 63; remainders of a vector,
+# fewer slabs than wavefronts and more than two rounds of them, slices across workgroups with a short last one.  What
+# lies around the operands is NaN: nothing read from there may reach a result, and nothing may be written there.
+@pytest.mark.parametrize("tile", ["16x64_64x2r2k8_w1x1_nn_align1", "32x64_64x2r2k8_w1x1_nn_align1"])
+@pytest.mark.parametrize("M,N,K", [(1, 8, 8), (16, 64, 64), (17, 63, 63), (33, 65, 126), (5, 127, 127), (40, 130, 1032),
+                                   (31, 66, 1150), (64, 126, 1009), (15, 1001, 777), (70, 72, 2002)])
+def test_gemm_waves_split_k(gpu, rt, oracle, monkeypatch, tile, M, N, K):
+    g = np.random.default_rng(M + N + K)
+    names = {n.rsplit("_", 1)[1]: (i + 1, n) for i, n, _, _ in rt.manifest() if f"_{tile}_" in n}
+    A, B = g.standard_normal((1, M, K)).astype(np.float16), (g.standard_normal((1, K, N)) * 0.1).astype(np.float16)
+    R, bias = g.standard_normal((1, M, N)).astype(np.float16), g.standard_normal((1, 1, N)).astype(np.float16)
+    Bt = np.ascontiguousarray(B[0].T)[None]
+    Mr = rt.MemRef.from_tensor
+    full, erf, plain = (oracle.gemm(A[0], B[0], R[0], beta=0.5),
+                        oracle.gemm(A[0], B[0], bias[0], beta=1.0, act="gelu_erf"), oracle.gemm(A[0], B[0]))
+
+    def place(a, off):  # between NaN, `off` elements behind a 256-byte boundary
+        t = torch.full((a.size + 256,), float("nan"), dtype=torch.float16, device="cuda")
+        v = t[128 + off:128 + off + a.size].view(a.shape)
+        v.copy_(torch.from_numpy(a))
+        return t, v
+
+    def check(t, v, want):
+        np.testing.assert_allclose(host(v)[0].astype(np.float64), want, rtol=1e-3, atol=1e-2)
+        assert int(torch.isnan(t).sum()) == 256
+
+    for off in (0, 1, 2):
+        (_, ta), (_, tb), (_, tr), (_, tbias), (_, tbt) = (place(x, off) for x in (A, B, R, bias, Bt))
+        for sk in (1, 2, 5):
+            t, td = place(np.zeros((1, M, N), np.float16), off)
+            gpu.cutlassGemmF16(*Mr(ta).args(), False, *Mr(tb).args(), False, *Mr(tr).args(), *Mr(td).args(), 0, 1.0,
+                               0.5, names["linear"][0], sk)
+            check(t, td, full)
+            gpu.cutlassGemmF16(*Mr(ta).args(), False, *Mr(tb).args(), False, *Mr(tbias).args(), *Mr(td).args(), 0, 1.0,
+                               1.0, names["gelu"][0], sk)
+            check(t, td, erf)
+            monkeypatch.setenv("HOM_NVTE_GEMM_KERNEL", f"{names['linear'][1]},{sk}")
+            gpu.nvteGemmF16(*Mr(ta).args(), False, *Mr(tbt).args(), True, *Mr(td).args(), *Mr(td).args(), 0, 1.0, 0.0,
+                            0, 0)
+            check(t, td, plain)
+
+
+# a first call inside a capture: a split across workgroups would need memory that cannot be allocated there
+def test_gemm_waves_split_k_first_call_captured(gpu, rt, oracle):
+    M, N, K = 33, 1001, 3001
+    idx, sk = ctypes.c_int64(), ctypes.c_int32()
+    gpu.homGemmSelect(M, N, K, 0, ctypes.byref(idx), ctypes.byref(sk))
+    assert "k8_w1x1_" in gpu.homGemmManifestName(idx.value).decode() and sk.value > 1
+    g = np.random.default_rng(3)
+    A, B = g.standard_normal((1, M, K)).astype(np.float16), (g.standard_normal((1, K, N)) * 0.1).astype(np.float16)
+    Mr = rt.MemRef.from_tensor
+    ta, tb, td = dev(A), dev(B), torch.zeros((1, M, N), dtype=torch.float16, device="cuda")
+    calls = [Mr(ta), Mr(tb), Mr(td)]
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    try:
+        gpu.homSetStream(ctypes.c_void_p(stream.cuda_stream))
+        with torch.cuda.graph(graph, stream=stream):
+            gpu.cutlassGemmF16(*calls[0].args(), False, *calls[1].args(), False, *calls[2].args(), *calls[2].args(), 0,
+                               1.0, 0.0, 0, 1)
+    finally:
+        gpu.homSetStream(None)
+    want = oracle.gemm(A[0], B[0])
+    for _ in range(3):
+        td.zero_()
+        graph.replay()
+        np.testing.assert_allclose(host(td)[0].astype(np.float64), want, rtol=1e-3, atol=1e-2)
 
 
 def fragment_order(a):
