@@ -130,6 +130,9 @@ constexpr int kEpiRowAffine = 4;
 constexpr int kEpiFoldA = 5;
 constexpr int kEpiFoldAGelu = 6;
 constexpr int kEpiFoldCStats = 7;
+// kEpiRowAffine with the column sums of B formed on the way, from the fragments
+// that the wavefronts multiply (row-major B).
+constexpr int kEpiRowAffineOwn = 8;
 
 template <int EPI> __device__ __forceinline__ float activate(float v) {
   if (EPI == int(Epilogue::kGeluErf))
@@ -590,15 +593,18 @@ foldRowStatFinish(const GemmParams &p, int m0, int tid,
 // scheme as epilogueFast (buffer descriptors per wavefront, 16-byte accesses,
 // every source vector requested before the transposition): N, ldd and ldc
 // multiples of 8, C / D 16-byte aligned, C absent or a full [M, N] matrix; the
-// host checks this.  myStat: foldRowStat() of this thread's row; the pairs of
+// host checks this.  kEpiRowAffineOwn: colAcc[j] is the sum of column l32 of block
+// column j over the k this lane has seen, `given` the rows' pairs in LDS.  myStat: foldRowStat() of this thread's row; the pairs of
 // the workgroup's BM rows meet in LDS, behind the wavefronts' accumulator
 // strips.
 template <int MI, int NI, int WTM, int WTN, int EPI, int BM, int THREADS>
 __device__ __forceinline__ void
 epilogueFold(const GemmParams &p, float16v (&acc)[MI][NI], int m0, int n0,
              int waveM, int waveN, int lane, int wave, int tid,
-             float2v myStat, unsigned char *smem) {
-  constexpr bool kFoldA = EPI == kEpiFoldA || EPI == kEpiFoldAGelu;
+             float2v myStat, unsigned char *smem, const float *colAcc = nullptr,
+             unsigned char *given = nullptr) {
+  constexpr bool kOwn = EPI == kEpiRowAffineOwn;
+  constexpr bool kFoldA = EPI == kEpiFoldA || EPI == kEpiFoldAGelu || kOwn;
   constexpr bool kFoldC = EPI == kEpiFoldCStats;
   constexpr bool kStats = EPI == kEpiFoldCStats;
   constexpr int ROW_B = WTN * 4 + 16;
@@ -611,7 +617,7 @@ epilogueFold(const GemmParams &p, float16v (&acc)[MI][NI], int m0, int n0,
   constexpr int kStripBytes = (THREADS / kWave) * 32 * ROW_B;
   constexpr int WN_ = (THREADS / kWave) / (BM / WTM); // wavefront columns
   unsigned char *mine = smem + wave * (32 * ROW_B);
-  float2v *rowStat = reinterpret_cast<float2v *>(smem + kStripBytes);
+  float2v *rowStat = reinterpret_cast<float2v *>(kOwn ? given : smem + kStripBytes);
   // (kStats) partial sums of the tile's rows per wavefront column, [BM][WN]
   float2v *tileSums = rowStat + BM;
   const int l32 = lane % 32, kb = lane / 32;
@@ -630,10 +636,10 @@ epilogueFold(const GemmParams &p, float16v (&acc)[MI][NI], int m0, int n0,
   const uint32_t colOff = n < p.N ? uint32_t(cc) * 2u : kOob;
   typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
   const bool useC = p.beta != 0.f;
-  const bool folded = p.foldStats != nullptr;
+  const bool folded = kOwn || p.foldStats != nullptr;
   // column sums of B for this lane's 8 columns (the same in every pass)
   float cs[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  if constexpr (kFoldA) {
+  if constexpr (kFoldA && !kOwn) {
     if (folded && n < p.N) {
       const float4v *src = reinterpret_cast<const float4v *>(p.colSum + n);
       const float4v a = src[0], b = src[1];
@@ -660,9 +666,29 @@ epilogueFold(const GemmParams &p, float16v (&acc)[MI][NI], int m0, int n0,
       }
   }
   __syncthreads(); // no wavefront still reads operands from the main loop's LDS
-  if (tid < BM)
+  if (!kOwn && tid < BM)
     rowStat[tid] = myStat;
+  float *colSums = reinterpret_cast<float *>(smem + kStripBytes); // (kOwn) [BN]
+  if constexpr (kOwn) {
+    // (the lanes 32 apart have the two halves of every 16 k; the wavefront rows
+    // have the same columns)
+#pragma unroll
+    for (int j = 0; j < NI; j++) {
+      const float total = colAcc[j] + __shfl_xor(colAcc[j], 32, kWave);
+      if (waveM == 0 && lane < 32)
+        colSums[waveN * WTN + j * 32 + lane] = total;
+    }
+  }
   __syncthreads();
+  if constexpr (kOwn) {
+    const float4v *src = reinterpret_cast<const float4v *>(colSums + waveN * WTN + cc);
+    const float4v a = src[0], b = src[1];
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      cs[e] = a[e];
+      cs[e + 4] = b[e];
+    }
+  }
 #pragma unroll
   for (int i = 0; i < MI; i++) {
 #pragma unroll

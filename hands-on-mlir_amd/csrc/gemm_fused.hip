@@ -109,12 +109,11 @@ FusedTile fusedTileFor(int likeKernel) {
     return {128, 32};
   return {64, 32};
 }
-template <int EPI>
-Status launchFusedTile(int likeKernel, const GemmProblem &p, hipStream_t s) {
+template <int EPI> Status launchFusedEdge(int edge, const GemmProblem &p, hipStream_t s) {
   // the folded-layer-norm epilogues run on the DMA-staged variants of the two
   // smaller tiles (the faster ones at the sizes those tiles serve)
   constexpr bool kDma = EPI >= kEpiFoldA;
-  switch (fusedTileFor(likeKernel).edge) {
+  switch (edge) {
   case 256:
     return launchPipe<256, 256, 2, 4, 1, EPI, false>(p, s);
   case 128:
@@ -124,8 +123,47 @@ Status launchFusedTile(int likeKernel, const GemmProblem &p, hipStream_t s) {
   }
 }
 
+// The pair's kernels with an epilogue of the folded layer norm: staged through
+// registers, which is the same on every box (128 x 128 tiles staged by DMA: 8 % faster
+// to 10 % slower).
+template <int EPI> Status launchPairFolded(int edge, const GemmProblem &p, hipStream_t s) {
+  if constexpr (EPI == kEpiRowAffineOwn) {
+    if (edge == 256)
+      return launchPipe<256, 256, 2, 4, 1, EPI, false>(p, s);
+    if (edge == 64)
+      return launchPipe<64, 64, 2, 2, 2, EPI, false>(p, s);
+  }
+  return launchPipe<128, 128, 2, 4, 2, EPI, false>(p, s);
+}
+template <int EPI>
+Status launchFusedTile(int likeKernel, const GemmProblem &p, hipStream_t s) {
+  return launchFusedEdge<EPI>(fusedTileFor(likeKernel).edge, p, s);
+}
+// The layer-norm pair's tile: the largest, up to `most` on a side, of which there is
+// one for ten (256) or nine (128) in sixteen CUs.  Second GEMM, 256 against 128,
+// us: 4096 x 4096 x 1024 (256 tiles of 256) 40.8 / 54.9, 4096 x 3072 x 768 (192) 28.2 / 34.1,
+// 2500 x 3072 x 1024 (120) 30.9 / 29.4; the first never gains by 256 (16384 x 768 x 768
+// 40.5 / 30.6), whose registers do not hold the source's vectors as well.
+FusedTile pairTile(const GemmProblem &p, int most) {
+  const int64_t cus = deviceInfo().computeUnits > 0 ? deviceInfo().computeUnits : 256;
+  auto tiles = [&](int64_t edge) {
+    return ((p.M + edge - 1) / edge) * ((p.N + edge - 1) / edge);
+  };
+  if (most >= 256 && tiles(256) * 16 >= cus * 10)
+    return {256, 64};
+  return tiles(128) * 16 >= cus * 9 ? FusedTile{128, 32} : FusedTile{64, 32};
+}
+
 inline bool aligned16(const void *p) {
   return (reinterpret_cast<uintptr_t>(p) & 15) == 0;
+}
+
+// What the epilogues of the folded layer norm ask for beyond fusedGemmFits(): no
+// source or a full matrix, 32-bit byte offsets inside a tile's rows.
+bool foldFits(const GemmProblem &p) {
+  return (p.beta == 0.f || (p.cRowPeriod >= p.M && p.ldc % 8 == 0 &&
+                            int64_t(256) * p.ldc * 2 < (int64_t(1) << 31))) &&
+         int64_t(256) * p.ldd * 2 < (int64_t(1) << 31);
 }
 
 } // namespace
@@ -139,15 +177,19 @@ bool fusedGemmFits(const GemmProblem &p) {
          (p.beta == 0.f || (p.C && p.ldc % 8 == 0 && aligned16(p.C)));
 }
 
-Status launchGemmRowStats(int likeKernel, const GemmProblem &p, _Float16 *var,
-                          _Float16 *mean, float eps, hipStream_t s) {
-  HOM_CHECK_RET(likeKernel >= 0 && likeKernel < gemmKernelCount() && fusedGemmFits(p),
-                Status::kInvalidArgument,
+Status launchGemmRowStats(const GemmProblem &p, _Float16 *var, _Float16 *mean, float eps,
+                          hipStream_t s) {
+  HOM_CHECK_RET(fusedGemmFits(p), Status::kInvalidArgument,
                 "gemm + row statistics: problem does not fit the fused kernels");
-  // every tile writes all of its wavefront columns, also those past N
-  const FusedTile t = fusedTileFor(likeKernel);
-  const int pieces =
-      int((p.N + t.edge - 1) / t.edge) * (t.edge / t.pieceWidth);
+  // No source or a full matrix, on 128 x 128 tiles: the epilogue of the folded
+  // layer norm with nothing folded in, which requests the source ahead of everything
+  // and adds up a tile's columns before it writes them (4096 x 1024 x 1024 17.4 -> 15.4
+  // us, 16384 x 1024 x 1024 61.0 -> 52.8, 3000 x 768 x 768 13.3 -> 11.8).  Others, a bias row
+  // or small tiles (64 x 768 x 768 8.2 / 9.1), write a partial sum per wavefront column,
+  // also of those past N.
+  const FusedTile t = pairTile(p, foldFits(p) ? 128 : 256);
+  const bool whole = t.edge == 128 && foldFits(p);
+  const int pieces = int((p.N + t.edge - 1) / t.edge) * (whole ? 1 : t.edge / t.pieceWidth);
   float *partials = static_cast<float *>(
       libraryScratch(kTemp, size_t(pieces) * size_t(p.M) * 2 * sizeof(float), false));
   if (!partials)
@@ -155,7 +197,8 @@ Status launchGemmRowStats(int likeKernel, const GemmProblem &p, _Float16 *var,
   GemmProblem q = p;
   q.splitK = 1;
   q.rowStatPartials = partials;
-  Status st = launchFusedTile<kEpiRowStats>(likeKernel, q, s);
+  Status st = whole ? launchPairFolded<kEpiFoldCStats>(t.edge, q, s)
+                    : launchFusedEdge<kEpiRowStats>(t.edge, q, s);
   if (st != Status::kSuccess)
     return st;
   rowStatsFinalizeKernel<<<dim3((unsigned)((p.M + 15) / 16)), dim3(kWave), 0,
@@ -165,14 +208,24 @@ Status launchGemmRowStats(int likeKernel, const GemmProblem &p, _Float16 *var,
   return Status::kSuccess;
 }
 
-Status launchGemmRowAffine(int likeKernel, const GemmProblem &p,
-                           const _Float16 *var, const _Float16 *mean,
+Status launchGemmRowAffine(const GemmProblem &p, const _Float16 *var, const _Float16 *mean,
                            hipStream_t s) {
-  HOM_CHECK_RET(likeKernel >= 0 && likeKernel < gemmKernelCount() && fusedGemmFits(p),
-                Status::kInvalidArgument,
+  HOM_CHECK_RET(fusedGemmFits(p), Status::kInvalidArgument,
                 "layernorm + gemm: problem does not fit the fused kernels");
-  // 128 rows of B per column-sum workgroup (four 16-byte loads per lane), at
-  // most 16 slices
+  GemmProblem q = p;
+  q.splitK = 1;
+  q.rowScale = var;
+  q.rowShift = mean;
+  const int edge = pairTile(p, 256).edge;
+  // No source or a full matrix: the column sums are formed on the way, four dot
+  // products per fragment of B in the shadow of its MFMAs; by a kernel of their own
+  // they took 4.5 us of a launch.  With the pairs kept in LDS and the epilogue of
+  // the folded layer norm, us: 64 x 768 x 768 9.2 -> 6.2, 1024 x 4096 x 1024 17.8 -> 12.8,
+  // 4096 x 4096 x 1024 43.8 -> 39.2, 16384 x 4096 x 1024 156 -> 147.
+  if (foldFits(p))
+    return launchPairFolded<kEpiRowAffineOwn>(edge, q, s);
+  // A source of another form: the column sums by a kernel of their own, 128 rows of
+  // B per workgroup (four 16-byte loads per lane), at most 16 slices.
   int slices = int((p.K + 127) / 128);
   if (slices > 16)
     slices = 16;
@@ -184,13 +237,9 @@ Status launchGemmRowAffine(int likeKernel, const GemmProblem &p,
   colSumKernel<<<dim3((unsigned)((p.N + 63) / 64), (unsigned)slices), dim3(256),
                  0, s>>>(p.B, p.ldb, int(p.K), int(p.N), kPer, colSum);
   HOM_HIP_RET(hipGetLastError(), Status::kInternal);
-  GemmProblem q = p;
-  q.splitK = 1;
-  q.rowScale = var;
-  q.rowShift = mean;
   q.colSum = colSum;
   q.colSumSlices = slices;
-  return launchFusedTile<kEpiRowAffine>(likeKernel, q, s);
+  return launchFusedEdge<kEpiRowAffine>(edge, q, s);
 }
 
 int foldedPieces(int likeKernel, int64_t N) {

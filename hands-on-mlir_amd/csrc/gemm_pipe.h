@@ -369,7 +369,16 @@ __global__ __launch_bounds__(WM *WN *kWave) void gemmPipeKernel(
   constexpr bool kFoldEarly = BM >= 128;
   float2v foldRaw[EPI >= kEpiFoldA ? FoldBatch<BM>::value : 1];
   float2v foldStat{1.f, 0.f};
-  if constexpr (EPI >= kEpiFoldA) {
+  constexpr bool kOwnColSums = EPI == kEpiRowAffineOwn;
+  static_assert(!kOwnColSums || !B_NK, "column sums from the fragments of a row-major B");
+  if constexpr (kOwnColSums) {
+    // (into LDS behind the slabs: 256 x 256 tiles have no registers to keep them in)
+    if (tid < BM) {
+      const int m = m0 + tid < p.M ? m0 + tid : p.M - 1;
+      reinterpret_cast<float2v *>(smem + NBUF * STAGE_BYTES)[tid] =
+          float2v{float(p.rowScale[m]), float(p.rowShift[m])};
+    }
+  } else if constexpr (EPI >= kEpiFoldA) {
     foldRowStatRequest<BM>(p, m0, tid, foldRaw);
     if constexpr (kFoldEarly) {
       foldStat = foldRowStatFinish<BM>(p, m0, tid, foldRaw);
@@ -385,6 +394,17 @@ __global__ __launch_bounds__(WM *WN *kWave) void gemmPipeKernel(
 #pragma unroll
       for (int e = 0; e < 16; e++)
         acc[i][j][e] = 0.f;
+  float colAcc[NI] = {}; // (kOwnColSums)
+  auto addColumns = [&](half8 (&b)[NI]) {
+    if constexpr (kOwnColSums) {
+      const half2v one = {_Float16(1), _Float16(1)};
+#pragma unroll
+      for (int j = 0; j < NI; j++)
+#pragma unroll
+        for (int e = 0; e < 8; e += 2)
+          colAcc[j] = __builtin_amdgcn_fdot2(half2v{b[j][e], b[j][e + 1]}, one, colAcc[j], false);
+    }
+  };
 
   // ---- fragment addresses: a few per-lane bases, the rest are immediates ----
   // K-contiguous tiles: the swizzle term (row >> 1) & 7 only involves bits of
@@ -587,6 +607,7 @@ __global__ __launch_bounds__(WM *WN *kWave) void gemmPipeKernel(
     constexpr int NR = RD ? MI + NI : 0;
     constexpr int N = NR + (V1 - V0);
     tieFragments(a, b, allowC);
+    addColumns(b);
     staticFor<NM>([&](auto mC) {
       constexpr int m = decltype(mC)::value;
       if constexpr (N > 0) {
@@ -733,6 +754,7 @@ __global__ __launch_bounds__(WM *WN *kWave) void gemmPipeKernel(
     for (int kk = 0; kk < KSTEPS; kk++) {
       loadFrags(0, kk, fa[0], fb[0]);
       tieFragments(fa[0], fb[0], TieNow{});
+      addColumns(fb[0]);
 #pragma unroll
       for (int m = 0; m < NM; m++)
         acc[m / NI][m % NI] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
@@ -802,11 +824,12 @@ __global__ __launch_bounds__(WM *WN *kWave) void gemmPipeKernel(
                 "epilogue strips (and the row statistics of the folded "
                 "epilogues behind them) must fit the main loop's LDS");
   if constexpr (EPI >= kEpiFoldA) {
-    if constexpr (!kFoldEarly)
+    if constexpr (!kFoldEarly && !kOwnColSums)
       foldStat = foldRowStatFinish<BM>(p, m0, tid, foldRaw);
     epilogueFold<MI, NI, WTM, WTN, EPI, BM, THREADS>(p, acc, m0, n0, waveM,
                                                      waveN, lane, wave, tid,
-                                                     foldStat, smem);
+                                                     foldStat, smem, colAcc,
+                                                     smem + NBUF * STAGE_BYTES);
   } else if (numSlices > 1) {
     storePartial<MI, NI, THREADS>(p, acc, tile, slice, numSlices, tid);
     if constexpr (EPI < kEpiRowStats) {
@@ -828,7 +851,8 @@ template <int BM, int BN, int WM, int WN, int DIST, int EPI, bool B_NK,
           bool DMA = false, bool ANY = false>
 Status launchPipe(const GemmProblem &pr, hipStream_t s) {
   static_assert(!ANY || !DMA, "DMA staging needs aligned rows");
-  constexpr int SMEM = (DMA ? DIST + 1 : 2) * (BM + BN) * 64 * 2;
+  constexpr int SMEM = (DMA ? DIST + 1 : 2) * (BM + BN) * 64 * 2 +
+                       (EPI == kEpiRowAffineOwn ? BM * 8 : 0);
   static_assert(!DMA || ((BM * 8) % (WM * WN * kWave) == 0 &&
                          (BN * 8) % (WM * WN * kWave) == 0 &&
                          (B_NK || 1024 % (BN * 2) == 0 || (BN * 2) % 1024 == 0)),

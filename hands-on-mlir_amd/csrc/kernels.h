@@ -139,20 +139,18 @@ Status noAllocWorkspace(float **ptr, size_t *bytes);
 
 // The layer-norm pair with the normalisation folded into the two GEMMs'
 // epilogues.  Both need the vector alignment class (K, N and the leading
-// dimensions multiples of 8, B row-major) -- fusedGemmFits() says whether a
-// problem qualifies -- and `likeKernel`, a manifest index whose tile size they
-// imitate.
+// dimensions multiples of 8, B row-major): fusedGemmFits() says whether a problem
+// qualifies.
 bool fusedGemmFits(const GemmProblem &p);
 // D = alpha A B + beta C, plus per-row statistics of the stored D:
 // var[m] = 1 / sqrt(E[d^2] - E[d]^2 + eps), mean[m] = -E[d] * var[m]
 // (the statistic is accumulated in the epilogue, a second small kernel turns
 // the per-tile partial sums into var / mean).
-Status launchGemmRowStats(int likeKernel, const GemmProblem &p, _Float16 *var,
-                          _Float16 *mean, float eps, hipStream_t s);
+Status launchGemmRowStats(const GemmProblem &p, _Float16 *var, _Float16 *mean, float eps,
+                          hipStream_t s);
 // D = alpha (A * var[m] + mean[m]) B + beta C, computed as
 // alpha (var[m] (A B) + mean[m] colsum(B)) + beta C.
-Status launchGemmRowAffine(int likeKernel, const GemmProblem &p,
-                           const _Float16 *var, const _Float16 *mean,
+Status launchGemmRowAffine(const GemmProblem &p, const _Float16 *var, const _Float16 *mean,
                            hipStream_t s);
 
 // A layer norm without affine parameters folded into the GEMMs around it (no

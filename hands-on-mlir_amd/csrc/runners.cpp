@@ -587,10 +587,7 @@ Status runGemmWithVarMean(int64_t rankA, void *dstA, int64_t rankB, void *dstB,
   pr.alpha = alpha;
   pr.beta = beta;
   if (fusedGemmFits(pr)) {
-    int64_t like;
-    int32_t sk;
-    selectGemm(pr.M, pr.N, pr.K, 0, &like, &sk);
-    return launchGemmRowStats(int(like), pr, Var.data, Mean.data, eps, stream());
+    return launchGemmRowStats(pr, Var.data, Mean.data, eps, stream());
   }
   st = runGemmManifest(rankA, dstA, rankB, dstB, rankC, dstC, rankD, dstD, 0,
                        alpha, beta, 0, 1);
@@ -872,10 +869,7 @@ Status runLayernormGemm(int64_t rankA, void *dstA, int64_t rankB, void *dstB,
   pr.alpha = alpha;
   pr.beta = beta;
   if (fusedGemmFits(pr)) {
-    int64_t like;
-    int32_t sk;
-    selectGemm(pr.M, pr.N, pr.K, 0, &like, &sk);
-    return launchGemmRowAffine(int(like), pr, Var.data, Mean.data, stream());
+    return launchGemmRowAffine(pr, Var.data, Mean.data, stream());
   }
   HOM_CHECK_RET(A.contiguous(), Status::kInvalidArgument,
                 "layernorm-gemm: A must be a contiguous rank-3 tensor");

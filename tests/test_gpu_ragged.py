@@ -212,6 +212,38 @@ def test_gemm_waves_split_k(gpu, rt, oracle, monkeypatch, tile, M, N, K):
             check(t, td, plain)
 
 
+# both halves of the layer-norm pair on each of their tiles (64, 128 and 256 on a side, ragged rows, columns and K),
+# without a source, with a bias row (column sums and row sums by the general epilogue) and with a full matrix
+@pytest.mark.parametrize("M,N,K", [(70, 136, 72), (1100, 2056, 200), (4100, 2568, 136)])
+@pytest.mark.parametrize("source", ["none", "bias", "full"])
+def test_layernorm_pair_tiles_and_sources(gpu, rt, M, N, K, source):
+    g = torch.Generator(device="cuda").manual_seed(M)
+    rand = lambda *s: torch.randn(*s, generator=g, device="cuda")  # noqa: E731
+    A, B = rand(1, M, K).half(), (rand(1, K, N) * 0.1).half()
+    var, mean = (1 + 0.2 * rand(1, M, 1)).half(), (0.5 * rand(1, M, 1)).half()
+    D = torch.zeros(1, M, N, dtype=torch.float16, device="cuda")
+    C = {"none": D, "bias": rand(1, 1, N).half(), "full": rand(1, M, N).half()}[source]
+    beta = 0.0 if source == "none" else 0.75
+    add = 0.0 if source == "none" else beta * C[0].double()
+    Mr = rt.MemRef.from_tensor
+    gpu.cutlassLayernormGemmF16(*Mr(A).args(), *Mr(B).args(), *Mr(C).args(), *Mr(D).args(), *Mr(var).args(),
+                                *Mr(mean).args(), 1.5, beta, 0)
+    want = 1.5 * ((A[0].double() * var[0].double() + mean[0].double()) @ B[0].double()) + add
+    # half a unit of the fp16 result; fp32 sums of K products and of K column values, a few units of their sizes
+    np.testing.assert_allclose(host(D)[0].astype(np.float64), want.cpu().numpy(), rtol=2**-10, atol=2e-3)
+    v, m = torch.zeros_like(var), torch.zeros_like(mean)
+    D.zero_()
+    gpu.cutlassGemmWithVarMeanF16(*Mr(A).args(), *Mr(B).args(), *Mr(C).args(), *Mr(D).args(), *Mr(v).args(),
+                                  *Mr(m).args(), 1.5, beta, 0, 1e-6)
+    want = 1.5 * (A[0].double() @ B[0].double()) + add
+    np.testing.assert_allclose(host(D)[0].astype(np.float64), want.cpu().numpy(), rtol=2**-10, atol=2e-3)
+    x = D[0].double()  # the statistics are those of the stored values
+    rstd = 1 / torch.sqrt(x.var(1, unbiased=False) + 1e-6)
+    np.testing.assert_allclose(host(v)[0, :, 0].astype(np.float64), rstd.cpu().numpy(), rtol=2**-10)
+    np.testing.assert_allclose(host(m)[0, :, 0].astype(np.float64), (-x.mean(1) * rstd).cpu().numpy(), rtol=2**-10,
+                               atol=1e-5)
+
+
 # a first call inside a capture: a split across workgroups would need memory that cannot be allocated there
 def test_gemm_waves_split_k_first_call_captured(gpu, rt, oracle):
     M, N, K = 33, 1001, 3001
