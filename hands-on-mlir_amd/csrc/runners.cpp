@@ -234,6 +234,55 @@ const std::vector<TileModel> &tileModels() {
   return models;
 }
 
+// More 64 x 64 tiles than CUs: K is not split, and the tiles differ by what a round
+// of them costs beyond its slabs, above all where all CUs write (and read a full
+// source) at once.  t = fixed + rounds (slab K / 64 + round + gelu + source) + out M N +
+// outSource M N + traffic of all tiles, us; a round is a tile on every CU.  Fitted to
+// 198 problems x 7 tiles, M = 500 .. 16384, N and K = 256 .. 4096, three sets of
+// operands in turn: 3 to 5 % off in the mean, the choice 0.8 % off the best (the
+// model below: 2.9 %; 15068 x 896 x 960 with a source 47.5 -> 38.6 us, 4813 x 3072 x 320
+// 29.6 -> 21.4).
+bool modelFullChip(int64_t M, int64_t N, int64_t K, Epilogue epi, int cls, bool fullSource,
+                   int64_t *idx, int32_t *splitK) {
+  struct Fit {
+    double fixed, slab, round, gelu, source, out, outSource, traffic;
+  };
+  static const Fit fits[] = { // in the order of tileModels()
+      {1.96, 0.118, 0.558, 0.152, 0, 0, 0.226, 0.0213},
+      {2.94, 0.201, 0, 0.313, 0, 0.362, 0.201, 0.0199},
+      {2.82, 0.190, 0, 0.379, 0.087, 0.339, 0.150, 0.0222},
+      {1.24, 0.281, 2.30, 0.704, 0.139, 0, 0.176, 0.0321},
+      {0, 0.468, 4.49, 2.00, 0.687, 0.075, 0.134, 0.0321},
+      {0, 0.455, 4.46, 1.96, 0.887, 0.0814, 0.108, 0.0346},
+      {0, 0.865, 9.23, 4.75, 2.78, 0.228, 0.427, 0.0332},
+  };
+  const int cus = deviceInfo().computeUnits > 0 ? deviceInfo().computeUnits : 256;
+  if (cls == 1 || ((M + 63) / 64) * ((N + 63) / 64) <= cus)
+    return false;
+  double best = 1e300;
+  const double outputs = double(M) * double(N) * 1e-6, slabs = double((K + 63) / 64);
+  for (size_t t = 0; t < tileModels().size(); t++) {
+    const TileModel &m = tileModels()[t];
+    const Fit &f = fits[t];
+    const int kernel = m.aligned[int(epi)];
+    if (kernel < 0)
+      continue;
+    const double tiles = double((M + m.tileM - 1) / m.tileM) * double((N + m.tileN - 1) / m.tileN);
+    const double traffic = tiles * (m.tileM + m.tileN) * double(K) * 2e-6;
+    const double cost =
+        f.fixed +
+        std::ceil(tiles / cus) * (f.slab * slabs + f.round + (epi == Epilogue::kLinear ? 0 : f.gelu) +
+                                  (fullSource ? f.source : 0)) +
+        (f.out + (fullSource ? f.outSource : 0)) * outputs + f.traffic * traffic;
+    if (cost < best) {
+      best = cost;
+      *idx = kernel;
+      *splitK = 1;
+    }
+  }
+  return best < 1e300;
+}
+
 // Kernel and split-K for an untuned shape of alignment class cls, from a timing
 // model of the register-staged kernels, fitted to measurements of every tile
 // over BERT-base / BERT-large sized problems (it reproduces them within 10 %):
@@ -377,8 +426,10 @@ bool ksplitPays(int64_t M, int64_t N, int64_t K, Epilogue epi, int cls,
   return true;
 }
 
-void modelGemm(int64_t M, int64_t N, int64_t K, Epilogue epi, int cls,
+void modelGemm(int64_t M, int64_t N, int64_t K, Epilogue epi, int cls, bool fullSource,
                int64_t *idx, int32_t *splitK) {
+  if (modelFullChip(M, N, K, epi, cls, fullSource, idx, splitK))
+    return;
   const double pipe = modelPipe(M, N, K, epi, cls, idx, splitK);
   if (ksplitFits(M, N))
     ksplitPays(M, N, K, epi, cls, pipe, *splitK, idx, splitK);
@@ -408,12 +459,12 @@ bool gemmPrefersNvte(int64_t M, int64_t N, int64_t K, int64_t activation) {
 }
 
 bool selectGemm(int64_t M, int64_t N, int64_t K, int64_t activation,
-                int64_t *idx, int32_t *splitK, bool bIsNK) {
+                int64_t *idx, int32_t *splitK, bool bIsNK, bool fullSource) {
   const Epilogue epi = epilogueFor(activation, false);
   const TunedEntry *t = findTuned(M, N, K, activation);
   // (the table holds kernels with slabs in sequence only)
   if (t && ksplitFits(M, N)) {
-    modelGemm(M, N, K, epi, naturalClass(N, K), idx, splitK);
+    modelGemm(M, N, K, epi, naturalClass(N, K), fullSource, idx, splitK);
     if (wavesSplitK(gemmKernelInfo(int(*idx))))
       return false;
   }
@@ -426,7 +477,7 @@ bool selectGemm(int64_t M, int64_t N, int64_t K, int64_t activation,
       return true;
     }
   }
-  modelGemm(M, N, K, epi, naturalClass(N, K), idx, splitK);
+  modelGemm(M, N, K, epi, naturalClass(N, K), fullSource, idx, splitK);
   return false;
 }
 
@@ -465,10 +516,11 @@ Status runGemmManifest(int64_t rankA, void *dstA, int64_t rankB, void *dstB,
                   "gemm: negative kernel number %d", gemmNum);
     int64_t sel;
     int32_t sk;
-    selectGemm(pr.M, pr.N, pr.K, activation, &sel, &sk);
+    const bool fullSource = beta != 0.f && pr.cRowPeriod > 1;
+    selectGemm(pr.M, pr.N, pr.K, activation, &sel, &sk, false, fullSource);
     const int cls = alignmentClass(pr);
     if (!kernelFits(gemmKernelInfo(int(sel)), cls))
-      modelGemm(pr.M, pr.N, pr.K, gemmKernelInfo(int(sel)).epilogue, cls, &sel,
+      modelGemm(pr.M, pr.N, pr.K, gemmKernelInfo(int(sel)).epilogue, cls, fullSource, &sel,
                 &sk);
     idx = int(sel);
     pr.splitK = sk;
@@ -518,7 +570,7 @@ int chooseNvteKernel(GemmProblem *pr, int64_t activation) {
   }
   const int cls = alignmentClass(*pr);
   if (!kernelFits(gemmKernelInfo(idx), cls)) {
-    modelGemm(pr->M, pr->N, pr->K, epi, cls, &sel, &sk);
+    modelGemm(pr->M, pr->N, pr->K, epi, cls, false, &sel, &sk);
     idx = int(sel);
     pr->splitK = sk;
   }

@@ -61,9 +61,10 @@ Status runColumnSums(int64_t rankB, void *dstB, float *out);
 
 // Kernel choice without timing: tuned table first, heuristic otherwise.
 // `activation`: 0 linear, 1 GELU (erf), 2 GELU (tanh).  Returns true when the
-// shape was found in the tuned table.
+// shape was found in the tuned table.  fullSource: beta C reads as much as D writes.
 bool selectGemm(int64_t M, int64_t N, int64_t K, int64_t activation,
-                int64_t *idx, int32_t *splitK, bool bIsNK = false);
+                int64_t *idx, int32_t *splitK, bool bIsNK = false,
+                bool fullSource = false);
 // What nvteGemmF16 runs for a shape (B as [N, K]; activation 1 is the tanh
 // form there), before the per-call alignment fallback.
 bool selectGemmNvte(int64_t M, int64_t N, int64_t K, int64_t activation,
