@@ -6,6 +6,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <stdint.h>
 
 namespace hom {
 
@@ -42,6 +43,23 @@ __device__ __forceinline__ float pairSum(float v) {
   const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v),
                                                   __float_as_uint(v), false, false);
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+// Two lanes l, l ^ 32 that each hold half of two 16-byte vectors (dwords even0, even1 of the
+// one, odd0, odd1 of the other; the lower lane the lower half): the lower lane gets
+// the even vector, the upper one the odd.
+typedef uint32_t lanes4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ lanes4 joinHalves(uint32_t even0, uint32_t even1, uint32_t odd0,
+                                             uint32_t odd1) {
+  const auto a = __builtin_amdgcn_permlane32_swap(even0, odd0, false, false);
+  const auto b = __builtin_amdgcn_permlane32_swap(even1, odd1, false, false);
+  return lanes4{a[0], b[0], a[1], b[1]};
+}
+// The way back: a lane has the even (lower lane) or odd vector v and gets the dwords
+// even0, even1, odd0, odd1 of its half.
+__device__ __forceinline__ lanes4 splitHalves(lanes4 v) {
+  const auto a = __builtin_amdgcn_permlane32_swap(v[0], v[2], false, false);
+  const auto b = __builtin_amdgcn_permlane32_swap(v[1], v[3], false, false);
+  return lanes4{a[0], b[0], a[1], b[1]};
 }
 // v_permlane16_swap exchanges the odd rows of its first operand with the even
 // rows of its second: the same value twice gives (even-row values, odd-row

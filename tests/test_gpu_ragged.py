@@ -427,6 +427,28 @@ def test_encoder_many_rows_equals_row_major(synth, bs, seq):
     np.testing.assert_allclose(got[0][live], got[1][live], rtol=1e-2, atol=1e-2)
 
 
+# the result is stored 16 bytes a lane from any 8-byte boundary: the same values there, padding rows included, and
+# nothing beside them (each way of the dispatch)
+@pytest.mark.parametrize("bs,seq,heads,d", [(1, 50, 2, 64), (3, 100, 4, 64), (30, 128, 12, 64), (2, 300, 4, 64),
+                                            (2, 200, 4, 128), (3, 130, 3, 192), (2, 70, 2, 256), (8, 384, 16, 256)])
+def test_attention_result_on_8_bytes(gpu, rt, bs, seq, heads, d):
+    g = torch.Generator(device="cuda").manual_seed(seq)
+    qkv = torch.randn(bs, seq, 3 * heads * d, generator=g, device="cuda").half()
+    lens = torch.randint(1, seq + 1, (bs,), generator=g, device="cuda")
+    cu = torch.zeros(bs + 1, dtype=torch.int32, device="cuda")
+    cu[1:] = torch.cumsum(lens, 0)
+    n, Mr, results = bs * seq * heads * d, rt.MemRef.from_tensor, []
+    for off in (0, 4):
+        t = torch.full((n + 64,), float("nan"), dtype=torch.float16, device="cuda")
+        out = t[32 + off:32 + off + n].view(bs, seq, heads * d)
+        gpu.nvteBertAttentionF16(*Mr(qkv).args(), *Mr(cu).args(), *Mr(out).args(), d ** -0.5, heads)
+        results.append(host(out))
+        assert int(torch.isnan(t).sum()) == 64
+    np.testing.assert_array_equal(results[0], results[1])
+    for b in range(bs):
+        assert not results[0][b, int(lens[b]):].any()
+
+
 # every way the attention is split, lengths around its chunk ends; what lies behind a sequence must not matter
 @pytest.mark.parametrize("bs,seq,heads,d", [(2, 60, 4, 64), (3, 100, 4, 64), (30, 128, 12, 64), (2, 300, 4, 64),
                                             (40, 200, 8, 64), (2, 64, 4, 128), (3, 130, 4, 128), (40, 256, 8, 128),
