@@ -299,14 +299,16 @@ __global__ __launch_bounds__(WM *WN *kWave, NBUF *(BM + BN) * SB > 1280 ? 1 : WM
     const int wideBlocks = p.N / 32; // 32-column blocks of C and D
     const int block0 = tm * kBlocksA + waveM * (WTM / 16) + l32 / 16;
     const int col0 = (tn * BN + waveN * WTN) / 32;
-    const uint32_t laneOff = uint32_t(lane % 16) * 16u + uint32_t(kb) * 8u;
+    // ... in accumulator order; lane and lane ^ 32 swap halves, so that each loads and
+    // stores whole 16 bytes, of the even (kb = 0) or odd g.
+    const uint32_t laneOff = uint32_t(lane % 16) * 16u + uint32_t(kb) * 256u;
     const uint32_t bytesCD = uint32_t(rowBlocks) * uint32_t(wideBlocks) * 1024u;
     const auto rsrcD = __builtin_amdgcn_make_buffer_rsrc(p.D, 0, int32_t(bytesCD), 0x00020000);
     auto offsetOf = [&](int i, int j) {
       return (uint32_t(block0 + 2 * i) * uint32_t(wideBlocks) + uint32_t(col0 + j)) * 1024u +
              laneOff;
     };
-    half4 cv[SRC ? MI : 1][SRC ? NI : 1][4];
+    lanes4 cw[SRC ? MI : 1][SRC ? NI : 1][2];
     float2v rowStat[MI];
     float4v cs[NORM_A ? NI : 1][4];
     if constexpr (SRC) {
@@ -317,10 +319,9 @@ __global__ __launch_bounds__(WM *WN *kWave, NBUF *(BM + BN) * SB > 1280 ? 1 : WM
 #pragma unroll
         for (int j = 0; j < NI; j++)
 #pragma unroll
-          for (int g = 0; g < 4; g++)
-            cv[i][j][g] = __builtin_bit_cast(
-                half4, __builtin_amdgcn_raw_buffer_load_b64(
-                           rsrcC, col0 + j < wideBlocks ? offsetOf(i, j) + g * 256u : kOob, 0, 0));
+          for (int g = 0; g < 2; g++)
+            cw[i][j][g] = __builtin_amdgcn_raw_buffer_load_b128(
+                rsrcC, col0 + j < wideBlocks ? offsetOf(i, j) + g * 512u : kOob, 0, 0);
 #pragma unroll
       for (int i = 0; i < MI; i++) {
         rowStat[i] = float2v{1.f, 0.f};
@@ -391,27 +392,33 @@ __global__ __launch_bounds__(WM *WN *kWave, NBUF *(BM + BN) * SB > 1280 ? 1 : WM
 #pragma unroll
       for (int i = 0; i < MI; i++)
 #pragma unroll
-        for (int g = 0; g < 4; g++) {
-          half4 o;
+        for (int g = 0; g < 4; g += 2) {
+          half4 o[2];
+          [[maybe_unused]] half8 c = {}; // g, then g + 1
+          if constexpr (SRC)
+            c = __builtin_bit_cast(half8, splitHalves(cw[i][j][g / 2]));
 #pragma unroll
-          for (int e = 0; e < 4; e++) {
-            float x = acc[i][j][4 * g + e];
-            if constexpr (NORM_A)
-              x = fmaf(rowStat[i][0], x, rowStat[i][1] * cs[j][g][e]);
-            if constexpr (ACT == 1)
-              x = geluErf(x);
-            if constexpr (ACT == 2)
-              x = geluTanh(x);
-            if constexpr (SRC)
-              x += float(_Float16(fmaf(float(cv[i][j][g][e]), rowStat[i][0], rowStat[i][1])));
-            o[e] = _Float16(x);
-          }
+          for (int h = 0; h < 2; h++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+              float x = acc[i][j][4 * (g + h) + e];
+              if constexpr (NORM_A)
+                x = fmaf(rowStat[i][0], x, rowStat[i][1] * cs[j][g + h][e]);
+              if constexpr (ACT == 1)
+                x = geluErf(x);
+              if constexpr (ACT == 2)
+                x = geluTanh(x);
+              if constexpr (SRC)
+                x += float(_Float16(fmaf(float(c[4 * h + e]), rowStat[i][0], rowStat[i][1])));
+              o[h][e] = _Float16(x);
+            }
           // (written through, see store_policy.h: a wavefront's store is whole runs of
           // 256 bytes.  BERT-base 32 x 128 1430 -> 1379 us, 8 x 128 597 -> 585,
           // BERT-large 32 x 512 11.54 -> 11.42 ms)
           typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
-          __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, o), rsrcD,
-                                                offsetOf(i, j) + g * 256u, 0, kWriteThroughAux);
+          const u32x2 even = __builtin_bit_cast(u32x2, o[0]), odd = __builtin_bit_cast(u32x2, o[1]);
+          __builtin_amdgcn_raw_buffer_store_b128(joinHalves(even[0], even[1], odd[0], odd[1]), rsrcD,
+                                                 offsetOf(i, j) + g * 256u, 0, kWriteThroughAux);
         }
     }
   }
