@@ -35,8 +35,11 @@ namespace gemmk {
 // with the scalar staging of gemm_staged.h, 9.9 us this way (1000 x 1000 x 1000
 // on the aligned kernel: 7.9 us; a misaligned vector touches two cache lines);
 // 16000 x 4095 x 1023 with bias and GELU 1432 -> 208 us.
+//
+// EARLY == true (register-staged 64 x 64 tiles): the partial slab of a ragged K is
+// requested ahead of the full ones, see below.
 template <int BM, int BN, int WM, int WN, int DIST, int EPI, bool B_NK,
-          bool DMA = false, bool ANY = false>
+          bool DMA = false, bool ANY = false, bool EARLY = false>
 __global__ __launch_bounds__(WM *WN *kWave) void gemmPipeKernel(
     const _Float16 *argA, const _Float16 *argB, int argM, int argN, int argK,
     int argLda, int argLdb, int argTilesN, int argXcdQ, uint32_t argTileWalk,
@@ -86,7 +89,7 @@ __global__ __launch_bounds__(WM *WN *kWave) void gemmPipeKernel(
   // to the first memory request and back counts as much as the main loop;
   // larger tiles keep the order that suits their register budget.
   constexpr bool kLatencyFirst = BM * BN <= 128 * 128;
-  constexpr bool kTailFirst = BM * BN <= 64 * 64; // the partial slab's requests
+  static_assert(!EARLY || (kLatencyFirst && !DMA), "an early partial slab: small staged tiles");
 
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
 
@@ -208,7 +211,7 @@ __global__ __launch_bounds__(WM *WN *kWave) void gemmPipeKernel(
   }
 
   half8 regA[DMA ? 1 : DIST][A_PER_T], regB[DMA ? 1 : DIST][B_PER_T];
-  half8 tailA[A_PER_T], tailB[B_PER_T]; // the partial slab
+  half8 earlyA[EARLY ? A_PER_T : 1], earlyB[EARLY ? B_PER_T : 1]; // the partial slab
   // Slabs of this slice that lie inside [0, kEnd) entirely, and whether a
   // partial one follows them (only the last slice of a ragged K has one).
   const int kFullEnd = ANY && !B_NK && kEnd == p.K ? kEnd - 1 : kEnd;
@@ -270,21 +273,22 @@ __global__ __launch_bounds__(WM *WN *kWave) void gemmPipeKernel(
   };
   // The partial slab, behind the full ones, with a range test per vector.  ANY:
   // elements of a vector inside the range: none, 8, or the last 1..7, which are
-  // read ending at the last one and shifted down when they are needed.
+  // read ending at the last one and shifted down (EARLY: when they are needed).
   auto tailInside = [&](bool isA, int i) -> int {
     const int k = (ktBegin + nkFull) * BK + (isA ? aK[i] : bK[i]);
     if (isA || B_NK)
       return kEnd - k;
     return k < kEnd ? p.N - (n0 + (tid + i * THREADS) % B_VPR * 8) : 0;
   };
-  auto loadTail = [&]() {
+  auto loadTail = [&](half8 (&tailA)[A_PER_T], half8 (&tailB)[B_PER_T]) {
     const int k0 = (ktBegin + nkFull) * BK;
     if constexpr (ANY) {
       auto fetch = [&](auto rsrc, uint32_t off, int inside) {
         const int back = inside > 0 && inside < 8 ? 8 - inside : 0;
-        return __builtin_bit_cast(
+        const half8 v = __builtin_bit_cast(
             half8, __builtin_amdgcn_raw_buffer_load_b128(
                        rsrc, inside > 0 ? off - uint32_t(back) * 2u : kOob, 0, 0));
+        return !EARLY && back > 0 ? shiftDown(v, inside) : v;
       };
 #pragma unroll
       for (int i = 0; i < A_PER_T; i++)
@@ -330,13 +334,15 @@ __global__ __launch_bounds__(WM *WN *kWave) void gemmPipeKernel(
   };
 
   // Small tiles: the first DIST slabs are requested before anything else is
-  // set up.  The smallest request the partial slab even ahead of them, into
-  // registers of its own: it is multiplied last, where its round trip to memory
-  // would stand alone (1000 x 1001 x 1003 11.0 -> 10.5 us, 600 x 600 x 600 5.1 -> 4.95; 128 x
-  // 128 tiles lose up to 3 % by it: 900 x 2312 x 600 9.4 -> 9.8).
+  // set up.  EARLY requests the partial slab even ahead of them, into registers of
+  // its own: it is multiplied last, where its round trip to memory would stand
+  // alone.  Those registers live through the main loop and cost a third wavefront
+  // per SIMD (144 -> 160), which is why launchPipe() has it only where the grid
+  // does not fill two.
   if constexpr (kLatencyFirst) {
-    if (kTailFirst && hasTail)
-      loadTail();
+    if constexpr (EARLY)
+      if (hasTail)
+        loadTail(earlyA, earlyB);
     if (nkFull > 0) {
       staticFor<DIST>(
           [&](auto d) { loadGlobal(ktBegin + decltype(d)::value, d); });
@@ -735,20 +741,24 @@ __global__ __launch_bounds__(WM *WN *kWave) void gemmPipeKernel(
   auto raggedSlab = [&]() {
     if constexpr (DMA) // nothing may still be on its way into buffer 0
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    if constexpr (!kTailFirst)
-      loadTail();
-    __syncthreads(); // no wavefront still reads a full slab from buffer 0
-    if constexpr (ANY) {
+    if constexpr (EARLY) {
+      __syncthreads(); // no wavefront still reads a full slab from buffer 0
+      if constexpr (ANY) {
 #pragma unroll
-      for (int i = 0; i < A_PER_T; i++)
-        if (tailInside(true, i) > 0 && tailInside(true, i) < 8)
-          tailA[i] = shiftDown(tailA[i], tailInside(true, i));
+        for (int i = 0; i < A_PER_T; i++)
+          if (tailInside(true, i) > 0 && tailInside(true, i) < 8)
+            earlyA[i] = shiftDown(earlyA[i], tailInside(true, i));
 #pragma unroll
-      for (int i = 0; i < B_PER_T; i++)
-        if (tailInside(false, i) > 0 && tailInside(false, i) < 8)
-          tailB[i] = shiftDown(tailB[i], tailInside(false, i));
+        for (int i = 0; i < B_PER_T; i++)
+          if (tailInside(false, i) > 0 && tailInside(false, i) < 8)
+            earlyB[i] = shiftDown(earlyB[i], tailInside(false, i));
+      }
+      storeLds(0, earlyA, earlyB);
+    } else {
+      loadTail(regA[0], regB[0]);
+      __syncthreads(); // no wavefront still reads a full slab from buffer 0
+      storeLds(0, regA[0], regB[0]);
     }
-    storeLds(0, tailA, tailB);
     __syncthreads();
 #pragma unroll
     for (int kk = 0; kk < KSTEPS; kk++) {
@@ -868,27 +878,54 @@ Status launchPipe(const GemmProblem &pr, hipStream_t s) {
   HOM_CHECK_RET((int64_t(BM) * pr.lda + pr.K) * 2 < (int64_t(1) << 31) &&
                     (int64_t(BN) * pr.ldb + pr.K) * 2 < (int64_t(1) << 31),
                 Status::kInvalidArgument, "gemm: leading dimension too large");
-  auto kernel = gemmPipeKernel<BM, BN, WM, WN, DIST, EPI, B_NK, DMA, ANY>;
-  static bool attrSet = false;
-  st = allowLds(kernel, SMEM, &attrSet);
-  if (st != Status::kSuccess)
-    return st;
-  if (plan.nTiles == 0)
-    return Status::kSuccess;
+  struct Variant {
+    decltype(&gemmPipeKernel<BM, BN, WM, WN, DIST, EPI, B_NK, DMA, ANY>) kernel;
+    bool attrSet;
+    int resident;
+  };
   // Workgroups that fit on the chip at once (rounded down to a multiple of the
   // XCD count, which the tile order relies on); more tiles than that are walked
   // by the same workgroups.
-  static int resident = 0;
-  if (resident == 0) {
+  auto prepare = [&](Variant *v) -> Status {
+    Status ready = allowLds(v->kernel, SMEM, &v->attrSet);
+    if (ready != Status::kSuccess || v->resident != 0)
+      return ready;
     int perCu = 0;
     HOM_HIP_RET(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                    &perCu, kernel, WM * WN * kWave, SMEM),
+                    &perCu, v->kernel, WM * WN * kWave, SMEM),
                 Status::kInternal);
     const int cus = deviceInfo().computeUnits > 0 ? deviceInfo().computeUnits : 256;
-    resident = perCu > 0 ? perCu * cus / kNumXcd * kNumXcd : 0;
-    if (resident < kNumXcd)
-      resident = 1 << 30; // unknown: one workgroup per tile
+    v->resident = perCu > 0 ? perCu * cus / kNumXcd * kNumXcd : 0;
+    if (v->resident < kNumXcd)
+      v->resident = 1 << 30; // unknown: one workgroup per tile
+    return Status::kSuccess;
+  };
+  static Variant late = {gemmPipeKernel<BM, BN, WM, WN, DIST, EPI, B_NK, DMA, ANY>, false, 0};
+  Variant *use = &late;
+  if (plan.nTiles == 0)
+    return Status::kSuccess;
+  // The smallest tiles the library chooses request a partial slab early (with a
+  // row-major B at any alignment there always is one) where all workgroups are
+  // resident at once all the same.  Late against early, three sets of operands in
+  // turn, us: 1000 x 1001 x 1003 9.5 -> 9.1, 1200 x 1201 x 1001 14.4 -> 14.0, 600 x 600 x 600
+  // 4.8 -> 4.7, 1200 x 1200 x 1000 equal.  Early kernels for everything lost their third
+  // wavefront: 1400 x 1400 x 704, without a partial slab, 8.2 -> 8.4.  128 x 128 tiles lose
+  // up to 3 % by it (900 x 2312 x 600 9.4 -> 9.8).
+  if constexpr (BM * BN <= 64 * 64 && DIST == 2 && !DMA && EPI < kEpiRowStats) {
+    static Variant early = {
+        gemmPipeKernel<BM, BN, WM, WN, DIST, EPI, B_NK, DMA, ANY, true>, false, 0};
+    if (pr.K % 64 != 0 || (ANY && !B_NK)) {
+      st = prepare(&early);
+      if (st != Status::kSuccess)
+        return st;
+      if (plan.nTiles * plan.splitK <= early.resident)
+        use = &early;
+    }
   }
+  st = prepare(use);
+  if (st != Status::kSuccess)
+    return st;
+  const int resident = use->resident;
   int64_t gridX = plan.nTiles;
   if (gridX * plan.splitK > resident)
     gridX = std::max<int64_t>(kNumXcd, resident / plan.splitK / kNumXcd * kNumXcd);
@@ -913,12 +950,12 @@ Status launchPipe(const GemmProblem &pr, hipStream_t s) {
     }
   }
   // (leading dimensions fit 31 bits: checked above)
-  kernel<<<dim3((unsigned)gridX, (unsigned)plan.splitK), dim3(WM * WN * kWave),
-           SMEM, s>>>(q.A, q.B, q.M, q.N, q.K, int(q.lda), int(q.ldb), q.tilesN,
-                      q.xcdQ,
-                      uint32_t(q.xcdR) | uint32_t(q.lastRows) << 4 |
-                          uint32_t(q.fullGroups) << 8,
-                      q.groupMagic, q.kTilesPerSlice, q);
+  use->kernel<<<dim3((unsigned)gridX, (unsigned)plan.splitK), dim3(WM * WN * kWave),
+                SMEM, s>>>(q.A, q.B, q.M, q.N, q.K, int(q.lda), int(q.ldb), q.tilesN,
+                           q.xcdQ,
+                           uint32_t(q.xcdR) | uint32_t(q.lastRows) << 4 |
+                               uint32_t(q.fullGroups) << 8,
+                           q.groupMagic, q.kTilesPerSlice, q);
   HOM_HIP_RET(hipGetLastError(), Status::kInternal);
   if (plan.splitK > 1 && !sumInKernel)
     return launchReduce<BM, BN, WM, WN, EPI, 8>(plan, s);

@@ -170,6 +170,28 @@ def test_gemm_any_alignment(gpu, rt, oracle, tile, M, N, K):
     np.testing.assert_allclose(host(td)[0].astype(np.float64), oracle.gemm(A[0], B[0]), rtol=1e-3, atol=1e-2)
 
 
+# 64 x 64 tiles with a partial slab: requested ahead of the full ones (up to two workgroups per CU), or behind them
+@pytest.mark.parametrize("tile,step", [("64x64_64x2r2_w2x2_nn_align8", 8), ("64x64_64x2u2_w2x2_nn_align1", 1)])
+@pytest.mark.parametrize("tilesM,tilesN", [(2, 3), (16, 32), (19, 27), (40, 39)])
+@pytest.mark.parametrize("K", [8, 72, 120, 392])
+def test_gemm_partial_slab_early_and_late(gpu, rt, monkeypatch, tile, step, tilesM, tilesN, K):
+    M, N, K = tilesM * 64 - 5, tilesN * 64 - step, K + (step == 1)
+    num, name = next((i + 1, n) for i, n, _, _ in rt.manifest() if f"_{tile}_linear" in n)
+    g = torch.Generator("cuda").manual_seed(M + K)
+    A = torch.randn(1, M, K, device="cuda", generator=g).half()
+    B = (torch.randn(1, K, N, device="cuda", generator=g) * 0.1).half()
+    want = (A[0].double() @ B[0].double()).cpu().numpy()
+    Mr, D, Bt = rt.MemRef.from_tensor, torch.zeros(1, M, N, dtype=torch.float16, device="cuda"), B[0].t().contiguous()[None]
+    for sk in (1, 2):
+        gpu.cutlassGemmF16(*Mr(A).args(), False, *Mr(B).args(), False, *Mr(D).args(), *Mr(D).args(), 0, 1.0, 0.0, num, sk)
+        # (half a unit of the fp16 result, and fp32 sums of up to 393 products of about 0.1)
+        np.testing.assert_allclose(host(D)[0].astype(np.float64), want, rtol=2**-10, atol=1e-4)
+        D.zero_()
+        monkeypatch.setenv("HOM_NVTE_GEMM_KERNEL", f"{name},{sk}")
+        gpu.nvteGemmF16(*Mr(A).args(), False, *Mr(Bt).args(), True, *Mr(D).args(), *Mr(D).args(), 0, 1.0, 0.0, 0, 0)
+        np.testing.assert_allclose(host(D)[0].astype(np.float64), want, rtol=2**-10, atol=1e-4)
+
+
 # the kernels whose wavefronts split K: tiles and slabs of 64 and, rows at odd elements, of 63; remainders of a vector,
 # fewer slabs than wavefronts and more than two rounds of them, slices across workgroups with a short last one.  What
 # lies around the operands is NaN: nothing read from there may reach a result, and nothing may be written there.
