@@ -5,6 +5,7 @@
 // var/mean per row through the column sums of B.  Both use the register-staged
 // pipeline kernels with the two extra epilogue codes.
 #include "gemm_pipe.h"
+#include "pair_tile.h"
 
 namespace hom {
 namespace {
@@ -139,21 +140,6 @@ template <int EPI>
 Status launchFusedTile(int likeKernel, const GemmProblem &p, hipStream_t s) {
   return launchFusedEdge<EPI>(fusedTileFor(likeKernel).edge, p, s);
 }
-// The layer-norm pair's tile: the largest, up to `most` on a side, of which there is
-// one for ten (256) or nine (128) in sixteen CUs.  Second GEMM, 256 against 128,
-// us: 4096 x 4096 x 1024 (256 tiles of 256) 40.8 / 54.9, 4096 x 3072 x 768 (192) 28.2 / 34.1,
-// 2500 x 3072 x 1024 (120) 30.9 / 29.4; the first never gains by 256 (16384 x 768 x 768
-// 40.5 / 30.6), whose registers do not hold the source's vectors as well.
-FusedTile pairTile(const GemmProblem &p, int most) {
-  const int64_t cus = deviceInfo().computeUnits > 0 ? deviceInfo().computeUnits : 256;
-  auto tiles = [&](int64_t edge) {
-    return ((p.M + edge - 1) / edge) * ((p.N + edge - 1) / edge);
-  };
-  if (most >= 256 && tiles(256) * 16 >= cus * 10)
-    return {256, 64};
-  return tiles(128) * 16 >= cus * 9 ? FusedTile{128, 32} : FusedTile{64, 32};
-}
-
 inline bool aligned16(const void *p) {
   return (reinterpret_cast<uintptr_t>(p) & 15) == 0;
 }
@@ -164,6 +150,15 @@ bool foldFits(const GemmProblem &p) {
   return (p.beta == 0.f || (p.cRowPeriod >= p.M && p.ldc % 8 == 0 &&
                             int64_t(256) * p.ldc * 2 < (int64_t(1) << 31))) &&
          int64_t(256) * p.ldd * 2 < (int64_t(1) << 31);
+}
+// The pair's tile (second: of its second GEMM).
+FusedTile pairTile(const GemmProblem &p, bool second) {
+  const int cus = deviceInfo().computeUnits > 0 ? deviceInfo().computeUnits : 256;
+  const PairSource source = p.beta == 0.f ? PairSource::kNone
+                            : foldFits(p) ? PairSource::kMatrix
+                                          : PairSource::kRow;
+  const int edge = pairTileEdge(p.M, p.N, p.K, second, source, cus);
+  return {edge, edge == 256 ? 64 : 32};
 }
 
 } // namespace
@@ -184,10 +179,11 @@ Status launchGemmRowStats(const GemmProblem &p, _Float16 *var, _Float16 *mean, f
   // No source or a full matrix, on 128 x 128 tiles: the epilogue of the folded
   // layer norm with nothing folded in, which requests the source ahead of everything
   // and adds up a tile's columns before it writes them (4096 x 1024 x 1024 17.4 -> 15.4
-  // us, 16384 x 1024 x 1024 61.0 -> 52.8, 3000 x 768 x 768 13.3 -> 11.8).  Others, a bias row
-  // or small tiles (64 x 768 x 768 8.2 / 9.1), write a partial sum per wavefront column,
+  // us, 8192 x 768 x 768 with a source 25.0 -> 22.5, 3000 x 768 x 768 13.3 -> 11.8).  Others, a
+  // bias row, small tiles (64 x 768 x 768 8.2 / 9.1) or 256 x 256 ones (whose registers do
+  // not hold the source's vectors as well), write a partial sum per wavefront column,
   // also of those past N.
-  const FusedTile t = pairTile(p, foldFits(p) ? 128 : 256);
+  const FusedTile t = pairTile(p, false);
   const bool whole = t.edge == 128 && foldFits(p);
   const int pieces = int((p.N + t.edge - 1) / t.edge) * (whole ? 1 : t.edge / t.pieceWidth);
   float *partials = static_cast<float *>(
@@ -216,7 +212,7 @@ Status launchGemmRowAffine(const GemmProblem &p, const _Float16 *var, const _Flo
   q.splitK = 1;
   q.rowScale = var;
   q.rowShift = mean;
-  const int edge = pairTile(p, 256).edge;
+  const int edge = pairTile(p, true).edge;
   // No source or a full matrix: the column sums are formed on the way, four dot
   // products per fragment of B in the shadow of its MFMAs; by a kernel of their own
   // they took 4.5 us of a launch.  With the pairs kept in LDS and the epilogue of

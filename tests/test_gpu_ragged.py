@@ -236,7 +236,8 @@ def test_gemm_waves_split_k(gpu, rt, oracle, monkeypatch, tile, M, N, K):
 
 # both halves of the layer-norm pair on each of their tiles (64, 128 and 256 on a side, ragged rows, columns and K),
 # without a source, with a bias row (column sums and row sums by the general epilogue) and with a full matrix
-@pytest.mark.parametrize("M,N,K", [(70, 136, 72), (1100, 2056, 200), (4100, 2568, 136)])
+@pytest.mark.parametrize("M,N,K", [(70, 136, 72), (1100, 2056, 200), (2500, 3080, 712), (4100, 2568, 136),
+                                   (4090, 4096, 520)])
 @pytest.mark.parametrize("source", ["none", "bias", "full"])
 def test_layernorm_pair_tiles_and_sources(gpu, rt, M, N, K, source):
     g = torch.Generator(device="cuda").manual_seed(M)
