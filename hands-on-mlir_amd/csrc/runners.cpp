@@ -238,24 +238,36 @@ const std::vector<TileModel> &tileModels() {
 // of them costs beyond its slabs, above all where all CUs write (and read a full
 // source) at once.  t = fixed + rounds (slab K / 64 + round + gelu + source) + out M N +
 // outSource M N + traffic of all tiles, us; a round is a tile on every CU.  Fitted to
-// 198 problems x 7 tiles, M = 500 .. 16384, N and K = 256 .. 4096, three sets of
-// operands in turn: 3 to 5 % off in the mean, the choice 0.8 % off the best (the
-// model below: 2.9 %; 15068 x 896 x 960 with a source 47.5 -> 38.6 us, 4813 x 3072 x 320
-// 29.6 -> 21.4).
+// 560 problems x 7 tiles, M = 400 .. 20000, N = 64 .. 4500, K = 8 .. 4500, three sets of
+// operands in turn: 6 to 8 % off in the mean, the choice 1.3 % off the best, 18 % at
+// worst, on short K (the model below: 5.0 % and 38 %; 15866 x 3288 x 328 with GELU 119.8 ->
+// 87.9 us, 10289 x 912 x 1256 with GELU 1.31 x less, 8372 x 1936 x 904 with a source 1.12 x);
+// and to 130 problems whose rows of C and D are not on 16 bytes, which cost the larger
+// tiles more (0.7 % off the best, the model below 10.7 %; 4622 x 502 x 272 with a source 64 x 64
+// 10.5 us, 64 x 128 13.3).
 bool modelFullChip(int64_t M, int64_t N, int64_t K, Epilogue epi, int cls, bool fullSource,
                    int64_t *idx, int32_t *splitK) {
   struct Fit {
     double fixed, slab, round, gelu, source, out, outSource, traffic;
   };
-  static const Fit fits[] = { // in the order of tileModels()
-      {1.96, 0.118, 0.558, 0.152, 0, 0, 0.226, 0.0213},
-      {2.94, 0.201, 0, 0.313, 0, 0.362, 0.201, 0.0199},
-      {2.82, 0.190, 0, 0.379, 0.087, 0.339, 0.150, 0.0222},
-      {1.24, 0.281, 2.30, 0.704, 0.139, 0, 0.176, 0.0321},
-      {0, 0.468, 4.49, 2.00, 0.687, 0.075, 0.134, 0.0321},
-      {0, 0.455, 4.46, 1.96, 0.887, 0.0814, 0.108, 0.0346},
-      {0, 0.865, 9.23, 4.75, 2.78, 0.228, 0.427, 0.0332},
-  };
+  // in the order of tileModels(); rows on 16 bytes, and others
+  static const Fit fits[2][7] = {{
+      {1.87, 0.191, 0.518, 0.128, 0, 0.0454, 0.199, 0.0188},
+      {2.63, 0.320, 0, 0.229, 0, 0.509, 0.213, 0.0180},
+      {2.51, 0.278, 0.132, 0.282, 0, 0.414, 0.179, 0.0195},
+      {1.37, 0.382, 2.32, 0.459, 0, 0.127, 0.201, 0.0301},
+      {1.44, 0.577, 3.16, 1.45, 0, 0.0616, 0.293, 0.0357},
+      {1.34, 0.697, 3.10, 1.50, 0, 0.0692, 0.307, 0.0312},
+      {0.32, 0.999, 7.65, 3.14, 4.03, 0.239, 0.436, 0.0395},
+  }, {
+      {2.82, 0.182, 0.373, 0.215, 0.159, 0.313, 0.189, 0.0232},
+      {4.18, 0.331, 0.195, 0.568, 0.484, 0.499, 0.339, 0.0147},
+      {3.99, 0.273, 0.600, 0.515, 0.502, 0.360, 0.357, 0.0189},
+      {3.23, 0.439, 1.24, 1.11, 1.41, 0.478, 0.209, 0.0231},
+      {5.19, 0.581, 2.24, 2.08, 3.16, 0.322, 0.282, 0.0310},
+      {5.66, 0.730, 1.89, 2.15, 3.30, 0.332, 0.247, 0.0173},
+      {9.14, 0.929, 3.86, 4.23, 6.72, 0.295, 0.458, 0.0386},
+  }};
   const int cus = deviceInfo().computeUnits > 0 ? deviceInfo().computeUnits : 256;
   if (cls == 1 || ((M + 63) / 64) * ((N + 63) / 64) <= cus)
     return false;
@@ -263,7 +275,7 @@ bool modelFullChip(int64_t M, int64_t N, int64_t K, Epilogue epi, int cls, bool 
   const double outputs = double(M) * double(N) * 1e-6, slabs = double((K + 63) / 64);
   for (size_t t = 0; t < tileModels().size(); t++) {
     const TileModel &m = tileModels()[t];
-    const Fit &f = fits[t];
+    const Fit &f = fits[cls == 8 ? 0 : 1][t];
     const int kernel = m.aligned[int(epi)];
     if (kernel < 0)
       continue;

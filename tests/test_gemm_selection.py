@@ -38,6 +38,23 @@ def test_every_size_gets_a_kernel_that_takes_it(rt, largest, step):
     assert largest > 1500 or seen == {16, 32}
 
 
+# Problems of more 64 x 64 tiles than CUs, no source or a bias row, all seven tiles timed on an MI355X: those within 5 % of
+# the fastest (sizes, activation, tiles)
+@pytest.mark.parametrize("M,N,K,act,tiles", [
+    (15866, 3288, 328, 1, "128x256"), (15440, 4040, 336, 1, "128x256"), (13520, 3656, 176, 2, "128x256 256x128"),
+    (13802, 3536, 56, 2, "128x256 256x128"), (9165, 424, 1176, 0, "128x256"), (10289, 912, 1256, 1, "256x256"),
+    (16873, 440, 1016, 0, "256x256"), (3037, 2920, 880, 2, "256x256"), (5339, 296, 712, 0, "64x128"),
+    (8930, 1728, 96, 0, "128x256 256x128"), (6580, 4168, 344, 0, "128x256 256x128"), (8534, 272, 32, 0, "64x64 64x128"),
+    (588, 4184, 16, 0, "64x64 64x128"), (3396, 1608, 176, 1, "128x256"),
+    # rows off 16 bytes
+    (19540, 420, 112, 1, "64x64"), (2673, 3938, 8, 2, "64x64"), (17143, 86, 80, 0, "64x64"), (2356, 2588, 64, 2, "64x64")])
+def test_large_problems_take_a_fast_tile(rt, M, N, K, act, tiles):
+    lib = rt.load_runtime()
+    idx, sk = choice(lib, "homGemmSelect", M, N, K, act)
+    name = lib.homGemmManifestName(idx).decode()
+    assert sk == 1 and re.search(r"f16_(\d+x\d+)_64x2r", name).group(1) in tiles.split(), name
+
+
 # The layer-norm pair's tiles where all that fit were timed on an MI355X and one is 8 % faster at least than the others:
 # (second GEMM, source: 0 none, 1 a bias row, 2 a full matrix; sizes, the fastest)
 PAIR_TILES = [(0, 0, 5535, 2408, 2960, 256), (0, 0, 16384, 4096, 1024, 256), (0, 0, 5189, 1968, 728, 256),
