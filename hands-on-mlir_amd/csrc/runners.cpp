@@ -479,14 +479,7 @@ bool gemmPrefersNvte(int64_t M, int64_t N, int64_t K, int64_t activation) {
 bool selectGemm(int64_t M, int64_t N, int64_t K, int64_t activation,
                 int64_t *idx, int32_t *splitK, bool bIsNK, bool fullSource) {
   const Epilogue epi = epilogueFor(activation, false);
-  const TunedEntry *t = findTuned(M, N, K, activation);
-  // (the table holds kernels with slabs in sequence only)
-  if (t && ksplitFits(M, N)) {
-    modelGemm(M, N, K, epi, naturalClass(N, K), fullSource, idx, splitK);
-    if (wavesSplitK(gemmKernelInfo(int(*idx))))
-      return false;
-  }
-  if (t) {
+  if (const TunedEntry *t = findTuned(M, N, K, activation)) {
     const int nk = bIsNK ? kernelByName(t->nkKernel) : -1;
     const int i = nk >= 0 ? nk : kernelByName(t->kernel);
     if (i >= 0) {

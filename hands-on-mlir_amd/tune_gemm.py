@@ -172,10 +172,6 @@ def main():
     for (M, N, K, act) in bert_shapes():
         if only_rows and M not in only_rows:
             continue
-        sel, split = ctypes.c_int64(), ctypes.c_int32()
-        lib.homGemmSelect(M, N, K, act, ctypes.byref(sel), ctypes.byref(split))
-        if "k8_w1x1_" in names[sel.value]:
-            continue  # the kernels whose wavefronts split K are chosen by their model, ahead of the table
         beta = 1.0 if (act == 0 and N in (768, 1024) and K != N // 3) else 0.0
         res = []
         for nk in (0, 1):

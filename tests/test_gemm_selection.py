@@ -38,6 +38,23 @@ def test_every_size_gets_a_kernel_that_takes_it(rt, largest, step):
     assert largest > 1500 or seen == {16, 32}
 
 
+def test_shipped_table_answers_first(rt):
+    lib = rt.load_runtime()
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    with open(os.path.join(root, "hands-on-mlir_amd", "csrc", "gemm_tuned_table.inc")) as f:
+        rows = re.findall(r'\{(\d+), (\d+), (\d+), (\d), "(\w+)", (\d+), "(\w+)", (\d+), (\d)\}', f.read())
+    assert len(rows) == 51
+    for M, N, K, act, *kernels, prefers in rows:
+        size = tuple(map(int, (M, N, K, act)))
+        for select, kernel, split in (("homGemmSelect", *kernels[:2]), ("homGemmSelectNvte", *kernels[2:])):
+            if select == "homGemmSelectNvte" and act == "1":
+                continue  # (GELU is the tanh form there)
+            idx, sk = ctypes.c_int64(-1), ctypes.c_int32(0)
+            assert getattr(lib, select)(*size, ctypes.byref(idx), ctypes.byref(sk)) == 1, size
+            assert (lib.homGemmManifestName(idx.value).decode(), sk.value) == (kernel, int(split)), size
+        assert lib.homGemmPrefersNvte(*size) == int(prefers), size
+
+
 # Few tiles: the wavefronts split K where there are slabs of 64 for most of them, on rows at odd places always
 @pytest.mark.parametrize("M,N", [(6, 72), (37, 952), (141, 168), (10, 320)])
 @pytest.mark.parametrize("select", ["homGemmSelect", "homGemmSelectNvte"])
