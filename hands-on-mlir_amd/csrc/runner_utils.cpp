@@ -354,6 +354,20 @@ int32_t homGemmSelectNvte(int64_t M, int64_t N, int64_t K, int64_t activation,
   return tuned ? 1 : 0;
 }
 
+int32_t homGemmSelectWithSource(int64_t M, int64_t N, int64_t K, int64_t activation,
+                                int32_t bIsNK, int32_t fullSource, int64_t *idx,
+                                int32_t *splitK) {
+  int64_t i = -1;
+  int32_t s = 1;
+  const bool tuned = bIsNK ? selectGemmNvte(M, N, K, activation, &i, &s, fullSource != 0)
+                           : selectGemm(M, N, K, activation, &i, &s, false, fullSource != 0);
+  if (idx)
+    *idx = i;
+  if (splitK)
+    *splitK = s;
+  return tuned ? 1 : 0;
+}
+
 int32_t homPackedGemmSelect(int64_t M, int64_t N, int64_t K, int64_t activation,
                             int32_t normA, int32_t source, int32_t packing,
                             int32_t readsAhead, int32_t *rows, int32_t *cols,

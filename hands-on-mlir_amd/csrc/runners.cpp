@@ -553,10 +553,10 @@ Status runGemmManifest(int64_t rankA, void *dstA, int64_t rankB, void *dstB,
 }
 
 bool selectGemmNvte(int64_t M, int64_t N, int64_t K, int64_t activation,
-                    int64_t *idx, int32_t *splitK) {
+                    int64_t *idx, int32_t *splitK, bool fullSource) {
   const Epilogue epi = epilogueFor(activation, true);
   return selectGemm(M, N, K, epi == Epilogue::kGeluTanh ? 2 : activation, idx,
-                    splitK, true);
+                    splitK, true, fullSource);
 }
 
 namespace {
@@ -564,7 +564,8 @@ int chooseNvteKernel(GemmProblem *pr, int64_t activation) {
   int64_t sel;
   int32_t sk;
   const Epilogue epi = epilogueFor(activation, true);
-  selectGemmNvte(pr->M, pr->N, pr->K, activation, &sel, &sk);
+  const bool fullSource = pr->beta != 0.f && pr->cRowPeriod > 1;
+  selectGemmNvte(pr->M, pr->N, pr->K, activation, &sel, &sk, fullSource);
   int idx = int(sel);
   pr->splitK = sk;
   // Profiling knob: HOM_NVTE_GEMM_KERNEL="<manifest name>[,<splitK>]" pins the
@@ -581,7 +582,7 @@ int chooseNvteKernel(GemmProblem *pr, int64_t activation) {
   }
   const int cls = alignmentClass(*pr);
   if (!kernelFits(gemmKernelInfo(idx), cls)) {
-    modelGemm(pr->M, pr->N, pr->K, epi, cls, false, &sel, &sk);
+    modelGemm(pr->M, pr->N, pr->K, epi, cls, fullSource, &sel, &sk);
     idx = int(sel);
     pr->splitK = sk;
   }

@@ -83,6 +83,21 @@ def test_large_problems_take_a_fast_tile(rt, M, N, K, act, tiles):
     assert sk == 1 and re.search(r"f16_(\d+x\d+)_64x2r", name).group(1) in tiles.split(), name
 
 
+# The same with a full matrix as source, whose price changes the fastest tile (the one named first is 9 % slower at least)
+@pytest.mark.parametrize("M,N,K,act,without,tile", [
+    (5945, 2312, 1408, 0, "256x256", "128x256"), (5475, 1576, 408, 0, "256x256", "64x128"), (3925, 2576, 608, 1, "256x256", "128x128"),
+    (9658, 1728, 80, 0, "128x256", "64x128"), (8967, 1208, 392, 1, "128x256", "128x128")])
+@pytest.mark.parametrize("nk", [0, 1])
+def test_a_source_is_priced(rt, M, N, K, act, without, tile, nk):
+    lib = rt.load_runtime()
+    idx, sk = ctypes.c_int64(-1), ctypes.c_int32(0)
+    for source, expected in ((0, without), (1, tile)):
+        assert lib.homGemmSelectWithSource(M, N, K, act, nk, source, ctypes.byref(idx), ctypes.byref(sk)) == 0
+        assert f"f16_{expected}_64x2r" in lib.homGemmManifestName(idx.value).decode()
+        if not source:
+            assert (idx.value, sk.value) == choice(lib, "homGemmSelectNvte" if nk else "homGemmSelect", M, N, K, act)
+
+
 # The layer-norm pair's tiles where all that fit were timed on an MI355X and one is 8 % faster at least than the others:
 # (second GEMM, source: 0 none, 1 a bias row, 2 a full matrix; sizes, the fastest)
 PAIR_TILES = [(0, 0, 5535, 2408, 2960, 256), (0, 0, 16384, 4096, 1024, 256), (0, 0, 5189, 1968, 728, 256),
