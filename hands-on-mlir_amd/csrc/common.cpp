@@ -26,6 +26,19 @@ struct StreamScratch {
 std::vector<StreamScratch> g_scratch;
 std::vector<void *> g_retired; // replaced scratch buffers, kept allocated
 int g_scratchGeneration = 0;
+
+// The calling stream's set; without one a set that a finished stream gave back
+// (releaseStreamScratch) serves it, buffers included.  nullptr: there is none.
+StreamScratch *scratchOfStream() {
+  StreamScratch *spare = nullptr;
+  for (StreamScratch &s : g_scratch) {
+    if (s.inUse && s.stream == g_stream)
+      return &s;
+    if (!s.inUse && !spare)
+      spare = &s;
+  }
+  return spare;
+}
 } // namespace
 
 int errorMode() { return g_errorMode; }
@@ -86,32 +99,21 @@ void releaseStreamScratch(hipStream_t s) {
 }
 
 bool libraryScratchReady(ScratchSlot slot, size_t bytes) {
-  for (const StreamScratch &e : g_scratch)
-    if (e.inUse && e.stream == g_stream && e.slot[slot].bytes >= bytes)
-      return true;
+  const StreamScratch *mine = scratchOfStream();
+  if (mine && mine->slot[slot].bytes >= bytes)
+    return true;
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   return hipStreamIsCapturing(g_stream, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone;
 }
 
 void *libraryScratch(ScratchSlot slot, size_t bytes, bool zero) {
-  StreamScratch *mine = nullptr, *spare = nullptr;
-  for (StreamScratch &s : g_scratch) {
-    if (s.inUse && s.stream == g_stream)
-      mine = &s;
-    else if (!s.inUse && !spare)
-      spare = &s;
-  }
+  StreamScratch *mine = scratchOfStream();
   if (!mine) {
-    // a set that a finished stream gave back (releaseStreamScratch) serves the
-    // next new stream, buffers included
-    if (!spare) {
-      g_scratch.emplace_back();
-      spare = &g_scratch.back();
-    }
-    mine = spare;
-    mine->stream = g_stream;
-    mine->inUse = true;
+    g_scratch.emplace_back();
+    mine = &g_scratch.back();
   }
+  mine->stream = g_stream;
+  mine->inUse = true;
   ScratchBuf &b = mine->slot[slot];
   if (bytes <= b.bytes)
     return b.ptr;

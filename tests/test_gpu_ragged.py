@@ -294,6 +294,37 @@ def test_gemm_waves_split_k_first_call_captured(gpu, rt, oracle):
         np.testing.assert_allclose(host(td)[0].astype(np.float64), want, rtol=1e-3, atol=1e-2)
 
 
+# a first call inside a capture on a stream that takes over another one's memory: the split, and the bits, of an eager call
+def test_gemm_waves_split_k_captured_on_handed_on_memory(gpu, rt):
+    M, N, K = 33, 1001, 3001
+    g = torch.Generator("cuda").manual_seed(5)
+    ta, tb = torch.randn(1, M, K, device="cuda", generator=g).half(), torch.randn(1, K, N, device="cuda", generator=g).half()
+    eager, td = (torch.zeros((1, M, N), dtype=torch.float16, device="cuda") for _ in range(2))
+    Mr = rt.MemRef.from_tensor
+
+    def call(out):
+        gpu.cutlassGemmF16(*Mr(ta).args(), False, *Mr(tb).args(), False, *Mr(out).args(), *Mr(out).args(), 0, 1.0, 0.0, 0, 1)
+
+    first, second, graph = torch.cuda.Stream(), torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    try:
+        gpu.homSetStream(ctypes.c_void_p(first.cuda_stream))
+        call(eager)
+        torch.cuda.synchronize()
+        gpu.homReleaseStreamScratch(ctypes.c_void_p(first.cuda_stream))
+        gpu.homSetStream(ctypes.c_void_p(second.cuda_stream))
+        with torch.cuda.graph(graph, stream=second):
+            call(td)
+    finally:
+        gpu.homSetStream(None)
+    for _ in range(3):
+        td.zero_()
+        graph.replay()
+        np.testing.assert_array_equal(host(td), host(eager))
+    del graph
+    gpu.homReleaseStreamScratch(ctypes.c_void_p(second.cuda_stream))
+
+
 def fragment_order(a):
     """[rows, cols] -> blocks of 16 rows x 32 columns as the packed GEMM takes them (rows padded to 16)."""
     rows, cols = a.shape
