@@ -234,6 +234,49 @@ def test_gemm_waves_split_k(gpu, rt, oracle, monkeypatch, tile, M, N, K):
             check(t, td, plain)
 
 
+# their slices added by the second kernel, with the in-kernel form off and where the caller brings the workspace: the sums
+# of the in-kernel form bit for bit; tiles of 64 and of 63 columns, ragged rows and columns, a short last slice
+@pytest.mark.parametrize("tile", ["16x64_64x2r2k8_w1x1_nn_align1", "32x64_64x2r2k8_w1x1_nn_align1"])
+@pytest.mark.parametrize("M,N,K", [(40, 130, 1032), (33, 1001, 777), (17, 63, 2002), (70, 72, 2002), (5, 127, 1150)])
+def test_gemm_waves_split_k_second_kernel(gpu, rt, oracle, monkeypatch, tile, M, N, K):
+    g = np.random.default_rng(M + N + K)
+    names = {n.rsplit("_", 1)[1]: (i + 1, n) for i, n, _, _ in rt.manifest() if f"_{tile}_" in n}
+    A, B = g.standard_normal((1, M, K)).astype(np.float16), (g.standard_normal((1, K, N)) * 0.1).astype(np.float16)
+    R = g.standard_normal((1, M, N)).astype(np.float16)
+    Mr, ta, tb, tr, tbt = rt.MemRef.from_tensor, dev(A), dev(B), dev(R), dev(np.ascontiguousarray(B[0].T)[None])
+    t = torch.full((M * N + 256,), float("nan"), dtype=torch.float16, device="cuda")
+    td = t[128:128 + M * N].view(1, M, N)
+
+    def result(fn, name, sk):
+        td.zero_()
+        if fn == "nvte":
+            monkeypatch.setenv("HOM_NVTE_GEMM_KERNEL", f"{names[name][1]},{sk}")
+            gpu.nvteGemmF16(*Mr(ta).args(), False, *Mr(tbt).args(), True, *Mr(td).args(), *Mr(td).args(), 0, 1.0, 0.0, 0, 0)
+        else:
+            getattr(gpu, fn)(*Mr(ta).args(), False, *Mr(tb).args(), False, *Mr(tr).args(), *Mr(td).args(), 0, 1.0, 0.5,
+                             names[name][0], sk)
+        out = host(td).copy()
+        assert int(torch.isnan(t).sum()) == 256
+        return out
+
+    for sk in (2, 5):
+        calls = [("cutlassGemmF16", "linear", sk), ("cutlassGemmF16", "gelu", sk), ("nvte", "linear", sk)]
+        launches = gpu.homSplitKInKernelLaunches()
+        in_kernel = [result(*c) for c in calls]
+        assert gpu.homSplitKInKernelLaunches() == launches + 3
+        np.testing.assert_allclose(in_kernel[0][0].astype(np.float64), oracle.gemm(A[0], B[0], R[0], beta=0.5), rtol=1e-3,
+                                   atol=1e-2)
+        try:
+            gpu.homSetSplitKInKernel(0)
+            for c, want in zip(calls, in_kernel):
+                np.testing.assert_array_equal(result(*c), want)
+        finally:
+            gpu.homSetSplitKInKernel(3)
+        assert gpu.homSplitKInKernelLaunches() == launches + 3
+        for c, want in zip(calls[:2], in_kernel):
+            np.testing.assert_array_equal(result("homGemmF16NoAlloc", *c[1:]), want)
+
+
 # both halves of the layer-norm pair on each of their tiles (64, 128 and 256 on a side, ragged rows, columns and K),
 # without a source, with a bias row (column sums and row sums by the general epilogue) and with a full matrix
 @pytest.mark.parametrize("M,N,K", [(70, 136, 72), (1100, 2056, 200), (2500, 3080, 712), (4100, 2568, 136),
