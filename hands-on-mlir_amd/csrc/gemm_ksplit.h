@@ -34,7 +34,7 @@ namespace gemmk {
 //
 // VEC: rows on 16-byte boundaries and K a multiple of 8; otherwise rows of any length
 // from 8 values up.  Every load is of whole dwords, in the tensor or, as part of
-// its last dword, two bytes behind it; what a vector of A (or of a [N, K] B) holds
+// its first or last dword, two bytes in front of it or behind it; what a vector of A (or of a [N, K] B) holds
 // behind the row's end is masked.  ODD_A, ODD_B: rows may start in the middle of a
 // dword.  16-byte loads from there run at 17 bytes a clock instead of 46, so such a
 // row is read from two bytes earlier and shifted into place, the last value of a
@@ -60,21 +60,18 @@ template <int MB, int NB> constexpr int ksplitWaveBytes() {
   constexpr int kSlab = (MB + NB) * 16 * 128, kPartial = MB * 16 * (NB * 64 + 16);
   return kSlab > kPartial ? kSlab : kPartial;
 }
-// Consecutive columns a thread finishes: 8 where that gives every thread work.
-template <int MB, int NB> constexpr int ksplitOutWidth() {
-  return MB * NB * 256 / 8 >= kKsplitThreads ? 8 : 4;
-}
+// Consecutive columns a thread finishes (all threads of a 32 x 64 tile have some).
+constexpr int kKsplitOut = 4;
 
-// alpha * v + beta * c, activated and stored: W consecutive columns of row m, those
+// alpha * v + beta * c, activated and stored: consecutive columns of row m, those
 // in front of nEnd.  onVectors: rows of D start on whole vectors.
-template <int W>
 __device__ __forceinline__ void ksplitFinish(const GemmParams &p, int activation, int m, int n,
-                                             int nEnd, bool onVectors, const float (&v)[W],
-                                             const _Float16 (&c)[W]) {
-  typedef _Float16 vec __attribute__((ext_vector_type(W)));
+                                             int nEnd, bool onVectors, const float (&v)[kKsplitOut],
+                                             const _Float16 (&c)[kKsplitOut]) {
+  typedef _Float16 vec __attribute__((ext_vector_type(kKsplitOut)));
   vec o;
 #pragma unroll
-  for (int e = 0; e < W; e++) {
+  for (int e = 0; e < kKsplitOut; e++) {
     float x = p.alpha * v[e];
     if (p.beta != 0.f)
       x += p.beta * float(c[e]);
@@ -85,15 +82,12 @@ __device__ __forceinline__ void ksplitFinish(const GemmParams &p, int activation
     o[e] = _Float16(x);
   }
   _Float16 *d = p.D + int64_t(m) * p.ldd + n;
-  if (n + W <= nEnd) {
-    // (rows that do not start on whole vectors: default policy, see store_policy.h)
+  if (n + kKsplitOut <= nEnd) {
+    // (8 bytes a lane, but sixteen lanes write a whole line: written through, 200 x
+    // 2048 x 768 5.40 -> 5.35 us, 500 x 1024 x 512 5.04 -> 4.99, tiles of 16 rows equal.  Rows
+    // that do not start on whole vectors: default policy, see store_policy.h)
     if (onVectors)
       storeWriteThrough(d, o);
-    else if constexpr (W == 8)
-      asm volatile("global_store_dwordx4 %0, %1, off\n\ts_nop 1"
-                   :
-                   : "v"(d), "v"(__builtin_bit_cast(uint4v, o))
-                   : "memory");
     else
       asm volatile("global_store_dwordx2 %0, %1, off"
                    :
@@ -101,31 +95,30 @@ __device__ __forceinline__ void ksplitFinish(const GemmParams &p, int activation
                    : "memory");
   } else {
 #pragma unroll
-    for (int e = 0; e < W; e++)
+    for (int e = 0; e < kKsplitOut; e++)
       if (n + e < nEnd)
         d[e] = o[e];
   }
 }
 // The source of the same outputs (zeros without one).
-template <int W>
 __device__ __forceinline__ void ksplitSource(const GemmParams &p, int m, int n, int nEnd,
-                                             _Float16 (&c)[W]) {
-  typedef _Float16 vec __attribute__((ext_vector_type(W)));
+                                             _Float16 (&c)[kKsplitOut]) {
+  typedef _Float16 vec __attribute__((ext_vector_type(kKsplitOut)));
   typedef vec vecAny __attribute__((aligned(2)));
 #pragma unroll
-  for (int e = 0; e < W; e++)
+  for (int e = 0; e < kKsplitOut; e++)
     c[e] = _Float16(0);
   if (p.beta == 0.f || m >= p.M || n >= nEnd)
     return;
   const _Float16 *src = p.C + int64_t(rowInPeriod(p, m)) * p.ldc + n;
-  if (n + W <= nEnd) {
+  if (n + kKsplitOut <= nEnd) {
     const vec x = *reinterpret_cast<const vecAny *>(src);
 #pragma unroll
-    for (int e = 0; e < W; e++)
+    for (int e = 0; e < kKsplitOut; e++)
       c[e] = x[e];
   } else {
 #pragma unroll
-    for (int e = 0; e < W; e++)
+    for (int e = 0; e < kKsplitOut; e++)
       if (n + e < nEnd)
         c[e] = src[e];
   }
@@ -144,7 +137,6 @@ __global__ __launch_bounds__(kKsplitThreads, 2) void gemmKsplitKernel(
   constexpr int A_BYTES = MT * 128;
   static_assert(B_NK || NT == 64, "rows of a row-major B slab are one cache line");
   constexpr int WAVE_BYTES = ksplitWaveBytes<MB, NB>();
-  constexpr int W = ksplitOutWidth<MB, NB>();
   constexpr uint32_t kOob = 0x80000000u;
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
   const int tid = threadIdx.x, lane = tid % kWave;
@@ -363,13 +355,14 @@ __global__ __launch_bounds__(kKsplitThreads, 2) void gemmKsplitKernel(
     p = *late;
   }
 #endif
-  // What this thread finishes: W columns of one row of the tile.
-  constexpr int OPR = NT / W;
-  const bool out = tid < MT * OPR;
-  const int row = tid / OPR, col = tid % OPR * W;
-  _Float16 c[W];
+  // What this thread finishes: some columns of one row of the tile.
+  constexpr int OPR = NT / kKsplitOut, kFinish = MT * OPR;
+  static_assert(kFinish <= kKsplitThreads, "one thread per outputs");
+  const bool out = tid < kFinish;
+  const int row = tid / OPR, col = tid % OPR * kKsplitOut;
+  _Float16 c[kKsplitOut];
   const int nEnd = n0 + COLS < N ? n0 + COLS : N;
-  ksplitSource<W>(p, out ? m0 + row : M, n0 + col, nEnd, c);
+  ksplitSource(p, out ? m0 + row : M, n0 + col, nEnd, c);
 #pragma unroll 1
   for (; s < last; s += 2 * kKsplitWaves) {
     stage(Set0{}, s);
@@ -390,50 +383,31 @@ __global__ __launch_bounds__(kKsplitThreads, 2) void gemmKsplitKernel(
     for (int j = 0; j < NB; j++)
       *reinterpret_cast<float4v *>(mine + (i * 16 + l16) * ROW_B + (j * 16 + kb * 4) * 4) = acc[i][j];
   __syncthreads();
-  float v[W] = {};
+  float4v v = {0.f, 0.f, 0.f, 0.f};
   if (out) {
 #pragma unroll
     for (int w = 0; w < kKsplitWaves; w++)
-#pragma unroll
-      for (int q = 0; q < W / 4; q++) {
-        const float4v x = *reinterpret_cast<const float4v *>(smem + w * WAVE_BYTES + row * ROW_B +
-                                                             (col + q * 4) * 4);
-#pragma unroll
-        for (int e = 0; e < 4; e++)
-          v[q * 4 + e] += x[e];
-      }
+      v += *reinterpret_cast<const float4v *>(smem + w * WAVE_BYTES + row * ROW_B + col * 4);
   }
   const int numSlices = gridDim.y;
   if (numSlices > 1) {
-    // (workspace: W values per finishing thread, slices of a tile one after the other)
+    // (workspace: a vector per finishing thread, slices of a tile one after the other)
     const int tile = m0 / MT + n0 / COLS * p.tilesM;
-    constexpr int kPerSlice = MT * NT / 4; // float4
-    float4v *part = reinterpret_cast<float4v *>(p.workspace) + int64_t(tile) * numSlices * kPerSlice;
-    if (out) {
-#pragma unroll
-      for (int q = 0; q < W / 4; q++)
-        part[slice * kPerSlice + q * (MT * OPR) + tid] =
-            float4v{v[q * 4], v[q * 4 + 1], v[q * 4 + 2], v[q * 4 + 3]};
-    }
+    float4v *part = reinterpret_cast<float4v *>(p.workspace) + int64_t(tile) * numSlices * kFinish;
+    if (out)
+      part[slice * kFinish + tid] = v;
     if (p.tileArrivals == nullptr || !arriveAtTile(p, tile, numSlices, tid, smem))
       return;
     if (out) {
-#pragma unroll
-      for (int e = 0; e < W; e++)
-        v[e] = 0.f;
+      v = float4v{0.f, 0.f, 0.f, 0.f};
 #pragma unroll 4
       for (int sl = 0; sl < numSlices; sl++)
-#pragma unroll
-        for (int q = 0; q < W / 4; q++) {
-          const float4v x = part[sl * kPerSlice + q * (MT * OPR) + tid];
-#pragma unroll
-          for (int e = 0; e < 4; e++)
-            v[q * 4 + e] += x[e];
-        }
+        v += part[sl * kFinish + tid];
     }
   }
   if (out && m0 + row < M && n0 + col < nEnd)
-    ksplitFinish<W>(p, activation, m0 + row, n0 + col, nEnd, COLS == NT && p.ldd % 8 == 0, v, c);
+    ksplitFinish(p, activation, m0 + row, n0 + col, nEnd, COLS == NT && p.ldd % 8 == 0,
+                 {v[0], v[1], v[2], v[3]}, c);
 }
 
 // The slices of a split-K launch, where the last workgroup to arrive does not add
@@ -441,30 +415,24 @@ __global__ __launch_bounds__(kKsplitThreads, 2) void gemmKsplitKernel(
 template <int MB, int NB>
 __global__ __launch_bounds__(256) void ksplitReduceKernel(GemmParams p, int numSlices, int activation,
                                                        int cols) {
-  constexpr int MT = MB * 16, NT = NB * 16, W = ksplitOutWidth<MB, NB>();
-  constexpr int OPR = NT / W, kFinish = MT * OPR, kPerSlice = MT * NT / 4;
+  constexpr int MT = MB * 16, NT = NB * 16;
+  constexpr int OPR = NT / kKsplitOut, kFinish = MT * OPR;
   const int64_t idx = int64_t(blockIdx.x) * 256 + threadIdx.x;
   if (idx >= int64_t(p.tilesM) * p.tilesN * kFinish)
     return;
   const int tile = int(idx / kFinish), t = int(idx % kFinish);
-  const int m = tile % p.tilesM * MT + t / OPR, n0 = tile / p.tilesM * cols, n = n0 + t % OPR * W;
+  const int m = tile % p.tilesM * MT + t / OPR, n0 = tile / p.tilesM * cols, n = n0 + t % OPR * kKsplitOut;
   const int nEnd = n0 + cols < p.N ? n0 + cols : p.N;
   if (m >= p.M || n >= nEnd)
     return;
-  _Float16 c[W];
-  ksplitSource<W>(p, m, n, nEnd, c);
-  const float4v *part = reinterpret_cast<const float4v *>(p.workspace) + int64_t(tile) * numSlices * kPerSlice;
-  float v[W] = {};
+  _Float16 c[kKsplitOut];
+  ksplitSource(p, m, n, nEnd, c);
+  const float4v *part = reinterpret_cast<const float4v *>(p.workspace) + int64_t(tile) * numSlices * kFinish;
+  float4v v = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll 4
   for (int sl = 0; sl < numSlices; sl++)
-#pragma unroll
-    for (int q = 0; q < W / 4; q++) {
-      const float4v x = part[sl * kPerSlice + q * kFinish + t];
-#pragma unroll
-      for (int e = 0; e < 4; e++)
-        v[q * 4 + e] += x[e];
-    }
-  ksplitFinish<W>(p, activation, m, n, nEnd, cols == NT && p.ldd % 8 == 0, v, c);
+    v += part[sl * kFinish + t];
+  ksplitFinish(p, activation, m, n, nEnd, cols == NT && p.ldd % 8 == 0, {v[0], v[1], v[2], v[3]}, c);
 }
 
 template <int MB, int NB, bool B_NK>
@@ -523,7 +491,7 @@ Status launchKsplit(const GemmProblem &pr, int activation, hipStream_t s) {
       r.chunkN, r.xmLog, q.kTilesPerSlice, activation, q);
   HOM_HIP_RET(hipGetLastError(), Status::kInternal);
   if (plan.splitK > 1 && !sumInKernel) {
-    const int64_t threads = plan.nTiles * (MT * NT / ksplitOutWidth<MB, NB>());
+    const int64_t threads = plan.nTiles * (MT * NT / kKsplitOut);
     ksplitReduceKernel<MB, NB><<<dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s>>>(
         plan.p, plan.splitK, activation, cols);
     HOM_HIP_RET(hipGetLastError(), Status::kInternal);

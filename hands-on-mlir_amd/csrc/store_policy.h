@@ -8,10 +8,11 @@
 // the end-of-kernel write-back finds nothing to do.  On the BERT-base encoder
 // (88 dependent launches of a few microseconds each) this takes 4 % off a
 // forward pass and 0.9 us off the 1024 x 3072 GEMM.  It pays for 16-byte
-// stores that together cover whole 64-byte segments; scattered 8-byte stores
-// (the attention output, the split-K reduction) and the 4-byte stores of
-// outputs whose rows are not 16-byte aligned got slower (1024 x 30522: 77 ->
-// 106 us) and keep the default policy.
+// stores that together cover whole 64-byte segments, and for the 8-byte stores of
+// gemm_ksplit.h, sixteen lanes of which write a line; scattered 8-byte stores (the
+// split-K reduction of the slab pipelines) and the 4-byte stores of outputs whose
+// rows are not 16-byte aligned got slower (1024 x 30522: 77 -> 106 us) and keep the
+// default policy, as does the attention output (see storeVector() there).
 #pragma once
 
 #include <hip/hip_runtime.h>
