@@ -78,11 +78,14 @@ template <int D> __device__ __forceinline__ int swzV(int k, int group) {
   return D == 64 || D == 192 ? group ^ ((k >> 1) & 1) : group ^ (k & 3);
 }
 
-// 16 bytes of the result, which starts on an 8-byte boundary: the hardware takes that, a
-// C++ store of the type would promise 16.  Default policy: written through,
-// BERT-base 1 x 64 took 265 us a request instead of 263, also in fragment order.
+// 16 bytes of the result, which starts on an 8-byte boundary: the hardware takes that,
+// and the type promises no more.  (As inline assembly the stores stayed in source
+// order with an address each: in fragment order 1 x 64 x 12 heads 3.28 us with 8-byte
+// stores, 3.35 so, 3.28 now.)  Default policy: written through, BERT-base 1 x 64 took
+// 265 us a request instead of 263, also in fragment order.
 __device__ __forceinline__ void storeVector(_Float16 *p, u32x4 v) {
-  asm volatile("global_store_dwordx4 %0, %1, off\n\ts_nop 1" : : "v"(p), "v"(v) : "memory");
+  typedef u32x4 onEight __attribute__((aligned(8)));
+  *reinterpret_cast<onEight *>(p) = v;
 }
 
 // NW wavefronts per workgroup, KS of them share each group of 32 query rows
@@ -106,10 +109,11 @@ __attribute__((amdgpu_waves_per_eu(D <= 128 || NW == 8 ? 2 : 1, D == 64 && KS ==
   constexpr int kChunk = DMA ? 64 : Chunk<D>::value;
   constexpr int SBW = DMA && KS == 2 ? 1 : 2; // 32-key sub-blocks a wavefront takes at a time
   // A wavefront at its MFMAs goes first, so that the other one of the SIMD is at its
-  // softmax meanwhile (head size 64: 20 x 700 x 12 27.3 -> 26.4 us, 32 x 512 x 16 37.3 ->
-  // 36.6; 128: equal; 192: 52.9 -> 53.3).
+  // softmax meanwhile (head size 64, chunks by DMA: 20 x 700 x 12 27.3 -> 26.4 us, 32 x 512
+  // x 16 37.3 -> 36.6; through registers 8 x 128 x 12 4.18 -> 4.25; head size 128: equal;
+  // 192: 52.9 -> 53.3).
   auto priority = [](auto pC) {
-    if constexpr (D == 64)
+    if constexpr (D == 64 && DMA)
       __builtin_amdgcn_s_setprio(decltype(pC)::value);
   };
   using First = std::integral_constant<int, 1>;
