@@ -79,10 +79,9 @@ template <int D> __device__ __forceinline__ int swzV(int k, int group) {
 }
 
 // 16 bytes of the result, which starts on an 8-byte boundary: the hardware takes that,
-// and the type promises no more.  (As inline assembly the stores stayed in source
-// order with an address each: in fragment order 1 x 64 x 12 heads 3.28 us with 8-byte
-// stores, 3.35 so, 3.28 now.)  Default policy: written through, BERT-base 1 x 64 took
-// 265 us a request instead of 263, also in fragment order.
+// and the type promises no more.  (As inline assembly the stores stay in source order
+// with an address each: 39 x 35 x 1 heads of 64 3.31 us, 3.27 so.)  Default policy:
+// written through, BERT-base 1 x 64 took 265 us a request instead of 263.
 __device__ __forceinline__ void storeVector(_Float16 *p, u32x4 v) {
   typedef u32x4 onEight __attribute__((aligned(8)));
   *reinterpret_cast<onEight *>(p) = v;
@@ -109,9 +108,9 @@ __attribute__((amdgpu_waves_per_eu(D <= 128 || NW == 8 ? 2 : 1, D == 64 && KS ==
   constexpr int kChunk = DMA ? 64 : Chunk<D>::value;
   constexpr int SBW = DMA && KS == 2 ? 1 : 2; // 32-key sub-blocks a wavefront takes at a time
   // A wavefront at its MFMAs goes first, so that the other one of the SIMD is at its
-  // softmax meanwhile (head size 64, chunks by DMA: 20 x 700 x 12 27.3 -> 26.4 us, 32 x 512
-  // x 16 37.3 -> 36.6; through registers 8 x 128 x 12 4.18 -> 4.25; head size 128: equal;
-  // 192: 52.9 -> 53.3).
+  // softmax meanwhile (head size 64, chunks by DMA: 20 x 700 x 12 30.2 -> 29.1 us, 32 x 512
+  // x 16 equal; through registers 8 x 128 x 12 4.18 -> 4.25; head size 128: equal; 192:
+  // 52.9 -> 53.3).
   auto priority = [](auto pC) {
     if constexpr (D == 64 && DMA)
       __builtin_amdgcn_s_setprio(decltype(pC)::value);
@@ -708,8 +707,10 @@ __attribute__((amdgpu_waves_per_eu(D <= 128 || NW == 8 ? 2 : 1, D == 64 && KS ==
     const float inv = valid ? 1.0f / rowSum : 0.f;
     // Lane and lane ^ 32 hold the halves of the same 16 bytes: they swap them, and a
     // lane stores those of the even or of the odd eight columns.  (8 bytes a lane
-    // before: 8 x 384 x 16 heads of 128 17.8 -> 17.0 us, 32 x 512 x 16 of 64 39.3 -> 37.7,
-    // 8 x 200 x 8 of 192 12.9 -> 11.6, 8 x 384 x 16 of 256 36.4 -> 33.6.)
+    // before: 8 x 384 x 16 heads of 128 17.7 -> 16.5 us, 32 x 512 x 16 of 64 41.7 -> 39.0,
+    // 8 x 200 x 8 of 192 13.3 -> 11.9, 8 x 384 x 16 of 256 40.4 -> 37.1.)  In fragment
+    // order the 8-byte stores of a wavefront are whole runs of 256 bytes as they are:
+    // 32 x 46 x 12 4.37 us, with the swap 4.43.
     _Float16 *const o16 = oRow - hb * 4 + hb * oEight;
 #pragma unroll
     for (int d = 0; d < DB; d++)
@@ -722,8 +723,13 @@ __attribute__((amdgpu_waves_per_eu(D <= 128 || NW == 8 ? 2 : 1, D == 64 && KS ==
 #pragma unroll
           for (int e = 0; e < 4; e++)
             o[h][e] = valid ? _Float16(accO[d][(g + h) * 4 + e] * inv) : _Float16(0);
-        const u32x2 even = __builtin_bit_cast(u32x2, o[0]), odd = __builtin_bit_cast(u32x2, o[1]);
-        storeVector(o16 + d * oWide + g * oEight, joinHalves(even[0], even[1], odd[0], odd[1]));
+        if constexpr (PACKED_IN) {
+          *reinterpret_cast<half4 *>(oRow + d * oWide + g * oEight) = o[0];
+          *reinterpret_cast<half4 *>(oRow + d * oWide + (g + 1) * oEight) = o[1];
+        } else {
+          const u32x2 even = __builtin_bit_cast(u32x2, o[0]), odd = __builtin_bit_cast(u32x2, o[1]);
+          storeVector(o16 + d * oWide + g * oEight, joinHalves(even[0], even[1], odd[0], odd[1]));
+        }
       }
   }
 }

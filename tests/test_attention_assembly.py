@@ -80,9 +80,11 @@ def test_no_use_of_a_transposing_read_before_its_wait(assembly):
 def test_priorities_and_stores_by_variant(assembly):
     """Priorities are raised where the chunks come by DMA at head size 64, and nowhere else; results leave in stores that
     the compiler places, not in statements of their own."""
-    kernels = re.findall(r"^(_ZN3hom\S*bertAttentionKernelILi\d+ELi\d+ELi(\d+)ELb\dELb(\d)E\S*):\s*;.*?$(.*?)^\.Lfunc_end", assembly,
-                         re.M | re.S)
+    kernels = re.findall(r"^(_ZN3hom\S*bertAttentionKernelILi\d+ELi\d+ELi(\d+)ELb(\d)ELb(\d)E\S*):\s*;.*?$(.*?)^\.Lfunc_end",
+                         assembly, re.M | re.S)
     assert len(kernels) >= 12
-    for name, head, dma, body in kernels:
+    for name, head, fragments, dma, body in kernels:
         assert ("s_setprio" in body) == (head == "64" and dma == "1"), name
-        assert "global_store_dwordx4" in body and "#ASMSTART\n\tglobal_store" not in body, name
+        stores = re.findall(r"^\s+(global_store_\w+)", body, re.M)
+        assert stores and "#ASMSTART\n\tglobal_store" not in body, name
+        assert ("global_store_dwordx2" in stores) == (fragments == "1"), name
