@@ -178,8 +178,8 @@ Status launchGemmRowStats(const GemmProblem &p, _Float16 *var, _Float16 *mean, f
                 "gemm + row statistics: problem does not fit the fused kernels");
   // No source or a full matrix, on 128 x 128 tiles: the epilogue of the folded
   // layer norm with nothing folded in, which requests the source ahead of everything
-  // and adds up a tile's columns before it writes them (4096 x 1024 x 1024 17.4 -> 15.4
-  // us, 8192 x 768 x 768 with a source 25.0 -> 22.5, 3000 x 768 x 768 13.3 -> 11.8).  Others, a
+  // and adds up a tile's columns before it writes them (with a source 1024 x 3072 x 768
+  // 14.8 -> 12.7 us, 8192 x 768 x 768 25.0 -> 22.5, 4096 x 1024 x 1024 17.8 -> 16.8).  Others, a
   // bias row, small tiles (64 x 768 x 768 8.2 / 9.1) or 256 x 256 ones (whose registers do
   // not hold the source's vectors as well), write a partial sum per wavefront column,
   // also of those past N.
@@ -216,8 +216,8 @@ Status launchGemmRowAffine(const GemmProblem &p, const _Float16 *var, const _Flo
   // No source or a full matrix: the column sums are formed on the way, four dot
   // products per fragment of B in the shadow of its MFMAs; by a kernel of their own
   // they took 4.5 us of a launch.  With the pairs kept in LDS and the epilogue of
-  // the folded layer norm, us: 64 x 768 x 768 9.2 -> 6.2, 1024 x 4096 x 1024 17.8 -> 12.8,
-  // 4096 x 4096 x 1024 43.8 -> 39.2, 16384 x 4096 x 1024 156 -> 147.
+  // the folded layer norm, us: 64 x 768 x 768 9.2 -> 6.1, 1024 x 4096 x 1024 20.2 -> 14.5,
+  // 4096 x 4096 x 1024 45.5 -> 41.6, 16384 x 4096 x 1024 165 -> 152.
   if (foldFits(p))
     return launchPairFolded<kEpiRowAffineOwn>(edge, q, s);
   // A source of another form: the column sums by a kernel of their own, 128 rows of

@@ -20,8 +20,9 @@ namespace gemmk {
 // behind the only barrier and are added in wavefront order.
 //
 // Slab pipeline before, this kernel, three sets of operands in turn, us: 100 x 768 x
-// 768 5.8 -> 4.8, 256 x 704 x 1504 9.3 -> 6.1, 256 x 700 x 1500 11.6 -> 7.3, 64 x 1001 x
-// 1003 7.2 -> 5.7, 1000 x 333 x 2777 15.9 -> 14.6; 3.5 us of a launch are not the K loop.
+// 768 5.6 -> 4.5, 256 x 704 x 1504 9.4 -> 6.2, 256 x 700 x 1500 10.0 -> 7.4, 64 x 1001 x
+// 1003 6.6 -> 5.3, 1000 x 333 x 2777 14.3 -> 13.4; 3.5 us of a launch are not the K loop.
+// On rows on 16 bytes it takes seven slabs for that, see ksplitPays() in runners.cpp.
 //
 // A tile is 16 MB x 16 NB.  What bounds it is the CU's L1 (60 bytes a clock where
 // whole 128-byte lines are asked for), so a row-major B is not cut into tiles
@@ -34,14 +35,14 @@ namespace gemmk {
 //
 // VEC: rows on 16-byte boundaries and K a multiple of 8; otherwise rows of any length
 // from 8 values up.  Every load is of whole dwords, in the tensor or, as part of
-// its first or last dword, two bytes in front of it or behind it; what a vector of A (or of a [N, K] B) holds
-// behind the row's end is masked.  ODD_A, ODD_B: rows may start in the middle of a
+// its first or last dword, two bytes in front of it or behind it; what a vector of A
+// (or of a [N, K] B) holds behind the row's end is masked.  ODD_A, ODD_B: rows may start in the middle of a
 // dword.  16-byte loads from there run at 17 bytes a clock instead of 46, so such a
 // row is read from two bytes earlier and shifted into place, the last value of a
 // vector coming from the next lane's.  The last value of a row's 128 bytes would be
 // missing: slabs are of 63 k then, or tiles of a row-major B of 63 columns (a load of
 // that value for each row cost more: 64 lines for 128 bytes).
-// 33 x 1001 x 3001 on 16 x 64 tiles: 13.5 -> 8.7 us (33 x 1002 x 3002: 7.9 us).
+// 33 x 1001 x 3001 unsplit on 16 x 64 tiles: 13.5 -> 8.7 us (33 x 1002 x 3002: 7.9 us).
 //
 // Split-K across workgroups (gridDim.y): the slices of a tile share an XCD (the
 // grid's x extent is a multiple of eight) and the last to arrive adds them in
