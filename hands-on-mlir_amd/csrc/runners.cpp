@@ -427,10 +427,11 @@ bool ksplitFits(int64_t M, int64_t N) {
 // On few slabs they lie below those lines, with most of the wavefronts here idle: over
 // 300 problems, this kernel / the pipelines by slabs of K, rows on 16 bytes 1: 1.16, 2:
 // 1.09, 3: 1.06, 4: 1.01, 5: 1.06, 6: 1.02, 7: 0.98, 8: 0.96; rows of C and D off them 1:
-// 1.00 (0.89 .. 1.17), 2: 1.02, 3: 1.00, 4: 0.95; any alignment gains from the first.
+// 1.00 (0.89 .. 1.17), 2: 1.02, 3: 1.00, 4: 0.95; any alignment, N a multiple of 8: 1: 1.07,
+// 2: 1.01, 3: 0.94, else 1: 0.93.
 bool ksplitPays(int64_t M, int64_t N, int64_t K, Epilogue epi, int cls,
                 double pipe, int32_t pipeSplitK, int64_t *idx, int32_t *splitK) {
-  if (K <= (cls == 8 ? 6 * 64 : cls == 2 ? 3 * 64 : 0))
+  if (K <= 64 * (cls == 8 ? 6 : cls == 2 ? 3 : N % 8 == 0 ? 2 : 0))
     return false;
   int64_t i = -1;
   int32_t sk = 1;
