@@ -319,7 +319,7 @@ bool chooseGemm(HomBertEncoder *e, int64_t M, int64_t N, int64_t K, int64_t act,
     if (layout == -1 && nkAllowed && homGemmPrefersNvte(M, N, K, act))
       out->nk = true;
     else
-      homGemmSelectWithSource(M, N, K, act, 0, beta != 0.f, &idx, &sk);
+      homGemmSelectWithSource(M, N, K, act, 0, beta != 0.f ? 2 : 0, &idx, &sk);
   }
   out->gemmNum = out->nk ? 0 : int32_t(idx + 1);
   out->splitK = out->nk ? 1 : sk;

@@ -355,12 +355,15 @@ int32_t homGemmSelectNvte(int64_t M, int64_t N, int64_t K, int64_t activation,
 }
 
 int32_t homGemmSelectWithSource(int64_t M, int64_t N, int64_t K, int64_t activation,
-                                int32_t bIsNK, int32_t fullSource, int64_t *idx,
+                                int32_t bIsNK, int32_t source, int64_t *idx,
                                 int32_t *splitK) {
   int64_t i = -1;
   int32_t s = 1;
-  const bool tuned = bIsNK ? selectGemmNvte(M, N, K, activation, &i, &s, fullSource != 0)
-                           : selectGemm(M, N, K, activation, &i, &s, false, fullSource != 0);
+  const GemmSource src = source == 0   ? GemmSource::kNone
+                         : source == 1 ? GemmSource::kRow
+                                       : GemmSource::kMatrix;
+  const bool tuned = bIsNK ? selectGemmNvte(M, N, K, activation, &i, &s, src)
+                           : selectGemm(M, N, K, activation, &i, &s, false, src);
   if (idx)
     *idx = i;
   if (splitK)

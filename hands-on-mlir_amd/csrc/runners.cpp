@@ -192,6 +192,12 @@ bool kernelFits(const GemmKernelInfo &k, int cls) {
 // The kernels of gemm_ksplit.h: one wavefront computes the whole tile.
 bool wavesSplitK(const GemmKernelInfo &k) { return k.wavesM * k.wavesN == 1; }
 
+GemmSource sourceOf(const GemmProblem &p) {
+  return p.beta == 0.f        ? GemmSource::kNone
+         : p.cRowPeriod == 1 ? GemmSource::kRow
+                             : GemmSource::kMatrix;
+}
+
 // Kernel and split-K (stored into pr) the [N, K]-B path runs for a problem.
 int chooseNvteKernel(GemmProblem *pr, int64_t activation);
 
@@ -245,7 +251,7 @@ const std::vector<TileModel> &tileModels() {
 // and to 130 problems whose rows of C and D are not on 16 bytes, which cost the larger
 // tiles more (0.7 % off the best, the model below 10.7 %; 4622 x 502 x 272 with a source 64 x 64
 // 10.5 us, 64 x 128 13.3).
-bool modelFullChip(int64_t M, int64_t N, int64_t K, Epilogue epi, int cls, bool fullSource,
+bool modelFullChip(int64_t M, int64_t N, int64_t K, Epilogue epi, int cls, GemmSource source,
                    int64_t *idx, int32_t *splitK) {
   struct Fit {
     double fixed, slab, round, gelu, source, out, outSource, traffic;
@@ -271,6 +277,7 @@ bool modelFullChip(int64_t M, int64_t N, int64_t K, Epilogue epi, int cls, bool 
   const int cus = deviceInfo().computeUnits > 0 ? deviceInfo().computeUnits : 256;
   if (cls == 1 || ((M + 63) / 64) * ((N + 63) / 64) <= cus)
     return false;
+  const bool fullSource = source == GemmSource::kMatrix;
   double best = 1e300;
   const double outputs = double(M) * double(N) * 1e-6, slabs = double((K + 63) / 64);
   for (size_t t = 0; t < tileModels().size(); t++) {
@@ -426,12 +433,16 @@ bool ksplitFits(int64_t M, int64_t N) {
 // their model (fitted to one set of operands, aligned rows) by the lines below.
 // On few slabs they lie below those lines, with most of the wavefronts here idle: over
 // 300 problems, this kernel / the pipelines by slabs of K, rows on 16 bytes 1: 1.16, 2:
-// 1.09, 3: 1.06, 4: 1.01, 5: 1.06, 6: 1.02, 7: 0.98, 8: 0.96; rows of C and D off them 1:
-// 1.00 (0.89 .. 1.17), 2: 1.02, 3: 1.00, 4: 0.95; any alignment, N a multiple of 8: 1: 1.07,
-// 2: 1.01, 3: 0.94, else 1: 0.93.
-bool ksplitPays(int64_t M, int64_t N, int64_t K, Epilogue epi, int cls,
+// 1.09, 3: 1.06, 4: 1.01, 5: 1.06, 6: 1.02, 7: 0.98, 8: 0.96; rows of C and D off them,
+// up to 16 rows 1: 1.05, 2: 1.06, 3: 1.03, 4: 0.95, more rows without a source 1: 1.00, 2:
+// 1.00, 3: 0.96, with one 1: 0.93, 2: 0.83, 3: 0.83; any alignment, N a multiple of 8: 1:
+// 1.07, 2: 1.01, 3: 0.94, else 1: 0.93.
+bool ksplitPays(int64_t M, int64_t N, int64_t K, Epilogue epi, int cls, GemmSource source,
                 double pipe, int32_t pipeSplitK, int64_t *idx, int32_t *splitK) {
-  if (K <= 64 * (cls == 8 ? 6 : cls == 2 ? 3 : N % 8 == 0 ? 2 : 0))
+  const int few = cls == 8   ? 6
+                  : cls == 2 ? (M <= 16 ? 3 : source == GemmSource::kNone ? 2 : 0)
+                             : (N % 8 == 0 ? 2 : 0);
+  if (K <= 64 * few)
     return false;
   int64_t i = -1;
   int32_t sk = 1;
@@ -445,13 +456,13 @@ bool ksplitPays(int64_t M, int64_t N, int64_t K, Epilogue epi, int cls,
   return true;
 }
 
-void modelGemm(int64_t M, int64_t N, int64_t K, Epilogue epi, int cls, bool fullSource,
+void modelGemm(int64_t M, int64_t N, int64_t K, Epilogue epi, int cls, GemmSource source,
                int64_t *idx, int32_t *splitK) {
-  if (modelFullChip(M, N, K, epi, cls, fullSource, idx, splitK))
+  if (modelFullChip(M, N, K, epi, cls, source, idx, splitK))
     return;
   const double pipe = modelPipe(M, N, K, epi, cls, idx, splitK);
   if (ksplitFits(M, N))
-    ksplitPays(M, N, K, epi, cls, pipe, *splitK, idx, splitK);
+    ksplitPays(M, N, K, epi, cls, source, pipe, *splitK, idx, splitK);
 }
 
 } // namespace
@@ -478,7 +489,7 @@ bool gemmPrefersNvte(int64_t M, int64_t N, int64_t K, int64_t activation) {
 }
 
 bool selectGemm(int64_t M, int64_t N, int64_t K, int64_t activation,
-                int64_t *idx, int32_t *splitK, bool bIsNK, bool fullSource) {
+                int64_t *idx, int32_t *splitK, bool bIsNK, GemmSource source) {
   const Epilogue epi = epilogueFor(activation, false);
   if (const TunedEntry *t = findTuned(M, N, K, activation)) {
     const int nk = bIsNK ? kernelByName(t->nkKernel) : -1;
@@ -489,7 +500,7 @@ bool selectGemm(int64_t M, int64_t N, int64_t K, int64_t activation,
       return true;
     }
   }
-  modelGemm(M, N, K, epi, naturalClass(N, K), fullSource, idx, splitK);
+  modelGemm(M, N, K, epi, naturalClass(N, K), source, idx, splitK);
   return false;
 }
 
@@ -528,11 +539,11 @@ Status runGemmManifest(int64_t rankA, void *dstA, int64_t rankB, void *dstB,
                   "gemm: negative kernel number %d", gemmNum);
     int64_t sel;
     int32_t sk;
-    const bool fullSource = beta != 0.f && pr.cRowPeriod > 1;
-    selectGemm(pr.M, pr.N, pr.K, activation, &sel, &sk, false, fullSource);
+    const GemmSource source = sourceOf(pr);
+    selectGemm(pr.M, pr.N, pr.K, activation, &sel, &sk, false, source);
     const int cls = alignmentClass(pr);
     if (!kernelFits(gemmKernelInfo(int(sel)), cls))
-      modelGemm(pr.M, pr.N, pr.K, gemmKernelInfo(int(sel)).epilogue, cls, fullSource, &sel,
+      modelGemm(pr.M, pr.N, pr.K, gemmKernelInfo(int(sel)).epilogue, cls, source, &sel,
                 &sk);
     idx = int(sel);
     pr.splitK = sk;
@@ -554,10 +565,10 @@ Status runGemmManifest(int64_t rankA, void *dstA, int64_t rankB, void *dstB,
 }
 
 bool selectGemmNvte(int64_t M, int64_t N, int64_t K, int64_t activation,
-                    int64_t *idx, int32_t *splitK, bool fullSource) {
+                    int64_t *idx, int32_t *splitK, GemmSource source) {
   const Epilogue epi = epilogueFor(activation, true);
   return selectGemm(M, N, K, epi == Epilogue::kGeluTanh ? 2 : activation, idx,
-                    splitK, true, fullSource);
+                    splitK, true, source);
 }
 
 namespace {
@@ -565,8 +576,8 @@ int chooseNvteKernel(GemmProblem *pr, int64_t activation) {
   int64_t sel;
   int32_t sk;
   const Epilogue epi = epilogueFor(activation, true);
-  const bool fullSource = pr->beta != 0.f && pr->cRowPeriod > 1;
-  selectGemmNvte(pr->M, pr->N, pr->K, activation, &sel, &sk, fullSource);
+  const GemmSource source = sourceOf(*pr);
+  selectGemmNvte(pr->M, pr->N, pr->K, activation, &sel, &sk, source);
   int idx = int(sel);
   pr->splitK = sk;
   // Profiling knob: HOM_NVTE_GEMM_KERNEL="<manifest name>[,<splitK>]" pins the
@@ -583,7 +594,7 @@ int chooseNvteKernel(GemmProblem *pr, int64_t activation) {
   }
   const int cls = alignmentClass(*pr);
   if (!kernelFits(gemmKernelInfo(idx), cls)) {
-    modelGemm(pr->M, pr->N, pr->K, epi, cls, fullSource, &sel, &sk);
+    modelGemm(pr->M, pr->N, pr->K, epi, cls, source, &sel, &sk);
     idx = int(sel);
     pr->splitK = sk;
   }

@@ -59,16 +59,19 @@ Status runPackedGemm(int64_t rankA, void *dstA, const void *packedB, int64_t ran
                      const void *ahead, int64_t aheadBytes);
 Status runColumnSums(int64_t rankB, void *dstB, float *out);
 
+// What beta C reads: nothing, a bias row, as much as D writes.
+enum class GemmSource { kNone, kRow, kMatrix };
+
 // Kernel choice without timing: tuned table first, timing models otherwise.
 // `activation`: 0 linear, 1 GELU (erf), 2 GELU (tanh).  Returns true when the
-// shape was found in the tuned table.  fullSource: beta C reads as much as D writes.
+// shape was found in the tuned table.
 bool selectGemm(int64_t M, int64_t N, int64_t K, int64_t activation,
                 int64_t *idx, int32_t *splitK, bool bIsNK = false,
-                bool fullSource = false);
+                GemmSource source = GemmSource::kNone);
 // What nvteGemmF16 runs for a shape (B as [N, K]; activation 1 is the tanh
 // form there), before the per-call alignment fallback.
 bool selectGemmNvte(int64_t M, int64_t N, int64_t K, int64_t activation,
-                    int64_t *idx, int32_t *splitK, bool fullSource = false);
+                    int64_t *idx, int32_t *splitK, GemmSource source = GemmSource::kNone);
 // Whether the tuned table says that, for this shape, the [N, K] path of
 // nvteGemmF16 beats every manifest kernel on row-major B (what the reference's
 // profiler reports as index -1).

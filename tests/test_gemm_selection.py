@@ -62,7 +62,11 @@ def test_few_slabs_stay_with_the_pipelines(rt, M, N, select):
     lib = rt.load_runtime()
     split = lambda n, K: "k8_w1x1_" in lib.homGemmManifestName(choice(lib, select, M, n, K, 0)[0]).decode()  # noqa: E731
     assert [split(N, K) for K in (8, 80, 136, 264, 384, 512, 696)] == [False] * 5 + [True] * 2
-    assert [split(N + 2, K) for K in (80, 192, 384, 512)] == [False] * 2 + [True] * 2
+    assert [split(N + 2, K) for K in (80, 128, 192, 384, 512)] == [False] * 2 + [M > 16] + [True] * 2
+    for source in (1, 2):  # which costs the pipelines more where the rows of C and D are off 16 bytes and not a few
+        idx, sk = ctypes.c_int64(-1), ctypes.c_int32(0)
+        lib.homGemmSelectWithSource(M, N + 2, 80, 0, int(select.endswith("Nvte")), source, ctypes.byref(idx), ctypes.byref(sk))
+        assert ("k8_w1x1_" in lib.homGemmManifestName(idx.value).decode()) == (M > 16)
     assert split(N + 1, 63) and split(N + 2, 93)  # (any alignment)
     assert not split(N, 60) and not split(N, 85) and split(N, 133)
 
@@ -92,7 +96,7 @@ def test_large_problems_take_a_fast_tile(rt, M, N, K, act, tiles):
 def test_a_source_is_priced(rt, M, N, K, act, without, tile, nk):
     lib = rt.load_runtime()
     idx, sk = ctypes.c_int64(-1), ctypes.c_int32(0)
-    for source, expected in ((0, without), (1, tile)):
+    for source, expected in ((0, without), (1, without), (2, tile)):
         assert lib.homGemmSelectWithSource(M, N, K, act, nk, source, ctypes.byref(idx), ctypes.byref(sk)) == 0
         assert f"f16_{expected}_64x2r" in lib.homGemmManifestName(idx.value).decode()
         if not source:
