@@ -273,7 +273,7 @@ __global__ __launch_bounds__(WM *WN *kWave) void gemmPipeKernel(
   };
   // The partial slab, behind the full ones, with a range test per vector.  ANY:
   // elements of a vector inside the range: none, 8, or the last 1..7, which are
-  // read ending at the last one and shifted down (EARLY: when they are needed).
+  // read ending at the last one and shifted down when they are needed.
   auto tailInside = [&](bool isA, int i) -> int {
     const int k = (ktBegin + nkFull) * BK + (isA ? aK[i] : bK[i]);
     if (isA || B_NK)
@@ -285,10 +285,9 @@ __global__ __launch_bounds__(WM *WN *kWave) void gemmPipeKernel(
     if constexpr (ANY) {
       auto fetch = [&](auto rsrc, uint32_t off, int inside) {
         const int back = inside > 0 && inside < 8 ? 8 - inside : 0;
-        const half8 v = __builtin_bit_cast(
+        return __builtin_bit_cast(
             half8, __builtin_amdgcn_raw_buffer_load_b128(
                        rsrc, inside > 0 ? off - uint32_t(back) * 2u : kOob, 0, 0));
-        return !EARLY && back > 0 ? shiftDown(v, inside) : v;
       };
 #pragma unroll
       for (int i = 0; i < A_PER_T; i++)
@@ -757,6 +756,18 @@ __global__ __launch_bounds__(WM *WN *kWave) void gemmPipeKernel(
     } else {
       loadTail(regA[0], regB[0]);
       __syncthreads(); // no wavefront still reads a full slab from buffer 0
+      // (the loads are on their way across the barrier: 10992 x 1487 x 39, [N, K], 22.4
+      // us with the shifts in front of it, 20.0)
+      if constexpr (ANY) {
+#pragma unroll
+        for (int i = 0; i < A_PER_T; i++)
+          if (tailInside(true, i) > 0 && tailInside(true, i) < 8)
+            regA[0][i] = shiftDown(regA[0][i], tailInside(true, i));
+#pragma unroll
+        for (int i = 0; i < B_PER_T; i++)
+          if (tailInside(false, i) > 0 && tailInside(false, i) < 8)
+            regB[0][i] = shiftDown(regB[0][i], tailInside(false, i));
+      }
       storeLds(0, regA[0], regB[0]);
     }
     __syncthreads();
@@ -906,7 +917,8 @@ Status launchPipe(const GemmProblem &pr, hipStream_t s) {
     return Status::kSuccess;
   // The smallest tiles the library chooses request a partial slab early (with a
   // row-major B at any alignment there always is one) where all workgroups are
-  // resident at once all the same.  Late against early, three sets of operands in
+  // resident at once all the same, or where it costs no wavefront ([N, K] at any
+  // alignment: 4466 x 1036 x 396 15.9 -> 15.3).  Late against early, three sets of operands in
   // turn, us: 1000 x 1001 x 1003 9.5 -> 9.1, 1200 x 1201 x 1001 14.4 -> 14.0, 600 x 600 x 600
   // 4.8 -> 4.7, 1200 x 1200 x 1000 equal.  Early kernels for everything lost their third
   // wavefront: 1400 x 1400 x 704, without a partial slab, 8.2 -> 8.4.  128 x 128 tiles lose
@@ -916,9 +928,11 @@ Status launchPipe(const GemmProblem &pr, hipStream_t s) {
         gemmPipeKernel<BM, BN, WM, WN, DIST, EPI, B_NK, DMA, ANY, true>, false, 0};
     if (pr.K % 64 != 0 || (ANY && !B_NK)) {
       st = prepare(&early);
+      if (st == Status::kSuccess)
+        st = prepare(&late);
       if (st != Status::kSuccess)
         return st;
-      if (plan.nTiles * plan.splitK <= early.resident)
+      if (plan.nTiles * plan.splitK <= early.resident || early.resident >= late.resident)
         use = &early;
     }
   }

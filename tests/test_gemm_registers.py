@@ -9,10 +9,10 @@ import pytest
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 CSRC = os.path.join(ROOT, "hands-on-mlir_amd", "csrc")
 
-# (slabs in flight, epilogue, [N, K] weights, staged by DMA, any alignment) -> wavefronts per SIMD
-KERNELS = {(2, 0, 0, 0, 0): 3, (2, 0, 1, 0, 0): 3, (2, 1, 0, 0, 0): 3, (2, 2, 1, 0, 0): 3, (2, 0, 0, 0, 1): 3,
-           (2, 0, 1, 0, 1): 3, (2, 1, 0, 0, 1): 3, (3, 0, 0, 1, 0): 4, (3, 0, 1, 1, 0): 4, (2, 3, 0, 0, 0): 4,
-           (2, 4, 0, 0, 0): 4}
+# (slabs in flight, epilogue, [N, K] weights, staged by DMA, any alignment, early partial slab) -> wavefronts per SIMD
+KERNELS = {(2, 0, 0, 0, 0, 0): 3, (2, 0, 1, 0, 0, 0): 3, (2, 1, 0, 0, 0, 0): 3, (2, 2, 1, 0, 0, 0): 3, (2, 0, 0, 0, 1, 0): 3,
+           (2, 0, 1, 0, 1, 0): 3, (2, 1, 0, 0, 1, 0): 3, (3, 0, 0, 1, 0, 0): 4, (3, 0, 1, 1, 0, 0): 4, (2, 3, 0, 0, 0, 0): 4,
+           (2, 4, 0, 0, 0, 0): 4, (2, 0, 0, 0, 0, 1): 2, (2, 0, 0, 0, 1, 1): 2, (2, 0, 1, 0, 1, 1): 3, (2, 1, 1, 0, 1, 1): 3}
 
 
 @pytest.fixture(scope="module")
@@ -23,17 +23,18 @@ def registers(tmp_path_factory):
     path = tmp_path_factory.mktemp("asm")
     source, out = path / "kernels.hip", path / "kernels.s"
     bools = ("false", "true")
-    lines = [f"template __global__ void gemmPipeKernel<64, 64, 2, 2, {d}, {e}, {bools[nk]}, {bools[dma]}, {bools[any_]}>("
+    lines = [f"template __global__ void gemmPipeKernel<64, 64, 2, 2, {d}, {e}, {bools[nk]}, {bools[dma]}, {bools[any_]}, "
+             f"{bools[early]}>("
              "const _Float16 *, const _Float16 *, int, int, int, int, int, int, int, uint32_t, uint32_t, int, GemmParams);"
-             for d, e, nk, dma, any_ in KERNELS]
+             for d, e, nk, dma, any_, early in KERNELS]
     source.write_text("\n".join(['#include "gemm_pipe.h"', "namespace hom { namespace gemmk {", *lines, "} }"]))
     res = subprocess.run(flags.stdout.split() + ["--offload-device-only", "-S", "-I", CSRC, str(source), "-o", str(out)],
                          capture_output=True, text=True, timeout=600)
     assert res.returncode == 0, res.stderr
     found = {}
     for name, body in re.findall(r"\.amdhsa_kernel (\S+)(.*?)\.end_amdhsa_kernel", out.read_text(), re.S):
-        d, e, nk, dma, any_ = re.search(r"gemmPipeKernelILi64ELi64ELi2ELi2ELi(\d)ELi(\d)ELb(\d)ELb(\d)ELb(\d)E", name).groups()
-        found[tuple(map(int, (d, e, nk, dma, any_)))] = int(re.search(r"next_free_vgpr (\d+)", body).group(1))
+        key = re.search(r"gemmPipeKernelILi64ELi64ELi2ELi2ELi(\d)ELi(\d)ELb(\d)ELb(\d)ELb(\d)ELb(\d)E", name).groups()
+        found[tuple(map(int, key))] = int(re.search(r"next_free_vgpr (\d+)", body).group(1))
     return found
 
 
