@@ -61,6 +61,16 @@ __device__ __forceinline__ lanes4 splitHalves(lanes4 v) {
   const auto b = __builtin_amdgcn_permlane32_swap(v[1], v[3], false, false);
   return lanes4{a[0], b[0], a[1], b[1]};
 }
+// Rows of 16 lanes: the odd ones of a against the even ones of b (its own inverse).
+typedef uint32_t lanes2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ void swapRows(lanes4 &a, lanes4 &b) {
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const auto r = __builtin_amdgcn_permlane16_swap(a[i], b[i], false, false);
+    a[i] = r[0];
+    b[i] = r[1];
+  }
+}
 // v_permlane16_swap exchanges the odd rows of its first operand with the even
 // rows of its second: the same value twice gives (even-row values, odd-row
 // values) in every lane pair (l, l ^ 16).

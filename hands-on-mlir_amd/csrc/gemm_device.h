@@ -523,6 +523,100 @@ epilogueFast(const GemmParams &p, float16v (&acc)[MI][NI], int m0, int n0,
 }
 
 
+// The same result without LDS: the arithmetic runs in accumulator order, then lanes
+// 32 apart exchange halves (joinHalves) and rows of 16 lanes change places (swapRows),
+// so that a lane has 8 consecutive columns and a store instruction writes 64 bytes of
+// 16 rows.  No barrier, and a wavefront's stores go out while others still multiply.
+template <int MI, int NI, int WTM, int WTN, int EPI, int CMODE>
+__device__ __forceinline__ void
+epilogueLanes(const GemmParams &p, float16v (&acc)[MI][NI], int m0, int n0,
+              int waveM, int waveN, int lane) {
+  constexpr uint32_t kOob = 0x80000000u;
+  const int l16 = lane % 16, kb = lane / 32;
+  // columns of this lane's 16 bytes in a block of 32
+  const int cc = (lane / 16 % 2) * 16 + kb * 8;
+  const int rowBase = m0 + waveM * WTM;
+  const int colBase = n0 + waveN * WTN;
+  auto clampBytes = [](int64_t b) -> int32_t {
+    return b > 0x7fffffffLL ? 0x7fffffff : (b < 0 ? 0 : int32_t(b));
+  };
+  const int rowsLeft = p.M - rowBase;
+  const auto rsrcD = __builtin_amdgcn_make_buffer_rsrc(
+      p.D + int64_t(rowBase) * p.ldd + colBase, 0,
+      clampBytes((int64_t(rowsLeft) * p.ldd - colBase) * 2), 0x00020000);
+  const uint32_t ldd2 = uint32_t(p.ldd) * 2u, ldc2 = uint32_t(p.ldc) * 2u;
+  auto offsetOf = [&](int i, int j, int h, uint32_t ld2) { // rows 16 h .. of block (i, j)
+    return colBase + j * 32 + cc < p.N
+               ? uint32_t(i * 32 + h * 16 + l16) * ld2 + uint32_t(j * 32 + cc) * 2u
+               : kOob;
+  };
+  half4 bias[CMODE == 1 ? NI : 1][4];
+  lanes4 cv[CMODE == 2 ? MI : 1][CMODE == 2 ? NI : 1][2];
+  if constexpr (CMODE == 1) {
+    const auto rsrcC = __builtin_amdgcn_make_buffer_rsrc(const_cast<_Float16 *>(p.C), 0, p.N * 2,
+                                                         0x00020000);
+#pragma unroll
+    for (int j = 0; j < NI; j++)
+#pragma unroll
+      for (int g = 0; g < 4; g++)
+        bias[j][g] = __builtin_bit_cast(
+            half4, __builtin_amdgcn_raw_buffer_load_b64(
+                       rsrcC, uint32_t(colBase + j * 32 + g * 8 + kb * 4) * 2u, 0, 0));
+  } else if constexpr (CMODE == 2) {
+    const auto rsrcC = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<_Float16 *>(p.C) + int64_t(rowBase) * p.ldc + colBase, 0,
+        clampBytes((int64_t(rowsLeft) * p.ldc - colBase) * 2), 0x00020000);
+#pragma unroll
+    for (int i = 0; i < MI; i++)
+#pragma unroll
+      for (int j = 0; j < NI; j++)
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+          cv[i][j][h] = __builtin_bit_cast(
+              lanes4, __builtin_amdgcn_raw_buffer_load_b128(rsrcC, offsetOf(i, j, h, ldc2), 0, 0));
+  }
+#pragma unroll
+  for (int i = 0; i < MI; i++)
+#pragma unroll
+    for (int j = 0; j < NI; j++) {
+      half4 c[4] = {};
+      if constexpr (CMODE == 1) {
+#pragma unroll
+        for (int g = 0; g < 4; g++)
+          c[g] = bias[j][g];
+      }
+      if constexpr (CMODE == 2) {
+        lanes4 lo = cv[i][j][0], hi = cv[i][j][1];
+        swapRows(lo, hi);
+        const lanes4 a = splitHalves(lo), b = splitHalves(hi);
+        c[0] = __builtin_bit_cast(half4, lanes2{a[0], a[1]});
+        c[1] = __builtin_bit_cast(half4, lanes2{a[2], a[3]});
+        c[2] = __builtin_bit_cast(half4, lanes2{b[0], b[1]});
+        c[3] = __builtin_bit_cast(half4, lanes2{b[2], b[3]});
+      }
+      lanes2 o[4];
+#pragma unroll
+      for (int g = 0; g < 4; g++) {
+        half4 r;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          float v = p.alpha * acc[i][j][4 * g + e];
+          if constexpr (CMODE != 0)
+            v = fmaf(p.beta, float(c[g][e]), v);
+          r[e] = _Float16(activate<EPI>(v));
+        }
+        o[g] = __builtin_bit_cast(lanes2, r);
+      }
+      // lower lanes columns 0 .. 7 and 16 .. 23, upper lanes 8 .. 15 and 24 .. 31 of row lane % 32;
+      // then of rows 0 .. 15 and 16 .. 31
+      lanes4 lo = joinHalves(o[0][0], o[0][1], o[1][0], o[1][1]);
+      lanes4 hi = joinHalves(o[2][0], o[2][1], o[3][0], o[3][1]);
+      swapRows(lo, hi);
+      __builtin_amdgcn_raw_buffer_store_b128(lo, rsrcD, offsetOf(i, j, 0, ldd2), 0, kWriteThroughAux);
+      __builtin_amdgcn_raw_buffer_store_b128(hi, rsrcD, offsetOf(i, j, 1, ldd2), 0, kWriteThroughAux);
+    }
+}
+
 // (rstd, -mean * rstd) of row m0 + tid of a folded layer norm, for the first BM
 // threads of the workgroup, in two steps: foldRowStatRequest asks for the
 // row's first pieces (no branch around a load: an index past the last piece
@@ -797,23 +891,61 @@ __host__ __device__ __forceinline__ int epilogueFastMode(const GemmParams &p,
   return -1;
 }
 
-// Dispatch: the fast epilogue where it applies, the general one otherwise.
-template <int MI, int NI, int WTM, int WTN, int EPI>
+// Whether a tile's results leave by lane exchanges (epilogueLanes) or through the
+// wavefronts' strips of LDS (epilogueFast), by wave tile, source and activation.
+// Lanes against strips, time of the launch, three shapes each:
+//   128 x 64 (256 x 256 tiles, eight wavefronts): DMA staged -1 .. -7 %, with a full
+//     source -7 .. -19; STAGED through registers, linear -9 .. -18 without a source, -1 .. -14
+//     with a full one, -7 .. +6 with a bias row, GELU +2 .. +6 with a bias row.  (One way for all sources of a
+//     kernel: with both in it, it spills as it did before and gains nothing.)
+//   64 x 64: GELU without a full source -1 .. -5; linear -7 .. +5 either way.
+//   64 x 32: -1 without a source, -1 .. -6 with a bias row, +1 .. +8 with a full one.
+//   32 x 96, 64 x 96: GELU -3 .. -9 (full source 0 .. -6), linear 0 .. +3.
+//   32 x 32: linear with a bias row -1 .. -4, else 0 .. +8, and four registers more, which cost some
+//     kernels their third wavefront per SIMD.
+//   128 x 128 (512 registers): 1.2 .. 2 times as long, what is exchanged no longer fits.
+template <int MI, int NI, int EPI, int CMODE, bool STAGED> constexpr bool leavesByLanes() {
+  constexpr bool gelu = EPI != int(Epilogue::kLinear);
+  if (MI == 4 && NI == 2)
+    return !STAGED || !gelu;
+  if (MI == 2 && NI == 2)
+    return gelu && CMODE != 2;
+  if (MI == 2 && NI == 1)
+    return CMODE != 2;
+  if (NI == 3)
+    return gelu;
+  return false;
+}
+
+// Dispatch: the fast epilogues where they apply, the general one otherwise.
+template <int MI, int NI, int WTM, int WTN, int EPI, bool STAGED = false>
 __device__ __forceinline__ void
 epilogueAuto(const GemmParams &p, float16v (&acc)[MI][NI], int m0, int n0,
              int waveM, int waveN, int lane, int wave, unsigned char *smem) {
   static_assert(EPI < kEpiFoldA, "folded epilogues are called directly");
   if constexpr (EPI <= int(Epilogue::kGeluTanh)) {
     const int mode = p.epiMode;
-    if (mode == 0)
-      return epilogueFast<MI, NI, WTM, WTN, EPI, 0>(p, acc, m0, n0, waveM, waveN,
-                                                    lane, wave, smem);
-    if (mode == 1)
-      return epilogueFast<MI, NI, WTM, WTN, EPI, 1>(p, acc, m0, n0, waveM, waveN,
-                                                    lane, wave, smem);
-    if (mode == 2)
-      return epilogueFast<MI, NI, WTM, WTN, EPI, 2>(p, acc, m0, n0, waveM, waveN,
-                                                    lane, wave, smem);
+    if (mode == 0) {
+      if constexpr (leavesByLanes<MI, NI, EPI, 0, STAGED>())
+        return epilogueLanes<MI, NI, WTM, WTN, EPI, 0>(p, acc, m0, n0, waveM, waveN, lane);
+      else
+        return epilogueFast<MI, NI, WTM, WTN, EPI, 0>(p, acc, m0, n0, waveM, waveN,
+                                                      lane, wave, smem);
+    }
+    if (mode == 1) {
+      if constexpr (leavesByLanes<MI, NI, EPI, 1, STAGED>())
+        return epilogueLanes<MI, NI, WTM, WTN, EPI, 1>(p, acc, m0, n0, waveM, waveN, lane);
+      else
+        return epilogueFast<MI, NI, WTM, WTN, EPI, 1>(p, acc, m0, n0, waveM, waveN,
+                                                      lane, wave, smem);
+    }
+    if (mode == 2) {
+      if constexpr (leavesByLanes<MI, NI, EPI, 2, STAGED>())
+        return epilogueLanes<MI, NI, WTM, WTN, EPI, 2>(p, acc, m0, n0, waveM, waveN, lane);
+      else
+        return epilogueFast<MI, NI, WTM, WTN, EPI, 2>(p, acc, m0, n0, waveM, waveN,
+                                                      lane, wave, smem);
+    }
   }
   epilogueStoreLds<MI, NI, WTM, WTN, EPI>(p, acc, m0, n0, waveM, waveN, lane,
                                           wave, smem);

@@ -857,12 +857,12 @@ __global__ __launch_bounds__(WM *WN *kWave) void gemmPipeKernel(
       if (p.tileArrivals != nullptr &&
           arriveAtTile(p, tile, numSlices, tid, smem)) {
         sumPartials<MI, NI, THREADS>(p, acc, tile, numSlices, tid);
-        epilogueAuto<MI, NI, WTM, WTN, EPI>(p, acc, m0, n0, waveM, waveN, lane,
+        epilogueAuto<MI, NI, WTM, WTN, EPI, !DMA>(p, acc, m0, n0, waveM, waveN, lane,
                                             wave, smem);
       }
     }
   } else
-    epilogueAuto<MI, NI, WTM, WTN, EPI>(p, acc, m0, n0, waveM, waveN, lane,
+    epilogueAuto<MI, NI, WTM, WTN, EPI, !DMA>(p, acc, m0, n0, waveM, waveN, lane,
                                         wave, smem);
   vpid += gridDim.x;
   } while (vpid < nTiles); // tiles of this workgroup

@@ -45,6 +45,37 @@ def sample_rows(g, rows, count=48):
     return np.unique(np.concatenate([fixed, g.integers(0, rows, size=count - len(fixed))]))
 
 
+@pytest.mark.parametrize("tile", ["256x256_64q1_w2x4", "256x256_64x2r1_w2x4", "256x128_64x2r2_w4x2",
+                                  "128x128_64x2r2_w2x4", "256x96_64x2r2_w4x1"])
+@pytest.mark.parametrize("act", [0, 1])
+@pytest.mark.parametrize("source", ["none", "bias", "full"])
+@pytest.mark.parametrize("M,N", [(8229, 4080),  # written past the last-level cache (> 64 MiB)
+                                 (301, 264)])   # edges in both directions inside a wavefront's blocks
+def test_gemm_results_by_lane_exchange(gpu, rt, tile, act, source, M, N):
+    """Every output of the epilogues without LDS: a block misplaced by an exchange shows as an error
+    of the size of the values.  Operands of K = 64 are exact in fp32, so the bound is one rounding to fp16
+    plus the activation's 3e-7."""
+    kernel = f"hom_gfx950_mfma_f16_s32x32x16gemm_f16_{tile}_nn_align8_{'gelu' if act else 'linear'}"
+    num = gpu.homGemmManifestFind(kernel.encode())
+    assert num >= 0
+    K, mr = 64, rt.MemRef.from_tensor
+    g = torch.Generator(device="cuda")
+    g.manual_seed(M + N)
+    rnd = lambda *s: torch.randint(-8, 9, s, generator=g, device="cuda").to(torch.float16) / 16  # noqa: E731
+    A, B, C = rnd(1, M, K), rnd(1, K, N), {"bias": rnd(1, 1, N), "full": rnd(1, M, N), "none": None}[source]
+    D = torch.full((1, M, N), float("nan"), dtype=torch.float16, device="cuda")
+    gpu.cutlassGemmF16(*mr(A).args(), False, *mr(B).args(), False, *mr(D if C is None else C).args(),
+                       *mr(D).args(), act, 1.0, 0.0 if C is None else 1.0, num + 1, 1)
+    torch.cuda.synchronize()
+    want = A[0].float() @ B[0].float()
+    if C is not None:
+        want = want + C[0].float()
+    if act:
+        want = torch.nn.functional.gelu(want)
+    err = (D[0].float() - want).abs()
+    assert bool((err <= 2.0 ** -11 * want.abs() + 1e-6).all()), f"max {err.max().item()}"
+
+
 @pytest.mark.parametrize("N,K,act,beta", [
     (4096, 1024, 1, 0.0),   # FFN1 + GELU-erf
     (1024, 4096, 0, 1.0),   # FFN2 + residual, in place
