@@ -135,6 +135,12 @@ constexpr int kEpiFoldCStats = 7;
 // kEpiRowAffine with the column sums of B formed on the way, from the fragments
 // that the wavefronts multiply (row-major B).
 constexpr int kEpiRowAffineOwn = 8;
+// ... without a source, its results by lane exchanges.  (A kernel of its own: with the strips in it as
+// well, 256 x 256 tiles spill, 4096 x 4096 x 1024 42.6 -> 46.7 us.)
+constexpr int kEpiRowAffineLanes = 9;
+constexpr bool ownColumnSums(int epi) {
+  return epi == kEpiRowAffineOwn || epi == kEpiRowAffineLanes;
+}
 
 template <int EPI> __device__ __forceinline__ float activate(float v) {
   if (EPI == int(Epilogue::kGeluErf))
@@ -871,6 +877,70 @@ epilogueFold(const GemmParams &p, float16v (&acc)[MI][NI], int m0, int n0,
                             p.rowStatPartials +
                             (int64_t(piece) * p.M + m0 + tid) * 2),
                         out);
+    }
+  }
+}
+
+// kEpiRowAffineLanes: alpha (var[m] (A B) + mean[m] colsum(B)) by lane exchanges, see epilogueLanes;
+// colAcc and `given` as for epilogueFold.
+template <int MI, int NI, int WTM, int WTN>
+__device__ __forceinline__ void
+epilogueAffineLanes(const GemmParams &p, float16v (&acc)[MI][NI], int m0, int n0, int waveM, int waveN,
+                    int lane, unsigned char *smem, const float *colAcc, const unsigned char *given) {
+  constexpr uint32_t kOob = 0x80000000u;
+  const int l32 = lane % 32, l16 = lane % 16, kb = lane / 32;
+  const int cc = (lane / 16 % 2) * 16 + kb * 8;
+  const int rowBase = m0 + waveM * WTM, colBase = n0 + waveN * WTN;
+  auto clampBytes = [](int64_t b) -> int32_t {
+    return b > 0x7fffffffLL ? 0x7fffffff : (b < 0 ? 0 : int32_t(b));
+  };
+  const auto rsrcD = __builtin_amdgcn_make_buffer_rsrc(
+      p.D + int64_t(rowBase) * p.ldd + colBase, 0,
+      clampBytes((int64_t(p.M - rowBase) * p.ldd - colBase) * 2), 0x00020000);
+  const uint32_t ldd2 = uint32_t(p.ldd) * 2u;
+  const float2v *rowStat = reinterpret_cast<const float2v *>(given);
+  float *colSums = reinterpret_cast<float *>(smem);
+  __syncthreads(); // no wavefront still reads operands from the main loop's LDS
+  // (the lanes 32 apart have the two halves of every 16 k; the wavefront rows
+  // have the same columns)
+#pragma unroll
+  for (int j = 0; j < NI; j++) {
+    const float total = colAcc[j] + __shfl_xor(colAcc[j], 32, kWave);
+    if (waveM == 0 && lane < 32)
+      colSums[waveN * WTN + j * 32 + lane] = total;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < NI; j++) {
+    float4v sums[4];
+#pragma unroll
+    for (int g = 0; g < 4; g++)
+      sums[g] = *reinterpret_cast<const float4v *>(colSums + waveN * WTN + j * 32 + g * 8 + kb * 4);
+#pragma unroll
+    for (int i = 0; i < MI; i++) {
+      const float2v st = rowStat[waveM * WTM + i * 32 + l32];
+      lanes2 o[4];
+#pragma unroll
+      for (int g = 0; g < 4; g++) {
+        half4 r;
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+          r[e] = _Float16(p.alpha * fmaf(st[0], acc[i][j][4 * g + e], st[1] * sums[g][e]));
+        o[g] = __builtin_bit_cast(lanes2, r);
+      }
+      lanes4 lo = joinHalves(o[0][0], o[0][1], o[1][0], o[1][1]);
+      lanes4 hi = joinHalves(o[2][0], o[2][1], o[3][0], o[3][1]);
+      swapRows(lo, hi);
+      const bool in = colBase + j * 32 + cc < p.N;
+      const uint32_t at = uint32_t(i * 32 + l16) * ldd2 + uint32_t(j * 32 + cc) * 2u;
+      const uint32_t below = in ? at + 16u * ldd2 : kOob;
+      if (p.streamD) {
+        __builtin_amdgcn_raw_buffer_store_b128(lo, rsrcD, in ? at : kOob, 0, kStreamingAux);
+        __builtin_amdgcn_raw_buffer_store_b128(hi, rsrcD, below, 0, kStreamingAux);
+      } else {
+        __builtin_amdgcn_raw_buffer_store_b128(lo, rsrcD, in ? at : kOob, 0, kWriteThroughAux);
+        __builtin_amdgcn_raw_buffer_store_b128(hi, rsrcD, below, 0, kWriteThroughAux);
+      }
     }
   }
 }

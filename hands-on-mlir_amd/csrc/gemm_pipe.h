@@ -374,7 +374,7 @@ __global__ __launch_bounds__(WM *WN *kWave) void gemmPipeKernel(
   constexpr bool kFoldEarly = BM >= 128;
   float2v foldRaw[EPI >= kEpiFoldA ? FoldBatch<BM>::value : 1];
   float2v foldStat{1.f, 0.f};
-  constexpr bool kOwnColSums = EPI == kEpiRowAffineOwn;
+  constexpr bool kOwnColSums = ownColumnSums(EPI);
   static_assert(!kOwnColSums || !B_NK, "column sums from the fragments of a row-major B");
   if constexpr (kOwnColSums) {
     // (into LDS behind the slabs: 256 x 256 tiles have no registers to keep them in)
@@ -844,7 +844,10 @@ __global__ __launch_bounds__(WM *WN *kWave) void gemmPipeKernel(
                     NBUF * STAGE_BYTES,
                 "epilogue strips (and the row statistics of the folded "
                 "epilogues behind them) must fit the main loop's LDS");
-  if constexpr (EPI >= kEpiFoldA) {
+  if constexpr (EPI == kEpiRowAffineLanes) {
+    epilogueAffineLanes<MI, NI, WTM, WTN>(p, acc, m0, n0, waveM, waveN, lane, smem, colAcc,
+                                          smem + NBUF * STAGE_BYTES);
+  } else if constexpr (EPI >= kEpiFoldA) {
     if constexpr (!kFoldEarly && !kOwnColSums)
       foldStat = foldRowStatFinish<BM>(p, m0, tid, foldRaw);
     epilogueFold<MI, NI, WTM, WTN, EPI, BM, THREADS>(p, acc, m0, n0, waveM,
@@ -873,7 +876,7 @@ template <int BM, int BN, int WM, int WN, int DIST, int EPI, bool B_NK,
 Status launchPipe(const GemmProblem &pr, hipStream_t s) {
   static_assert(!ANY || !DMA, "DMA staging needs aligned rows");
   constexpr int SMEM = (DMA ? DIST + 1 : 2) * (BM + BN) * 64 * 2 +
-                       (EPI == kEpiRowAffineOwn ? BM * 8 : 0);
+                       (ownColumnSums(EPI) ? BM * 8 : 0);
   static_assert(!DMA || ((BM * 8) % (WM * WN * kWave) == 0 &&
                          (BN * 8) % (WM * WN * kWave) == 0 &&
                          (B_NK || 1024 % (BN * 2) == 0 || (BN * 2) % 1024 == 0)),

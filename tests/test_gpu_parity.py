@@ -429,6 +429,7 @@ def test_ln_gemm_pair(gpu, rt, oracle, literals):
     (1024, 768, 768, 768, 0.0),      # 64x64 tiles for both halves
     (1024, 768, 768, 2304, 1.0),     # second half on 128x128 tiles, residual source
     (4096, 1024, 256, 2304, 0.0),    # second half on 256x256 tiles
+    (4101, 1024, 64, 2312, 0.0),     # ... with edges in both directions
     (1000, 776, 264, 520, 1.0),      # ragged rows and columns (still multiples of 8)
     (100, 250, 72, 30, 0.0),         # N not a multiple of 8: the unfused kernels
 ])
