@@ -14,9 +14,10 @@
 // sequences, many workgroups), or two wavefronts share 32 rows and take every
 // other key block (short sequences: fewer workgroups than CUs, the key walk of
 // one wavefront is the critical path; the two halves are merged through LDS).
-// Keys are walked in chunks of 128: the whole workgroup stages the chunk's K
-// and V rows into LDS (one barrier), then the wavefronts run over it in blocks
-// of 64 keys without further synchronisation.
+// Keys are walked in chunks of 128 (64 where they are copied straight into LDS): the
+// whole workgroup stages the chunk's K and V rows into LDS (one barrier), then the
+// wavefronts run over it in blocks of 64 keys (32 each) without further
+// synchronisation.
 // Both contractions run on v_mfma_f32_32x32x16_f16 and are issued transposed:
 //   S^T = K Q^T   (A operand = K rows from LDS, B operand = Q rows in registers)
 //   O^T = V^T P^T (A operand = V columns, B operand = P rows)
@@ -77,6 +78,17 @@ template <int D> __device__ __forceinline__ int swzK(int row, int chunk) {
 template <int D> __device__ __forceinline__ int swzV(int k, int group) {
   return D == 64 || D == 192 ? group ^ ((k >> 1) & 1) : group ^ (k & 3);
 }
+
+// Order of the workgroups: the query tiles of a (batch, head) back to back, or all
+// first tiles, then all second ones, .., so that those of nothing but padding come
+// last.  That pays where the workgroups of a launch do not all fit the chip at
+// once (two to a CU at head size 128, one above) and all K and V fit the L2s, as in the
+// launches the key-split variant takes: 16:200:12 heads of 128 14.4 -> 13.8 us, 8:384:16
+// 15.1 -> 14.7, 1:700:12 of 256 22.5 -> 21.9; at head size 64, where all are resident,
+// 8:500:12 takes 14.9 instead of 13.9, and 32:512:12 of 192 on eight wavefronts 104.8 instead
+// of 102.1.
+template <int NW, int KS, int D, bool DMA>
+constexpr bool kTilesOutside = DMA && KS == 2 && NW == 4 && D >= 128;
 
 // 16 bytes of the result, which starts on an 8-byte boundary: the hardware takes that,
 // and the type promises no more.  (As inline assembly the stores stay in source order
@@ -152,7 +164,10 @@ __attribute__((amdgpu_waves_per_eu(D <= 128 || NW == 8 ? 2 : 1, D == 64 && KS ==
       }
     }
     int pair;
-    if (pairs % 8 == 0) {
+    if (kTilesOutside<NW, KS, D, DMA>) {
+      qTile = int(divByMagic(uint32_t(id), uint32_t(pairs), numQMagic));
+      pair = id - qTile * pairs;
+    } else if (pairs % 8 == 0) {
       const uint32_t t = uint32_t(id) / 8, g = divByMagic(t, uint32_t(numQTiles), numQMagic);
       qTile = int(t - g * uint32_t(numQTiles));
       pair = int(g * 8 + uint32_t(id) % 8);
@@ -326,24 +341,250 @@ __attribute__((amdgpu_waves_per_eu(D <= 128 || NW == 8 ? 2 : 1, D == 64 && KS ==
                           : uint32_t(r) * rowBytes + uint32_t(cV) * 16u;
     }
   }
-  auto requestChunk = [&](int ch) {
+  constexpr float kSumLimit = 4096.0f;
+  // PIPE: the next chunk's scores between this chunk's exponentials, so that one
+  // wavefront has the matrix cores and the vector ALU at work at once (a kernel that
+  // takes them in turn is bound by the sum of both, also with two wavefronts on a SIMD).
+  // It costs the registers of another block's scores.  us without and with it, lengths
+  // uniform in [seq / 4, seq]: head size 128, 32:512:16 70.9 -> 68.3, 16:200:12 15.2 -> 14.4,
+  // 2:700:12 13.0 -> 11.9, 1:700:8 9.1 -> 8.25; 64 with split keys 2:700:16 9.2 -> 8.8, 8:500:12
+  // 14.1 -> 13.8; 256 with split keys 1:700:12 23.4 -> 22.5.  Not for head size 64 with whole
+  // rows (32:512:16 37.2 -> 40.1: two wavefronts a SIMD instead of four), 192 (32:512:12 102.1
+  // -> 104.7, spills) and fragment order (BERT-base 8 x 384 1315 -> 1328, 2 x 700 equal).
+  constexpr bool PIPE = DMA && (D == 128 || (KS == 2 && !PACKED_IN && D != 192));
+  auto requestTile = [&](auto valuesC, int ch) { // K or V rows of chunk ch
 #if defined(__HIP_DEVICE_COMPILE__) // (the builtin's LDS pointer type exists only for the GPU target)
     if constexpr (DMA) {
+      constexpr bool kValues = decltype(valuesC)::value;
       const uint32_t chunkOff = uint32_t(ch * kChunk) * rowBytes;
-      unsigned char *dst = smem + (ch % 2) * (2 * kTileBytes) + wave * 1024;
+      unsigned char *dst =
+          smem + (ch % 2) * (2 * kTileBytes) + (kValues ? kTileBytes : 0) + wave * 1024;
 #pragma unroll
       for (int i = 0; i < VPT; i++) {
         const bool out = PACKED_IN && ch * kChunk + (tid + i * kThreads) / CPR >= len;
         __builtin_amdgcn_raw_ptr_buffer_load_lds(
-            rsrcK, HOM_LDS_PTR(dst + i * (kThreads * 16)), 16,
-            out ? 0x80000000u : dmaK[i] + chunkOff, 0, 0, 0);
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(
-            rsrcV, HOM_LDS_PTR(dst + kTileBytes + i * (kThreads * 16)), 16,
-            out ? 0x80000000u : dmaV[i] + chunkOff, 0, 0, 0);
+            kValues ? rsrcV : rsrcK, HOM_LDS_PTR(dst + i * (kThreads * 16)), 16,
+            out ? 0x80000000u : (kValues ? dmaV[i] : dmaK[i]) + chunkOff, 0, 0, 0);
       }
     }
 #endif
   };
+  auto requestChunk = [&](int ch) {
+    requestTile(std::false_type{}, ch);
+    requestTile(std::true_type{}, ch);
+  };
+  // ---- O^T += V^T P^T: group g of 16 keys, whose probabilities are prob(g) ----
+  auto weighValues = [&](const unsigned char *sV, int blk, auto &&prob) {
+    // Transposing reads issued and waited for by hand: in front of its
+    // own the compiler would wait for every copy into LDS
+    // that is on its way, i.e. for the whole next chunk.
+    // INVARIANT: what an asm read writes is not valid until the wait.  Every
+    // destination is an in/out operand of a wait, so that no use of it can
+    // move ahead of that one; that the register allocator does not copy or
+    // spill one in between either is checked on the compiled kernels
+    // (tests/test_attention_assembly.py).
+    constexpr int kGroups = SBW * 2, kSets = D <= 128 ? 2 : 1;
+    static_assert(DB % 2 == 0, "a wait takes the reads of two column blocks");
+    const uint32_t vLane = uint32_t(uintptr_t(HOM_LDS_PTR(sV))) +
+                           uint32_t((blk + 4 * hb + trRow) * kRowB + trCol * 2);
+    short4v run[kSets][DB][2];
+    auto readGroup = [&](auto gC) {
+      constexpr int g = decltype(gC)::value;
+#pragma unroll
+      for (int d = 0; d < DB; d++) {
+        const uint32_t at = vLane + uint32_t((d ^ vSwz) * 64);
+        asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2"
+                     : "=v"(run[g % kSets][d][0])
+                     : "v"(at), "i"(g * 16 * kRowB));
+        asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2"
+                     : "=v"(run[g % kSets][d][1])
+                     : "v"(at), "i"((g * 16 + 8) * kRowB));
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    __builtin_amdgcn_sched_barrier(0);
+    readGroup(std::integral_constant<int, 0>{});
+    priority(First{});
+    auto pvGroup = [&](auto gC) {
+      constexpr int g = decltype(gC)::value;
+      constexpr bool kMore = g + 1 < kGroups;
+      using Next = std::integral_constant<int, kMore ? g + 1 : 0>;
+      const half8 fp = prob(gC);
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (kMore && kSets == 2)
+        readGroup(Next{});
+#pragma unroll
+      for (int d = 0; d < DB; d += 2) // (the first one waits for all of them)
+        asm volatile("s_waitcnt lgkmcnt(%4)"
+                     : "+v"(run[g % kSets][d][0]), "+v"(run[g % kSets][d][1]),
+                       "+v"(run[g % kSets][d + 1][0]), "+v"(run[g % kSets][d + 1][1])
+                     : "n"(kMore && kSets == 2 ? DB * 2 : 0)
+                     : "memory");
+#pragma unroll
+      for (int d = 0; d < DB; d++) {
+        const short4v lo = run[g % kSets][d][0], hi = run[g % kSets][d][1];
+        short8v both;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          both[e] = lo[e];
+          both[4 + e] = hi[e];
+        }
+        accO[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+            __builtin_bit_cast(half8, both), fp, accO[d], 0, 0, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (kMore && kSets == 1)
+        readGroup(Next{});
+    };
+    pvGroup(std::integral_constant<int, 0>{});
+    pvGroup(std::integral_constant<int, 1>{});
+    if constexpr (kGroups == 4) {
+      pvGroup(std::integral_constant<int, 2>{});
+      pvGroup(std::integral_constant<int, 3>{});
+    }
+    priority(Even{});
+  };
+  if constexpr (PIPE) {
+    // Chunk by chunk: the scores of the next one (matrix cores) between the
+    // exponentials of this one (vector ALU), K a chunk further ahead than V.
+    constexpr int kSteps = D / 16, NE = 16 * SBW, NM = kSteps * SBW;
+    constexpr int kDeep = SBW == 1 && D <= 128 ? kSteps : kSteps >= 8 ? kSteps / 2 : kSteps;
+    const int blk = kh * (SBW * 32); // this wavefront's keys of a chunk
+    auto tileOf = [&](int ch) { return smem + (ch % 2) * (2 * kTileBytes); };
+    float16v accS[SBW], accN[SBW];
+    half8 fk[SBW][kDeep];
+    auto readK = [&](const unsigned char *sK, int sb, int kk) {
+      fk[sb][kk % kDeep] = *reinterpret_cast<const half8 *>(
+          sK + (blk + sb * 32 + l32) * kRowB + ((kk * 2 + hb) ^ swzLane) * 16);
+    };
+    auto multiplyK = [&](const unsigned char *sK, int m) { // MFMA m of a block's scores
+      const int kk = m / SBW, sb = m % SBW;
+      accN[sb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+          fk[sb][kk % kDeep], fq[kk], kk == 0 ? float16v{} : accN[sb], 0, 0, 0);
+      if (kk + kDeep < kSteps)
+        readK(sK, sb, kk + kDeep);
+    };
+    auto firstReads = [&](const unsigned char *sK) {
+#pragma unroll
+      for (int kk = 0; kk < kDeep; kk++)
+#pragma unroll
+        for (int sb = 0; sb < SBW; sb++)
+          readK(sK, sb, kk);
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    auto hideKeys = [&](int key0) { // those past the sequence end
+#pragma unroll
+      for (int sb = 0; sb < SBW; sb++)
+#pragma unroll
+        for (int e = 0; e < 16; e++) {
+          const int key = key0 + blk + sb * 32 + 8 * (e / 4) + 4 * hb + (e % 4);
+          accN[sb][e] = key < len ? accN[sb][e] : -INFINITY;
+        }
+    };
+    requestTile(std::false_type{}, 0);
+    if (numChunks > 1) {
+      requestTile(std::false_type{}, 1);
+      requestTile(std::true_type{}, 0);
+      asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(2 * VPT) : "memory");
+    } else {
+      requestTile(std::true_type{}, 0);
+      asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(VPT) : "memory");
+    }
+    if (blk < len) {
+      firstReads(tileOf(0));
+#pragma unroll
+      for (int m = 0; m < NM; m++)
+        multiplyK(tileOf(0), m);
+      if (blk + SBW * 32 > len)
+        hideKeys(0);
+      float blockMax = -INFINITY;
+#pragma unroll
+      for (int sb = 0; sb < SBW; sb++)
+#pragma unroll
+        for (int e = 0; e < 16; e++)
+          blockMax = fmaxf(blockMax, accN[sb][e]);
+      rowMax = pairMax(blockMax);
+    }
+    auto step = [&](int ch, auto moreC) {
+      constexpr bool MORE = decltype(moreC)::value;
+      // the next chunk's K and this one's V have landed, and every wavefront is done
+      // with this one's K and the previous one's V
+      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      if constexpr (MORE) {
+        if (ch + 2 < numChunks)
+          requestTile(std::false_type{}, ch + 2);
+        requestTile(std::true_type{}, ch + 1);
+      }
+      const unsigned char *sKn = tileOf(ch + 1);
+      const int key0 = ch * kChunk;
+      if constexpr (!MORE) {
+        if (key0 + blk >= len)
+          return; // (the last chunk ends before this wavefront's keys)
+        if (ch > 0 && key0 + blk + SBW * 32 > len)
+          hideKeys(key0);
+      }
+#pragma unroll
+      for (int sb = 0; sb < SBW; sb++)
+        accS[sb] = accN[sb];
+      half8 p[SBW][2];
+      float sum = 0.f;
+      const float negMax = -rowMax * scaleLog2e;
+      if constexpr (MORE)
+        firstReads(sKn);
+#pragma unroll
+      for (int m = 0; m < NM; m++) {
+#pragma unroll
+        for (int x = m * NE / NM; x < (m + 1) * NE / NM; x++) {
+          const int sb = x / 16, e = x % 16;
+          const float pv = __builtin_amdgcn_exp2f(fmaf(accS[sb][e], scaleLog2e, negMax));
+          sum += pv;
+          p[sb][e / 8][e % 8] = _Float16(pv);
+        }
+        if constexpr (MORE) {
+          __builtin_amdgcn_sched_barrier(0);
+          multiplyK(sKn, m);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+      if (__builtin_expect(__any(!(sum <= kSumLimit)), 0)) {
+        float blockMax = -INFINITY;
+#pragma unroll
+        for (int sb = 0; sb < SBW; sb++)
+#pragma unroll
+          for (int e = 0; e < 16; e++)
+            blockMax = fmaxf(blockMax, accS[sb][e]);
+        const float newMax = fmaxf(rowMax, pairMax(blockMax));
+        const float corr = __builtin_amdgcn_exp2f((rowMax - newMax) * scaleLog2e);
+        rowSum *= corr;
+        rowMax = newMax;
+#pragma unroll
+        for (int d = 0; d < DB; d++)
+#pragma unroll
+          for (int e = 0; e < 16; e++)
+            accO[d][e] *= corr;
+        sum = 0.f;
+        const float toMax = -rowMax * scaleLog2e;
+#pragma unroll
+        for (int sb = 0; sb < SBW; sb++)
+#pragma unroll
+          for (int e = 0; e < 16; e++) {
+            const float pv = __builtin_amdgcn_exp2f(fmaf(accS[sb][e], scaleLog2e, toMax));
+            sum += pv;
+            p[sb][e / 8][e % 8] = _Float16(pv);
+          }
+      }
+      rowSum += sum;
+      weighValues(tileOf(ch) + kTileBytes, blk, [&](auto gC) {
+        constexpr int g = decltype(gC)::value;
+        return p[g / 2][g % 2];
+      });
+    };
+    int ch = 0;
+    for (; ch + 1 < numChunks; ch++)
+      step(ch, std::true_type{});
+    step(ch, std::false_type{});
+    rowSum = pairSum(rowSum); // (each lane has added up its own keys)
+  } else {
   requestChunk(0);
   // (at least one round in either variant: a loop that may run zero times
   // would put a test of the sequence length ahead of the prefetched loads)
@@ -499,7 +740,6 @@ __attribute__((amdgpu_waves_per_eu(D <= 128 || NW == 8 ? 2 : 1, D == 64 && KS ==
       // With real score distributions the slow path runs once per wavefront.
       // Every block that is visited has at least one valid key, so blockMax
       // is finite and the differences below are never inf - inf.
-      constexpr float kSumLimit = 4096.0f;
       const bool first = ch == 0 && blk == kh * (SBW * 32);
       float blockSum = 0.f;
       bool slow = first;
@@ -554,77 +794,14 @@ __attribute__((amdgpu_waves_per_eu(D <= 128 || NW == 8 ? 2 : 1, D == 64 && KS ==
 
       // ---- O^T += V^T P^T ----
       if constexpr (DMA) {
-        // The same reads as below, issued and waited for by hand: in front of its
-        // own transposing reads the compiler would wait for every copy into LDS
-        // that is on its way, i.e. for the whole next chunk.
-        // INVARIANT: what an asm read writes is not valid until the wait.  Every
-        // destination is an in/out operand of a wait, so that no use of it can
-        // move ahead of that one; that the register allocator does not copy or
-        // spill one in between either is checked on the compiled kernels
-        // (tests/test_attention_assembly.py).
-        constexpr int kGroups = SBW * 2, kSets = D <= 128 ? 2 : 1;
-        static_assert(DB % 2 == 0, "a wait takes the reads of two column blocks");
-        const uint32_t vLane = uint32_t(uintptr_t(HOM_LDS_PTR(sV))) +
-                               uint32_t((blk + 4 * hb + trRow) * kRowB + trCol * 2);
-        short4v run[kSets][DB][2];
-        auto readGroup = [&](auto gC) {
+        weighValues(sV, blk, [&](auto gC) {
           constexpr int g = decltype(gC)::value;
-#pragma unroll
-          for (int d = 0; d < DB; d++) {
-            const uint32_t at = vLane + uint32_t((d ^ vSwz) * 64);
-            asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2"
-                         : "=v"(run[g % kSets][d][0])
-                         : "v"(at), "i"(g * 16 * kRowB));
-            asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2"
-                         : "=v"(run[g % kSets][d][1])
-                         : "v"(at), "i"((g * 16 + 8) * kRowB));
-          }
-          __builtin_amdgcn_sched_barrier(0);
-        };
-        __builtin_amdgcn_sched_barrier(0);
-        readGroup(std::integral_constant<int, 0>{});
-        priority(First{});
-        auto pvGroup = [&](auto gC) {
-          constexpr int g = decltype(gC)::value;
-          constexpr bool kMore = g + 1 < kGroups;
-          using Next = std::integral_constant<int, kMore ? g + 1 : 0>;
           half8 fp;
 #pragma unroll
           for (int e = 0; e < 8; e++)
             fp[e] = _Float16(accS[g / 2][8 * (g % 2) + e]);
-          __builtin_amdgcn_sched_barrier(0);
-          if constexpr (kMore && kSets == 2)
-            readGroup(Next{});
-#pragma unroll
-          for (int d = 0; d < DB; d += 2) // (the first one waits for all of them)
-            asm volatile("s_waitcnt lgkmcnt(%4)"
-                         : "+v"(run[g % kSets][d][0]), "+v"(run[g % kSets][d][1]),
-                           "+v"(run[g % kSets][d + 1][0]), "+v"(run[g % kSets][d + 1][1])
-                         : "n"(kMore && kSets == 2 ? DB * 2 : 0)
-                         : "memory");
-#pragma unroll
-          for (int d = 0; d < DB; d++) {
-            const short4v lo = run[g % kSets][d][0], hi = run[g % kSets][d][1];
-            short8v both;
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-              both[e] = lo[e];
-              both[4 + e] = hi[e];
-            }
-            accO[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
-                __builtin_bit_cast(half8, both), fp, accO[d], 0, 0, 0);
-          }
-          __builtin_amdgcn_sched_barrier(0);
-          if constexpr (kMore && kSets == 1)
-            readGroup(Next{});
-        };
-        pvGroup(std::integral_constant<int, 0>{});
-        pvGroup(std::integral_constant<int, 1>{});
-        if constexpr (kGroups == 4) {
-          pvGroup(std::integral_constant<int, 2>{});
-          pvGroup(std::integral_constant<int, 3>{});
-        }
-        priority(Even{});
+          return fp;
+        });
       } else {
 #pragma unroll
       for (int sb = 0; sb < SBW; sb++) {
@@ -662,6 +839,7 @@ __attribute__((amdgpu_waves_per_eu(D <= 128 || NW == 8 ? 2 : 1, D == 64 && KS ==
       }
     }
   } while (++ch < numChunks);
+  }
 
   // ---- merge the key shares ----
   // Share 1 hands (reference, sum, O) of its rows to share 0 through LDS, in
@@ -770,7 +948,7 @@ template <int NW, int KS, int D, bool PACKED_IN, bool DMA> Status launchVariant(
   }
   kernel<<<grid, dim3(NW * kWave), kLds, l.stream>>>(l.qkv, l.cu, l.out, int(l.seq), int(l.heads),
                                                      int(nq), int(l.bs), l.scale, l.packedOut,
-                                                     magicFor(nq), magicFor(uint32_t(l.heads)),
+                                                     magicFor(kTilesOutside<NW, KS, D, DMA> ? uint32_t(pairs) : nq), magicFor(uint32_t(l.heads)),
                                                      l.ahead, l.aheadBytes);
   HOM_HIP_RET(hipGetLastError(), Status::kInternal);
   return Status::kSuccess;
@@ -822,29 +1000,40 @@ Status launchBertAttentionF16(const _Float16 *qkv, const int32_t *cuSeqlens,
   // in [seq / 4, seq], batch : seq : heads):
   //  - Prefetch: 64 rows per workgroup with the keys split over two wavefronts per
   //    32 rows, K and V of the first 128 keys requested before anything else is
-  //    known.  The fastest while that is all of them and workgroups are few
-  //    (head size 64, 8:128:12 4.2, against 5.0 - 5.3).
+  //    known.  The fastest while that is all of them and every workgroup has a CU of
+  //    its own (head size 64, 8:128:12 4.2, against 5.0 - 5.3; 26:105:8, where it has not,
+  //    6.4 against 4.8 by Dma, 11:119:16 6.45 against 4.9).
   //  - Wide: 128 rows, chunks of 128 keys through registers; head size 64 for so
   //    many short sequences that the workgroups of a CU cover each other
-  //    (64:128:12 10.5 against 10.8), and 256, whose chunks by DMA would leave too
-  //    few registers (8:384:16 42 against 47).
+  //    (64:70:12 7.7 against 7.9, but 32:128:16 8.3 against 7.95), and 256, whose chunks by
+  //    DMA would leave too few registers (8:384:16 42 against 47).
   //  - Dma: 128 rows, chunks of 64 keys straight into LDS while the one before is
   //    worked on (head size 64, 32:512:16 41.8 -> 40.6, 1:64:12 4.0 -> 3.6; 128,
   //    32:512:16 66.9 -> 60.9).  Head size 192: 8 wavefronts, two per 32 rows, which
   //    then fit two to a SIMD (32:512:12 117 -> 97).
-  //  - DmaSplit: the same with 64 rows and two wavefronts per 32 rows, for fewer
-  //    workgroups than fill the chip twice (head size 64, 2:700:16 13.1 -> 10.8;
-  //    128, 2:700:12 21.2 -> 17.6; 192, 2:100:8 10.0 -> 8.5; 256 12.5 -> 10.5).
+  //  - DmaSplit: the same with 64 rows and two wavefronts per 32 rows, where its
+  //    finer workgroups spread better over the CUs.  That is up to half a CU's worth of
+  //    128-row tiles (3:346:8 of 64 5.0 against 6.1, 3:615:8 of 128 10.8 against 13.9, 4:185:16
+  //    of 256 11.9 against 14.5, 8:200:8 of 192 10.1 against 11.8) and, at head sizes 64 and 128,
+  //    also up to 0.6 (2:707:12 of 64 7.6 against 9.6, of 128 2:657:12 9.7 against 12.0) and
+  //    from one to 1.4 tiles a CU, where a second tile would be all that some CUs do
+  //    (4:700:12 9.6 against 12.2, 9:189:16 6.3 against 6.5, 6:746:8 of 128 18.1 against 19.8).
+  //    Between and above those Dma: 7:235:12 6.4 against 6.8, 8:384:16 9.6 against 11.0, 16:200:12
+  //    7.5 against 9.4; of 128 7:241:16 9.2 against 10.6, 16:256:12 13.6 against 16.3, 8:384:16 14.8
+  //    against 15.2.  (64, long sequences of few batches up to a tile a CU: 2:747:16
+  //    8.3 against 9.7 split, 5:493:12 9.75 against 8.9.)
   enum { Prefetch, Wide, Dma, DmaSplit } way;
   const int64_t tiles = pairs * ((seq + 127) / 128);
+  const bool few = tiles <= cus / 2;
+  const bool finer = 10 * tiles <= 6 * cus || (tiles > cus && 10 * tiles <= 14 * cus);
   if (headDim == 64)
     way = seq <= 64    ? Dma
-          : seq <= 128 ? (tiles < cus ? Prefetch : Wide)
-                       : (tiles < 2 * cus ? DmaSplit : Dma);
+          : seq <= 128 ? (few ? Prefetch : tiles <= 2 * cus ? Dma : Wide)
+                       : (finer || (tiles <= cus && seq > 512) ? DmaSplit : Dma);
   else if (headDim == 128)
-    way = seq > 64 && (tiles < cus / 2 || (seq > 128 && tiles < 2 * cus)) ? DmaSplit : Dma;
+    way = seq > 64 && (tiles < cus / 2 || (seq > 128 && finer)) ? DmaSplit : Dma;
   else
-    way = tiles < cus / 2 ? DmaSplit : headDim == 192 ? Dma : Wide;
+    way = few ? DmaSplit : headDim == 192 ? Dma : Wide;
   // profiling knob: HOM_ATTENTION_VARIANT=wide | split
   if (const char *force = getenv("HOM_ATTENTION_VARIANT"))
     way = strcmp(force, "wide") == 0 ? (headDim == 256 ? Wide : Dma) : DmaSplit;

@@ -571,6 +571,33 @@ def test_attention_splits(gpu, rt, bs, seq, heads, d):
     torch.testing.assert_close(out.float(), want, rtol=2e-3, atol=2e-3)
 
 
+# lengths at the ends of 32-key blocks and 64-key chunks: split keys (64, 128, 256), whole rows (128; 64 up to 128
+# tokens with more tiles than half the CUs), and split keys between one and 1.4 tiles a CU
+@pytest.mark.parametrize("bs,seq,heads,d", [(13, 200, 2, 64), (13, 200, 2, 128), (13, 200, 2, 256), (48, 200, 2, 128),
+                                            (48, 100, 4, 64), (13, 200, 11, 128), (13, 200, 11, 64)])
+def test_attention_chunk_ends(gpu, rt, bs, seq, heads, d):
+    g = torch.Generator("cuda").manual_seed(seq + d)
+    qkv = torch.randn(bs, seq, 3, heads, d, device="cuda", generator=g)
+    qkv[:, :, 1] *= 1.0 + 4.0 * torch.arange(seq, device="cuda")[None, :, None, None] / seq  # the reference moves
+    qkv = qkv.half()
+    ends = [1, 31, 32, 33, 63, 64, 65, 96, 97, 128, 129, 192, 200]
+    lens = torch.tensor([min(seq, ends[i % 13]) for i in range(bs)], device="cuda")
+    live = torch.arange(seq, device="cuda")[None, :] < lens[:, None]
+    q, k, v = qkv.float().permute(2, 0, 3, 1, 4).contiguous()
+    s = torch.matmul(q, k.transpose(2, 3).contiguous()) / d ** 0.5
+    want = torch.matmul(s.masked_fill(~live[:, None, None, :], float("-inf")).softmax(-1), v).permute(0, 2, 1, 3)
+    want = want.reshape(bs, seq, heads * d) * live[:, :, None]
+    qkv[~live] = float("nan")
+    cu = torch.zeros(bs + 1, dtype=torch.int32, device="cuda")
+    cu[1:] = lens.cumsum(0)
+    out = torch.full((bs, seq, heads * d), 7.0, dtype=torch.float16, device="cuda")
+    Mr = rt.MemRef
+    gpu.nvteBertAttentionF16(*Mr.from_tensor(qkv.view(bs, seq, -1)).args(), *Mr.from_tensor(cu).args(),
+                             *Mr.from_tensor(out).args(), d ** -0.5, heads)
+    # probabilities and result in fp16: 2 * 2^-11 of values up to about 4
+    torch.testing.assert_close(out.float(), want, rtol=2e-3, atol=4e-3)
+
+
 @pytest.mark.parametrize("K,N", [(32, 16), (96, 48), (768, 2304), (1056, 320)])
 def test_pack_weight_and_back(gpu, rt, K, N):
     B = np.random.default_rng(K + N).standard_normal((1, K, N)).astype(np.float16)
