@@ -71,6 +71,15 @@ __device__ __forceinline__ void swapRows(lanes4 &a, lanes4 &b) {
     b[i] = r[1];
   }
 }
+// Lanes 8 .. 15 of a's rows against lanes 0 .. 7 of b's.
+__device__ __forceinline__ void swapHalfRows(lanes4 &a, lanes4 &b) {
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const int x = int(a[i]), y = int(b[i]); // (0x128: rotate a row of 16 lanes by 8)
+    a[i] = uint32_t(__builtin_amdgcn_update_dpp(x, y, 0x128, 0xf, 0xc, false));
+    b[i] = uint32_t(__builtin_amdgcn_update_dpp(y, x, 0x128, 0xf, 0x3, false));
+  }
+}
 // v_permlane16_swap exchanges the odd rows of its first operand with the even
 // rows of its second: the same value twice gives (even-row values, odd-row
 // values) in every lane pair (l, l ^ 16).

@@ -535,10 +535,11 @@ epilogueFast(const GemmParams &p, float16v (&acc)[MI][NI], int m0, int n0,
 // 32 apart exchange halves (joinHalves) and rows of 16 lanes change places (swapRows),
 // so that a lane has 8 consecutive columns and a store instruction writes 64 bytes of
 // 16 rows.  No barrier, and a wavefront's stores go out while others still multiply.
+// stream: past the last-level cache (GemmParams::streamD).
 template <int MI, int NI, int WTM, int WTN, int EPI, int CMODE>
 __device__ __forceinline__ void
 epilogueLanes(const GemmParams &p, float16v (&acc)[MI][NI], int m0, int n0,
-              int waveM, int waveN, int lane) {
+              int waveM, int waveN, int lane, bool stream) {
   constexpr uint32_t kOob = 0x80000000u;
   const int l16 = lane % 16, kb = lane / 32;
   // columns of this lane's 16 bytes in a block of 32
@@ -583,6 +584,12 @@ epilogueLanes(const GemmParams &p, float16v (&acc)[MI][NI], int m0, int n0,
           cv[i][j][h] = __builtin_bit_cast(
               lanes4, __builtin_amdgcn_raw_buffer_load_b128(rsrcC, offsetOf(i, j, h, ldc2), 0, 0));
   }
+  // 256 x 256 tiles: halves of those rows change places between two blocks of 32 columns
+  // (swapHalfRows), so that an instruction writes 8 rows' whole 128-byte lines.  By 64 bytes,
+  // results that the last-level cache has to make room for took longer: 16384 x 4096 x 1024 in
+  // requests 140 us through LDS, 162 by 64 bytes, 142 by lines; 16384 x 3072 x 768 91, 96, 86.
+  constexpr bool kLines = MI == 4 && NI == 2;
+  lanes4 left[2]; // the even block of a pair
 #pragma unroll
   for (int i = 0; i < MI; i++)
 #pragma unroll
@@ -620,9 +627,30 @@ epilogueLanes(const GemmParams &p, float16v (&acc)[MI][NI], int m0, int n0,
       lanes4 lo = joinHalves(o[0][0], o[0][1], o[1][0], o[1][1]);
       lanes4 hi = joinHalves(o[2][0], o[2][1], o[3][0], o[3][1]);
       swapRows(lo, hi);
-      if (MI * NI == 8 && p.streamD) {
-        __builtin_amdgcn_raw_buffer_store_b128(lo, rsrcD, offsetOf(i, j, 0, ldd2), 0, kStreamingAux);
-        __builtin_amdgcn_raw_buffer_store_b128(hi, rsrcD, offsetOf(i, j, 1, ldd2), 0, kStreamingAux);
+      if constexpr (kLines) {
+        if (j % 2 == 0) {
+          left[0] = lo;
+          left[1] = hi;
+        } else {
+          swapHalfRows(left[0], lo);
+          swapHalfRows(left[1], hi);
+          const int block = j - 1 + l16 / 8;
+          const uint32_t at = colBase + block * 32 + cc < p.N
+                                  ? uint32_t(i * 32 + l16 % 8) * ldd2 + uint32_t(block * 32 + cc) * 2u
+                                  : kOob;
+          const uint32_t step = at == kOob ? 0u : 8u * ldd2; // rows 0 .., 8 .., 16 .., 24 ..
+          auto store = [&](auto auxC) {
+            constexpr int kAux = decltype(auxC)::value;
+            __builtin_amdgcn_raw_buffer_store_b128(left[0], rsrcD, at, 0, kAux);
+            __builtin_amdgcn_raw_buffer_store_b128(lo, rsrcD, at + step, 0, kAux);
+            __builtin_amdgcn_raw_buffer_store_b128(left[1], rsrcD, at + 2 * step, 0, kAux);
+            __builtin_amdgcn_raw_buffer_store_b128(hi, rsrcD, at + 3 * step, 0, kAux);
+          };
+          if (EPI != int(Epilogue::kLinear) && stream)
+            store(std::integral_constant<int, kStreamingAux>{});
+          else
+            store(std::integral_constant<int, kWriteThroughAux>{});
+        }
       } else {
         __builtin_amdgcn_raw_buffer_store_b128(lo, rsrcD, offsetOf(i, j, 0, ldd2), 0, kWriteThroughAux);
         __builtin_amdgcn_raw_buffer_store_b128(hi, rsrcD, offsetOf(i, j, 1, ldd2), 0, kWriteThroughAux);
@@ -881,7 +909,9 @@ epilogueFold(const GemmParams &p, float16v (&acc)[MI][NI], int m0, int n0,
   }
 }
 
-// kEpiRowAffineLanes: alpha (var[m] (A B) + mean[m] colsum(B)) by lane exchanges, see epilogueLanes;
+// kEpiRowAffineLanes: alpha (var[m] (A B) + mean[m] colsum(B)) by lane exchanges and whole lines, see
+// epilogueLanes (both calls, 16384 x 1024 -> 4096 through LDS 209 us, by 64 bytes of a row 209, by lines
+// 203; 16384 x 768 -> 3072 135 -> 131, 4096 x 1024 -> 4096 57.0 -> 54.2);
 // colAcc and `given` as for epilogueFold.
 template <int MI, int NI, int WTM, int WTN>
 __device__ __forceinline__ void
@@ -910,38 +940,38 @@ epilogueAffineLanes(const GemmParams &p, float16v (&acc)[MI][NI], int m0, int n0
       colSums[waveN * WTN + j * 32 + lane] = total;
   }
   __syncthreads();
+  static_assert(NI == 2, "whole lines, see epilogueLanes");
+  const int block = l16 / 8;
+  const bool in = colBase + block * 32 + cc < p.N;
+  const uint32_t step = in ? 8u * ldd2 : 0u;
 #pragma unroll
-  for (int j = 0; j < NI; j++) {
-    float4v sums[4];
+  for (int i = 0; i < MI; i++) {
+    const float2v st = rowStat[waveM * WTM + i * 32 + l32];
+    lanes4 v[NI][2]; // rows 0 .. 15, rows 16 .. 31
 #pragma unroll
-    for (int g = 0; g < 4; g++)
-      sums[g] = *reinterpret_cast<const float4v *>(colSums + waveN * WTN + j * 32 + g * 8 + kb * 4);
-#pragma unroll
-    for (int i = 0; i < MI; i++) {
-      const float2v st = rowStat[waveM * WTM + i * 32 + l32];
+    for (int j = 0; j < NI; j++) {
       lanes2 o[4];
 #pragma unroll
       for (int g = 0; g < 4; g++) {
+        const float4v sums =
+            *reinterpret_cast<const float4v *>(colSums + waveN * WTN + j * 32 + g * 8 + kb * 4);
         half4 r;
 #pragma unroll
         for (int e = 0; e < 4; e++)
-          r[e] = _Float16(p.alpha * fmaf(st[0], acc[i][j][4 * g + e], st[1] * sums[g][e]));
+          r[e] = _Float16(p.alpha * fmaf(st[0], acc[i][j][4 * g + e], st[1] * sums[e]));
         o[g] = __builtin_bit_cast(lanes2, r);
       }
-      lanes4 lo = joinHalves(o[0][0], o[0][1], o[1][0], o[1][1]);
-      lanes4 hi = joinHalves(o[2][0], o[2][1], o[3][0], o[3][1]);
-      swapRows(lo, hi);
-      const bool in = colBase + j * 32 + cc < p.N;
-      const uint32_t at = uint32_t(i * 32 + l16) * ldd2 + uint32_t(j * 32 + cc) * 2u;
-      const uint32_t below = in ? at + 16u * ldd2 : kOob;
-      if (p.streamD) {
-        __builtin_amdgcn_raw_buffer_store_b128(lo, rsrcD, in ? at : kOob, 0, kStreamingAux);
-        __builtin_amdgcn_raw_buffer_store_b128(hi, rsrcD, below, 0, kStreamingAux);
-      } else {
-        __builtin_amdgcn_raw_buffer_store_b128(lo, rsrcD, in ? at : kOob, 0, kWriteThroughAux);
-        __builtin_amdgcn_raw_buffer_store_b128(hi, rsrcD, below, 0, kWriteThroughAux);
-      }
+      v[j][0] = joinHalves(o[0][0], o[0][1], o[1][0], o[1][1]);
+      v[j][1] = joinHalves(o[2][0], o[2][1], o[3][0], o[3][1]);
+      swapRows(v[j][0], v[j][1]);
     }
+    swapHalfRows(v[0][0], v[1][0]);
+    swapHalfRows(v[0][1], v[1][1]);
+    const uint32_t at =
+        in ? uint32_t(i * 32 + l16 % 8) * ldd2 + uint32_t(block * 32 + cc) * 2u : kOob;
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+      __builtin_amdgcn_raw_buffer_store_b128(v[q % 2][q / 2], rsrcD, at + q * step, 0, kWriteThroughAux);
   }
 }
 
@@ -971,8 +1001,9 @@ __host__ __device__ __forceinline__ int epilogueFastMode(const GemmParams &p,
 // Whether a tile's results leave by lane exchanges (epilogueLanes) or through the
 // wavefronts' strips of LDS (epilogueFast), by wave tile, source and activation.
 // Lanes against strips, time of the launch, three shapes each:
-//   128 x 64 (256 x 256 tiles, eight wavefronts): DMA staged -1 .. -7 %, with a full
-//     source -7 .. -19; STAGED through registers, linear -9 .. -18 without a source, -1 .. -14
+//   128 x 64 (256 x 256 tiles, eight wavefronts): DMA staged, linear -1 .. -7 % (+1 beyond results of
+//     112 MiB), with a full source -7 .. -19, GELU -1 .. 0; staged through registers, linear -9 .. -18
+//     without a source, -1 .. -14
 //     with a full one, -7 .. +6 with a bias row, GELU +2 .. +6 with a bias row.  (One way for all sources of a
 //     kernel: with both in it, it spills as it did before and gains nothing.)
 //   64 x 64: GELU without a full source -1 .. -5; linear -7 .. +5 either way.
@@ -998,27 +1029,27 @@ template <int MI, int NI, int EPI, int CMODE, bool STAGED> constexpr bool leaves
 template <int MI, int NI, int WTM, int WTN, int EPI, bool STAGED = false>
 __device__ __forceinline__ void
 epilogueAuto(const GemmParams &p, float16v (&acc)[MI][NI], int m0, int n0,
-             int waveM, int waveN, int lane, int wave, unsigned char *smem) {
+             int waveM, int waveN, int lane, int wave, unsigned char *smem, bool stream = false) {
   static_assert(EPI < kEpiFoldA, "folded epilogues are called directly");
   if constexpr (EPI <= int(Epilogue::kGeluTanh)) {
     const int mode = p.epiMode;
     if (mode == 0) {
       if constexpr (leavesByLanes<MI, NI, EPI, 0, STAGED>())
-        return epilogueLanes<MI, NI, WTM, WTN, EPI, 0>(p, acc, m0, n0, waveM, waveN, lane);
+        return epilogueLanes<MI, NI, WTM, WTN, EPI, 0>(p, acc, m0, n0, waveM, waveN, lane, stream);
       else
         return epilogueFast<MI, NI, WTM, WTN, EPI, 0>(p, acc, m0, n0, waveM, waveN,
                                                       lane, wave, smem);
     }
     if (mode == 1) {
       if constexpr (leavesByLanes<MI, NI, EPI, 1, STAGED>())
-        return epilogueLanes<MI, NI, WTM, WTN, EPI, 1>(p, acc, m0, n0, waveM, waveN, lane);
+        return epilogueLanes<MI, NI, WTM, WTN, EPI, 1>(p, acc, m0, n0, waveM, waveN, lane, stream);
       else
         return epilogueFast<MI, NI, WTM, WTN, EPI, 1>(p, acc, m0, n0, waveM, waveN,
                                                       lane, wave, smem);
     }
     if (mode == 2) {
       if constexpr (leavesByLanes<MI, NI, EPI, 2, STAGED>())
-        return epilogueLanes<MI, NI, WTM, WTN, EPI, 2>(p, acc, m0, n0, waveM, waveN, lane);
+        return epilogueLanes<MI, NI, WTM, WTN, EPI, 2>(p, acc, m0, n0, waveM, waveN, lane, stream);
       else
         return epilogueFast<MI, NI, WTM, WTN, EPI, 2>(p, acc, m0, n0, waveM, waveN,
                                                       lane, wave, smem);
@@ -1356,10 +1387,12 @@ inline Status planTiles(const GemmProblem &pr, int bm, int bn, int bk, int tileE
   p.cRowMagic = magicFor(uint32_t(p.cRowPeriod));
   // (the row range a wavefront addresses with 32-bit offsets is at most bm rows)
   p.epiMode = epilogueFastMode(p, bm);
-  // Results that leave nothing else in the 256 MB Infinity Cache are written past it:
-  // 16384 x 4096 x 1024 + GELU on three sets of operands in turn 158 -> 149 us, on one 150 ->
-  // 149; outputs of 15 to 56 MB differ by -5 to +2 % on three sets, so the line is drawn above them.
-  p.streamD = int64_t(p.M) * p.N * 2 > (int64_t(64) << 20);
+  // GELU results of more than half the 256 MB Infinity Cache are written past it, but for a
+  // workgroup's last tile (the launch would wait for memory at its end).  16384 x 4096 x 1024, 128
+  // MiB, three sets of operands in turn 162 us through LDS, 164 by lines, 158 past the cache (on
+  // another box 154 and 145); a call alone 161 -> 164, on a new buffer 176 -> 179.  Linear
+  // results: 149.9 -> 148.5, alone 157 -> 159.  Of 96 MiB (16384 x 3072 x 768): 90 -> 86, alone 92 -> 99.
+  p.streamD = int64_t(p.M) * p.N * 2 > (int64_t(120) << 20);
   p.workspace = nullptr;
   p.tileArrivals = nullptr;
   p.misplaced = nullptr;

@@ -866,7 +866,8 @@ __global__ __launch_bounds__(WM *WN *kWave) void gemmPipeKernel(
     }
   } else
     epilogueAuto<MI, NI, WTM, WTN, EPI, !DMA>(p, acc, m0, n0, waveM, waveN, lane,
-                                        wave, smem);
+                                        wave, smem,
+                                        p.streamD && vpid + int(gridDim.x) < nTiles);
   vpid += gridDim.x;
   } while (vpid < nTiles); // tiles of this workgroup
 }

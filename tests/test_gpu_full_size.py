@@ -49,7 +49,7 @@ def sample_rows(g, rows, count=48):
                                   "128x128_64x2r2_w2x4", "256x96_64x2r2_w4x1"])
 @pytest.mark.parametrize("act", [0, 1])
 @pytest.mark.parametrize("source", ["none", "bias", "full"])
-@pytest.mark.parametrize("M,N", [(8229, 4080),  # written past the last-level cache (> 64 MiB)
+@pytest.mark.parametrize("M,N", [(15501, 4080),  # GELU: written past the last-level cache (> 120 MiB)
                                  (301, 264)])   # edges in both directions inside a wavefront's blocks
 def test_gemm_results_by_lane_exchange(gpu, rt, tile, act, source, M, N):
     """Every output of the epilogues without LDS: a block misplaced by an exchange shows as an error
