@@ -574,7 +574,8 @@ def test_attention_splits(gpu, rt, bs, seq, heads, d):
 # lengths at the ends of 32-key blocks and 64-key chunks: split keys (64, 128, 256), whole rows (128; 64 up to 128
 # tokens with more tiles than half the CUs), and split keys between one and 1.4 tiles a CU
 @pytest.mark.parametrize("bs,seq,heads,d", [(13, 200, 2, 64), (13, 200, 2, 128), (13, 200, 2, 256), (48, 200, 2, 128),
-                                            (48, 100, 4, 64), (13, 200, 11, 128), (13, 200, 11, 64)])
+                                            (48, 100, 4, 64), (13, 200, 11, 128), (13, 200, 11, 64), (7, 64, 2, 128),
+                                            (10, 192, 2, 256)])
 def test_attention_chunk_ends(gpu, rt, bs, seq, heads, d):
     g = torch.Generator("cuda").manual_seed(seq + d)
     qkv = torch.randn(bs, seq, 3, heads, d, device="cuda", generator=g)
