@@ -586,7 +586,6 @@ __attribute__((amdgpu_waves_per_eu(D <= 128 || NW == 8 ? 2 : 1, D == 64 && KS ==
     for (; ch + 1 < numChunks; ch++)
       step(ch, std::true_type{});
     step(ch, std::false_type{});
-    rowSum = pairSum(rowSum); // (each lane has added up its own keys)
   } else {
   requestChunk(0);
   // (at least one round in either variant: a loop that may run zero times
@@ -734,7 +733,8 @@ __attribute__((amdgpu_waves_per_eu(D <= 128 || NW == 8 ? 2 : 1, D == 64 && KS ==
       //  - fast path (every block but a wavefront's first): p is computed
       //    against the reference as it stands, no maximum is taken at all, and
       //    the row sums that are needed anyway tell whether that was safe: if
-      //    some row's sum over the 64 keys exceeds kSumLimit (so a p could leave
+      //    some lane's sum (its half of a row's keys; the halves meet behind the last
+      //    block) exceeds kSumLimit (so a p could leave
       //    fp16's range; an overflowed exp2 gives inf and lands here too) the
       //    block's scores are recomputed from LDS and take the slow path;
       //  - slow path (the first block, and a block whose sums overflowed): the
@@ -757,7 +757,6 @@ __attribute__((amdgpu_waves_per_eu(D <= 128 || NW == 8 ? 2 : 1, D == 64 && KS ==
             accS[sb][e] = pv;
             blockSum += pv;
           }
-        blockSum = pairSum(blockSum);
         slow = __any(!(blockSum <= kSumLimit));
         if (slow)
           scores(); // the probabilities are discarded: raw scores again
@@ -791,7 +790,6 @@ __attribute__((amdgpu_waves_per_eu(D <= 128 || NW == 8 ? 2 : 1, D == 64 && KS ==
             accS[sb][e] = pv;
             blockSum += pv;
           }
-        blockSum = pairSum(blockSum);
       }
       rowSum += blockSum;
 
@@ -843,6 +841,7 @@ __attribute__((amdgpu_waves_per_eu(D <= 128 || NW == 8 ? 2 : 1, D == 64 && KS ==
     }
   } while (++ch < numChunks);
   }
+  rowSum = pairSum(rowSum); // (each lane has added up its own keys)
 
   // ---- merge the key shares ----
   // Share 1 hands (reference, sum, O) of its rows to share 0 through LDS, in
