@@ -1390,7 +1390,7 @@ inline Status planTiles(const GemmProblem &pr, int bm, int bn, int bk, int tileE
   // GELU results of more than half the 256 MB Infinity Cache are written past it, but for a
   // workgroup's last tile (the launch would wait for memory at its end).  16384 x 4096 x 1024, 128
   // MiB, three sets of operands in turn 162 us through LDS, 164 by lines, 158 past the cache (on
-  // another box 154 and 145); a call alone 161 -> 164, on a new buffer 176 -> 179.  Linear
+  // another box 154 and 145); a call alone 161 -> 164, on new buffers 168 .. 176 -> 179 .. 182.  Linear
   // results: 149.9 -> 148.5, alone 157 -> 159.  Of 96 MiB (16384 x 3072 x 768): 90 -> 86, alone 92 -> 99.
   p.streamD = int64_t(p.M) * p.N * 2 > (int64_t(120) << 20);
   p.workspace = nullptr;
