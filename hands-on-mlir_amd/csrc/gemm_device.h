@@ -97,8 +97,6 @@ struct GemmParams {
   int fullGroups, lastRows;
   // epilogueFastMode() evaluated on the host for the whole launch
   int epiMode;
-  // D is too large to be found in the last-level cache later (kStreamingAux)
-  int streamD;
   // layer-norm pair (kEpiRowStats / kEpiRowAffine kernels only)
   float *rowStatPartials;
   const _Float16 *rowScale;
@@ -535,11 +533,10 @@ epilogueFast(const GemmParams &p, float16v (&acc)[MI][NI], int m0, int n0,
 // 32 apart exchange halves (joinHalves) and rows of 16 lanes change places (swapRows),
 // so that a lane has 8 consecutive columns and a store instruction writes 64 bytes of
 // 16 rows.  No barrier, and a wavefront's stores go out while others still multiply.
-// stream: past the last-level cache (GemmParams::streamD).
 template <int MI, int NI, int WTM, int WTN, int EPI, int CMODE>
 __device__ __forceinline__ void
 epilogueLanes(const GemmParams &p, float16v (&acc)[MI][NI], int m0, int n0,
-              int waveM, int waveN, int lane, bool stream) {
+              int waveM, int waveN, int lane) {
   constexpr uint32_t kOob = 0x80000000u;
   const int l16 = lane % 16, kb = lane / 32;
   // columns of this lane's 16 bytes in a block of 32
@@ -588,6 +585,9 @@ epilogueLanes(const GemmParams &p, float16v (&acc)[MI][NI], int m0, int n0,
   // (swapHalfRows), so that an instruction writes 8 rows' whole 128-byte lines.  By 64 bytes,
   // results that the last-level cache has to make room for took longer: 16384 x 4096 x 1024 in
   // requests 140 us through LDS, 162 by 64 bytes, 142 by lines; 16384 x 3072 x 768 91, 96, 86.
+  // Always written through, never past that cache: with GELU (128 MiB of results) three sets of operands in
+  // turn took 153 us so instead of 160, but a first call on new buffers 188 instead of 170, and a call
+  // followed by the 16384 x 1024 x 4096 that reads it 296 instead of 283 for both (through LDS 159, 182, 289).
   constexpr bool kLines = MI == 4 && NI == 2;
   lanes4 left[2]; // the even block of a pair
 #pragma unroll
@@ -639,17 +639,10 @@ epilogueLanes(const GemmParams &p, float16v (&acc)[MI][NI], int m0, int n0,
                                   ? uint32_t(i * 32 + l16 % 8) * ldd2 + uint32_t(block * 32 + cc) * 2u
                                   : kOob;
           const uint32_t step = at == kOob ? 0u : 8u * ldd2; // rows 0 .., 8 .., 16 .., 24 ..
-          auto store = [&](auto auxC) {
-            constexpr int kAux = decltype(auxC)::value;
-            __builtin_amdgcn_raw_buffer_store_b128(left[0], rsrcD, at, 0, kAux);
-            __builtin_amdgcn_raw_buffer_store_b128(lo, rsrcD, at + step, 0, kAux);
-            __builtin_amdgcn_raw_buffer_store_b128(left[1], rsrcD, at + 2 * step, 0, kAux);
-            __builtin_amdgcn_raw_buffer_store_b128(hi, rsrcD, at + 3 * step, 0, kAux);
-          };
-          if (EPI != int(Epilogue::kLinear) && stream)
-            store(std::integral_constant<int, kStreamingAux>{});
-          else
-            store(std::integral_constant<int, kWriteThroughAux>{});
+          __builtin_amdgcn_raw_buffer_store_b128(left[0], rsrcD, at, 0, kWriteThroughAux);
+          __builtin_amdgcn_raw_buffer_store_b128(lo, rsrcD, at + step, 0, kWriteThroughAux);
+          __builtin_amdgcn_raw_buffer_store_b128(left[1], rsrcD, at + 2 * step, 0, kWriteThroughAux);
+          __builtin_amdgcn_raw_buffer_store_b128(hi, rsrcD, at + 3 * step, 0, kWriteThroughAux);
         }
       } else {
         __builtin_amdgcn_raw_buffer_store_b128(lo, rsrcD, offsetOf(i, j, 0, ldd2), 0, kWriteThroughAux);
@@ -1029,27 +1022,27 @@ template <int MI, int NI, int EPI, int CMODE, bool STAGED> constexpr bool leaves
 template <int MI, int NI, int WTM, int WTN, int EPI, bool STAGED = false>
 __device__ __forceinline__ void
 epilogueAuto(const GemmParams &p, float16v (&acc)[MI][NI], int m0, int n0,
-             int waveM, int waveN, int lane, int wave, unsigned char *smem, bool stream = false) {
+             int waveM, int waveN, int lane, int wave, unsigned char *smem) {
   static_assert(EPI < kEpiFoldA, "folded epilogues are called directly");
   if constexpr (EPI <= int(Epilogue::kGeluTanh)) {
     const int mode = p.epiMode;
     if (mode == 0) {
       if constexpr (leavesByLanes<MI, NI, EPI, 0, STAGED>())
-        return epilogueLanes<MI, NI, WTM, WTN, EPI, 0>(p, acc, m0, n0, waveM, waveN, lane, stream);
+        return epilogueLanes<MI, NI, WTM, WTN, EPI, 0>(p, acc, m0, n0, waveM, waveN, lane);
       else
         return epilogueFast<MI, NI, WTM, WTN, EPI, 0>(p, acc, m0, n0, waveM, waveN,
                                                       lane, wave, smem);
     }
     if (mode == 1) {
       if constexpr (leavesByLanes<MI, NI, EPI, 1, STAGED>())
-        return epilogueLanes<MI, NI, WTM, WTN, EPI, 1>(p, acc, m0, n0, waveM, waveN, lane, stream);
+        return epilogueLanes<MI, NI, WTM, WTN, EPI, 1>(p, acc, m0, n0, waveM, waveN, lane);
       else
         return epilogueFast<MI, NI, WTM, WTN, EPI, 1>(p, acc, m0, n0, waveM, waveN,
                                                       lane, wave, smem);
     }
     if (mode == 2) {
       if constexpr (leavesByLanes<MI, NI, EPI, 2, STAGED>())
-        return epilogueLanes<MI, NI, WTM, WTN, EPI, 2>(p, acc, m0, n0, waveM, waveN, lane, stream);
+        return epilogueLanes<MI, NI, WTM, WTN, EPI, 2>(p, acc, m0, n0, waveM, waveN, lane);
       else
         return epilogueFast<MI, NI, WTM, WTN, EPI, 2>(p, acc, m0, n0, waveM, waveN,
                                                       lane, wave, smem);
@@ -1387,12 +1380,6 @@ inline Status planTiles(const GemmProblem &pr, int bm, int bn, int bk, int tileE
   p.cRowMagic = magicFor(uint32_t(p.cRowPeriod));
   // (the row range a wavefront addresses with 32-bit offsets is at most bm rows)
   p.epiMode = epilogueFastMode(p, bm);
-  // GELU results of more than half the 256 MB Infinity Cache are written past it, but for a
-  // workgroup's last tile (the launch would wait for memory at its end).  16384 x 4096 x 1024, 128
-  // MiB, three sets of operands in turn 162 us through LDS, 164 by lines, 158 past the cache (on
-  // another box 154 and 145); a call alone 161 -> 164, on new buffers 168 .. 176 -> 179 .. 182.  Linear
-  // results: 149.9 -> 148.5, alone 157 -> 159.  Of 96 MiB (16384 x 3072 x 768): 90 -> 86, alone 92 -> 99.
-  p.streamD = int64_t(p.M) * p.N * 2 > (int64_t(120) << 20);
   p.workspace = nullptr;
   p.tileArrivals = nullptr;
   p.misplaced = nullptr;

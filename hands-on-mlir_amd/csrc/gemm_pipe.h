@@ -866,8 +866,7 @@ __global__ __launch_bounds__(WM *WN *kWave) void gemmPipeKernel(
     }
   } else
     epilogueAuto<MI, NI, WTM, WTN, EPI, !DMA>(p, acc, m0, n0, waveM, waveN, lane,
-                                        wave, smem,
-                                        p.streamD && vpid + int(gridDim.x) < nTiles);
+                                        wave, smem);
   vpid += gridDim.x;
   } while (vpid < nTiles); // tiles of this workgroup
 }

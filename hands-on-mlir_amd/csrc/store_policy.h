@@ -23,8 +23,6 @@ namespace hom {
 // auxiliary (cache policy) operand of the raw buffer store builtins:
 // bit 0 = sc0, bit 4 = sc1
 constexpr int kWriteThroughAux = 17;
-// (bit 1 = nt) what storeStreaming() does
-constexpr int kStreamingAux = 18;
 
 // *p = v with the sc0 sc1 bits.
 // (p: any element boundary, the hardware's wide stores take it)
