@@ -30,6 +30,7 @@
 // ds_read_b64_tr_b16 (the transposing LDS read) from the row-major V tile.
 // LDS rows are 128 bytes, unpadded; 16-byte chunks (K) / 64-byte groups (V) are
 // XOR-permuted by row so that the fragment reads are bank-conflict free.
+#include "attention_way.h"
 #include "cross_lane.h"
 #include "fast_div.h"
 #include "packed_args.h"
@@ -999,57 +1000,22 @@ Status launchBertAttentionF16(const _Float16 *qkv, const int32_t *cuSeqlens,
       ahead && pairs * ((seq + 127) / 128) <= 2 * cus ? aheadGroups<256>(aheadBytes, cus) : 0;
   const Launch l{qkv, cuSeqlens, out, bs, seq, heads, scale, packedOut,
                  static_cast<const char *>(ahead), aheadBytes, packedIn ? extra : 0, s};
-  // Four ways, all with the same arithmetic per 32 query rows (us, lengths uniform
-  // in [seq / 4, seq], batch : seq : heads):
-  //  - Prefetch: 64 rows per workgroup with the keys split over two wavefronts per
-  //    32 rows, K and V of the first 128 keys requested before anything else is
-  //    known.  The fastest while that is all of them and every workgroup has a CU of
-  //    its own (head size 64, 8:128:12 4.2, against 5.0 - 5.3; 26:105:8, where it has not,
-  //    6.4 against 4.8 by Dma, 11:119:16 6.45 against 4.9).
-  //  - Wide: 128 rows, chunks of 128 keys through registers; head size 64 for so
-  //    many short sequences that the workgroups of a CU cover each other
-  //    (64:70:12 7.7 against 7.9, but 32:128:16 8.3 against 7.95), and 256, whose chunks by
-  //    DMA would leave too few registers (8:384:16 42 against 47).
-  //  - Dma: 128 rows, chunks of 64 keys straight into LDS while the one before is
-  //    worked on (head size 64, 32:512:16 41.8 -> 40.6, 1:64:12 4.0 -> 3.6; 128,
-  //    32:512:16 66.9 -> 60.9).  Head size 192: 8 wavefronts, two per 32 rows, which
-  //    then fit two to a SIMD (32:512:12 117 -> 97).
-  //  - DmaSplit: the same with 64 rows and two wavefronts per 32 rows, where its
-  //    finer workgroups spread better over the CUs.  That is up to half a CU's worth of
-  //    128-row tiles (3:346:8 of 64 5.0 against 6.1, 3:615:8 of 128 10.8 against 13.9, 4:185:16
-  //    of 256 11.9 against 14.5, 8:200:8 of 192 10.1 against 11.8) and, at head sizes 64 and 128,
-  //    also up to 0.6 (2:707:12 of 64 7.6 against 9.6, of 128 2:657:12 9.7 against 12.0) and
-  //    from one to 1.4 tiles a CU, where a second tile would be all that some CUs do
-  //    (4:700:12 9.6 against 12.2, 9:189:16 6.3 against 6.5, 6:746:8 of 128 18.1 against 19.8).
-  //    Between and above those Dma: 7:235:12 6.4 against 6.8, 8:384:16 9.6 against 11.0, 16:200:12
-  //    7.5 against 9.4; of 128 7:241:16 9.2 against 10.6, 16:256:12 13.6 against 16.3, 8:384:16 14.8
-  //    against 15.2.  (64, long sequences of few batches up to a tile a CU: 2:747:16
-  //    8.3 against 9.7 split, 5:493:12 9.75 against 8.9.)
-  enum { Prefetch, Wide, Dma, DmaSplit } way;
-  const int64_t tiles = pairs * ((seq + 127) / 128);
-  const bool few = tiles <= cus / 2;
-  const bool finer = 10 * tiles <= 6 * cus || (tiles > cus && 10 * tiles <= 14 * cus);
-  if (headDim == 64)
-    way = seq <= 64    ? Dma
-          : seq <= 128 ? (few ? Prefetch : tiles <= 2 * cus ? Dma : Wide)
-                       : (finer || (tiles <= cus && seq > 512) ? DmaSplit : Dma);
-  else if (headDim == 128)
-    way = seq > 64 && (tiles < cus / 2 || (seq > 128 && finer)) ? DmaSplit : Dma;
-  else
-    way = few ? DmaSplit : headDim == 192 ? Dma : Wide;
+  AttentionWay way = attentionWay(pairs, seq, headDim, packedIn, cus);
   // profiling knob: HOM_ATTENTION_VARIANT=wide | split
   if (const char *force = getenv("HOM_ATTENTION_VARIANT"))
-    way = strcmp(force, "wide") == 0 ? (headDim == 256 ? Wide : Dma) : DmaSplit;
+    way = strcmp(force, "wide") != 0 ? AttentionWay::kDmaSplit
+          : headDim == 256          ? AttentionWay::kWide
+                                    : AttentionWay::kDma;
   switch (headDim) {
   case 64:
     switch (way) {
-    case Prefetch:
+    case AttentionWay::kPrefetch:
       return packedIn ? launchVariant<4, 2, 64, true, false>(l)
                       : launchVariant<4, 2, 64, false, false>(l);
-    case Wide:
+    case AttentionWay::kWide:
       return packedIn ? launchVariant<4, 1, 64, true, false>(l)
                       : launchVariant<4, 1, 64, false, false>(l);
-    case Dma:
+    case AttentionWay::kDma:
       return packedIn ? launchVariant<4, 1, 64, true, true>(l)
                       : launchVariant<4, 1, 64, false, true>(l);
     default:
@@ -1057,14 +1023,14 @@ Status launchBertAttentionF16(const _Float16 *qkv, const int32_t *cuSeqlens,
                       : launchVariant<4, 2, 64, false, true>(l);
     }
   case 128:
-    return way != Dma  ? launchVariant<4, 2, 128, false, true>(l)
+    return way != AttentionWay::kDma ? launchVariant<4, 2, 128, false, true>(l)
            : seq > 64 ? launchVariant<4, 1, 128, false, true, true>(l)
                       : launchVariant<4, 1, 128, false, true, false>(l);
   case 192:
-    return way == Dma ? launchVariant<8, 2, 192, false, true>(l)
+    return way == AttentionWay::kDma ? launchVariant<8, 2, 192, false, true>(l)
                       : launchVariant<4, 2, 192, false, true>(l);
   default:
-    return way == Wide ? launchVariant<4, 1, 256, false, false>(l)
+    return way == AttentionWay::kWide ? launchVariant<4, 1, 256, false, false>(l)
            : seq > 192 ? launchVariant<4, 2, 256, false, true, true>(l)
                        : launchVariant<4, 2, 256, false, true, false>(l);
   }
