@@ -80,14 +80,8 @@ template <int D> __device__ __forceinline__ int swzV(int k, int group) {
   return D == 64 || D == 192 ? group ^ ((k >> 1) & 1) : group ^ (k & 3);
 }
 
-// Order of the workgroups: the query tiles of a (batch, head) back to back, or all
-// first tiles, then all second ones, .., so that those of nothing but padding come
-// last.  That pays where the workgroups of a launch do not all fit the chip at
-// once (two to a CU at head size 128, one above) and all K and V fit the L2s, as in the
-// launches the key-split variant takes: 16:200:12 heads of 128 14.4 -> 13.8 us, 8:384:16
-// 15.1 -> 14.7, 1:700:12 of 256 22.5 -> 21.9; at head size 64, where all are resident,
-// 8:500:12 takes 14.9 instead of 13.9, and 32:512:12 of 192 on eight wavefronts 104.8 instead
-// of 102.1.
+// Kernels whose launches may have all first query tiles first (attentionTilesOutside).  On eight wavefronts
+// 32:512:12 of 192 takes 104.8 us so instead of 102.1.
 template <int NW, int KS, int D, bool DMA>
 constexpr bool kTilesOutside = DMA && KS == 2 && NW == 4 && D >= 128;
 
@@ -178,7 +172,7 @@ __attribute__((amdgpu_waves_per_eu(D <= 128 || NW == 8 ? 2 : 1, D == 64 && KS ==
       }
     }
     int pair;
-    if (kTilesOutside<NW, KS, D, DMA>) {
+    if (kTilesOutside<NW, KS, D, DMA> && attentionTilesOutside(pairs, numQTiles)) {
       qTile = int(divByMagic(uint32_t(id), uint32_t(pairs), numQMagic));
       pair = id - qTile * pairs;
     } else if (pairs % 8 == 0) {
@@ -950,9 +944,10 @@ Status launchVariant(const Launch &l) {
     const unsigned plane = nq * unsigned(l.heads);
     grid = dim3(nq, unsigned(l.heads), unsigned(l.bs) + (l.extra + plane - 1) / plane);
   }
+  const bool outside = kTilesOutside<NW, KS, D, DMA> && attentionTilesOutside(int(pairs), int(nq));
   kernel<<<grid, dim3(NW * kWave), kLds, l.stream>>>(l.qkv, l.cu, l.out, int(l.seq), int(l.heads),
                                                      int(nq), int(l.bs), l.scale, l.packedOut,
-                                                     magicFor(kTilesOutside<NW, KS, D, DMA> ? uint32_t(pairs) : nq), magicFor(uint32_t(l.heads)),
+                                                     magicFor(outside ? uint32_t(pairs) : nq), magicFor(uint32_t(l.heads)),
                                                      l.ahead, l.aheadBytes);
   HOM_HIP_RET(hipGetLastError(), Status::kInternal);
   return Status::kSuccess;

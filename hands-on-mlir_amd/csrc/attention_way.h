@@ -70,4 +70,15 @@ inline AttentionWay attentionWay(int64_t pairs, int64_t seq, int64_t headDim, bo
   return few ? AttentionWay::kDmaSplit : headDim == 192 ? AttentionWay::kDma : AttentionWay::kWide;
 }
 
+// Order of the workgroups of split keys at head sizes from 128 on: the query tiles of a pair
+// (batch entry, head) back to back, or (true) all first tiles, then all second ones, .., so that
+// those of nothing but padding come last.  That pays
+//  - up to one and a half workgroups a CU, where the last ones find a CU free: of 128, pairs a multiple of 8, eight
+//    draws of lengths uniform in [seq / 4, seq], 0.86 to 1.05 of the time with 257 to 320 workgroups (mean of
+//    11 shapes 0.94), 0.91 to 1.07 to 384 (13, 0.98), beyond means of 1.01 to 1.05 (118; 8:620:8 17.6 -> 20.5 us);
+//  - where the pairs are no multiple of 8: back to back a pair's tiles go to the XCDs in turn, and those past the
+//    end of its sequence to the same few of them (22 shapes 0.70 to 1.015; 1:700:12 10.0 -> 9.1 us, of 256 20.0 ->
+//    19.5, of 192 14.7 -> 14.3).
+constexpr bool attentionTilesOutside(int pairs, int tiles) { return pairs % 8 != 0 || pairs * tiles <= 384; }
+
 } // namespace hom
