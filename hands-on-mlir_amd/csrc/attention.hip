@@ -105,17 +105,13 @@ __device__ __forceinline__ void storeVector(_Float16 *p, u32x4 v) {
 // PIPE: the next chunk's scores between this chunk's exponentials, so that one
 // wavefront has the matrix cores and the vector ALU at work at once (a kernel that
 // takes them in turn is bound by the sum of both, also with two wavefronts on a SIMD).
-// It costs the registers of another block's scores.  us without and with it, lengths
-// uniform in [seq / 4, seq]: head size 128, 32:512:16 70.9 -> 68.3, 16:200:12 15.2 -> 14.4,
-// 2:700:12 13.0 -> 11.9, 1:700:8 9.1 -> 8.25, from 64 on (1:33:16 4.2 -> 4.3); 64 with split keys 2:700:16 9.2 -> 8.8, 8:500:12
-// 14.1 -> 13.8; 256 with split keys 1:700:12 23.4 -> 22.5, 2:300:8 13.0 -> 12.8, but 1:33:16 7.3
-// -> 7.6 and 1:106:8 8.5 -> 8.7, so from 192 on.  Not for head size 64 with whole
-// rows (32:512:16 37.2 -> 40.1: two wavefronts a SIMD instead of four), 192 (32:512:12 102.1
-// -> 104.7, spills) and fragment order (BERT-base 8 x 384 1315 -> 1328, 2 x 700 equal).
+// It costs the registers of another block's scores; from how many tokens on it pays:
+// attentionOverlapsScores().  Not for head size 64 with whole rows (us, lengths uniform in [seq / 4,
+// seq], 32:512:16 37.2 -> 40.1: two wavefronts a SIMD instead of four), 192 (32:512:12 102.1
+// -> 104.7, spills) and fragment order (requests, BERT-base 8 x 384 1315 -> 1328, 2 x 700 equal).
 template <int D, int KS, bool PACKED_IN, bool DMA>
-constexpr bool kPipe = DMA && (D == 128 || (KS == 2 && !PACKED_IN && D == 64));
-template <int NW, int KS, int D, bool PACKED_IN = false, bool DMA = false,
-          bool PIPE = kPipe<D, KS, PACKED_IN, DMA>>
+constexpr bool kPipe = DMA && !PACKED_IN && (D == 128 || (KS == 2 && (D == 64 || D == 256)));
+template <int NW, int KS, int D, bool PACKED_IN, bool DMA, bool PIPE>
 __global__ __launch_bounds__(NW *kWave)
 __attribute__((amdgpu_waves_per_eu(D <= 128 || NW == 8 ? 2 : 1, D == 64 && KS == 1 ? 4 : (D <= 128 || NW == 8 ? 2 : 1)))) void bertAttentionKernel(
     const _Float16 *__restrict__ qkv, const int32_t *__restrict__ cu,
@@ -921,8 +917,12 @@ struct Launch {
   unsigned extra; // workgroups that read ahead
   hipStream_t stream;
 };
-template <int NW, int KS, int D, bool PACKED_IN, bool DMA, bool PIPE = kPipe<D, KS, PACKED_IN, DMA>>
+template <int NW, int KS, int D, bool PACKED_IN, bool DMA, bool PIPE = false>
 Status launchVariant(const Launch &l) {
+  if constexpr (kPipe<D, KS, PACKED_IN, DMA> && !PIPE) {
+    if (attentionOverlapsScores(D, l.seq))
+      return launchVariant<NW, KS, D, PACKED_IN, DMA, true>(l);
+  }
   constexpr int QG = NW / KS;
   constexpr int kTileBytes = (DMA ? 64 : Chunk<D>::value) * D * 2;
   constexpr int kExchange = KS == 2 ? QG * (D / 2 + 2) * kWave * 4 : 0;
@@ -1018,16 +1018,14 @@ Status launchBertAttentionF16(const _Float16 *qkv, const int32_t *cuSeqlens,
                       : launchVariant<4, 2, 64, false, true>(l);
     }
   case 128:
-    return way != AttentionWay::kDma ? launchVariant<4, 2, 128, false, true>(l)
-           : seq > 64 ? launchVariant<4, 1, 128, false, true, true>(l)
-                      : launchVariant<4, 1, 128, false, true, false>(l);
+    return way == AttentionWay::kDma ? launchVariant<4, 1, 128, false, true>(l)
+                                     : launchVariant<4, 2, 128, false, true, true>(l); // (beyond 64 tokens only)
   case 192:
     return way == AttentionWay::kDma ? launchVariant<8, 2, 192, false, true>(l)
-                      : launchVariant<4, 2, 192, false, true>(l);
+                                     : launchVariant<4, 2, 192, false, true>(l);
   default:
     return way == AttentionWay::kWide ? launchVariant<4, 1, 256, false, false>(l)
-           : seq > 192 ? launchVariant<4, 2, 256, false, true, true>(l)
-                       : launchVariant<4, 2, 256, false, true, false>(l);
+                                      : launchVariant<4, 2, 256, false, true>(l);
   }
 }
 

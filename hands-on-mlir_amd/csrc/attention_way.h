@@ -81,4 +81,16 @@ inline AttentionWay attentionWay(int64_t pairs, int64_t seq, int64_t headDim, bo
 //    19.5, of 192 14.7 -> 14.3).
 constexpr bool attentionTilesOutside(int pairs, int tiles) { return pairs % 8 != 0 || pairs * tiles <= 384; }
 
+// Whether the chunked kernels issue the next chunk's scores between this chunk's exponentials (see
+// kPipe in attention.hip for those that never do).  A first and last chunk have nothing to overlap, so it depends on
+// the length.  Time with it over without, six draws of lengths uniform in [seq / 4, seq]:
+//  - 64, split keys: to 192 tokens 0.99 to 1.05 (9:129:16 5.3 -> 5.6 us), 193 to 256 0.97 to 0.99, beyond 0.95 to
+//    1.03 (mean 0.99; 2:520:12 7.0 -> 6.65).
+//  - 128, whole rows: 1.0 to 1.01 to 64 tokens, beyond 0.90 to 1.01 (1:720:16 13.6 -> 12.25).  Split keys, which
+//    are for more tokens than that anyway, 0.92 to 1.016 (1:720:16 10.5 -> 9.7).
+//  - 256, split keys: 1.03 to 1.05 to 65 tokens, 0.986 to 1.017 to 192, beyond 0.97 to 1.0 (3:620:8 23.8 -> 23.1).
+constexpr bool attentionOverlapsScores(int64_t headDim, int64_t seq) {
+  return headDim == 128 ? seq > 64 : seq > 192;
+}
+
 } // namespace hom

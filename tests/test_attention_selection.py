@@ -55,3 +55,10 @@ def test_attention_takes_the_faster_way(tmp_path, d, packed):
                                           (False, [(8, 620, 8), (4, 582, 16), (4, 575, 16), (4, 700, 12), (6, 384, 16)])])
 def test_order_of_the_query_tiles(tmp_path, faster, sizes):
     assert answers(tmp_path, (f"attentionTilesOutside({b * h}, {-(-s // 64)})" for b, s, h in sizes)) == [faster] * len(sizes)
+
+
+# (head size, seq) -> scores under the softmax: where both were timed, at the ends of the ranges
+def test_lengths_with_scores_under_the_softmax(tmp_path):
+    want = {(64, 129): 0, (64, 192): 0, (64, 193): 1, (64, 720): 1, (128, 64): 0, (128, 80): 1, (128, 720): 1, (256, 65): 0,
+            (256, 192): 0, (256, 256): 1, (256, 720): 1}
+    assert answers(tmp_path, (f"attentionOverlapsScores({d}, {s})" for d, s in want)) == list(want.values())
