@@ -28,9 +28,9 @@ enum class AttentionWay { kPrefetch, kWide, kDma, kDmaSplit };
 // leave less idle where a sequence ends inside a tile; but all K and V are read twice as often.
 // Both timed in turn at 200 shapes of each head size (130 to 770 tokens, 0.4 to 2.2 tiles of 128 rows a
 // CU), eight draws of lengths and full ones.  Whole rows over split keys, by tiles a CU:
-//  - to 0.6: 1.08 to 1.29.  Up to 192 tokens also while the 64-row workgroups have a CU each, 1.09 to 1.15.
-//  - to 1: of 128 0.87 to 1.08 (full lengths 0.84 to 0.96); of 64 0.94 to 1.0 up to 256 tokens, 1.03 to 1.13 beyond
-//    384 (full 0.92 to 1.03), between those 0.99 to 1.08 up to 0.8 tiles and 0.99 to 1.03 (full 0.94 to 0.98) above.
+//  - to 0.6: 1.08 to 1.29.  Up to 192 tokens also to 1.1 workgroups of 64 rows a CU, 1.08 to 1.15.
+//  - to 1: of 128 0.87 to 1.08 (full lengths 0.84 to 0.96); of 64 0.94 to 1.0 up to 256 tokens, 0.99 to 1.13 beyond
+//    (full 0.87 to 1.03).
 //  - to 1.4, where a second tile would be all that some CUs do: 1.0 to 1.2 (full 0.74 to 1.24), but 0.83 to 0.87 from
 //    193 to 256 tokens, two full tiles.
 //  - to 1.8: 1.0 to 1.15 where the last tile is at most half full (full lengths 0.77 to 0.96), 0.8 to 1.03 where
@@ -46,7 +46,7 @@ inline bool attentionSplitsKeys(int64_t pairs, int64_t seq, int64_t headDim, boo
   if (10 * tiles <= 6 * cus || (seq <= 192 && 10 * tiles64 <= 11 * cus))
     return true;
   if (tiles <= cus)
-    return packed || (headDim == 64 && (seq > 384 || (seq > 256 && 10 * tiles <= 8 * cus)));
+    return packed || (headDim == 64 && seq > 256);
   if (seq > 192 && seq <= 256)
     return false;
   if (10 * tiles <= 14 * cus)

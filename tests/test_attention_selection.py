@@ -28,7 +28,7 @@ def ways(tmp_path, problems):
 # sequence on; the other way took 5 % more at least in the mean, in fragment order 0.7 % of a request of six layers.
 TIMED = {
     (64, False): {"split": [(4, 135, 16), (6, 223, 8), (2, 345, 16), (1, 706, 16), (5, 150, 16), (7, 307, 8), (4, 543, 12),
-                            (11, 157, 16), (8, 294, 12), (3, 776, 16), (19, 132, 12), (16, 290, 8)],
+                            (11, 157, 16), (8, 294, 12), (3, 776, 16), (19, 132, 12), (16, 290, 8), (6, 300, 12)],
                   "whole": [(10, 150, 12), (7, 195, 16), (11, 193, 16), (26, 251, 8), (16, 380, 8), (5, 749, 12),
                             (30, 171, 8), (21, 228, 12), (11, 258, 16), (16, 442, 8)]},
     (128, False): {"split": [(8, 153, 8), (8, 220, 8), (4, 307, 8), (1, 706, 16), (10, 165, 8), (12, 147, 12), (12, 362, 8),
