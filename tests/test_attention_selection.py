@@ -62,3 +62,15 @@ def test_lengths_with_scores_under_the_softmax(tmp_path):
     want = {(64, 129): 0, (64, 192): 0, (64, 193): 1, (64, 720): 1, (128, 64): 0, (128, 80): 1, (128, 720): 1, (256, 65): 0,
             (256, 192): 0, (256, 256): 1, (256, 720): 1}
     assert answers(tmp_path, (f"attentionOverlapsScores({d}, {s})" for d, s in want)) == list(want.values())
+
+
+# Sizes (batch, seq, heads, head size, fragment order) that tests of the kernels use for each way
+@pytest.mark.parametrize("way,sizes", [
+    ("prefetch", [(3, 100, 4, 64, False), (5, 99, 16, 64, True)]),
+    ("wide", [(44, 100, 12, 64, False), (48, 100, 11, 64, False), (44, 100, 12, 64, True), (48, 200, 2, 256, False)]),
+    ("whole", [(30, 128, 12, 64, False), (24, 128, 12, 64, True), (40, 200, 8, 64, True), (48, 200, 2, 128, False),
+               (13, 200, 11, 64, False), (13, 200, 5, 192, False)]),
+    ("split", [(13, 160, 11, 64, False), (13, 160, 11, 128, False), (2, 300, 4, 64, True), (13, 200, 2, 128, False),
+               (16, 100, 8, 192, False), (10, 192, 2, 256, False)])])
+def test_sizes_that_stand_for_a_way(tmp_path, way, sizes):
+    assert ways(tmp_path, sizes) == [way] * len(sizes)

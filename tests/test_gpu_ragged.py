@@ -482,9 +482,9 @@ def test_packed_layernorm(gpu, rt, M, H):
     np.testing.assert_array_equal(got, host(rows))
 
 
-# both variants of the attention kernel; batch entries that start inside a row block, chunk ends inside one
+# every way of the attention kernel; batch entries that start inside a row block, chunk ends inside one
 @pytest.mark.parametrize("bs,seq,heads", [(1, 1, 1), (3, 33, 2), (2, 64, 12), (5, 99, 16), (2, 300, 4), (24, 128, 12),
-                                          (40, 200, 8), (257, 17, 3)])
+                                          (40, 200, 8), (257, 17, 3), (44, 100, 12)])
 def test_attention_in_fragment_order(gpu, rt, bs, seq, heads):
     g, H = np.random.default_rng(bs + seq), heads * 64
     rows, Mr = bs * seq, rt.MemRef
@@ -527,7 +527,8 @@ def test_encoder_many_rows_equals_row_major(synth, bs, seq):
 # the result is stored 16 bytes a lane from any 8-byte boundary: the same values there, padding rows included, and
 # nothing beside them (each way of the dispatch)
 @pytest.mark.parametrize("bs,seq,heads,d", [(1, 50, 2, 64), (3, 100, 4, 64), (30, 128, 12, 64), (2, 300, 4, 64),
-                                            (2, 200, 4, 128), (3, 130, 3, 192), (2, 70, 2, 256), (8, 384, 16, 256)])
+                                            (2, 200, 4, 128), (3, 130, 3, 192), (2, 70, 2, 256), (8, 384, 16, 256),
+                                            (44, 100, 12, 64)])
 def test_attention_result_on_8_bytes(gpu, rt, bs, seq, heads, d):
     g = torch.Generator(device="cuda").manual_seed(seq)
     qkv = torch.randn(bs, seq, 3 * heads * d, generator=g, device="cuda").half()
@@ -550,7 +551,7 @@ def test_attention_result_on_8_bytes(gpu, rt, bs, seq, heads, d):
 @pytest.mark.parametrize("bs,seq,heads,d", [(2, 60, 4, 64), (3, 100, 4, 64), (30, 128, 12, 64), (2, 300, 4, 64),
                                             (40, 200, 8, 64), (2, 64, 4, 128), (3, 130, 4, 128), (40, 256, 8, 128),
                                             (2, 70, 3, 192), (16, 129, 9, 192), (2, 70, 3, 256), (16, 129, 9, 256),
-                                            (5, 193, 2, 256)])
+                                            (5, 193, 2, 256), (44, 100, 12, 64)])
 def test_attention_splits(gpu, rt, bs, seq, heads, d):
     g = torch.Generator("cuda").manual_seed(seq + d)
     qkv = torch.randn(bs, seq, 3, heads, d, device="cuda", generator=g).half()
@@ -572,10 +573,12 @@ def test_attention_splits(gpu, rt, bs, seq, heads, d):
 
 
 # lengths at the ends of 32-key blocks and 64-key chunks: split keys (64, 128, 256), whole rows (128; 64 up to 128
-# tokens with more tiles than half the CUs), and split keys between one and 1.4 tiles a CU
+# tokens with more tiles than half the CUs), split keys between one and 1.4 tiles a CU, chunks through registers (64 with
+# more than two tiles a CU, 256 from half a tile on), and both ways of 192 at the line between them
 @pytest.mark.parametrize("bs,seq,heads,d", [(13, 200, 2, 64), (13, 200, 2, 128), (13, 200, 2, 256), (48, 200, 2, 128),
                                             (48, 100, 4, 64), (13, 200, 11, 128), (13, 200, 11, 64), (7, 64, 2, 128),
-                                            (10, 192, 2, 256)])
+                                            (10, 192, 2, 256), (13, 160, 11, 64), (13, 160, 11, 128), (48, 100, 11, 64),
+                                            (48, 200, 2, 256), (16, 100, 8, 192), (13, 200, 5, 192)])
 def test_attention_chunk_ends(gpu, rt, bs, seq, heads, d):
     g = torch.Generator("cuda").manual_seed(seq + d)
     qkv = torch.randn(bs, seq, 3, heads, d, device="cuda", generator=g)
