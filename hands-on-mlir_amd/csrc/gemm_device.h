@@ -993,12 +993,13 @@ __host__ __device__ __forceinline__ int epilogueFastMode(const GemmParams &p,
 
 // Whether a tile's results leave by lane exchanges (epilogueLanes) or through the
 // wavefronts' strips of LDS (epilogueFast), by wave tile, source and activation.
-// Lanes against strips, time of the launch, three shapes each:
-//   128 x 64 (256 x 256 tiles, eight wavefronts): DMA staged, linear -1 .. -7 % (+1 beyond results of
-//     112 MiB), with a full source -7 .. -19, GELU -1 .. 0; staged through registers, linear -9 .. -18
-//     without a source, -1 .. -14
-//     with a full one, -7 .. +6 with a bias row, GELU +2 .. +6 with a bias row.  (One way for all sources of a
-//     kernel: with both in it, it spills as it did before and gains nothing.)
+// Lanes against strips, time of the launch, three shapes each (linear 128 x 64: 14, M = 4096 .. 16384, N =
+// 768 .. 4096, K = 264 .. 4096, three sets of operands in turn):
+//   128 x 64 (256 x 256 tiles, eight wavefronts): DMA staged, linear -1 .. -15 %, with a bias row 0 .. -14, with a
+//     full source 0 .. -27, GELU -1 .. 0; staged through registers, linear -4 .. -15, with a full source
+//     -1 .. -15, with a bias row, in a kernel of its own, -3 .. -17 (4295 x 2208 x 552 19.1 -> 17.6 us,
+//     16384 x 3072 x 768 83 -> 78; beside the other sources -8 .. +4: that kernel spills 33 registers, its own
+//     3), GELU +2 .. +6 with a bias row.
 //   64 x 64: GELU without a full source -1 .. -5; linear -7 .. +5 either way.
 //   64 x 32: -1 without a source, -1 .. -6 with a bias row, +1 .. +8 with a full one.
 //   32 x 96, 64 x 96: GELU -3 .. -9 (full source 0 .. -6), linear 0 .. +3.
@@ -1018,14 +1019,15 @@ template <int MI, int NI, int EPI, int CMODE, bool STAGED> constexpr bool leaves
   return false;
 }
 
-// Dispatch: the fast epilogues where they apply, the general one otherwise.
-template <int MI, int NI, int WTM, int WTN, int EPI, bool STAGED = false>
+// Dispatch: the fast epilogues where they apply, the general one otherwise.  MODE: the kernel is
+// for launches of that epiMode only (-1: any).
+template <int MI, int NI, int WTM, int WTN, int EPI, bool STAGED = false, int MODE = -1>
 __device__ __forceinline__ void
 epilogueAuto(const GemmParams &p, float16v (&acc)[MI][NI], int m0, int n0,
              int waveM, int waveN, int lane, int wave, unsigned char *smem) {
   static_assert(EPI < kEpiFoldA, "folded epilogues are called directly");
   if constexpr (EPI <= int(Epilogue::kGeluTanh)) {
-    const int mode = p.epiMode;
+    const int mode = MODE >= 0 ? MODE : p.epiMode;
     if (mode == 0) {
       if constexpr (leavesByLanes<MI, NI, EPI, 0, STAGED>())
         return epilogueLanes<MI, NI, WTM, WTN, EPI, 0>(p, acc, m0, n0, waveM, waveN, lane);

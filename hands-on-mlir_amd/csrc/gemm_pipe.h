@@ -38,8 +38,10 @@ namespace gemmk {
 //
 // EARLY == true (register-staged 64 x 64 tiles): the partial slab of a ragged K is
 // requested ahead of the full ones, see below.
+//
+// MODE: see epilogueAuto().
 template <int BM, int BN, int WM, int WN, int DIST, int EPI, bool B_NK,
-          bool DMA = false, bool ANY = false, bool EARLY = false>
+          bool DMA = false, bool ANY = false, bool EARLY = false, int MODE = -1>
 __global__ __launch_bounds__(WM *WN *kWave) void gemmPipeKernel(
     const _Float16 *argA, const _Float16 *argB, int argM, int argN, int argK,
     int argLda, int argLdb, int argTilesN, int argXcdQ, uint32_t argTileWalk,
@@ -860,12 +862,12 @@ __global__ __launch_bounds__(WM *WN *kWave) void gemmPipeKernel(
       if (p.tileArrivals != nullptr &&
           arriveAtTile(p, tile, numSlices, tid, smem)) {
         sumPartials<MI, NI, THREADS>(p, acc, tile, numSlices, tid);
-        epilogueAuto<MI, NI, WTM, WTN, EPI, !DMA>(p, acc, m0, n0, waveM, waveN, lane,
+        epilogueAuto<MI, NI, WTM, WTN, EPI, !DMA, MODE>(p, acc, m0, n0, waveM, waveN, lane,
                                             wave, smem);
       }
     }
   } else
-    epilogueAuto<MI, NI, WTM, WTN, EPI, !DMA>(p, acc, m0, n0, waveM, waveN, lane,
+    epilogueAuto<MI, NI, WTM, WTN, EPI, !DMA, MODE>(p, acc, m0, n0, waveM, waveN, lane,
                                         wave, smem);
   vpid += gridDim.x;
   } while (vpid < nTiles); // tiles of this workgroup
@@ -938,6 +940,15 @@ Status launchPipe(const GemmProblem &pr, hipStream_t s) {
       if (plan.nTiles * plan.splitK <= early.resident || early.resident >= late.resident)
         use = &early;
     }
+  }
+  // Linear 256 x 256 tiles on eight wavefronts with a bias row have a kernel of their own (see
+  // leavesByLanes).  (A source of [N, K] weights is the result itself.)
+  if constexpr (BM == 256 && BN == 256 && WM == 2 && WN == 4 && !DMA && !B_NK &&
+                EPI == int(Epilogue::kLinear)) {
+    static Variant row = {
+        gemmPipeKernel<BM, BN, WM, WN, DIST, EPI, B_NK, DMA, ANY, false, 1>, false, 0};
+    if (plan.p.epiMode == 1)
+      use = &row;
   }
   st = prepare(use);
   if (st != Status::kSuccess)

@@ -1,5 +1,6 @@
 """GEMM kernels from what they compile to: register use of the 64 x 64 ones, as problems of many tiles are walked by as
-many workgroups as the registers leave room for, and the cache policy of the 256 x 256 ones' results."""
+many workgroups as the registers leave room for, of the 256 x 256 ones for a bias row, and the cache policy of the latter's
+results."""
 import os
 import re
 import subprocess
@@ -56,3 +57,15 @@ def test_results_stay_in_the_last_level_cache(tmp_path, epilogue, dma):
         "const _Float16 *, const _Float16 *, int, int, int, int, int, int, int, uint32_t, uint32_t, int, GemmParams);"])
     stores = re.findall(r"^\s*(?:buffer|global)_store_dwordx4 .*$", text, re.M)
     assert stores and not [s for s in stores if re.search(r"\bnt\b", s)]
+
+
+@pytest.mark.parametrize("any_", ["false", "true"])
+def test_bias_row_without_spills(tmp_path, any_):
+    """256 x 256 linear tiles, results by lane exchanges: with the code for every source one kernel keeps some thirty
+    registers in memory, the one for a bias row alone (last argument) next to none."""
+    text = compiled(tmp_path, [
+        f"template __global__ void gemmPipeKernel<256, 256, 2, 4, 1, 0, false, false, {any_}, false, {mode}>("
+        "const _Float16 *, const _Float16 *, int, int, int, int, int, int, int, uint32_t, uint32_t, int, GemmParams);"
+        for mode in (-1, 1)])
+    spilled = list(map(int, re.findall(r"\.vgpr_spill_count: (\d+)", text)))
+    assert spilled[1] <= 8 and spilled[1] < spilled[0], spilled

@@ -49,7 +49,7 @@ def sample_rows(g, rows, count=48):
                                   "128x128_64x2r2_w2x4", "256x96_64x2r2_w4x1"])
 @pytest.mark.parametrize("act", [0, 1])
 @pytest.mark.parametrize("source", ["none", "bias", "full"])
-@pytest.mark.parametrize("M,N", [(15501, 4080),  # GELU: written past the last-level cache (> 120 MiB)
+@pytest.mark.parametrize("M,N", [(15501, 4080),  # several tiles a workgroup
                                  (301, 264)])   # edges in both directions inside a wavefront's blocks
 def test_gemm_results_by_lane_exchange(gpu, rt, tile, act, source, M, N):
     """Every output of the epilogues without LDS: a block misplaced by an exchange shows as an error
@@ -74,6 +74,28 @@ def test_gemm_results_by_lane_exchange(gpu, rt, tile, act, source, M, N):
         want = torch.nn.functional.gelu(want)
     err = (D[0].float() - want).abs()
     assert bool((err <= 2.0 ** -11 * want.abs() + 1e-6).all()), f"max {err.max().item()}"
+
+
+# linear 256 x 256 tiles with a bias row have kernels of their own, aligned and any alignment: nothing but a partial slab,
+# full slabs and a partial one, slices of K, several tiles a workgroup
+@pytest.mark.parametrize("tile,step", [("256x256_64x2r1_w2x4_nn_align8", 8), ("256x256_64x2u1_w2x4_nn_align1", 1)])
+@pytest.mark.parametrize("M,N,K,slices", [(301, 264, 40, 1), (301, 520, 64, 1), (515, 264, 200, 1), (301, 264, 200, 2),
+                                          (15501, 4080, 72, 1)])
+def test_gemm_bias_row_of_its_own(gpu, rt, tile, step, M, N, K, slices):
+    num = gpu.homGemmManifestFind(f"hom_gfx950_mfma_f16_s32x32x16gemm_f16_{tile}_linear".encode())
+    assert num >= 0
+    mr, K = rt.MemRef.from_tensor, K + (step == 1)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(M + N + K)
+    rnd = lambda *s: torch.randint(-8, 9, s, generator=g, device="cuda").to(torch.float16) / 16  # noqa: E731
+    A, B, C = rnd(1, M, K), rnd(1, K, N), rnd(1, 1, N)
+    want = A[0].float() @ B[0].float() + 0.5 * C[0].float()  # (exact: multiples of 2^-8 below 2^6)
+    D = torch.full((1, M, N), float("nan"), dtype=torch.float16, device="cuda")
+    gpu.cutlassGemmF16(*mr(A).args(), False, *mr(B).args(), False, *mr(C).args(), *mr(D).args(), 0, 1.0, 0.5, num + 1,
+                       slices)
+    torch.cuda.synchronize()
+    err = (D[0].float() - want).abs()
+    assert bool((err <= 2.0 ** -11 * want.abs()).all()), f"max {err.max().item()}"
 
 
 @pytest.mark.parametrize("N,K,act,beta", [
