@@ -129,8 +129,8 @@ template <int EPI> Status launchFusedEdge(int edge, const GemmProblem &p, hipStr
 // to 10 % slower).
 template <int EPI> Status launchPairFolded(int edge, const GemmProblem &p, hipStream_t s) {
   if constexpr (EPI == kEpiRowAffineOwn) {
-    // Without a source 256 x 256 tiles leave by lane exchanges, us: 4096 x 4096 x 1024 41.1 -> 38.8,
-    // 8192 x 3072 x 1024 68.9 -> 65.8, 16384 x 768 x 768 27.6 -> 26.2, 16384 x 4096 x 1024 (written past the last-level cache) 149.7 -> 145.7.
+    // Without a source 256 x 256 tiles leave by lane exchanges, through LDS -> so, us: 4096 x 4096 x 1024 40.8 -> 38.5,
+    // 8192 x 3072 x 1024 68.7 -> 65.8, 16384 x 768 x 768 27.6 -> 25.4, 16384 x 4096 x 1024 153 -> 148.
     // (Staged by DMA the same to 2 % slower; 128 x 128 tiles, 700 x 4096 x 1024: 11.8 -> 12.0.)
     if (edge == 256 && p.beta == 0.f)
       return launchPipe<256, 256, 2, 4, 1, kEpiRowAffineLanes, false>(p, s);
